@@ -10,19 +10,21 @@
 // read with ds_read_b64_tr_b16 exactly as V is in the attention kernel.  The reference writes C column-major
 // (:386-389); C and D are row-major here.  gfx950 has no tf32/xf32 MFMA: fp32 operands multiply in full fp32.
 //
-// Workgroup = 4 waves (one per SIMD) on a 256 x 256 macro tile; wave (wm, wn) of a 2 x 2 grid owns 128 x 128 of C, its
-// 256 accumulator registers in the AGPR half of the register file.  fp16 operands multiply on 16x16x32 MFMAs
-// (gemm_kernel16, 8 x 8 blocks per wave: the power-efficient shape on this board), fp32 operands on 32x32x2
-// (gemm_kernel_f32, 4 x 4 blocks).  K tiles are 128 bytes deep (64 halves / 32 floats) and go global -> registers -> LDS:
-// 16-byte buffer loads a tile ahead (scalar resource + 32-bit lane offset, no vector address arithmetic), parked in
-// one of two 64 KB LDS stages by ds_write_b128 while the other stage multiplies, one barrier per tile; every multiply
-// is followed by at most one fragment read or one store/load pair, see the pipeline comments in the kernels.
+// Two kernels.  gemm_kernel16 (fp16): 4 waves, one per SIMD, on a 256 x 256 macro tile, for as many of those as fill the CUs
+// in whole rounds; wave (wm, wn) of a 2 x 2 grid owns 128 x 128 of C, its 256 accumulator registers in the AGPR half of the
+// register file, 8 x 8 blocks of 16x16x32 MFMAs (the power-efficient shape on this board).  K tiles are 128 bytes deep and go
+// global -> registers -> LDS: 16-byte buffer loads a tile ahead (scalar resource + 32-bit lane offset, no vector address
+// arithmetic), parked in one of two 64 KB LDS stages by ds_write_b128 while the other stage multiplies, one barrier per tile;
+// every multiply is followed by at most one fragment read or one store/load pair, see the pipeline comment in the kernel.
 // (Global -> LDS copy instructions instead of the register path, through a ring of four 32-deep stages and spread the
 // same way, measured 1.57 against 1.94 PFLOP/s on constant operands: with one wave per SIMD an LDS-destination load
-// holds up the issuing wave and with it the MFMA pipe.)  The MFMA computes the TRANSPOSED block (rows = n, columns =
-// m); the epilogue stages each row of blocks through LDS and stores whole rows, 16 bytes per lane.
+// holds up the issuing wave and with it the MFMA pipe.)
+// gemm_tile (gemm_kernel16_tile, gemm_kernel_f32): the smaller macro tiles, for what 256 x 256 blocks leave over and for all
+// fp32 products (v_mfma_f32_32x32x2_f32), whose 16 times slower multiplies any tile can feed.
+// The MFMA computes the TRANSPOSED block (rows = n, columns = m); the epilogue stages blocks through LDS and stores whole
+// rows, 16 bytes per lane.
 // Measured on MI355X, M=N=K=8192 fp16 TN: 1.34-1.40 PFLOP/s on U(-1,1) operands, where the board is power-limited
-// (the vendor library's kernel for this shape, also on 16x16x32 MFMAs: 1.55); fp32: 152 TFLOP/s.
+// (the vendor library's kernel for this shape, also on 16x16x32 MFMAs: 1.55); fp32: 150 TFLOP/s.
 #include <type_traits>
 
 #include <mutex>
@@ -47,245 +49,11 @@ constexpr int BM = 256, BN = 256;
 template <int PITCH>
 __device__ __forceinline__ int swz_k(int row) { return PITCH == 128 ? (row >> 1) & 7 : (row >> 2) & 3; }
 
-// The fp32 kernel (TN only), on v_mfma_f32_32x32x2_f32: 4 x 4 blocks of 32 x 32 per wave.  BKB = bytes of a K-contiguous
-// tile row (32 floats at 128).  blockIdx.y = problem of a batch.  4 waves of 128 x 128, one per SIMD.
-template <int BKB>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-gemm_kernel_f32(const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ Cin, float *__restrict__ D,
-                int M, int N, int K, float alpha, float beta) {
-  using T = float;
-  constexpr int ES = sizeof(T);
-  constexpr int BK = BKB / ES;
-  using Frag = f32x4;  // 16 bytes of a row: the operand of one K-step
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 31, g = lane >> 5;
-  constexpr int WN = 2, NWAVES = 4;
-  constexpr int NB = 4;                // 32-column blocks per wave
-  constexpr int PITCH = BKB;           // bytes per K-contiguous LDS row
-  constexpr int A_TILE = BM * PITCH;   // B tile likewise (n rows)
-  constexpr int STAGE = 2 * A_TILE;
-  constexpr int CPW = A_TILE / 1024 / NWAVES;  // 16-byte pieces per lane and operand tile
-  constexpr int RPC = 1024 / PITCH;    // rows per wave-wide 1 KB piece
-  constexpr int KS = PITCH / 32;       // K-steps per tile: 32 bytes of a row (one 16-byte fragment per lane half) each
-  const int wm = wave / WN, wn = wave % WN;
-
-  // tile order: groups of 8 tile rows, column-major inside a group, so concurrently running workgroups share A and
-  // B panels in L2; workgroup ids are first remapped so that each XCD owns a contiguous range of that order
-  const int tiles_n = N / BN, tiles_m = M / BM;
-  int t = xcd_remap(blockIdx.x, gridDim.x);
-  constexpr int GROUP = 8;
-  const int per_group = GROUP * tiles_n;
-  const int grp = t / per_group;
-  const int first_m = grp * GROUP;
-  const int rows_in_group = tiles_m - first_m < GROUP ? tiles_m - first_m : GROUP;
-  const int in_grp = t - grp * per_group;
-  const int tm = first_m + in_grp % rows_in_group;
-  const int tn = in_grp / rows_in_group;
-  const int m0 = tm * BM, n0 = tn * BN;
-
-  const int64_t batch = blockIdx.y;  // packed strides M*K, N*K, M*N (reference: gemm.cu:519-521)
-  A += batch * M * K;
-  B += batch * N * K;
-  D += batch * M * N;
-  if (Cin) Cin += batch * M * N;
-  const char *Ap = (const char *)(A + (int64_t)m0 * K);
-  const char *Bp = (const char *)(B + (int64_t)n0 * K);
-
-  // ---- global -> register -> LDS staging, 16 B per lane and piece.  Piece i of wave w covers tile rows
-  // (i*NWAVES + w)*RPC .. +RPC; lane l owns LDS slot (row l / CPR, chunk position l % CPR) of the piece and fetches
-  // chunk position ^ swz(row) of that row: the XOR swizzle is applied on the global side, LDS writes are linear.
-  // The loads are ordinary loads into registers (compiler-tracked), issued a tile ahead of the ds_write that parks
-  // them in LDS: unlike LDS-destination loads they do not hold up the issuing wave, which with one wave per SIMD
-  // would hold up the MFMA pipe.
-  uint32_t goff_a[CPW], goff_b[CPW];
-#pragma unroll
-  for (int i = 0; i < CPW; ++i) {
-    const int row = (i * NWAVES + wave) * RPC + lane / (PITCH / 16);
-    const int cp = lane % (PITCH / 16);
-    goff_a[i] = (uint32_t)row * (uint32_t)(K * ES) + (uint32_t)((cp ^ swz_k<PITCH>(row)) * 16);
-    goff_b[i] = goff_a[i];
-  }
-  const uint32_t st_off = wave * 1024 + lane * 16;  // + (piece * NWAVES) * 1024 (+ A_TILE for B) + stage * STAGE
-  int4v stg[2 * CPW];                               // the tile in flight: A pieces, then B pieces
-  // Buffer loads: a scalar resource per operand tile (rebuilt per tile by the scalar unit) plus the lane's 32-bit
-  // offset, so that a load costs no vector address arithmetic.
-  using Rsrc = __amdgpu_buffer_rsrc_t;
-  auto tile_ptrs = [&](int kt, Rsrc &ga, Rsrc &gb) {
-    const char *pa = Ap + (size_t)kt * PITCH;
-    const char *pb = Bp + (size_t)kt * PITCH;
-    ga = __builtin_amdgcn_make_buffer_rsrc((void *)pa, 0, -1, 0x00020000);
-    gb = __builtin_amdgcn_make_buffer_rsrc((void *)pb, 0, -1, 0x00020000);
-  };
-  auto load_piece = [&](Rsrc ga, Rsrc gb, int c) {
-    const u32x4 x = c < CPW ? __builtin_amdgcn_raw_buffer_load_b128(ga, (int)goff_a[c], 0, 0)
-                            : __builtin_amdgcn_raw_buffer_load_b128(gb, (int)goff_b[c - CPW], 0, 0);
-    stg[c] = __builtin_bit_cast(int4v, x);
-  };
-  auto store_piece = [&](int stage, int c) {
-    char *dst = smem + stage * STAGE + st_off + (c < CPW ? c * NWAVES * 1024 : A_TILE + (c - CPW) * NWAVES * 1024);
-    *(int4v *)dst = stg[c];
-  };
-
-  // ---- LDS read addresses.  K-step s: lane (r, g) needs bytes 32s + 16g .. +16 of its row (fp16: k = 16s + 8g .. +8;
-  // fp32: k = 8s + 4g .. +4, used one element per 32x32x2 MFMA: which contraction slot means which k is free as long
-  // as A and B agree).
-  int a_rd[KS], b_rd[KS];
-#pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    a_rd[s] = (wm * 128 + r) * PITCH + (((2 * s + g) ^ swz_k<PITCH>(r)) * 16);               // + 32 rows per m block
-    b_rd[s] = A_TILE + (wn * NB * 32 + r) * PITCH + (((2 * s + g) ^ swz_k<PITCH>(r)) * 16);  // + 32 rows per n block (TN)
-  }
-  f32x16 acc[4][NB];
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mb][nb][v] = 0.f;
-
-  const int k_tiles = K / BK;
-  // One 16-byte operand fragment of K-step s of the tile in LDS stage `st`, in the order the multiplies first need
-  // them: i = 0: B block 0, 1: A block 0, 2..4: B blocks 1..3, 5..7: A blocks 1..3
-  auto fetch_one = [&](const char *st, int s, int i, Frag (&aop)[4], Frag (&bop)[NB]) {
-    const bool is_a = i == 1 || i >= 5;
-    const int blk = i == 0 ? 0 : i == 1 ? 0 : i <= 4 ? i - 1 : i - 4;
-    if (is_a) {
-      aop[blk] = *(const Frag *)(st + a_rd[s] + blk * 32 * PITCH);
-    } else {
-      bop[blk] = *(const Frag *)(st + b_rd[s] + blk * 32 * PITCH);
-    }
-  };
-  // One block multiply (one MFMA, or 4 for fp32 operands).  Transposed block: MFMA rows = n (B operand first)
-  auto mma_block = [&](const Frag (&aop)[4], const Frag (&bop)[NB], int mb, int nb) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(bop[nb][e], aop[mb][e], acc[mb][nb], 0, 0, 0);
-  };
-
-  // Pipeline: two LDS stages and one tile in registers.  While tile kt multiplies out of stage kt % 2, the registers
-  // (tile kt+1, loaded a tile ago) are written to the other stage -- whose readers passed the barrier that opened
-  // this tile -- and refilled with tile kt+2, all before the tile's one barrier.  With one wave per SIMD nothing but
-  // this wave's own instruction stream keeps the MFMA pipe fed: a run of LDS and memory instructions between two
-  // multiplies stalls it.  So every K-step is laid out as 16 slots of one block multiply plus at most a piece of the
-  // other work, pinned in that order: the even slots carry the eight fragment reads of the next K-step (or, behind
-  // the barrier, of the next tile's first); the odd slots of all K-steps but the last carry the staging, the
-  // ds_write of a piece of tile kt+1 and, LD_LAG odd slots later, the load of the same piece of tile kt+2 (a load
-  // issued right behind the store that frees its register waits for that store to have read it).
-  // Measured (8192^3, constant operands): 1.64 PFLOP/s with reads and staging in runs of 8 and 3 instructions, 1.94
-  // with one per slot, 2.04 with the lagged load.
-  constexpr int CPT = 2 * CPW;
-  constexpr int ST_STEPS = KS > 1 ? KS - 1 : 1;
-  constexpr int ST_PER = (CPT + ST_STEPS - 1) / ST_STEPS;     // pieces per K-step
-  constexpr int LD_LAG = 2;
-  static_assert(ST_PER + LD_LAG <= 8, "stores and lagged loads of a K-step must fit its eight odd slots");
-  auto st_slot = [](int c) { return (c / ST_PER) * 8 + c % ST_PER; };  // odd slot (of the tile) of piece c's store
-  Rsrc ga, gb;
-  tile_ptrs(0, ga, gb);
-#pragma unroll
-  for (int c = 0; c < CPT; ++c) load_piece(ga, gb, c);
-#pragma unroll
-  for (int c = 0; c < CPT; ++c) store_piece(0, c);
-  tile_ptrs(k_tiles > 1 ? 1 : 0, ga, gb);
-#pragma unroll
-  for (int c = 0; c < CPT; ++c) load_piece(ga, gb, c);
-  __syncthreads();
-  Frag aop[2][4], bop[2][NB];  // two operand register sets: K-step s+1 is fetched while K-step s multiplies
-#pragma unroll
-  for (int i = 0; i < 8; ++i) fetch_one(smem, 0, i, aop[0], bop[0]);
-  int stage = 0;
-  for (int kt = 0; kt < k_tiles; ++kt) {
-    const char *st = smem + stage * STAGE;
-    const int nstage = stage ^ 1;
-    tile_ptrs(kt + 2 < k_tiles ? kt + 2 : k_tiles - 1, ga, gb);  // clamped at the end: a surplus tile is loaded and dropped
-#pragma unroll
-    for (int s2 = 0; s2 < KS; ++s2) {
-      const bool last = s2 + 1 == KS;
-      // tile kt+1 is in LDS for everybody; all reads of this tile's stage have completed
-      if (last) __syncthreads();
-      const char *src = last ? smem + nstage * STAGE : st;
-      const int s_next = last ? 0 : s2 + 1;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        mma_block(aop[s2 & 1], bop[s2 & 1], i / 4, i % 4);
-        if (i % 2 == 0) {
-          fetch_one(src, s_next, i / 2, aop[(s2 + 1) & 1], bop[(s2 + 1) & 1]);
-        } else {
-          const int t = s2 * 8 + i / 2;  // odd slot number within the tile
-#pragma unroll
-          for (int c = 0; c < CPT; ++c)
-            if (st_slot(c) == t) store_piece(nstage, c);
-#pragma unroll
-          for (int c = 0; c < CPT; ++c)
-            if (st_slot(c) + LD_LAG == t) load_piece(ga, gb, c);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    stage = nstage;
-  }
-
-  // ---- epilogue: D = alpha * acc + beta * C in fp32 (src/cutlass-gemm/gemm.cu:318-324).  Lane (m = r, g) holds
-  // n = 8i + 4g + j of each block: stored directly, a wave-wide store would touch 32 rows with 16 or 32 bytes each.
-  // Each 32 x 128 row of blocks goes through the wave's own LDS region (the stages are dead: every wave passed the last
-  // tile's barrier after its last stage reads and writes) as raw fp32 accumulators and leaves as whole rows, 16 bytes
-  // per lane; alpha, beta and the single rounding to T are applied on the way out.
-  constexpr int E_PITCH = 128 * 4 + 16;          // bytes per staged row of 128 floats, padded
-  constexpr int EPL = 16 / ES;                   // elements per lane and store (8 halves / 4 floats)
-  constexpr int LPR = 128 / EPL, RPP = 64 / LPR; // lanes per row, rows per wave-wide store
-  using OutV = f32x4;
-  const bool with_c = Cin != nullptr && beta != 0.f;
-  char *et = smem + wave * (32 * E_PITCH);
-  const int e_row = lane / LPR, e_col = (lane % LPR) * EPL;
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        f32x4 v4;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v4[j] = acc[mb][nb][4 * i + j];
-        *(f32x4 *)(et + r * E_PITCH + (nb * 32 + 8 * i + 4 * g) * 4) = v4;
-      }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int pass = 0; pass < 32 / RPP; ++pass) {
-      const int row = pass * RPP + e_row;
-      const int64_t off = (int64_t)(m0 + wm * 128 + mb * 32 + row) * N + n0 + wn * NB * 32 + e_col;
-      float v[EPL];
-#pragma unroll
-      for (int q = 0; q < EPL / 4; ++q) {
-        const f32x4 x = *(const f32x4 *)(et + row * E_PITCH + (e_col + 4 * q) * 4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[4 * q + j] = alpha * x[j];
-      }
-      if (with_c) {
-        const OutV c = *(const OutV *)(Cin + off);
-#pragma unroll
-        for (int j = 0; j < EPL; ++j) v[j] += beta * (float)c[j];
-      }
-      OutV o;
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) o[j] = (T)v[j];
-      *(OutV *)(D + off) = o;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();  // the region is rewritten by the next row of blocks
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
-}
-
 // 512-byte rows read with ds_read_b64_tr_b16 in the 16x16x32 lane map: a 32-lane half of the wave touches rows
 // 8g .. 8g+3 of two k groups g x 32 contiguous bytes; bit 0 stays clear so the 32 bytes stay contiguous
 __device__ __forceinline__ int swz512n(int row) { return ((row & 3) | (((row >> 3) & 1) << 2)) << 1; }
 
-// The fp16 kernel on 16x16x32 MFMAs (v_mfma_f32_16x16x32_f16): the same workgroup tile, staging path and epilogue as
-// gemm_kernel_f32, with the wave's 128 x 128 of C as 8 x 8 blocks (NWAVES = 4; NWAVES = 8 runs two waves per SIMD on
+// The fp16 kernel on 16x16x32 MFMAs (v_mfma_f32_16x16x32_f16): the wave's 128 x 128 of C as 8 x 8 blocks (NWAVES = 4; NWAVES = 8 runs two waves per SIMD on
 // 128 x 64 each and measured the same).  Measured, 8192^3 TN, same session: 1401 TFLOP/s on U(-1,1) operands against
 // 1309 for the same kernel on 32x32x16 MFMAs (8 waves: 1390); on constant operands 1837 against 2048 (LDS writes between the
 // short multiplies hold the MFMA pipe up for about 20 cycles each).  On U(-1,1) operands this board is
@@ -314,9 +82,13 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
   constexpr int KS = PITCH / 64;       // K-steps per tile: 64 bytes of a row (four 16-byte fragments, one per g) each
   const int wm = wave / WN, wn = wave % WN;
 
-  // tile order and XCD remap as in gemm_kernel_f32
+  // tile order: groups of 8 tile rows, column-major inside a group, so concurrently running workgroups share A and
+  // B panels in L2; workgroup ids are first remapped so that each XCD owns a contiguous range of that order (the problems
+  // of a batch one after the other)
   const int tiles_n = N / BN, tiles_m = M / BM;
   int t = xcd_remap(blockIdx.x, gridDim.x);
+  const int64_t batch = t / (tiles_m * tiles_n);  // packed strides M*K, N*K, M*N (reference: gemm.cu:519-521)
+  t -= (int)batch * tiles_m * tiles_n;
   constexpr int GROUP = 8;
   const int per_group = GROUP * tiles_n;
   const int grp = t / per_group;
@@ -327,7 +99,6 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
   const int tn = in_grp / rows_in_group;
   const int m0 = tm * BM, n0 = tn * BN;
 
-  const int64_t batch = blockIdx.y;
   A += batch * M * K;
   B += batch * N * K;
   D += batch * M * N;
@@ -335,7 +106,12 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
   const char *Ap = (const char *)(A + (int64_t)m0 * K);
   const char *Bp = NN ? (const char *)(B + n0) : (const char *)(B + (int64_t)n0 * K);
 
-  // ---- global -> register -> LDS staging (see gemm_kernel_f32)
+  // ---- global -> register -> LDS staging, 16 B per lane and piece.  Piece i of wave w covers tile rows
+  // (i*NWAVES + w)*RPC .. +RPC; lane l owns LDS slot (row l / CPR, chunk position l % CPR) of the piece and fetches
+  // chunk position ^ swz(row) of that row: the XOR swizzle is applied on the global side, LDS writes are linear.
+  // The loads are ordinary loads into registers (compiler-tracked), issued a tile ahead of the ds_write that parks
+  // them in LDS: unlike LDS-destination loads they do not hold up the issuing wave, which with one wave per SIMD
+  // would hold up the MFMA pipe.
   uint32_t goff_a[CPW], goff_b[CPW];
 #pragma unroll
   for (int i = 0; i < CPW; ++i) {
@@ -413,9 +189,13 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
     }
   };
 
-  // Pipeline as in gemm_kernel_f32 (two LDS stages, one tile in registers, one barrier per tile), laid out as slots of
-  // one multiply each (K-step major, then m block, then n block; SPM = NBN slots per m block) with at most one piece
-  // of other work behind each multiply, pinned in that order.  Fragment registers: the n-side fragments of a K-step
+  // Pipeline: two LDS stages and one tile in registers.  While tile kt multiplies out of stage kt % 2, the registers
+  // (tile kt+1, loaded a tile ago) are written to the other stage -- whose readers passed the barrier that opened
+  // this tile -- and refilled with tile kt+2, all before the tile's one barrier.  With one wave per SIMD nothing but
+  // this wave's own instruction stream keeps the MFMA pipe fed: a run of LDS and memory instructions between two
+  // multiplies stalls it.  So a tile is laid out as slots of one multiply each (K-step major, then m block, then n block;
+  // SPM = NBN slots per m block) with at most one piece of other work behind each multiply, pinned in that order; a load is
+  // issued LD_LAG pieces behind the store that frees its register (right behind it, it waits for that store to have read it).  Fragment registers: the n-side fragments of a K-step
   // are live throughout it and double-buffered (bop[K-step parity]); the m-side fragment of block mb is only needed
   // for its NBN multiplies and lives in a ring of four (aop[mb % 4]), read two blocks ahead.
   //   K-step 0:  first slot of m block mb: m fragment mb+2 (the last two: blocks 0, 1 of K-step 1);  slot SPM/2 of
@@ -494,7 +274,7 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
   // the dependency through the asm statements)
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
   // ---- epilogue: D = alpha * acc + beta * C in fp32, each 16 x 128 row of blocks staged through the wave's own LDS
-  // region (see gemm_kernel_f32) and stored as whole rows, 16 bytes per lane
+  // region and stored as whole rows, 16 bytes per lane
   constexpr int E_PITCH = 128 * 4 + 16;
   constexpr int EPL = 8;                          // halves per lane and store
   constexpr int WCOLS = NBN * 16;                   // columns of the wave tile
@@ -536,44 +316,414 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
   }
 }
 
-template <class T, bool NN>
-struct GemmLaunch {
-  static constexpr int BKB = 128;  // 64-deep K tiles for fp16, 32-deep for fp32
-  static constexpr int LDS_BYTES = 2 * 2 * BM * BKB;
-  static constexpr int WAVES16 = 4;  // waves of the fp16 kernel
-  static constexpr auto kern = [] {
-    if constexpr (sizeof(T) == 2) return gemm_kernel16<NN, WAVES16>;
-    else return gemm_kernel_f32<BKB>;
-  }();
-  // one-time set-up, thread-safe and callable ahead of any launch
-  static hipError_t prepare() {
-    static std::once_flag once;
-    static hipError_t status = hipSuccess;
-    std::call_once(once, [] {
-      status = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
-    });
-    return status;
-  }
-  static hipError_t launch(const GemmArgs &g, hipStream_t s) {
-    const hipError_t e = prepare();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((g.M / BM) * (g.N / BN), g.batch), dim3(sizeof(T) == 2 ? WAVES16 * 64 : 256), LDS_BYTES, s, (const T *)g.A,
-                       (const T *)g.B, (const T *)g.C, (T *)g.D, g.M, g.N, g.K, g.alpha, g.beta);
-    return hipGetLastError();
-  }
+// ---- Smaller macro tiles (which of them a call takes: launch_f16 and launch_f32 below).
+// 8 waves (two per SIMD) or 4: WM x WN of them share a tile of K, each with TM x TN of C, and KG such groups take the
+// 128-byte deep K tiles in turn; their partial sums meet in the LDS.  Splitting the waves over K instead of over C keeps
+// the wave tile large -- an operand fragment feeds TM/16 or TN/16 multiplies -- where the macro tile is small, and puts KG
+// times the bytes in flight.  Tiles go global -> LDS by copy instructions (1 KB a wave, whole 128-byte row pieces: a
+// lane-per-row load of operand fragments straight into registers runs at 16 bytes per clock and CU, a quarter of this)
+// through ST stages, waited for by count.
+template <class T_, bool NN_, int WM_, int WN_, int TM_, int TN_, int KG_, int ST_>
+struct TileCfg {
+  using T = T_;
+  static constexpr bool NN = NN_;
+  static constexpr int ES = sizeof(T), WM = WM_, WN = WN_, TM = TM_, TN = TN_, KG = KG_, ST = ST_;
+  static constexpr int BMT = WM * TM, BNT = WN * TN, SUB = (BM / BMT) * (BN / BNT);  // tiles of a 256 x 256 block
+  static constexpr int WPG = WM * WN, NW = WPG * KG, THREADS = NW * 64;
+  static constexpr int BK = 128 / ES;
+  static constexpr int A_BYTES = BMT * 128, G_BYTES = (BMT + BNT) * 128, STAGE = KG * G_BYTES;
+  static constexpr int A_PPW = BMT / 8 / WPG, PPW = (BMT + BNT) / 8 / WPG;   // 1 KB copies per wave and stage
+  static constexpr int E_PITCH = BNT * 4 + 16, E_BYTES = KG * BMT * E_PITCH;  // epilogue: fp32 sums, rows padded
+  static constexpr int LDS_BYTES = ST * STAGE > E_BYTES ? ST * STAGE : E_BYTES;
+  static constexpr int FB = ES == 2 ? 16 : 32;                                // block edge of the MFMA
+  static_assert(A_PPW * WPG * 8 == BMT && PPW * WPG * 8 == BMT + BNT, "whole 1 KB copies per wave");
+  static_assert(LDS_BYTES <= 160 * 1024 && ST >= 2, "stages");
 };
+
+// B rows [k][n] of PITCH bytes read with ds_read_b64_tr_b16 in the 16x16x32 lane map (see swz512n): rows 8g .. 8g+3 of
+// two k groups g x 32 contiguous bytes spread over the 256-byte bank period, of which 256/PITCH rows share one
+template <int PITCH>
+__device__ __forceinline__ int swz_bn(int row) {
+  if (PITCH >= 256) return ((row & 3) | (((row >> 3) & 1) << 2)) << 1;
+  if (PITCH == 128) return (((row >> 1) & 1) | (((row >> 3) & 1) << 1)) << 1;
+  return ((row >> 3) & 1) << 1;
+}
+
+template <class C>
+__device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, const typename C::T *__restrict__ B,
+                                          const typename C::T *__restrict__ Cin, typename C::T *__restrict__ D, int M, int N, int K,
+                                          float alpha, float beta, int block0) {
+  using T = typename C::T;
+  constexpr bool F16 = C::ES == 2, NN = C::NN;
+  constexpr int ES = C::ES, FB = C::FB, MB = C::TM / FB, NB = C::TN / FB;
+  constexpr int BPITCH = C::BNT * 2;               // NN: bytes of a k row of the B tile
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave / C::WPG, wi = wave % C::WPG, wm = wi / C::WN, wn = wi % C::WN;
+  const int c = lane % FB, g = lane / FB;
+
+  // tile order: the 256 x 256 blocks in the order of the kernels above (from block0 on, the batch's problems one after the
+  // other), the tiles of a block next to each other
+  const int tiles_n = N / BN, tiles_m = M / BM;
+  const int w = xcd_remap(blockIdx.x, gridDim.x);
+  int t = block0 + w / C::SUB;
+  const int s_idx = w % C::SUB;
+  const int64_t batch = t / (tiles_m * tiles_n);
+  t -= (int)batch * tiles_m * tiles_n;
+  constexpr int GROUP = 8;
+  const int per_group = GROUP * tiles_n;
+  const int grp = t / per_group;
+  const int first_m = grp * GROUP;
+  const int rows_in_group = tiles_m - first_m < GROUP ? tiles_m - first_m : GROUP;
+  const int in_grp = t - grp * per_group;
+  const int m0 = (first_m + in_grp % rows_in_group) * BM + s_idx / (BN / C::BNT) * C::BMT;
+  const int n0 = in_grp / rows_in_group * BN + s_idx % (BN / C::BNT) * C::BNT;
+  A += batch * M * K;
+  B += batch * N * K;
+  D += batch * M * N;
+  if (Cin) Cin += batch * M * N;
+  const char *Ap = (const char *)(A + (int64_t)m0 * K);
+  const char *Bp = NN ? (const char *)(B + n0) : (const char *)(B + (int64_t)n0 * K);
+
+  // ---- copies: group kg fills its own part of a stage; piece i of a wave is 8 rows of A or B (NN: 1 KB of k rows of B)
+  uint32_t goff[C::PPW];
+#pragma unroll
+  for (int i = 0; i < C::PPW; ++i) {
+    const int p = i < C::A_PPW ? i * C::WPG + wi : (i - C::A_PPW) * C::WPG + wi;
+    if (!NN || i < C::A_PPW) {
+      const int row = p * 8 + lane / 8;
+      goff[i] = (uint32_t)row * (uint32_t)(K * ES) + (uint32_t)(((lane % 8) ^ swz_k<128>(row)) * 16);
+    } else {
+      constexpr int CPR = BPITCH / 16;
+      const int krow = p * (64 / CPR) + lane / CPR;
+      goff[i] = (uint32_t)krow * (uint32_t)(N * 2) + (uint32_t)(((lane % CPR) ^ swz_bn<BPITCH>(krow)) * 16);
+    }
+  }
+  const uint32_t lds_base = (uint32_t)(uintptr_t)LDS_PTR(char, smem);
+  const uint32_t lds_wave = lds_base + kg * C::G_BYTES + wi * 1024;
+  const int chunks = K / C::BK, n_st = (chunks + C::KG - 1) / C::KG;
+  auto load_piece = [&](int j, int slot, int i) __attribute__((always_inline)) {
+    int ch = j * C::KG + kg;
+    ch = ch < chunks ? ch : chunks - 1;   // (a group without a tile in the last turn copies one it does not multiply)
+    const bool is_a = i < C::A_PPW;
+    const char *gp = is_a ? Ap + (size_t)ch * 128 : NN ? Bp + (size_t)ch * ((size_t)C::BK * N * 2) : Bp + (size_t)ch * 128;
+    lds_dma16(gp, goff[i], lds_wave + slot * C::STAGE, is_a ? i * C::WPG * 1024 : C::A_BYTES + (i - C::A_PPW) * C::WPG * 1024);
+  };
+  auto load_stage = [&](int j, int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < C::PPW; ++i) load_piece(j, slot, i);
+  };
+
+  // ---- LDS read addresses, relative to the group's part of a stage (see gemm_kernel16; fp32: lane (c, g) needs bytes
+  // 32s + 16g .. +16 of its row, k = 8s + 4g .. +4, used one element per 32x32x2 MFMA: which contraction slot means which k
+  // is free as long as A and B agree)
+  constexpr int KS = F16 ? 2 : 4;                  // K-steps (one 16-byte fragment per operand block) of a tile
+  constexpr int FPS = F16 ? 4 : 2;                 // fragments of a row in a K-step
+  int a_rd[KS], b_rd[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    a_rd[s] = (wm * C::TM + c) * 128 + (((FPS * s + g) ^ swz_k<128>(c)) * 16);
+    b_rd[s] = C::A_BYTES + (wn * C::TN + c) * 128 + (((FPS * s + g) ^ swz_k<128>(c)) * 16);
+  }
+  int bt_rd[NB];
+  if constexpr (NN) {
+    const int bk_row = 8 * g + (c >> 2), cg = c & 3;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const int chunk = (wn * C::TN + 16 * nb) / 8 + (cg >> 1);
+      bt_rd[nb] = C::A_BYTES + bk_row * BPITCH + ((chunk ^ swz_bn<BPITCH>(bk_row)) * 16) + (cg & 1) * 8;
+    }
+  }
+  using Frag = std::conditional_t<F16, half8, f32x4>;
+  using Acc = std::conditional_t<F16, f32x4, f32x16>;
+  constexpr int AV = F16 ? 4 : 16;
+  Acc acc[MB][NB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int v = 0; v < AV; ++v) acc[mb][nb][v] = 0.f;
+
+  Frag af[2][MB], bf[2][NB];
+  // fragment i of K-step s of the stage in `slot`, in the order the multiplies want them: B 0, A 0, B 1 .., A 1 ..
+  constexpr int FRAGS = MB + NB;
+  auto fetch_piece = [&](int slot, int s, int i, Frag (&fa)[MB], Frag (&fb)[NB]) __attribute__((always_inline)) {
+    const char *st = smem + slot * C::STAGE + kg * C::G_BYTES;
+    if (i == 1 || i > NB) {
+      const int mb = i == 1 ? 0 : i - NB;
+      fa[mb] = *(const Frag *)(st + a_rd[s] + mb * FB * 128);
+      return;
+    }
+    const int nb = i == 0 ? 0 : i - 1;
+    if constexpr (!NN) {
+      fb[nb] = *(const Frag *)(st + b_rd[s] + nb * FB * 128);
+    } else {
+      union {
+        struct { short4v lo, hi; } p;
+        half8 h;
+      } u;
+      const char *bp = st + bt_rd[nb] + s * 32 * BPITCH;
+      u.p.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4v, bp));
+      u.p.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4v, bp + 4 * BPITCH));
+      fb[nb] = u.h;
+    }
+  };
+  auto multiply_block = [&](int mb, int nb, const Frag (&fa)[MB], const Frag (&fb)[NB]) __attribute__((always_inline)) {
+    if constexpr (F16) {
+      acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[nb], fa[mb], acc[mb][nb], 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[nb][e], fa[mb][e], acc[mb][nb], 0, 0, 0);
+    }
+  };
+  // The multiplies of one K-step with the other work (fragment reads of the next, copies).  Where all waves work on one tile
+  // of K it is spread between them, order pinned: a run of LDS reads in front of the multiplies leaves the matrix cores idle
+  // while all eight waves queue for the LDS (256 x 128, M=4096 N=2048 K=4096: 60.5 us against 62.7).  With several groups
+  // the compiler's order is the faster one (128 x 128, M=N=2048 K=8192: 68.7 us against 71.9).
+  auto multiply_with = [&](const Frag (&fa)[MB], const Frag (&fb)[NB], auto n_pieces, auto &&piece) __attribute__((always_inline)) {
+    constexpr int P = decltype(n_pieces)::value, NS = MB * NB;
+    if constexpr (C::KG > 1) {
+#pragma unroll
+      for (int k = 0; k < P; ++k) piece(k);
+    }
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      multiply_block(i / NB, i % NB, fa, fb);
+      if constexpr (C::KG == 1) {
+#pragma unroll
+        for (int k = 0; k < P; ++k)
+          if (k * NS / (P ? P : 1) == i) piece(k);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  // Waits until all but this wave's copies of the `behind` newest stages have landed and its LDS reads have returned, and
+  // meets the others: then everybody's copies have, and a slot whose reads lie in front of the barrier is free.
+  auto arrive = [&](int behind) __attribute__((always_inline)) {
+    if (C::ST >= 5 && behind >= 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(3 * C::PPW) : "memory");
+    else if (C::ST >= 4 && behind >= 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * C::PPW) : "memory");
+    else if (C::ST >= 3 && behind >= 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::PPW) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  // Fragments are read one K-step ahead, across the barrier too, so that the reads of one step lie beside the multiplies
+  // of the one before.
+#pragma unroll
+  for (int j = 0; j < C::ST; ++j)
+    if (j < n_st) load_stage(j, j);
+  if (n_st >= C::ST) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((C::ST - 1) * C::PPW) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < FRAGS; ++i) fetch_piece(0, 0, i, af[0], bf[0]);
+  using std::integral_constant;
+  int slot = 0;
+  for (int j = 0; j + 1 < n_st; ++j) {
+    const int next = slot == C::ST - 1 ? 0 : slot + 1;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if (s + 1 < KS) {
+        multiply_with(af[s & 1], bf[s & 1], integral_constant<int, FRAGS>{},
+                      [&](int k) __attribute__((always_inline)) { fetch_piece(slot, s + 1, k, af[(s + 1) & 1], bf[(s + 1) & 1]); });
+      } else {
+        const int behind = n_st - 2 - j;
+        arrive(behind < C::ST - 2 ? behind : C::ST - 2);
+        const bool more = j + C::ST < n_st;
+        multiply_with(af[s & 1], bf[s & 1], integral_constant<int, FRAGS + C::PPW>{}, [&](int k) __attribute__((always_inline)) {
+          if (k < FRAGS) fetch_piece(next, 0, k, af[0], bf[0]);
+          else if (more) load_piece(j + C::ST, slot, k - FRAGS);
+        });
+      }
+    }
+    slot = next;
+  }
+  if (C::KG == 1 || (n_st - 1) * C::KG + kg < chunks) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if (s + 1 < KS)
+        multiply_with(af[s & 1], bf[s & 1], integral_constant<int, FRAGS>{},
+                      [&](int k) __attribute__((always_inline)) { fetch_piece(slot, s + 1, k, af[(s + 1) & 1], bf[(s + 1) & 1]); });
+      else multiply_with(af[s & 1], bf[s & 1], integral_constant<int, 0>{}, [](int) {});
+    }
+  }
+
+  // ---- epilogue: every group leaves its fp32 sums in the LDS as rows of C; they are added up, scaled and rounded once on
+  // the way out, 16 bytes per lane of whole tile rows
+  __syncthreads();
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int i = 0; i < AV / 4; ++i) {
+        f32x4 v4;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v4[x] = acc[mb][nb][4 * i + x];
+        // lane (m = c, g): n = 4 g .. +3 of a 16-wide block, 8 i + 4 g .. +3 of a 32-wide one
+        *(f32x4 *)(smem + (kg * C::BMT + wm * C::TM + mb * FB + c) * C::E_PITCH + (wn * C::TN + nb * FB + 8 * i + 4 * g) * 4) = v4;
+      }
+  __syncthreads();
+  constexpr int EPL = 16 / ES, LPR = C::BNT / EPL, RPP = C::THREADS / LPR;
+  using OutV = std::conditional_t<F16, half8, f32x4>;
+  const bool with_c = Cin != nullptr && beta != 0.f;
+  const int e_row = tid / LPR, e_col = (tid % LPR) * EPL;
+  static_assert(C::BMT % RPP == 0 || RPP > C::BMT, "whole passes");
+#pragma unroll
+  for (int pass = 0; pass < (C::BMT + RPP - 1) / RPP; ++pass) {
+    const int row = pass * RPP + e_row;
+    if (RPP > C::BMT && row >= C::BMT) break;
+    const int64_t off = (int64_t)(m0 + row) * N + n0 + e_col;
+    float v[EPL];
+#pragma unroll
+    for (int q = 0; q < EPL / 4; ++q) {
+      f32x4 x = *(const f32x4 *)(smem + row * C::E_PITCH + (e_col + 4 * q) * 4);
+#pragma unroll
+      for (int k = 1; k < C::KG; ++k) x += *(const f32x4 *)(smem + (k * C::BMT + row) * C::E_PITCH + (e_col + 4 * q) * 4);
+#pragma unroll
+      for (int x2 = 0; x2 < 4; ++x2) v[4 * q + x2] = alpha * x[x2];
+    }
+    if (with_c) {
+      const OutV cv = *(const OutV *)(Cin + off);
+#pragma unroll
+      for (int x = 0; x < EPL; ++x) v[x] += beta * (float)cv[x];
+    }
+    OutV o;
+#pragma unroll
+    for (int x = 0; x < EPL; ++x) o[x] = (T)v[x];
+    *(OutV *)(D + off) = o;
+  }
+}
+
+// The macro tiles built: <operand type, NN, waves along m and n, rows and columns per wave, wave groups over K, stages>.
+// Measured and not built (fp16, TN): 128 x 128 by 8 waves on one K tile, 4 stages, 67.8 us against 68.7 at M=N=2048 K=8192 but
+// 90 against 73.5 for NN; 64 x 64 by four K groups of two waves, 31.9 us against 27.7 at M=N=1024 K=8192 (two stages, half
+// the bytes in flight).
+template <bool NN, int ROWS, int COLS> struct HTile;
+template <bool NN> struct HTile<NN, 256, 128> : TileCfg<_Float16, NN, 4, 2, 64, 64, 1, 3> {};
+template <bool NN> struct HTile<NN, 128, 128> : TileCfg<_Float16, NN, 2, 2, 64, 64, 2, 2> {};
+template <bool NN> struct HTile<NN, 128, 64> : TileCfg<_Float16, NN, 2, 2, 64, 32, 2, 3> {};
+template <bool NN> struct HTile<NN, 64, 64> : TileCfg<_Float16, NN, 2, 2, 32, 32, 2, 4> {};
+template <bool NN> struct HTile<NN, 32, 32> : TileCfg<_Float16, NN, 1, 1, 32, 32, 4, 4> {};
+template <int EDGE> struct FTile;
+template <> struct FTile<128> : TileCfg<float, false, 2, 2, 64, 64, 1, 2> {};
+template <> struct FTile<64> : TileCfg<float, false, 2, 2, 32, 32, 2, 2> {};
+template <> struct FTile<32> : TileCfg<float, false, 1, 1, 32, 32, 4, 2> {};
+
+template <bool NN, int ROWS, int COLS>
+__global__ void __launch_bounds__((HTile<NN, ROWS, COLS>::THREADS))
+gemm_kernel16_tile(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
+                   _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta, int block0) {
+  gemm_tile<HTile<NN, ROWS, COLS>>(A, B, Cin, D, M, N, K, alpha, beta, block0);
+}
+
+template <int EDGE>
+__global__ void __launch_bounds__(FTile<EDGE>::THREADS)
+gemm_kernel_f32(const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ Cin, float *__restrict__ D,
+                int M, int N, int K, float alpha, float beta, int block0) {
+  gemm_tile<FTile<EDGE>>(A, B, Cin, D, M, N, K, alpha, beta, block0);
+}
+
+constexpr int kWaves16 = 4;                          // waves of gemm_kernel16
+constexpr int kLds16 = 2 * 2 * BM * 128;             // two stages of an A and a B tile, 128 bytes deep
+
+// one-time set-up of a kernel (its dynamic-LDS limit), thread-safe and callable ahead of any launch
+template <auto Kern, int Lds>
+hipError_t prepare_kernel() {
+  static std::once_flag once;
+  static hipError_t status = hipSuccess;
+  std::call_once(once, [] { status = hipFuncSetAttribute((const void *)Kern, hipFuncAttributeMaxDynamicSharedMemorySize, Lds); });
+  return status;
+}
+
+// the 256 x 256 blocks 0 .. blocks-1 of the batch
+template <bool NN>
+hipError_t launch_blocks(const GemmArgs &g, hipStream_t s, int blocks) {
+  const hipError_t e = prepare_kernel<gemm_kernel16<NN, kWaves16>, kLds16>();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((gemm_kernel16<NN, kWaves16>), dim3(blocks), dim3(kWaves16 * 64), kLds16, s, (const _Float16 *)g.A, (const _Float16 *)g.B,
+                     (const _Float16 *)g.C, (_Float16 *)g.D, g.M, g.N, g.K, g.alpha, g.beta);
+  return hipGetLastError();
+}
+
+// `blocks` 256 x 256 blocks from block0 on, in tiles of configuration C by kernel Kern
+template <class C, auto Kern>
+hipError_t launch_tiles(const GemmArgs &g, hipStream_t s, int block0, int blocks) {
+  const hipError_t e = prepare_kernel<Kern, C::LDS_BYTES>();
+  if (e != hipSuccess) return e;
+  using T = typename C::T;
+  hipLaunchKernelGGL(Kern, dim3(blocks * C::SUB), dim3(C::THREADS), C::LDS_BYTES, s, (const T *)g.A, (const T *)g.B, (const T *)g.C,
+                     (T *)g.D, g.M, g.N, g.K, g.alpha, g.beta, block0);
+  return hipGetLastError();
+}
+template <bool NN, int ROWS, int COLS>
+hipError_t launch_tiles16(const GemmArgs &g, hipStream_t s, int block0, int blocks) {
+  return launch_tiles<HTile<NN, ROWS, COLS>, gemm_kernel16_tile<NN, ROWS, COLS>>(g, s, block0, blocks);
+}
+template <int EDGE>
+hipError_t launch_tiles32(const GemmArgs &g, hipStream_t s, int blocks) {
+  return launch_tiles<FTile<EDGE>, gemm_kernel_f32<EDGE>>(g, s, 0, blocks);
+}
+
+constexpr int kCus = 256;
+
+// fp16: 256 x 256 blocks run in whole rounds of the CUs, one to a CU; the blocks of a last round that at most half fills the
+// CUs are cut into the largest tiles that still go round the CUs once.  The time of such a round over K, relative to one of
+// 256 x 256 blocks (85 us at K=4096): 256 x 128 0.70, 128 x 128 0.47, 128 x 64 0.26, 64 x 64 0.17, 32 x 32 0.10; a tile size
+// down costs two rounds of its own.  Measured, us (TN), against 256 x 256 blocks alone: M=N=K=1024 8.4 / 25.1, M=N=512 K=4096
+// 8.7 / 75.4, M=N=2048 K=4096 39.5 / 79.5, 5120 x 4096 x 4096 (256 blocks, then 64 in 128 x 128 tiles) 144 / 175 and with C 155 / 199.
+template <bool NN>
+hipError_t launch_f16(const GemmArgs &g, hipStream_t s, int blocks) {
+  const int left = blocks % kCus, whole = left > kCus / 2 ? blocks : blocks - left;
+  if (whole) {
+    const hipError_t e = launch_blocks<NN>(g, s, whole);
+    if (e != hipSuccess || whole == blocks) return e;
+  }
+  if (left * HTile<NN, 32, 32>::SUB <= kCus) return launch_tiles16<NN, 32, 32>(g, s, whole, left);
+  if (left * HTile<NN, 64, 64>::SUB <= kCus) return launch_tiles16<NN, 64, 64>(g, s, whole, left);
+  if (left * HTile<NN, 128, 64>::SUB <= kCus) return launch_tiles16<NN, 128, 64>(g, s, whole, left);
+  if (left * HTile<NN, 128, 128>::SUB <= kCus) return launch_tiles16<NN, 128, 128>(g, s, whole, left);
+  return launch_tiles16<NN, 256, 128>(g, s, whole, left);
+}
+
+// fp32: the multiplies bound every tile size, so what counts is how full the last round of the CUs is: the tile whose rounds,
+// at their measured times relative to 128 x 128 (66 us per 1024 of K), add up to least.  Three problems of M=1024 N=768 K=1536
+// (576 tiles of 64 x 64, 2304 of 32 x 32) 64.6 us by 32 x 32 against 76.3 and 97; M=N=5120 K=4096 1532 us by 64 x 64 against
+// 1615 and 1717; M=N=K=8192 7.31 ms by 128 x 128.  (256 x 256 blocks, 4 waves of 128 x 128 with registers between global memory
+// and LDS: 345 us, 1989 us and 7.89 ms for the three.)
+hipError_t launch_f32(const GemmArgs &g, hipStream_t s, int blocks) {
+  const auto rounds = [&](int sub) { return (double)(((long long)blocks * sub + kCus - 1) / kCus); };
+  const double t128 = rounds(FTile<128>::SUB), t64 = 0.267 * rounds(FTile<64>::SUB), t32 = 0.072 * rounds(FTile<32>::SUB);
+  if (t128 <= t64 && t128 <= t32) return launch_tiles32<128>(g, s, blocks);
+  return t64 <= t32 ? launch_tiles32<64>(g, s, blocks) : launch_tiles32<32>(g, s, blocks);
+}
+
+template <bool NN>
+hipError_t prepare_f16() {
+  const hipError_t e[] = {prepare_kernel<gemm_kernel16<NN, kWaves16>, kLds16>(),
+                          prepare_kernel<gemm_kernel16_tile<NN, 256, 128>, HTile<NN, 256, 128>::LDS_BYTES>(),
+                          prepare_kernel<gemm_kernel16_tile<NN, 128, 128>, HTile<NN, 128, 128>::LDS_BYTES>(),
+                          prepare_kernel<gemm_kernel16_tile<NN, 128, 64>, HTile<NN, 128, 64>::LDS_BYTES>(),
+                          prepare_kernel<gemm_kernel16_tile<NN, 64, 64>, HTile<NN, 64, 64>::LDS_BYTES>(),
+                          prepare_kernel<gemm_kernel16_tile<NN, 32, 32>, HTile<NN, 32, 32>::LDS_BYTES>()};
+  for (hipError_t x : e)
+    if (x != hipSuccess) return x;
+  return hipSuccess;
+}
 
 }  // namespace
 
 hipError_t launch_gemm(const GemmArgs &g, hipStream_t s) {
-  if (g.f32) return g.layout == 0 ? GemmLaunch<float, false>::launch(g, s) : hipErrorNotSupported;
-  return g.layout == 0 ? GemmLaunch<_Float16, false>::launch(g, s) : GemmLaunch<_Float16, true>::launch(g, s);
+  const int blocks = (g.M / BM) * (g.N / BN) * g.batch;
+  if (g.f32) return g.layout == 0 ? launch_f32(g, s, blocks) : hipErrorNotSupported;
+  return g.layout == 0 ? launch_f16<false>(g, s, blocks) : launch_f16<true>(g, s, blocks);
 }
 
 hipError_t prepare_gemm() {
-  hipError_t e = GemmLaunch<float, false>::prepare();
-  if (e == hipSuccess) e = GemmLaunch<_Float16, false>::prepare();
-  if (e == hipSuccess) e = GemmLaunch<_Float16, true>::prepare();
+  hipError_t e = prepare_f16<false>();
+  if (e == hipSuccess) e = prepare_f16<true>();
+  if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32<128>, FTile<128>::LDS_BYTES>();
+  if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32<64>, FTile<64>::LDS_BYTES>();
+  if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32<32>, FTile<32>::LDS_BYTES>();
   return e;
 }
 

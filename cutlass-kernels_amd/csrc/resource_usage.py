@@ -31,7 +31,7 @@ def demangle(names):
 def short_name(d):
     """cfk::fmha_fwd_kernel16<cfk::FmhaCfg<128, 64, 8, 2, false, ...>>(cfk::FmhaArgs) -> fmha_fwd_kernel16<128,64,8,2,0,0,0,0,2,0,1>"""
     m = re.match(r"_ZN3cfk12_GLOBAL__N_1\d+([a-z_0-9]+?)I(.*?)EEv", d)   # (the system's c++filt does not know _Float16 parameters)
-    if m: return m.group(1) + "<" + m.group(2).replace("Lb0E", "0,").replace("Lb1E", "1,").replace("Li4E", "4").rstrip(",") + ">"
+    if m: return m.group(1) + "<" + ",".join(re.findall(r"L[bi](\d+)", m.group(2))) + ">"
     d = re.sub(r"^void ", "", d).replace("(anonymous namespace)::", "")
     d = re.sub(r"\(.*\)$", "", d)
     direct = "DirectCfg<" in d     # the build with e4m3 weights written as codes: shown as <...>/direct

@@ -77,6 +77,31 @@ def test_alpha_beta_batch_integer_inputs_bit_exact(dtype):
     assert np.array_equal(got.cpu().numpy(), np.stack([oracle.gemm_f32(a[i], b[i]) for i in range(L)]).astype(dtype))
 
 
+@pytest.mark.parametrize("K", [64, 192, 320])
+@pytest.mark.parametrize("dtype,layout", [(np.float16, 0), (np.float16, 1), (np.float32, 0)])
+@pytest.mark.parametrize("L,M,N", [
+    (1, 256, 256), (1, 512, 512), (1, 256, 1280), (1, 1024, 1024), (17, 256, 256), (2, 1024, 1024), (1, 256, 8448),
+    (4, 1024, 1024), (65, 256, 256), (1, 4096, 2048), (129, 256, 256), (257, 256, 256)])
+def test_macro_tiles_integer_inputs_bit_exact(L, M, N, K, dtype, layout):
+    # 1 to 257 blocks of 256 x 256 on either side of every line where the macro tile changes (4, 16, 32, 64, 128 blocks, and
+    # one block beyond a whole round of the CUs), with fewer K tiles than wave groups, a last turn that not all groups have
+    # a tile for, and whole turns.  Integers: every sum is exact in fp32 in any order.
+    import torch
+    rng = np.random.default_rng(L + M + N + K)
+    if L > 4 and K > 64:
+        K = 64 if L > 100 else K                         # (the oracle's time)
+    a = rng.integers(-8, 9, (L, M, K)).astype(np.float32)
+    b = rng.integers(-8, 9, (L, N, K)).astype(np.float32)
+    c = rng.integers(-8, 9, (L, M, N)).astype(np.float32)
+    bt = b if layout == 0 else np.ascontiguousarray(b.transpose(0, 2, 1))
+    got = pkg.gemm(to_dev(a.astype(dtype)), to_dev(bt.astype(dtype)), c=to_dev(c.astype(dtype)), alpha=0.5, beta=-1.0, layout=layout)
+    torch.cuda.synchronize()
+    got = got.cpu().numpy()
+    for i in sorted({0, L // 2, L - 1}):
+        want = (0.5 * oracle.gemm_f32(a[i], b[i]) - c[i]).astype(dtype)
+        assert np.array_equal(got[i], want), i
+
+
 def test_fp32_uniform_inputs():
     # the CuTe example's type 1 (float operands, gemm.cu:677-684), U(-1,1) data (:482-485).  Both sides accumulate in
     # fp32 in different orders: |error| <~ sqrt(K) * 2^-24 * |terms|
