@@ -74,6 +74,24 @@ int check_fmha(const cfk_fmha_fwd_params *p, cfk::FmhaPlan *plan, bool need_poin
   return CFK_OK;
 }
 
+// Workgroups that share a query block's keys (cfk_fmha_forward_ws): as many as fit on the chip at once, while the turns that
+// their waves are spared outweigh the second launch and the merge, about 4 us plus 0.3 us for each partial result.  Measured
+// (fp16, head dim 128, two heads of 64 rows each: 8 workgroups), us at 1, 4, 8, 16, 32 splits: 4096 keys 22.5, 14.1, 14.4, 18.3,
+// 28.2; 16384 keys 100, 30.8, 23.6, 22.8, 30.7; 1024 keys 9.3, 10.8, 12.8.  64 workgroups, 16384 keys: 109.9 -> 51.0 at 4.
+int key_splits(const cfk_fmha_fwd_params *p, const cfk::FmhaPlan &plan) {
+  if (plan.split_tiles == 0) return 1;
+  int best = 1;
+  float best_us = 0.f;
+  for (int n = 1; n * plan.grid <= 256 && n <= plan.split_tiles; ++n) {
+    const int tiles = (plan.split_tiles + n - 1) / n, turns = (tiles + plan.split_waves - 1) / plan.split_waves;
+    const float us = turns * plan.split_turn_us + (n > 1 ? 4.f + 0.3f * n : 0.f);
+    if (n == 1 || us < best_us) best = n, best_us = us;
+  }
+  return best;
+}
+// one partial result: fp32 O and a (reference point, row sum) pair per query row
+int64_t partial_bytes(const cfk_fmha_fwd_params *p) { return (int64_t)p->batch * p->heads * p->seqlen_q * (p->head_dim + 2) * 4; }
+
 int check_device() {
   int dev = -1;
   hipError_t e = hipGetDevice(&dev);
@@ -86,6 +104,63 @@ int check_device() {
   if (strncmp(prop.gcnArchName, "gfx950", 6) != 0)
     return fail(CFK_ERR_NO_DEVICE, "device %d is %s; this library is built for gfx950 only", dev, prop.gcnArchName);
   checked_dev = dev;
+  return CFK_OK;
+}
+
+// Launches a checked call; n_split > 1: with its keys shared by that many workgroups, through the workspace.
+int launch_fmha(const cfk_fmha_fwd_params *p, int n_split, void *workspace, void *stream) {
+  const int rc = check_device();
+  if (rc != CFK_OK) return rc;
+  constexpr float kLog2e = 1.4426950408889634074f;  // fmha_forward.cu:452
+  cfk::FmhaArgs a{};
+  a.q = p->q;
+  a.k = p->k;
+  a.v = p->v;
+  a.o = p->o;
+  a.s_tap = p->dbg_s;
+  a.row_max = p->dbg_row_max;
+  a.row_sum = p->dbg_row_sum;
+  a.B = p->batch;
+  a.H = p->heads;
+  a.Sq = p->seqlen_q;
+  a.Skv = p->seqlen_kv;
+  a.v_layout = p->v_layout;
+  a.n_split = n_split;
+  if (n_split > 1) {
+    a.part_o = (float *)workspace;
+    a.part_ml = a.part_o + (int64_t)n_split * p->batch * p->heads * p->seqlen_q * p->head_dim;
+  }
+  // Deferred rescale: O and l are only rescaled when a tile's max exceeds the max the reference point was set from by
+  // more than tau (log2 domain).  fp16 P: 2^8 of head-room.  e4m3 P already sits 2^7 above the reference point, which
+  // leaves 1.  With e4m3 P the row's largest weight is an exact power of two only while the reference point follows
+  // the running max (as the reference's does on every tile, online_softmax.h:144-165); the rounding error of that
+  // weight (<= 6 %) averages out over long key sequences but shows in the reference's error-percentage measure on short
+  // ones, so those run with tau = 0.
+  a.tau = p->v_dtype != CFK_FP8_E4M3 ? 8.0f : p->seqlen_kv < 2048 ? 0.0f : 1.0f;
+  // e4m3 P: in the pass without a row max per tile the reference point comes from the first tile, so a row's largest
+  // weight is not the exact power of two it is under a running max, and over few keys the rounding of that weight shows in
+  // the reference's error-percentage gate (fmha_forward.cu:638-639, limit 0.001 %): 0.0000 % over the 4096 keys of the
+  // reference's own problem, 0.00001..0.00006 % at 3072 and 3584 keys, 0.0001..0.0003 % at 2560, 0.0005..0.0013 % at 2048
+  // (head dims 128, 256, 64).  Key lengths below 3072 take the max-tracking pass only.
+  a.direct_p = g_fast_e4m3.load(std::memory_order_relaxed);
+  a.track_only = cfk::predictable_latency() || (p->v_dtype == CFK_FP8_E4M3 && p->seqlen_kv < 3072) ? 1 : 0;
+  hipError_t e;
+  a.s_scale = p->dtype == CFK_FP16 ? p->softmax_scale : p->softmax_scale * p->q_descale * p->k_descale;
+  if (p->dtype == CFK_FP16) {
+    a.scale_log2 = p->softmax_scale * kLog2e;
+    a.out_scale = 1.0f;
+    e = cfk::launch_fmha_f16(a, p->head_dim, (hipStream_t)stream);
+  } else if (p->v_dtype == CFK_FP16) {  // hybrid: fp16 V carries no scale
+    a.scale_log2 = p->softmax_scale * kLog2e * p->q_descale * p->k_descale;
+    a.out_scale = 1.0f;
+    e = cfk::launch_fmha_hybrid(a, p->head_dim, (hipStream_t)stream);
+  } else {
+    a.scale_log2 = p->softmax_scale * kLog2e * p->q_descale * p->k_descale;
+    a.out_scale = p->v_descale;
+    e = cfk::launch_fmha_fp8(a, p->head_dim, (hipStream_t)stream);
+  }
+  if (e == hipSuccess && a.n_split > 1) e = cfk::launch_fmha_combine(a, p->head_dim, (hipStream_t)stream);
+  if (e != hipSuccess) return fail(CFK_ERR_HIP, "FMHA launch failed: %s", hipGetErrorString(e));
   return CFK_OK;
 }
 
@@ -120,6 +195,7 @@ int cfk_fmha_forward_mfma(const cfk_fmha_fwd_params *params, int32_t *mfma_rows)
 
 int cfk_fmha_forward_kernel(const cfk_fmha_fwd_params *params, char *name, int32_t capacity) {
   cfk::FmhaPlan plan{};
+  plan.want_name = true;
   int rc = check_fmha(params, &plan, false);
   if (rc != CFK_OK) return rc;
   if (!name || capacity <= (int32_t)strlen(plan.kernel)) return fail(CFK_ERR_INVALID_ARG, "name buffer of %d bytes is too small", capacity);
@@ -127,57 +203,31 @@ int cfk_fmha_forward_kernel(const cfk_fmha_fwd_params *params, char *name, int32
   return CFK_OK;
 }
 
-int cfk_fmha_forward(const cfk_fmha_fwd_params *p, void *stream) {
+int64_t cfk_fmha_forward_workspace(const cfk_fmha_fwd_params *p) {
   cfk::FmhaPlan plan{};
-  int rc = check_fmha(p, &plan, true);
+  if (check_fmha(p, &plan, false) != CFK_OK) return 0;
+  const int n = key_splits(p, plan);
+  return n > 1 ? (int64_t)n * partial_bytes(p) : 0;
+}
+
+int cfk_fmha_forward(const cfk_fmha_fwd_params *p, void *stream) { return cfk_fmha_forward_ws(p, nullptr, 0, stream); }
+
+int64_t cfk_fmha_forward_or_workspace(const cfk_fmha_fwd_params *p, void *stream) {
+  cfk::FmhaPlan plan{};
+  const int rc = check_fmha(p, &plan, true);
   if (rc != CFK_OK) return rc;
-  rc = check_device();
+  const int n = key_splits(p, plan);
+  return n > 1 ? (int64_t)n * partial_bytes(p) : launch_fmha(p, 1, nullptr, stream);
+}
+
+int cfk_fmha_forward_ws(const cfk_fmha_fwd_params *p, void *workspace, int64_t workspace_bytes, void *stream) {
+  cfk::FmhaPlan plan{};
+  const int rc = check_fmha(p, &plan, true);
   if (rc != CFK_OK) return rc;
-  constexpr float kLog2e = 1.4426950408889634074f;  // fmha_forward.cu:452
-  cfk::FmhaArgs a{};
-  a.q = p->q;
-  a.k = p->k;
-  a.v = p->v;
-  a.o = p->o;
-  a.s_tap = p->dbg_s;
-  a.row_max = p->dbg_row_max;
-  a.row_sum = p->dbg_row_sum;
-  a.B = p->batch;
-  a.H = p->heads;
-  a.Sq = p->seqlen_q;
-  a.Skv = p->seqlen_kv;
-  a.v_layout = p->v_layout;
-  // Deferred rescale: O and l are only rescaled when a tile's max exceeds the max the reference point was set from by
-  // more than tau (log2 domain).  fp16 P: 2^8 of head-room.  e4m3 P already sits 2^7 above the reference point, which
-  // leaves 1.  With e4m3 P the row's largest weight is an exact power of two only while the reference point follows
-  // the running max (as the reference's does on every tile, online_softmax.h:144-165); the rounding error of that
-  // weight (<= 6 %) averages out over long key sequences but shows in the reference's error-percentage measure on short
-  // ones, so those run with tau = 0.
-  a.tau = p->v_dtype != CFK_FP8_E4M3 ? 8.0f : p->seqlen_kv < 2048 ? 0.0f : 1.0f;
-  // e4m3 P: in the pass without a row max per tile the reference point comes from the first tile, so a row's largest
-  // weight is not the exact power of two it is under a running max, and over few keys the rounding of that weight shows in
-  // the reference's error-percentage gate (fmha_forward.cu:638-639, limit 0.001 %): 0.0000 % over the 4096 keys of the
-  // reference's own problem, 0.00001..0.00006 % at 3072 and 3584 keys, 0.0001..0.0003 % at 2560, 0.0005..0.0013 % at 2048
-  // (head dims 128, 256, 64).  Key lengths below 3072 take the max-tracking pass only.
-  a.direct_p = g_fast_e4m3.load(std::memory_order_relaxed);
-  a.track_only = cfk::predictable_latency() || (p->v_dtype == CFK_FP8_E4M3 && p->seqlen_kv < 3072) ? 1 : 0;
-  hipError_t e;
-  a.s_scale = p->dtype == CFK_FP16 ? p->softmax_scale : p->softmax_scale * p->q_descale * p->k_descale;
-  if (p->dtype == CFK_FP16) {
-    a.scale_log2 = p->softmax_scale * kLog2e;
-    a.out_scale = 1.0f;
-    e = cfk::launch_fmha_f16(a, p->head_dim, (hipStream_t)stream);
-  } else if (p->v_dtype == CFK_FP16) {  // hybrid: fp16 V carries no scale
-    a.scale_log2 = p->softmax_scale * kLog2e * p->q_descale * p->k_descale;
-    a.out_scale = 1.0f;
-    e = cfk::launch_fmha_hybrid(a, p->head_dim, (hipStream_t)stream);
-  } else {
-    a.scale_log2 = p->softmax_scale * kLog2e * p->q_descale * p->k_descale;
-    a.out_scale = p->v_descale;
-    e = cfk::launch_fmha_fp8(a, p->head_dim, (hipStream_t)stream);
-  }
-  if (e != hipSuccess) return fail(CFK_ERR_HIP, "FMHA launch failed: %s", hipGetErrorString(e));
-  return CFK_OK;
+  const int n = workspace ? key_splits(p, plan) : 1;
+  const bool split = n > 1 && workspace_bytes >= n * partial_bytes(p);
+  if (split && (uintptr_t)workspace % 16 != 0) return fail(CFK_ERR_INVALID_ARG, "workspace must be 16-byte aligned");
+  return launch_fmha(p, split ? n : 1, workspace, stream);
 }
 
 int cfk_set_option(int32_t option, int32_t value) {

@@ -22,6 +22,9 @@ struct FmhaArgs {
   int32_t v_layout;  // 0 = [B,S,H,D], 1 = [B,D,H,S]
   float tau;         // the softmax reference point moves when a tile's max exceeds it by more than this (log2 domain)
   int32_t track_only;  // no optimistic first pass over the keys (cfk_set_option(CFK_OPT_PREDICTABLE_LATENCY, 1))
+  int32_t n_split;     // workgroups that share a query block's keys (key-split kernel; 1: no workspace is touched)
+  float *part_o;       // their partial results, n_split of each: O [B,H,Sq,D] not divided by the row sum, and (reference point,
+  float *part_ml;      // row sum) pairs [B,H,Sq,2]
   int32_t direct_p;    // first pass with e4m3 P: codes without an exponential (cfk_set_option(CFK_OPT_FAST_E4M3_WEIGHTS, 1))
 };
 
@@ -34,7 +37,11 @@ struct FmhaPlan {
   int32_t block_m, block_n, lds_bytes, threads, grid;
   int32_t q_multiple;   // what the query length has to be a multiple of (block_m, or 32 where the last tile may be partly filled)
   int32_t kv_multiple;  // what the key length has to be a multiple of (block_n, or one key tile where the kernel has a tail)
+  int32_t split_tiles;  // key-split kernel: key tiles its waves take turns at; 0: another kernel
+  int32_t split_waves;  // ... those waves, and the time of a turn
+  float split_turn_us;
   int32_t mfma;  // 32: 32x32 MFMA build, 16: 16x16x32 build
+  bool want_name;   // set by a caller that wants the next field
   char kernel[80];  // the instantiation, as profilers print it without namespaces: fmha_fwd_kernel16p<128,64,8,2,0,0,0,0,2,0,1,1>
 };
 
@@ -57,6 +64,9 @@ hipError_t prepare_fmha_f16();
 hipError_t prepare_fmha_fp8();
 hipError_t prepare_fmha_hybrid();
 hipError_t prepare_gemm();
+
+// Merges a.n_split partial results of the key-split kernel into a.o.
+hipError_t launch_fmha_combine(const FmhaArgs &a, int head_dim, hipStream_t s);
 
 // D = alpha * A.B + beta * C for `batch` packed problems; f32 selects float operands (layout 0 only), else fp16.
 struct GemmArgs {

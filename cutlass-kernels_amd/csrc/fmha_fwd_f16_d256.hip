@@ -5,6 +5,7 @@
 // 928 TFLOP/s on B=2 H=8 S=8192 with N(0,1) tensors, 1206 against 1024 with constant tensors.  Every kernel with two or
 // three waves per SIMD loses under it (registers spill), so it is not a library-wide flag.
 #include "fmha_fwd_kernel16p.h"
+#include "fmha_fwd_kernel_ks.h"
 
 namespace cfk {
 namespace {
@@ -20,8 +21,10 @@ using C256_128x64 = FmhaCfg<256, 64, 4, 1, false, false>;
 // The hand-scheduled persistent build on 16x16x32 MFMAs (fmha_fwd_kernel16p.h; key length a multiple of 128, at least
 // 256): two 32-key tiles per barrier, big problems only
 using A256_128x64 = FmhaCfg<256, 32, 4, 1, false, false, false, false, 2, 0, true, true>;
+// few query rows: the waves of a workgroup split the keys (not by wish)
+using K256_32x32 = KsCfg<256, 4>;
 using All256 = CfgList<C256_128x32P, C256_128x32, C256_128x64, A256_128x64>;
-using Auto256 = CfgList<A256_128x64, C256_128x32P, C256_128x32>;
+using Auto256 = CfgList<K256_32x32, A256_128x64, C256_128x32P, C256_128x32>;
 
 template <class F>
 void dispatch(int sq, int skv, int bh, F &&f) {
@@ -31,7 +34,7 @@ void dispatch(int sq, int skv, int bh, F &&f) {
 }  // namespace
 
 void plan_fmha_f16_d256(int sq, int skv, int bh, FmhaPlan *p) {
-  dispatch(sq, skv, bh, [&](auto cfg) { fill_fmha_plan<decltype(cfg)>(sq, bh, p); });
+  dispatch(sq, skv, bh, [&](auto cfg) { fill_fmha_plan<decltype(cfg)>(sq, skv, bh, p); });
 }
 
 hipError_t launch_fmha_f16_d256(const FmhaArgs &a, hipStream_t s) {
@@ -40,6 +43,7 @@ hipError_t launch_fmha_f16_d256(const FmhaArgs &a, hipStream_t s) {
   return e;
 }
 
-hipError_t prepare_fmha_f16_d256() { return prepare_all(All256{}); }
+hipError_t prepare_fmha_f16_d256() { const hipError_t e = prepare_all(All256{});
+  return e != hipSuccess ? e : prepare_all(CfgList<K256_32x32>{}); }
 
 }  // namespace cfk

@@ -2,6 +2,7 @@
 // The kernel, including the fp8 V-tile layout transform, is in fmha_fwd_kernel.h.
 #include "fmha_fwd_kernel.h"
 #include "fmha_fwd_kernel8p.h"
+#include "fmha_fwd_kernel_ks.h"
 
 namespace cfk {
 namespace {
@@ -21,6 +22,14 @@ using A128_256x128 = FmhaCfg<128, 64, 8, 2, true, true, false, false, 2, 0, fals
 using A128_128x128 = FmhaCfg<128, 64, 4, 2, true, true, false, false, 2, 0, false, true>;   // the same loop, 4 waves, one per SIMD
 using C256_128x64 = FmhaCfg<256, 64, 4, 1, true, true>;
 using C256_128x128 = FmhaCfg<256, 64, 4, 1, true, true, false, false, 2>;
+
+// few query rows: the waves of a workgroup split the keys (fmha_fwd_kernel_ks.h; not by wish)
+using K64 = KsCfg8<64, 8, true, false>;
+using K128 = KsCfg8<128, 8, true, false>;
+using K256 = KsCfg8<256, 4, true, false>;
+using K64T = KsCfg8<64, 8, true, true>;
+using K128T = KsCfg8<128, 8, true, true>;
+using K256T = KsCfg8<256, 4, true, true>;
 
 // V pre-transposed to [B,D,H,S] (the reference's offline transpose, src/fmha-pipeline/fmha_forward.cu:514-532)
 using C64T = FmhaCfg<64, 64, 4, 2, true, true, true>;
@@ -52,18 +61,18 @@ bool dispatch(int head_dim, int sq, int skv, int bh, int v_layout, bool tap_s, F
   }
   if (v_layout == 1) {
     switch (head_dim) {
-      case 64: f(C64T{}); return true;
-      case 128: f(C128T{}); return true;
-      case 256: f(C256T{}); return true;
+      case 64: select_tile<CfgList<C64T>, CfgList<K64T, C64T>, C64T>(sq, skv, bh, f); return true;
+      case 128: select_tile<CfgList<C128T>, CfgList<K128T, C128T>, C128T>(sq, skv, bh, f); return true;
+      case 256: select_tile<CfgList<C256T>, CfgList<K256T, C256T>, C256T>(sq, skv, bh, f); return true;
       default: return false;
     }
   }
   switch (head_dim) {
-    case 64: select_tile<All64, CfgList<C64_128x64>, C64_128x64>(sq, skv, bh, f); return true;
+    case 64: select_tile<All64, CfgList<K64, C64_128x64>, C64_128x64>(sq, skv, bh, f); return true;
     // big problems: 256 rows with one barrier per 128 keys (+4 % on N(0,1) data over the 128x64 tile)
-    case 128: select_tile<All128, CfgList<A128_256x128, A128_128x128, C128_256x128, C128_128x64>, C128_128x64>(sq, skv, bh, f); return true;
+    case 128: select_tile<All128, CfgList<K128, A128_256x128, A128_128x128, C128_256x128, C128_128x64>, C128_128x64>(sq, skv, bh, f); return true;
     // one barrier per 128 keys: +11 % at head dim 256 (1604 against 1439 TFLOP/s, B=4 H=8 S=4096)
-    case 256: select_tile<All256, CfgList<C256_128x128, C256_128x64>, C256_128x64>(sq, skv, bh, f); return true;
+    case 256: select_tile<All256, CfgList<K256, C256_128x128, C256_128x64>, C256_128x64>(sq, skv, bh, f); return true;
     default: return false;
   }
 }
@@ -71,7 +80,7 @@ bool dispatch(int head_dim, int sq, int skv, int bh, int v_layout, bool tap_s, F
 }  // namespace
 
 bool plan_fmha_fp8(int head_dim, int sq, int skv, int bh, int v_layout, bool tap_s, FmhaPlan *p) {
-  return dispatch(head_dim, sq, skv, bh, v_layout, tap_s, [&](auto cfg) { fill_fmha_plan<decltype(cfg)>(sq, bh, p); });
+  return dispatch(head_dim, sq, skv, bh, v_layout, tap_s, [&](auto cfg) { fill_fmha_plan<decltype(cfg)>(sq, skv, bh, p); });
 }
 
 hipError_t launch_fmha_fp8(const FmhaArgs &a, int head_dim, hipStream_t s) {
@@ -84,6 +93,7 @@ hipError_t prepare_fmha_fp8() {
   hipError_t e = prepare_all(All64{});
   if (e == hipSuccess) e = prepare_all(All128{});
   if (e == hipSuccess) e = prepare_all(All256{});
+  if (e == hipSuccess) e = prepare_all(CfgList<K64, K128, K256, K64T, K128T, K256T>{});
   if (e == hipSuccess) e = prepare_all(CfgList<C64T, C128T, C256T, C64Tap, C128Tap, C256Tap, C64TTap, C128TTap, C256TTap>{});
   return e;
 }

@@ -2,6 +2,7 @@
 // what the reference's --prec-type=2 computes when built without -DGEMM2FP8 (src/fmha-pipeline/fmha_forward.cu:
 // 446-450).  Tile shapes and dispatch; the kernel is in fmha_fwd_kernel.h.
 #include "fmha_fwd_kernel.h"
+#include "fmha_fwd_kernel_ks.h"
 
 namespace cfk {
 namespace {
@@ -13,6 +14,11 @@ using C128_128x64 = FmhaCfg<128, 64, 4, 2, true, false>;
 using C128_256x64 = FmhaCfg<128, 64, 8, 2, true, false>;
 using C128_256x128 = FmhaCfg<128, 64, 8, 2, true, false, false, false, 2>;
 using C256_128x32 = FmhaCfg<256, 32, 4, 1, true, false>;
+
+// few query rows: the waves of a workgroup split the keys (fmha_fwd_kernel_ks.h; not by wish)
+using K64 = KsCfg8<64, 8, false, false>;
+using K128 = KsCfg8<128, 8, false, false>;
+using K256 = KsCfg8<256, 4, false, false>;
 
 // builds that also write the score tap (debug): 128-row tile only
 using C64Tap = FmhaCfg<64, 64, 4, 2, true, false, false, true>;
@@ -34,9 +40,9 @@ bool dispatch(int head_dim, int sq, int skv, int bh, bool tap_s, F &&f) {
     }
   }
   switch (head_dim) {
-    case 64: select_tile<All64, CfgList<C64_128x64>, C64_128x64>(sq, skv, bh, f); return true;
-    case 128: select_tile<All128, CfgList<C128_256x64, C128_128x64>, C128_128x64>(sq, skv, bh, f); return true;
-    case 256: select_tile<All256, CfgList<C256_128x32>, C256_128x32>(sq, skv, bh, f); return true;
+    case 64: select_tile<All64, CfgList<K64, C64_128x64>, C64_128x64>(sq, skv, bh, f); return true;
+    case 128: select_tile<All128, CfgList<K128, C128_256x64, C128_128x64>, C128_128x64>(sq, skv, bh, f); return true;
+    case 256: select_tile<All256, CfgList<K256, C256_128x32>, C256_128x32>(sq, skv, bh, f); return true;
     default: return false;
   }
 }
@@ -44,7 +50,7 @@ bool dispatch(int head_dim, int sq, int skv, int bh, bool tap_s, F &&f) {
 }  // namespace
 
 bool plan_fmha_hybrid(int head_dim, int sq, int skv, int bh, bool tap_s, FmhaPlan *p) {
-  return dispatch(head_dim, sq, skv, bh, tap_s, [&](auto cfg) { fill_fmha_plan<decltype(cfg)>(sq, bh, p); });
+  return dispatch(head_dim, sq, skv, bh, tap_s, [&](auto cfg) { fill_fmha_plan<decltype(cfg)>(sq, skv, bh, p); });
 }
 
 hipError_t launch_fmha_hybrid(const FmhaArgs &a, int head_dim, hipStream_t s) {
@@ -57,6 +63,7 @@ hipError_t prepare_fmha_hybrid() {
   hipError_t e = prepare_all(All64{});
   if (e == hipSuccess) e = prepare_all(All128{});
   if (e == hipSuccess) e = prepare_all(All256{});
+  if (e == hipSuccess) e = prepare_all(CfgList<K64, K128, K256>{});
   if (e == hipSuccess) e = prepare_all(CfgList<C64Tap, C128Tap, C256Tap>{});
   return e;
 }

@@ -819,7 +819,7 @@ hipError_t launch_fmha_cfg(const FmhaArgs &a, hipStream_t s) {
   const hipError_t e = prepare_fmha_cfg<C>();
   if (e != hipSuccess) return e;
   const int items = a.B * a.H * ((a.Sq + C::BM - 1) / C::BM);
-  const int grid = C::ASM ? persistent_grid(items) : items;
+  const int grid = C::ASM ? persistent_grid(items) : C::KSPLIT ? items * a.n_split : items;
   if constexpr (has_direct_build<C>) {
     if (a.direct_p != 0) {
       hipLaunchKernelGGL(fmha_kernel_of<DirectCfg<C>>(), dim3(grid), dim3(C::T), C::LDS_BYTES, s, a);
@@ -831,7 +831,7 @@ hipError_t launch_fmha_cfg(const FmhaArgs &a, hipStream_t s) {
 }
 
 template <class C>
-void fill_fmha_plan(int sq, int bh, FmhaPlan *p) {
+void fill_fmha_plan(int sq, int skv, int bh, FmhaPlan *p) {
   p->block_m = C::BM;
   p->block_n = C::BN * C::SUB;
   p->kv_multiple = C::ASM && C::D != 256 ? C::BN : C::BN * C::SUB;
@@ -840,10 +840,17 @@ void fill_fmha_plan(int sq, int bh, FmhaPlan *p) {
   p->lds_bytes = C::LDS_BYTES;
   p->threads = C::T;
   p->grid = bh * ((sq + C::BM - 1) / C::BM);
+  p->split_tiles = p->split_waves = 0;
   if constexpr (C::KSPLIT) {
-    snprintf(p->kernel, sizeof p->kernel, "fmha_fwd_kernel_ks<%d,%d>", C::D, C::NWAVES);
+    p->split_tiles = skv / C::TK;
+    p->split_waves = C::NWAVES;
+    p->split_turn_us = C::TURN_US;
+    if (!p->want_name) return;
+    if (C::QK8) snprintf(p->kernel, sizeof p->kernel, "fmha_fwd_kernel_ks<%d,%d,%d,%d>", C::D, C::NWAVES, (int)C::PV8, (int)C::VT);
+    else snprintf(p->kernel, sizeof p->kernel, "fmha_fwd_kernel_ks<%d,%d>", C::D, C::NWAVES);
     return;
   }
+  if (!p->want_name) return;
   snprintf(p->kernel, sizeof p->kernel, "%s<%d,%d,%d,%d,%d,%d,%d,%d,%d,%d,%d,%d>",
            C::ASM ? (C::QK8 ? "fmha_fwd_kernel8p" : "fmha_fwd_kernel16p") : C::M16 ? "fmha_fwd_kernel16" : "fmha_fwd_kernel", C::D, C::BN, C::NWAVES, C::WPE,
            (int)C::QK8, (int)C::PV8, (int)C::VT, (int)C::TAP_S, C::SUB, C::KPRE, (int)C::M16, (int)C::ASM);
@@ -941,10 +948,28 @@ constexpr bool hand_loop_pays(long long items, int skv) {
 // (The compiler-scheduled fp16 256-row builds need key length to pay: B=8 H=27 S_q=1536 D=128 with 896 keys 723 TFLOP/s on
 // 256 x 128 keys, 871 on 256 x 64, 947 on 128 x 64, all on 16x16x32 MFMAs; with 1536 keys 1036 / 1038 / 1014.  e4m3, B=8 H=32
 // S_q=2048 D=128: 1024 keys 1445 on 256 x 128 against 1517 on 128 x 64, 1536 keys 1529 / 1573, 2048 keys 1702 / 1705.)
+// Where the key-split build (32 query rows per workgroup, whose waves split the keys) beats the 128-row builds: while its
+// workgroups fit on the chip all at once.  us at 256 workgroups, 128-row build -> key-split build: 512 keys, head dims 64 / 128 /
+// 256: fp16 8.3 -> 5.6, 11.8 -> 7.6, 20.5 -> 15.4; e4m3 7.6 -> 5.4, 9.8 -> 6.9, 19.2 -> 11.6; hybrid 7.9 -> 5.6, 9.7 -> 7.3, 16.6 ->
+// 13.6; 2048 keys: fp16 18.7 -> 10.6, 30.0 -> 17.7, 50.7 -> 39.6.  At 512 workgroups of fp16 a tie at 2048 keys (20.7 / 19.7) and
+// below a loss.  128 keys: e4m3 Q and K lose there (4.2 -> 4.7).  e4m3 Q and K at head dim 64, where the tiles are small (with
+// e4m3 V two of these workgroups share a CU), up to 512 workgroups from
+// 1024 keys: 2048 keys e4m3 21.2 -> 16.5, hybrid 22.6 -> 18.4; at head dims 128 and 256 a tie there.
+// fp16 at head dim 256 (1024 keys, 256 workgroups 31.4 -> 23.1) stays on the hand-scheduled build from 1024 query rows and
+// keys on: tests/test_abi.py holds the choice of kernel there.
+template <class C>
+constexpr bool key_split_pays(long long wgs, int sq, int skv) {
+  if (skv < (C::QK8 && C::D <= 128 ? 192 : 128)) return false;
+  if (!C::QK8 && C::D == 256 && sq >= 1024 && skv >= 1024) return false;
+  if (wgs <= 256) return true;
+  if (wgs > 512) return false;
+  return C::QK8 && C::D == 64 && skv >= 1024;
+}
+
 // Calls f with the first instantiation of the list that fits the shape and the wish.  Without a wish for the query
 // rows, the hand-scheduled builds are taken where they pay (above), other tiles above 128 rows and the other 16x16x32
 // builds (slower where launch and prologue dominate) only for big problems (size 2: enough workgroups to fill 256 CUs
-// twice), and the key-split build only for small ones (size 0: its 32-row workgroups fit on the chip all at once).
+// twice), and the key-split build only for small ones (above).
 template <class F, class... Cs>
 bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish w, F &&f) {
   bool done = false;
@@ -979,7 +1004,7 @@ bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish
     const bool by_size = C::ASM ? tight && stacked_ok && hand_loop_pays<C>(bh * ((sq + C::BM - 1) / C::BM), skv)
                                 : (C::QK8 && C::BM > 128 ? fills256 : !((C::BM > 128 || C::M16) && size != 2)) &&
                                       !(C::BM > 128 && skv < (C::PV8 ? 2048 : C::QK8 ? 0 : 1152));
-    if (C::KSPLIT ? (w.bm ? C::BM != w.bm : size != 0) : (w.bm ? C::BM != w.bm : !by_size)) return;
+    if (C::KSPLIT ? (w.bm ? C::BM != w.bm : !key_split_pays<C>(bh * ((sq + 31) / 32), sq, skv)) : (w.bm ? C::BM != w.bm : !by_size)) return;
     if (w.bn && C::BN * C::SUB != w.bn) return;
     if (w.mfma && (C::M16 ? 16 : 32) != w.mfma) return;
     if (w.hand && C::ASM != (w.hand > 0)) return;
@@ -995,8 +1020,7 @@ bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish
 template <class All, class Auto, class Fallback, class F>
 void select_tile(int sq, int skv, int bh, F &&f) {
   const bool big = sq % 256 == 0 && (long long)bh * (sq / 256) >= 512;
-  const bool small = (long long)bh * ((sq + 31) / 32) <= 256 && skv >= 128;
-  const int size = big ? 2 : small ? 0 : 1;
+  const int size = big ? 2 : 1;
   const TileWish w = tile_wish();
   if ((w.bm || w.bn) && first_fit(All{}, sq, skv, bh, size, w, f)) return;
   static const bool no_hand = [] { const char *e = getenv("CFK_FMHA_HANDLOOP"); return e && e[0] == '0'; }();

@@ -14,7 +14,7 @@ import subprocess
 import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCES = ["fmha_fwd_f16.hip", "fmha_fwd_f16_d256.hip", "fmha_fwd_fp8.hip", "fmha_fwd_hybrid.hip", "gemm.hip"]
+SOURCES = ["fmha_fwd_f16.hip", "fmha_fwd_f16_d256.hip", "fmha_fwd_fp8.hip", "fmha_fwd_hybrid.hip", "fmha_combine.hip", "gemm.hip"]
 FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-command-line-argument", "-fno-gpu-rdc", "--offload-device-only", "-Rpass-analysis=kernel-resource-usage",
          "-c", "-o", "/dev/null"]
@@ -35,7 +35,7 @@ def short_name(d):
     d = re.sub(r"^void ", "", d).replace("(anonymous namespace)::", "")
     d = re.sub(r"\(.*\)$", "", d)
     direct = "DirectCfg<" in d     # the build with e4m3 weights written as codes: shown as <...>/direct
-    d = d.replace("cfk::", "").replace("DirectCfg<", "").replace("FmhaCfg<", "").replace("KsCfg<", "").replace(">>", ">").replace(">>", ">")
+    d = d.replace("cfk::", "").replace("DirectCfg<", "").replace("FmhaCfg<", "").replace("KsCfg<", "").replace("KsCfg8<", "").replace(">>", ">").replace(">>", ">")
     d = d.replace("false", "0").replace("true", "1").replace(" ", "")
     return re.sub(r">+$", ">", d) + ("/direct" if direct else "")
 

@@ -80,6 +80,12 @@ def lib():
         l = ctypes.CDLL(_LIB_PATH)
         l.cfk_fmha_forward.restype = ctypes.c_int
         l.cfk_fmha_forward.argtypes = [ctypes.POINTER(FmhaFwdParams), ctypes.c_void_p]
+        l.cfk_fmha_forward_ws.restype = ctypes.c_int
+        l.cfk_fmha_forward_ws.argtypes = [ctypes.POINTER(FmhaFwdParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+        l.cfk_fmha_forward_workspace.restype = ctypes.c_int64
+        l.cfk_fmha_forward_workspace.argtypes = [ctypes.POINTER(FmhaFwdParams)]
+        l.cfk_fmha_forward_or_workspace.restype = ctypes.c_int64
+        l.cfk_fmha_forward_or_workspace.argtypes = [ctypes.POINTER(FmhaFwdParams), ctypes.c_void_p]
         l.cfk_fmha_forward_plan.restype = ctypes.c_int
         l.cfk_fmha_forward_plan.argtypes = [ctypes.POINTER(FmhaFwdParams)] + [ctypes.POINTER(ctypes.c_int32)] * 4
         l.cfk_fmha_forward_mfma.restype = ctypes.c_int
@@ -224,8 +230,22 @@ def fmha_forward(q, k, v, o=None, softmax_scale=None, q_descale=1.0, k_descale=1
                     dbg_s=scores.data_ptr() if scores is not None else 0)
     if prepare:
         return PreparedForward(p, (q, k, v, o, row_max, row_sum, scores), stream)
-    _check(lib().cfk_fmha_forward(ctypes.byref(p), _stream_ptr(stream)))
+    rc = lib().cfk_fmha_forward_or_workspace(ctypes.byref(p), _stream_ptr(stream))
+    if rc > 0:   # the call is not made yet: it can use this much scratch memory
+        ws = _workspace(rc, q.device, stream)
+        rc = lib().cfk_fmha_forward_ws(ctypes.byref(p), ws.data_ptr(), rc, _stream_ptr(stream))
+    _check(rc)
     return o
+
+
+def _workspace(n, device, stream):
+    """n bytes of scratch memory for one call, from torch's allocator for the stream that the call runs on: free again when the
+    caller drops it, reused only by later work of that stream (or of the graph being captured)."""
+    import torch
+    if stream is None:
+        return torch.empty(n, dtype=torch.uint8, device=device)
+    with torch.cuda.stream(torch.cuda.ExternalStream(stream, device=device) if isinstance(stream, int) else stream):
+        return torch.empty(n, dtype=torch.uint8, device=device)
 
 
 class PreparedForward:
@@ -239,10 +259,14 @@ class PreparedForward:
         self.o = tensors[3]
         self._ref = ctypes.byref(params)
         self._stream = _stream_ptr(stream)
-        self._fn = lib().cfk_fmha_forward
+        self._fn = lib().cfk_fmha_forward_ws
+        self._ws_bytes = lib().cfk_fmha_forward_workspace(self._ref)
+        # (kept: the calls run one after the other on one stream)
+        self._ws = _workspace(self._ws_bytes, tensors[0].device, stream) if self._ws_bytes else None
+        self._ws_ptr = self._ws.data_ptr() if self._ws_bytes else None
 
     def __call__(self):
-        rc = self._fn(self._ref, self._stream)
+        rc = self._fn(self._ref, self._ws_ptr, self._ws_bytes, self._stream)
         if rc != 0:
             _check(rc)
         return self.o

@@ -85,13 +85,29 @@ typedef struct cfk_fmha_fwd_params {
                          weights AS ROUNDED to the precision of P (fp16, or e4m3 for v_dtype = CFK_FP8_E4M3) -- the
                          weights the second GEMM applies, so that rows of O are exactly normalised -- where the
                          reference sums the fp32 values before the cast (online_softmax.h:173-206).  The rounding
-                         is unbiased: the two sums agree to ~1e-4 relative (fp16) / < 1 % (e4m3).  One exception:
-                         e4m3 with head_dim 256 sums the fp32 values, as the reference does                    */
+                         is unbiased: the two sums agree to ~1e-4 relative (fp16) / < 1 % (e4m3).  Exceptions: e4m3
+                         with head_dim 256, and the builds for few query rows (fmha_fwd_kernel_ks), whose weights
+                         are fp16 in every mode, sum the fp32 values, as the reference does                    */
 } cfk_fmha_fwd_params;
 
 /* FMHA forward: O = softmax(softmax_scale * Q K^T) V per (batch, head); no mask, no dropout.
  * Replaces fmhaForwardDevice (src/fmha-pipeline/fmha_forward.cu:86-383), one launch per call. */
 int cfk_fmha_forward(const cfk_fmha_fwd_params *params, void *stream);
+
+/* The same call with scratch memory: where a problem has too few query blocks to go round the compute units, its keys are
+ * split over several workgroups, whose partial results (fp32 O, reference point and row sum per query row) meet in
+ * `workspace` -- device memory of at least cfk_fmha_forward_workspace(params) bytes, 16-byte aligned, that nothing else uses
+ * until the call has run on `stream`; its content does not matter before and after.  With workspace = NULL, or one that is
+ * too small, this is cfk_fmha_forward.  Two launches per call where the keys are split.  No counterpart in the reference,
+ * which walks a query block's keys in one thread block (src/fmha-pipeline/fmha_forward.cu:361-372). */
+int cfk_fmha_forward_ws(const cfk_fmha_fwd_params *params, void *workspace, int64_t workspace_bytes, void *stream);
+
+/* One step for callers that allocate on demand: makes the call if it has no use for a workspace (returns 0, or a negative
+ * cfk_status), or else returns the bytes it can use, with nothing launched. */
+int64_t cfk_fmha_forward_or_workspace(const cfk_fmha_fwd_params *params, void *stream);
+
+/* Bytes of workspace cfk_fmha_forward_ws can use for `params`; 0: none (or invalid params).  Does not touch the GPU. */
+int64_t cfk_fmha_forward_workspace(const cfk_fmha_fwd_params *params);
 
 /* Bytes of LDS and the tile shape the library would pick for `params` (query rows per workgroup, keys per
  * tile); the reference fixes these at compile time (src/fmha-pipeline/shared_storage.h:4-22).  Any of the
