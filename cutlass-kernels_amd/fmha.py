@@ -9,11 +9,14 @@ from __future__ import annotations
 import ctypes
 import math
 import os
+import struct
 import subprocess
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_HERE, "libcfk_fmha.so")
 _lib = None
+_launch = None   # (fmha, fmha with workspace, gemm): the launching entry points taking their parameter block as bytes
+_torch = None
 
 CFK_FP16 = 1
 CFK_FP8_E4M3 = 2
@@ -54,6 +57,12 @@ class GemmParams(ctypes.Structure):
         ("alpha", ctypes.c_float), ("beta", ctypes.c_float),
         ("a", ctypes.c_void_p), ("b", ctypes.c_void_p), ("c", ctypes.c_void_p), ("d", ctypes.c_void_p),
     ]
+
+
+# The same two blocks for the launch path: packing bytes takes a fraction of the time of filling a ctypes structure.
+_FMHA_BLOCK = struct.Struct("=8i4Q4f3Q")
+_GEMM_BLOCK = struct.Struct("=6i2f4Q")
+assert _FMHA_BLOCK.size == ctypes.sizeof(FmhaFwdParams) and _GEMM_BLOCK.size == ctypes.sizeof(GemmParams)
 
 
 def lib_path() -> str:
@@ -171,11 +180,25 @@ def fmha_forward_kernel(dtype, batch, heads, seqlen_q, seqlen_kv, head_dim, v_la
     return buf.value.decode()
 
 
-def _stream_ptr(stream):
-    if stream is None:
+def _launchers():
+    """torch and the launching entry points, looked up once."""
+    global _torch, _launch
+    if _launch is None:
         import torch
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return ctypes.c_void_p(stream if isinstance(stream, int) else stream.cuda_stream)
+        l = lib()
+        _torch = torch
+        _launch = (ctypes.CFUNCTYPE(ctypes.c_int64, ctypes.c_char_p, ctypes.c_void_p)(("cfk_fmha_forward_or_workspace", l)),
+                   ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_char_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p)(("cfk_fmha_forward_ws", l)),
+                   ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_char_p, ctypes.c_void_p)(("cfk_gemm", l)))
+    return _launch
+
+
+def _stream_ptr(stream):
+    """The hipStream_t of ``stream`` (a torch stream or a pointer; None: torch's current stream of the current device)."""
+    if stream is None:
+        # (torch.cuda.current_stream() builds a Stream object: 2.5 us, as much as the launch itself)
+        return _torch._C._cuda_getCurrentRawStream(_torch._C._cuda_getDevice())
+    return stream if isinstance(stream, int) else stream.cuda_stream
 
 
 def fmha_forward(q, k, v, o=None, softmax_scale=None, q_descale=1.0, k_descale=1.0, v_descale=1.0,
@@ -187,65 +210,66 @@ def fmha_forward(q, k, v, o=None, softmax_scale=None, q_descale=1.0, k_descale=1
     q,k: hybrid mode).  ``v`` is [B,D,H,S] when
     ``v_layout == CFK_V_BDHS``.  ``row_max`` / ``row_sum`` / ``scores`` are the optional debug taps.  Returns ``o`` (float16 [B,Sq,H,D]); launches asynchronously on ``stream``
     (default: torch's current stream)."""
-    import torch
+    launch, launch_ws, _ = _launch or _launchers()
+    f16 = _torch.float16
     if not (q.is_cuda and k.is_cuda and v.is_cuda):
         raise ValueError("q, k, v must be device tensors (there is no CPU path)")
     if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
         raise ValueError("q, k, v must be contiguous [B,S,H,D]")
-    if q.dtype == torch.float16:
+    qt, vt = q.dtype, v.dtype
+    if qt == f16:
         dtype = CFK_FP16
-    elif q.dtype in (torch.float8_e4m3fn, torch.uint8):
+    elif qt in (_torch.float8_e4m3fn, _torch.uint8):
         dtype = CFK_FP8_E4M3
     else:
-        raise ValueError(f"unsupported dtype {q.dtype}")
-    if k.dtype != q.dtype:
+        raise ValueError(f"unsupported dtype {qt}")
+    if k.dtype != qt:
         raise ValueError("q and k must share one dtype")
-    if v.dtype == q.dtype:
+    if vt == qt:
         v_dtype = dtype
-    elif dtype == CFK_FP8_E4M3 and v.dtype == torch.float16:
+    elif dtype == CFK_FP8_E4M3 and vt == f16:
         v_dtype = CFK_FP16  # hybrid mode: e4m3 Q,K with fp16 P,V (the reference's fp8 build without GEMM2FP8)
     else:
         raise ValueError("v must have the dtype of q, or float16 with fp8 q/k")
-    B, Sq, H, D = q.shape
-    Skv = k.shape[1]
-    if tuple(k.shape) != (B, Skv, H, D):
+    B, Sq, H, D = q_shape = q.shape
+    k_shape = k.shape
+    Skv = k_shape[1]
+    if k_shape != (B, Skv, H, D):
         raise ValueError("k shape mismatch")
-    want_v = (B, Skv, H, D) if v_layout == CFK_V_BSHD else (B, D, H, Skv)
-    if tuple(v.shape) != want_v:
-        raise ValueError(f"v shape {tuple(v.shape)} does not match layout {v_layout}: expected {want_v}")
+    if v.shape != (k_shape if v_layout == CFK_V_BSHD else (B, D, H, Skv)):
+        raise ValueError(f"v shape {tuple(v.shape)} does not match layout {v_layout}: expected "
+                         f"{(B, Skv, H, D) if v_layout == CFK_V_BSHD else (B, D, H, Skv)}")
     if o is None:
-        o = torch.empty((B, Sq, H, D), dtype=torch.float16, device=q.device)
-    elif o.dtype != torch.float16 or tuple(o.shape) != (B, Sq, H, D) or not o.is_contiguous() or not o.is_cuda:
+        o = _torch.empty_like(q, dtype=f16)
+    elif o.dtype != f16 or o.shape != q_shape or not o.is_contiguous() or not o.is_cuda:
         raise ValueError("o must be a contiguous float16 device tensor [B,Sq,H,D]")
     for t in (row_max, row_sum):
-        if t is not None and (t.dtype != torch.float32 or tuple(t.shape) != (B, H, Sq) or not t.is_contiguous()):
+        if t is not None and (t.dtype != _torch.float32 or t.shape != (B, H, Sq) or not t.is_contiguous()):
             raise ValueError("row_max/row_sum must be contiguous float32 [B,H,Sq]")
-    if scores is not None and (scores.dtype != torch.float32 or tuple(scores.shape) != (B, H, Sq, Skv)
+    if scores is not None and (scores.dtype != _torch.float32 or scores.shape != (B, H, Sq, Skv)
                                or not scores.is_contiguous()):
         raise ValueError("scores must be contiguous float32 [B,H,Sq,Skv]")
-    p = make_params(dtype, B, H, Sq, Skv, D, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), softmax_scale,
-                    q_descale, k_descale, v_descale, v_layout, v_dtype=v_dtype,
-                    dbg_row_max=row_max.data_ptr() if row_max is not None else 0,
-                    dbg_row_sum=row_sum.data_ptr() if row_sum is not None else 0,
-                    dbg_s=scores.data_ptr() if scores is not None else 0)
+    scale = 1.0 / math.sqrt(D) if softmax_scale is None else softmax_scale
+    block = _FMHA_BLOCK.pack(dtype, v_dtype, B, H, Sq, Skv, D, v_layout, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+                             scale, q_descale, k_descale, v_descale, *(0 if t is None else t.data_ptr() for t in (scores, row_max, row_sum)))
     if prepare:
-        return PreparedForward(p, (q, k, v, o, row_max, row_sum, scores), stream)
-    rc = lib().cfk_fmha_forward_or_workspace(ctypes.byref(p), _stream_ptr(stream))
+        return PreparedForward(FmhaFwdParams.from_buffer_copy(block), (q, k, v, o, row_max, row_sum, scores), stream)
+    rc = launch(block, _stream_ptr(stream))
     if rc > 0:   # the call is not made yet: it can use this much scratch memory
         ws = _workspace(rc, q.device, stream)
-        rc = lib().cfk_fmha_forward_ws(ctypes.byref(p), ws.data_ptr(), rc, _stream_ptr(stream))
-    _check(rc)
+        rc = launch_ws(block, ws.data_ptr(), rc, _stream_ptr(stream))
+    if rc != 0:
+        _check(rc)
     return o
 
 
 def _workspace(n, device, stream):
     """n bytes of scratch memory for one call, from torch's allocator for the stream that the call runs on: free again when the
     caller drops it, reused only by later work of that stream (or of the graph being captured)."""
-    import torch
     if stream is None:
-        return torch.empty(n, dtype=torch.uint8, device=device)
-    with torch.cuda.stream(torch.cuda.ExternalStream(stream, device=device) if isinstance(stream, int) else stream):
-        return torch.empty(n, dtype=torch.uint8, device=device)
+        return _torch.empty(n, dtype=_torch.uint8, device=device)
+    with _torch.cuda.stream(_torch.cuda.ExternalStream(stream, device=device) if isinstance(stream, int) else stream):
+        return _torch.empty(n, dtype=_torch.uint8, device=device)
 
 
 class PreparedForward:
@@ -258,7 +282,7 @@ class PreparedForward:
         self.params, self.tensors = params, tensors   # (the tensors are held so that their memory stays alive)
         self.o = tensors[3]
         self._ref = ctypes.byref(params)
-        self._stream = _stream_ptr(stream)
+        self._stream = ctypes.c_void_p(_stream_ptr(stream))
         self._fn = lib().cfk_fmha_forward_ws
         self._ws_bytes = lib().cfk_fmha_forward_workspace(self._ref)
         # (kept: the calls run one after the other on one stream)
@@ -274,8 +298,8 @@ class PreparedForward:
 
 def gemm_f16(a, b, c=None, layout=CFK_GEMM_TN, stream=None):
     """C[M,N] = A[M,K] . B  with B as [N,K] (TN, the reference's form) or [K,N] (NN); fp16 in, fp32 accumulate, fp16 out."""
-    import torch
-    if a.dtype != torch.float16 or b.dtype != torch.float16 or not (a.is_cuda and b.is_cuda):
+    _launch or _launchers()
+    if a.dtype != _torch.float16 or b.dtype != _torch.float16 or not (a.is_cuda and b.is_cuda):
         raise ValueError("a, b must be float16 device tensors")
     if not (a.is_contiguous() and b.is_contiguous()):
         raise ValueError("a, b must be contiguous")
@@ -284,7 +308,7 @@ def gemm_f16(a, b, c=None, layout=CFK_GEMM_TN, stream=None):
     if tuple(b.shape) != ((N, K) if layout == CFK_GEMM_TN else (K, N)):
         raise ValueError("b shape mismatch")
     if c is None:
-        c = torch.empty((M, N), dtype=torch.float16, device=a.device)
+        c = a.new_empty((M, N))
     _check(lib().cfk_gemm_f16(M, N, K, a.data_ptr(), b.data_ptr(), c.data_ptr(), layout, _stream_ptr(stream)))
     return c
 
@@ -296,30 +320,28 @@ def gemm(a, b, c=None, alpha=1.0, beta=0.0, out=None, layout=CFK_GEMM_TN, stream
     [K,N] (NN, fp16 only), with the same leading batch dimension; ``c`` / ``out`` are [M,N] or [L,M,N].  float16 or
     float32 device tensors, all of one dtype (the reference's types 3 and 1, gemm.cu:677-684).
     """
-    import torch
-    if a.dtype not in (torch.float16, torch.float32) or b.dtype != a.dtype or not (a.is_cuda and b.is_cuda):
+    _, _, launch = _launch or _launchers()
+    dt = a.dtype
+    if dt not in (_torch.float16, _torch.float32) or b.dtype != dt or not (a.is_cuda and b.is_cuda):
         raise ValueError("a, b must be float16 or float32 device tensors of one dtype")
-    if a.dim() not in (2, 3) or b.dim() != a.dim():
+    a_shape, b_shape = a.shape, b.shape
+    if len(a_shape) not in (2, 3) or len(b_shape) != len(a_shape):
         raise ValueError("a, b must both be 2-D or both 3-D (leading batch dimension)")
     if not (a.is_contiguous() and b.is_contiguous()):
         raise ValueError("a, b must be contiguous")
-    L = a.shape[0] if a.dim() == 3 else 1
-    M, K = a.shape[-2:]
-    N = b.shape[-2] if layout == CFK_GEMM_TN else b.shape[-1]
-    if tuple(b.shape[-2:]) != ((N, K) if layout == CFK_GEMM_TN else (K, N)) or (b.dim() == 3 and b.shape[0] != L):
+    lead = a_shape[:-2]
+    M, K = a_shape[-2:]
+    N = b_shape[-2] if layout == CFK_GEMM_TN else b_shape[-1]
+    if b_shape != (lead + ((N, K) if layout == CFK_GEMM_TN else (K, N))):
         raise ValueError("b shape mismatch")
-    shape = (L, M, N) if a.dim() == 3 else (M, N)
+    shape = lead + (M, N)
     if out is None:
-        out = torch.empty(shape, dtype=a.dtype, device=a.device)
+        out = a.new_empty(shape)
     for t in (c, out):
-        if t is not None and (t.dtype != a.dtype or tuple(t.shape) != shape or not t.is_contiguous() or not t.is_cuda):
-            raise ValueError("c / out must be contiguous device tensors of a's dtype and shape " + str(shape))
-    p = GemmParams()
-    p.dtype = CFK_FP16 if a.dtype == torch.float16 else CFK_FP32
-    p.layout = layout
-    p.m, p.n, p.k, p.batch = M, N, K, L
-    p.alpha, p.beta = float(alpha), float(beta)
-    p.a, p.b, p.d = a.data_ptr(), b.data_ptr(), out.data_ptr()
-    p.c = c.data_ptr() if c is not None else None
-    _check(lib().cfk_gemm(ctypes.byref(p), _stream_ptr(stream)))
+        if t is not None and (t.dtype != dt or t.shape != shape or not t.is_contiguous() or not t.is_cuda):
+            raise ValueError("c / out must be contiguous device tensors of a's dtype and shape " + str(tuple(shape)))
+    rc = launch(_GEMM_BLOCK.pack(CFK_FP16 if dt == _torch.float16 else CFK_FP32, layout, M, N, K, lead[0] if lead else 1, alpha, beta,
+                                 a.data_ptr(), b.data_ptr(), 0 if c is None else c.data_ptr(), out.data_ptr()), _stream_ptr(stream))
+    if rc != 0:
+        _check(rc)
     return out
