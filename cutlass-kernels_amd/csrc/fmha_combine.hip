@@ -27,7 +27,7 @@ __global__ void __launch_bounds__(kThreads) fmha_combine(const FmhaArgs a) {
 #pragma unroll 4
   for (int s = 0; s < a.n_split; ++s) {
     const f32x2 x = ml[s * rows + row];
-    const float w = __builtin_amdgcn_exp2f(x[0] - m_all);
+    const float w = x[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x[0] - m_all);   // (no finite score among the part's keys)
     const f32x4 *po = (const f32x4 *)(a.part_o + (s * rows + row) * D + d8 * 8);
     l_all += x[1] * w;
     o0 += po[0] * w;

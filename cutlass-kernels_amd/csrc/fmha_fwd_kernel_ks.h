@@ -7,7 +7,7 @@
 // tiles).  The chain per wave is then one eighth as long, and no barrier sits inside it.
 //
 // A query block's keys can further be split over a.n_split workgroups: each leaves its unnormalised fp32 O, reference point
-// and row sum in the caller's workspace, and fmha_combine (fmha_split.hip) merges them the same way.
+// and row sum in the caller's workspace, and fmha_combine (fmha_combine.hip) merges them the same way.
 //
 // What bounds it: with few workgroups the latency of that chain, with long key sequences the stream of K and V.  Both are
 // copied global -> LDS into tiles of the wave's own, 1 KB of whole rows per instruction: loading K fragments straight into
@@ -189,14 +189,17 @@ __global__ void __launch_bounds__(C::T) fmha_fwd_kernel_ks(const FmhaArgs a) {
     half8 pb[QB][PS];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
+      const float m_old = m_ref[qb];
       float mx = s_[0][qb][0];
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int t = 0; t < 4; ++t) mx = __builtin_fmaxf(mx, s_[kb][qb][t]);
-      const float m_new = fmaxf(m_ref[qb], quad_max(mx) * c_log2);
-      const float alpha = __builtin_amdgcn_exp2f(m_ref[qb] - m_new);
-      m_ref[qb] = m_new;
+      // (while all of a row's scores are -inf -- keys masked by an infinite K -- the point stays there and the weights, taken
+      // against 0, are 0: which keys a wave meets first is this kernel's choice, and -inf minus -inf would be NaN)
+      m_ref[qb] = fmaxf(m_old, quad_max(mx) * c_log2);
+      const float m_new = m_ref[qb] == -INFINITY ? 0.f : m_ref[qb];
+      const float alpha = __builtin_amdgcn_exp2f(m_old - m_new);
 #pragma unroll
       for (int db = 0; db < DB; ++db) oacc[db][qb] *= alpha;
       float rs = 0.f;
@@ -247,7 +250,6 @@ __global__ void __launch_bounds__(C::T) fmha_fwd_kernel_ks(const FmhaArgs a) {
   // ---- the partial results meet: wave u leaves O_u as fp32 rows (chunks of 4 XOR-swizzled by the row) and per query its
   // reference point m_u and row sum l_u; a wave without tiles leaves m = -inf, l = 0, O = 0
   __syncthreads();   // (the rows lie over other waves' tiles)
-  constexpr int O_CPR = D / 4;
   {
     char *op = smem + wave * (32 * D * 4);
 #pragma unroll

@@ -135,3 +135,20 @@ def test_workspace_streams_graphs_and_small_workspaces():
         torch.cuda.synchronize()
         assert max_abs(o.float().cpu().numpy(), want) <= tol
     assert pkg.lib().cfk_fmha_forward_ws(ctypes.byref(p), ws.data_ptr() + 4, need, stream) == -1
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv,D", [(1, 2, 64, 576, 64), (1, 2, 64, 576, 128), (1, 2, 64, 576, 256), (1, 1, 32, 8192, 128)])
+def test_masked_key_ranges(B, H, Sq, Skv, D):
+    """Keys taken out by a -inf in K (one element of Q positive throughout): whole tiles of a wave, and of a workgroup where
+    the keys are shared, have no finite score.  The first 64 keys stay: every other kernel starts from their row max."""
+    import torch
+    q, k, v = (x.astype(np.float16) for x in pkg.testbed.qkv(B, Sq, H, D, seqlen_kv=Skv))
+    q[..., 0] = 1.0
+    k[..., 0] = 0.0
+    keep = list(range(64)) + list(range(Skv - 128, Skv - 100))
+    masked = np.setdiff1d(np.arange(Skv), keep)
+    k[:, masked, :, 0] = -np.inf
+    o = pkg.fmha_forward(*(to_dev(x) for x in (q, k, v)))
+    torch.cuda.synchronize()
+    want = oracle.attention_f32(*(x.astype(np.float32) for x in (q, k[:, keep], v[:, keep])))["O"]
+    assert max_abs(o.float().cpu().numpy(), want) <= TOL_FP16
