@@ -78,7 +78,7 @@ int check_fmha(const cfk_fmha_fwd_params *p, cfk::FmhaPlan *plan, bool need_poin
 // their waves are spared outweigh the second launch and the merge, about 4 us plus 0.3 us for each partial result.  Measured
 // (fp16, head dim 128, two heads of 64 rows each: 8 workgroups), us at 1, 4, 8, 16, 32 splits: 4096 keys 22.5, 14.1, 14.4, 18.3,
 // 28.2; 16384 keys 100, 30.8, 23.6, 22.8, 30.7; 1024 keys 9.3, 10.8, 12.8.  64 workgroups, 16384 keys: 109.9 -> 51.0 at 4.
-int key_splits(const cfk_fmha_fwd_params *p, const cfk::FmhaPlan &plan) {
+int key_splits(const cfk::FmhaPlan &plan) {
   if (plan.split_tiles == 0) return 1;
   int best = 1;
   float best_us = 0.f;
@@ -89,8 +89,18 @@ int key_splits(const cfk_fmha_fwd_params *p, const cfk::FmhaPlan &plan) {
   }
   return best;
 }
+using cfk::KeySplit;
+int query_blocks(const cfk_fmha_fwd_params *p, int bm) { return p->batch * p->heads * ((p->seqlen_q + bm - 1) / bm); }
+
+KeySplit plan_key_split(const cfk_fmha_fwd_params *p, const cfk::FmhaPlan &plan) {
+  KeySplit k{key_splits(plan), 32, 0};
+  if (p->dtype == CFK_FP16 && !p->dbg_s) cfk::plan_fmha_f16_split(p->head_dim, p->seqlen_q, p->seqlen_kv, p->batch * p->heads, plan, &k);
+  return k;
+}
 // one partial result: fp32 O and a (reference point, row sum) pair per query row
-int64_t partial_bytes(const cfk_fmha_fwd_params *p) { return (int64_t)p->batch * p->heads * p->seqlen_q * (p->head_dim + 2) * 4; }
+int64_t partial_bytes(const cfk_fmha_fwd_params *p, const KeySplit &k) {
+  return (int64_t)(query_blocks(p, k.bm) - k.from) * k.bm * (p->head_dim + 2) * 4;
+}
 
 int check_device() {
   int dev = -1;
@@ -107,8 +117,8 @@ int check_device() {
   return CFK_OK;
 }
 
-// Launches a checked call; n_split > 1: with its keys shared by that many workgroups, through the workspace.
-int launch_fmha(const cfk_fmha_fwd_params *p, int n_split, void *workspace, void *stream) {
+// Launches a checked call; split.n > 1: with keys shared by that many units of work, through the workspace.
+int launch_fmha(const cfk_fmha_fwd_params *p, const KeySplit &split, void *workspace, void *stream) {
   const int rc = check_device();
   if (rc != CFK_OK) return rc;
   constexpr float kLog2e = 1.4426950408889634074f;  // fmha_forward.cu:452
@@ -125,10 +135,12 @@ int launch_fmha(const cfk_fmha_fwd_params *p, int n_split, void *workspace, void
   a.Sq = p->seqlen_q;
   a.Skv = p->seqlen_kv;
   a.v_layout = p->v_layout;
-  a.n_split = n_split;
-  if (n_split > 1) {
+  a.n_split = split.n;
+  a.split_bm = split.bm;
+  a.split_from = split.from;
+  if (split.n > 1) {
     a.part_o = (float *)workspace;
-    a.part_ml = a.part_o + (int64_t)n_split * p->batch * p->heads * p->seqlen_q * p->head_dim;
+    a.part_ml = a.part_o + (int64_t)split.n * (query_blocks(p, split.bm) - split.from) * split.bm * p->head_dim;
   }
   // Deferred rescale: O and l are only rescaled when a tile's max exceeds the max the reference point was set from by
   // more than tau (log2 domain).  fp16 P: 2^8 of head-room.  e4m3 P already sits 2^7 above the reference point, which
@@ -206,8 +218,8 @@ int cfk_fmha_forward_kernel(const cfk_fmha_fwd_params *params, char *name, int32
 int64_t cfk_fmha_forward_workspace(const cfk_fmha_fwd_params *p) {
   cfk::FmhaPlan plan{};
   if (check_fmha(p, &plan, false) != CFK_OK) return 0;
-  const int n = key_splits(p, plan);
-  return n > 1 ? (int64_t)n * partial_bytes(p) : 0;
+  const KeySplit k = plan_key_split(p, plan);
+  return k.n > 1 ? k.n * partial_bytes(p, k) : 0;
 }
 
 int cfk_fmha_forward(const cfk_fmha_fwd_params *p, void *stream) { return cfk_fmha_forward_ws(p, nullptr, 0, stream); }
@@ -216,18 +228,18 @@ int64_t cfk_fmha_forward_or_workspace(const cfk_fmha_fwd_params *p, void *stream
   cfk::FmhaPlan plan{};
   const int rc = check_fmha(p, &plan, true);
   if (rc != CFK_OK) return rc;
-  const int n = key_splits(p, plan);
-  return n > 1 ? (int64_t)n * partial_bytes(p) : launch_fmha(p, 1, nullptr, stream);
+  const KeySplit k = plan_key_split(p, plan);
+  return k.n > 1 ? k.n * partial_bytes(p, k) : launch_fmha(p, KeySplit{1, 0, 0}, nullptr, stream);
 }
 
 int cfk_fmha_forward_ws(const cfk_fmha_fwd_params *p, void *workspace, int64_t workspace_bytes, void *stream) {
   cfk::FmhaPlan plan{};
   const int rc = check_fmha(p, &plan, true);
   if (rc != CFK_OK) return rc;
-  const int n = workspace ? key_splits(p, plan) : 1;
-  const bool split = n > 1 && workspace_bytes >= n * partial_bytes(p);
+  const KeySplit k = workspace ? plan_key_split(p, plan) : KeySplit{1, 0, 0};
+  const bool split = k.n > 1 && workspace_bytes >= k.n * partial_bytes(p, k);
   if (split && (uintptr_t)workspace % 16 != 0) return fail(CFK_ERR_INVALID_ARG, "workspace must be 16-byte aligned");
-  return launch_fmha(p, split ? n : 1, workspace, stream);
+  return launch_fmha(p, split ? k : KeySplit{1, 0, 0}, workspace, stream);
 }
 
 int cfk_set_option(int32_t option, int32_t value) {

@@ -14,11 +14,15 @@ constexpr int kThreads = 256;
 
 template <int D>
 __global__ void __launch_bounds__(kThreads) fmha_combine(const FmhaArgs a) {
-  const int64_t rows = (int64_t)a.B * a.H * a.Sq;
+  const int q_blocks = (a.Sq + a.split_bm - 1) / a.split_bm;
+  const int64_t rows = (int64_t)(a.B * a.H * q_blocks - a.split_from) * a.split_bm;
   const int64_t e = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   const int64_t row = e / (D / 8);
   if (row >= rows) return;
   const int d8 = (int)(e % (D / 8));
+  const int block = (int)(row / a.split_bm), bh = (a.split_from + block) / q_blocks;
+  const int q = (a.split_from + block - bh * q_blocks) * a.split_bm + (int)(row - (int64_t)block * a.split_bm);
+  if (q >= a.Sq) return;   // (behind the last row of a partly filled block)
   const f32x2 *ml = (const f32x2 *)a.part_ml;
   float m_all = -INFINITY;
   for (int s = 0; s < a.n_split; ++s) m_all = fmaxf(m_all, ml[s * rows + row][0]);
@@ -37,18 +41,20 @@ __global__ void __launch_bounds__(kThreads) fmha_combine(const FmhaArgs a) {
   half8 o8;
 #pragma unroll
   for (int t = 0; t < 4; ++t) o8[t] = (_Float16)(o0[t] * inv), o8[4 + t] = (_Float16)(o1[t] * inv);
-  const int64_t bh = row / a.Sq, q = row - bh * a.Sq, b = bh / a.H, h = bh - b * a.H;
-  *(half8 *)((_Float16 *)a.o + ((b * a.Sq + q) * a.H + h) * D + d8 * 8) = o8;
+  const int b = bh / a.H, h = bh - b * a.H;
+  *(half8 *)((_Float16 *)a.o + (((int64_t)b * a.Sq + q) * a.H + h) * D + d8 * 8) = o8;
   if (d8 == 0) {   // (the parts' reference points are the row maxima of their keys)
-    if (a.row_max) a.row_max[row] = m_all;
-    if (a.row_sum) a.row_sum[row] = l_all;
+    const int64_t si = (int64_t)bh * a.Sq + q;
+    if (a.row_max) a.row_max[si] = m_all;
+    if (a.row_sum) a.row_sum[si] = l_all;
   }
 }
 
 }  // namespace
 
 hipError_t launch_fmha_combine(const FmhaArgs &a, int head_dim, hipStream_t s) {
-  const int64_t threads = (int64_t)a.B * a.H * a.Sq * (head_dim / 8);
+  const int blocks = a.B * a.H * ((a.Sq + a.split_bm - 1) / a.split_bm) - a.split_from;
+  const int64_t threads = (int64_t)blocks * a.split_bm * (head_dim / 8);
   const dim3 grid((unsigned)((threads + kThreads - 1) / kThreads)), block(kThreads);
   switch (head_dim) {
     case 64: hipLaunchKernelGGL(fmha_combine<64>, grid, block, 0, s, a); break;

@@ -22,9 +22,11 @@ struct FmhaArgs {
   int32_t v_layout;  // 0 = [B,S,H,D], 1 = [B,D,H,S]
   float tau;         // the softmax reference point moves when a tile's max exceeds it by more than this (log2 domain)
   int32_t track_only;  // no optimistic first pass over the keys (cfk_set_option(CFK_OPT_PREDICTABLE_LATENCY, 1))
-  int32_t n_split;     // workgroups that share a query block's keys (key-split kernel; 1: no workspace is touched)
-  float *part_o;       // their partial results, n_split of each: O [B,H,Sq,D] not divided by the row sum, and (reference point,
-  float *part_ml;      // row sum) pairs [B,H,Sq,2]
+  int32_t n_split;     // units of work that share a query block's keys (1: no workspace is touched) ...
+  int32_t split_bm;    // ... of so many rows; 32: the key-split kernel, else a SplitCfg build
+  int32_t split_from;  // ... from this query block on, in the order [B,H,query block]
+  float *part_o;       // their partial results [n_split][query blocks from split_from on][split_bm]: O not divided by the row sum,
+  float *part_ml;      // and (reference point, row sum) pairs
   int32_t direct_p;    // first pass with e4m3 P: codes without an exponential (cfk_set_option(CFK_OPT_FAST_E4M3_WEIGHTS, 1))
 };
 
@@ -41,9 +43,17 @@ struct FmhaPlan {
   int32_t split_waves;  // ... those waves, and the time of a turn
   float split_turn_us;
   int32_t mfma;  // 32: 32x32 MFMA build, 16: 16x16x32 build
+  bool hand;     // a build with a hand-scheduled main loop
   bool want_name;   // set by a caller that wants the next field
   char kernel[80];  // the instantiation, as profilers print it without namespaces: fmha_fwd_kernel16p<128,64,8,2,0,0,0,0,2,0,1,1>
 };
+
+// How a call with a workspace shares keys out: the query blocks of bm rows from block `from` on are n units of work each.
+struct KeySplit {
+  int n, bm, from;   // n = 1: no block is cut
+};
+// For a fp16 call that would launch `plan`: whether cutting query blocks of a hand-scheduled build pays, and how.
+bool plan_fmha_f16_split(int head_dim, int sq, int skv, int bh, const FmhaPlan &plan, KeySplit *out);
 
 // Each launcher validates nothing: the C-ABI layer has already checked shapes against the plan.
 // `tap_s` (plan) / a.s_tap (launch) selects the build of the kernel that also writes the score tap.

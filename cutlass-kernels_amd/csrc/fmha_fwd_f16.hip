@@ -6,6 +6,8 @@
 namespace cfk {
 namespace {
 
+constexpr int kCus = 256;
+
 // <head dim, keys per tile, waves, waves per SIMD, e4m3 Q/K, e4m3 P/V, V transposed, score tap, tiles per barrier,
 //  K fragments read ahead of the barrier, 16x16x32 build>.  4 waves = 128 query rows (two workgroups share a CU),
 // 8 waves = 256 rows (one workgroup per CU, half the K/V traffic per query row).  Two waves per SIMD, except head dim
@@ -74,15 +76,61 @@ bool plan_fmha_f16(int head_dim, int sq, int skv, int bh, bool tap_s, FmhaPlan *
 
 hipError_t launch_fmha_f16(const FmhaArgs &a, int head_dim, hipStream_t s) {
   if (head_dim == 256 && !a.s_tap) return launch_fmha_f16_d256(a, s);
+  if (a.n_split > 1 && a.split_bm == 256) return head_dim == 64 ? launch_fmha_split<A64_256x128>(a, s) : launch_fmha_split<A128_256x128>(a, s);
+  if (a.n_split > 1 && a.split_bm == 128) return head_dim == 64 ? launch_fmha_split<A64_128x128>(a, s) : launch_fmha_split<A128_128x128>(a, s);
   hipError_t e = hipErrorInvalidValue;
   dispatch(head_dim, a.Sq, a.Skv, a.B * a.H, a.s_tap != nullptr, [&](auto cfg) { e = launch_fmha_cfg<decltype(cfg)>(a, s); });
   return e;
+}
+
+// The hand-scheduled builds run one workgroup per CU in rounds of 256 units of work.  The whole rounds take items as they are; the
+// items left over -- all of them, where there are fewer than CUs -- are cut into n units along the keys, at least two groups
+// of four key tiles each, as many as still make one round.  n, and the rows per item, are what the times below add up to least
+// for; the call is cut if that is less than its time otherwise by a twentieth.  Times, us, by head dim: a key tile of a unit while
+// all CUs work and while at most half do (the clock is higher then), a unit's start and end, tiles behind the last group of four
+// as two and a half, the merge 5 and 4 TB/s for the partial results.  Measured, N(0,1), us before -> after: D=128, 36 heads of 256
+// rows, 10176 keys 127.6 -> 65.5 (3 units); 16 heads of 1024 rows, 8192 keys 99.2 -> 71.0; 20 heads of 6528 rows, 6144 keys (520
+// items of 256 rows) 399 -> 334; D=64, 16 heads of 4512 rows, 6976 keys 174.0 -> 132.4; 160 heads of 1216 rows, 4864 keys 259 -> 234;
+// D=256, 36 heads of 256 rows, 8192 keys 225.8 -> 114.4; 15 heads of 2976 rows, 4096 keys 202.1 -> 181.7.  No gain, and the rule
+// keeps off: 256 items of 128 rows, D=128, 4096 keys 64.0 / 70.5.
+// (Only calls that run a hand-scheduled build anyway: its Q is rounded once more, rms error of O 3.6e-4 of its size against
+// 2.9e-4 of the compiler-scheduled builds.)
+bool plan_fmha_f16_split(int head_dim, int sq, int skv, int bh, const FmhaPlan &plan, KeySplit *out) {
+  const TileWish w = tile_wish();
+  const int bn = head_dim == 256 ? 32 : 64, tiles = skv / bn, groups = tiles / 4, left = tiles % 4;
+  if (!plan.hand || w.bm || w.bn || groups < 4) return false;
+  struct Build { int bm; float full, low, fixed; };
+  const Build b256 = head_dim == 64 ? Build{256, 0.885f, 0.62f, 3.f} : Build{256, 1.66f, 1.05f, 5.f};
+  const Build b128 = head_dim == 64 ? Build{128, 0.48f, 0.45f, 4.f} : head_dim == 128 ? Build{128, 0.95f, 0.74f, 4.f} : Build{128, 0.884f, 0.67f, 4.f};
+  const auto round_us = [&](const Build &b, int units, int loop_tiles, int tail) {
+    const float busy = 2.f * units / kCus - 1.f, tile = b.low + (b.full - b.low) * (busy > 0.f ? busy : 0.f);
+    return units ? b.fixed + (loop_tiles + 2.5f * tail) * tile : 0.f;
+  };
+  const auto rounds_us = [&](const Build &b, int items) {
+    return items / kCus * round_us(b, kCus, 4 * groups, left) + round_us(b, items % kCus, 4 * groups, left);
+  };
+  float best_us = 0.95f * rounds_us(plan.block_m == 256 ? b256 : b128, plan.grid);
+  bool found = false;
+  for (const Build &b : {b256, b128}) {
+    if (head_dim == 256 && b.bm == 256) continue;
+    const int items = bh * ((sq + b.bm - 1) / b.bm), from = items / kCus * kCus, cut = items - from;
+    const float whole_us = rounds_us(b, from);
+    for (int n = 2; n * cut <= kCus && 2 * n <= groups && cut; ++n) {
+      const float merge_us = 5.f + (float)n * cut * b.bm * head_dim * 4.f / 4e6f;
+      const float us = whole_us + round_us(b, n * cut, 4 * ((groups + n - 1) / n), left) + merge_us;
+      if (us < best_us) best_us = us, *out = KeySplit{n, b.bm, from}, found = true;
+    }
+  }
+  return found;
 }
 
 hipError_t prepare_fmha_f16() {
   hipError_t e = prepare_all(All64{});
   if (e == hipSuccess) e = prepare_all(All128{});
   if (e == hipSuccess) e = prepare_fmha_f16_d256();
+  const hipError_t split[] = {prepare_fmha_split<A64_256x128>(), prepare_fmha_split<A64_128x128>(), prepare_fmha_split<A128_256x128>(), prepare_fmha_split<A128_128x128>()};
+  for (hipError_t x : split)
+    if (e == hipSuccess) e = x;
   if (e == hipSuccess) e = prepare_all(CfgList<C64Tap, C128Tap, C256Tap>{});
   return e;
 }

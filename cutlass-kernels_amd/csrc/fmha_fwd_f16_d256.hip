@@ -38,12 +38,16 @@ void plan_fmha_f16_d256(int sq, int skv, int bh, FmhaPlan *p) {
 }
 
 hipError_t launch_fmha_f16_d256(const FmhaArgs &a, hipStream_t s) {
+  if (a.n_split > 1 && a.split_bm == 128) return launch_fmha_split<A256_128x64>(a, s);
   hipError_t e = hipErrorInvalidValue;
   dispatch(a.Sq, a.Skv, a.B * a.H, [&](auto cfg) { e = launch_fmha_cfg<decltype(cfg)>(a, s); });
   return e;
 }
 
-hipError_t prepare_fmha_f16_d256() { const hipError_t e = prepare_all(All256{});
-  return e != hipSuccess ? e : prepare_all(CfgList<K256_32x32>{}); }
+hipError_t prepare_fmha_f16_d256() {
+  hipError_t e = prepare_all(All256{});
+  if (e == hipSuccess) e = prepare_all(CfgList<K256_32x32>{});
+  return e != hipSuccess ? e : prepare_fmha_split<A256_128x64>();
+}
 
 }  // namespace cfk

@@ -92,6 +92,7 @@ struct FmhaCfg {
   static constexpr int WPE = WPE_;                              // waves per SIMD the register budget is sized for
   static constexpr bool QK8 = QK8_, PV8 = PV8_;                 // e4m3 (true) or fp16 (false) operands of GEMM-I / II
   static constexpr bool DIRECT = false;                         // (DirectCfg below)
+  static constexpr bool SPLIT = false;                          // (SplitCfg below)
   static constexpr bool VT = VT_;                               // V given pre-transposed, [B,D,H,S] (e4m3 only)
   static constexpr bool TAP_S = TAP_S_;                         // also write the pre-softmax scores (debug build)
   static constexpr int T = NWAVES * 64;
@@ -770,6 +771,11 @@ template <class C>
 struct DirectCfg : C {
   static constexpr bool DIRECT = true;
 };
+// The hand-scheduled persistent build with the keys of some items cut into units of work of their own (FmhaArgs::n_split).
+template <class C>
+struct SplitCfg : C {
+  static constexpr bool SPLIT = true;
+};
 template <class C>
 constexpr bool has_direct_build = C::PV8 && C::D <= 128 && !C::TAP_S && !C::KSPLIT;
 
@@ -831,6 +837,26 @@ hipError_t launch_fmha_cfg(const FmhaArgs &a, hipStream_t s) {
 }
 
 template <class C>
+hipError_t prepare_fmha_split() {
+  static std::once_flag once;
+  static hipError_t status = hipSuccess;
+  std::call_once(once, [] {
+    status = hipFuncSetAttribute((const void *)fmha_kernel_of<SplitCfg<C>>(), hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES);
+  });
+  return status;
+}
+
+// a call with a.split_from whole items and a.n_split units of each further one
+template <class C>
+hipError_t launch_fmha_split(const FmhaArgs &a, hipStream_t s) {
+  const hipError_t e = prepare_fmha_split<C>();
+  if (e != hipSuccess) return e;
+  const int items = a.B * a.H * ((a.Sq + C::BM - 1) / C::BM), units = a.split_from + (items - a.split_from) * a.n_split;
+  hipLaunchKernelGGL(fmha_kernel_of<SplitCfg<C>>(), dim3(persistent_grid(units)), dim3(C::T), C::LDS_BYTES, s, a);
+  return hipGetLastError();
+}
+
+template <class C>
 void fill_fmha_plan(int sq, int skv, int bh, FmhaPlan *p) {
   p->block_m = C::BM;
   p->block_n = C::BN * C::SUB;
@@ -841,6 +867,7 @@ void fill_fmha_plan(int sq, int skv, int bh, FmhaPlan *p) {
   p->threads = C::T;
   p->grid = bh * ((sq + C::BM - 1) / C::BM);
   p->split_tiles = p->split_waves = 0;
+  p->hand = C::ASM;
   if constexpr (C::KSPLIT) {
     p->split_tiles = skv / C::TK;
     p->split_waves = C::NWAVES;

@@ -256,8 +256,11 @@ def fmha_forward(q, k, v, o=None, softmax_scale=None, q_descale=1.0, k_descale=1
         return PreparedForward(FmhaFwdParams.from_buffer_copy(block), (q, k, v, o, row_max, row_sum, scores), stream)
     rc = launch(block, _stream_ptr(stream))
     if rc > 0:   # the call is not made yet: it can use this much scratch memory
-        ws = _workspace(rc, q.device, stream)
-        rc = launch_ws(block, ws.data_ptr(), rc, _stream_ptr(stream))
+        try:
+            ws = _workspace(rc, q.device, stream)
+        except _torch.OutOfMemoryError:   # no room: the call without it
+            ws, rc = None, 0
+        rc = launch_ws(block, 0 if ws is None else ws.data_ptr(), rc, _stream_ptr(stream))
     if rc != 0:
         _check(rc)
     return o

@@ -94,8 +94,8 @@ typedef struct cfk_fmha_fwd_params {
  * Replaces fmhaForwardDevice (src/fmha-pipeline/fmha_forward.cu:86-383), one launch per call. */
 int cfk_fmha_forward(const cfk_fmha_fwd_params *params, void *stream);
 
-/* The same call with scratch memory: where a problem has too few query blocks to go round the compute units, its keys are
- * split over several workgroups, whose partial results (fp32 O, reference point and row sum per query row) meet in
+/* The same call with scratch memory: where a problem has too few query blocks to go round the compute units, or its last
+ * round leaves most of them idle, the keys of those blocks are split over several workgroups, whose partial results (fp32 O, reference point and row sum per query row) meet in
  * `workspace` -- device memory of at least cfk_fmha_forward_workspace(params) bytes, 16-byte aligned, that nothing else uses
  * until the call has run on `stream`; its content does not matter before and after.  With workspace = NULL, or one that is
  * too small, this is cfk_fmha_forward.  Two launches per call where the keys are split.  No counterpart in the reference,

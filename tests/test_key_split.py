@@ -152,3 +152,47 @@ def test_masked_key_ranges(B, H, Sq, Skv, D):
     torch.cuda.synchronize()
     want = oracle.attention_f32(*(x.astype(np.float32) for x in (q, k[:, keep], v[:, keep])))["O"]
     assert max_abs(o.float().cpu().numpy(), want) <= TOL_FP16
+
+
+@pytest.mark.parametrize("D,B,H,Sq,Skv", [
+    (128, 1, 16, 1024, 8192),   # fewer blocks than CUs: every block cut
+    (128, 1, 9, 1312, 8320),    # ... the last one partly filled, key tiles behind the last group of four
+    (128, 2, 65, 512, 3328),    # one whole round, 4 further blocks cut
+    (64, 2, 8, 1024, 8192),
+    (64, 1, 33, 2016, 4160),
+    (256, 2, 8, 1024, 4096),
+    (256, 1, 37, 928, 2048),
+])
+@pytest.mark.parametrize("keys", ["plain", "climbing", "masked"])
+def test_cut_query_blocks_of_the_hand_scheduled_builds(D, B, H, Sq, Skv, keys):
+    import torch
+    q, k, v = pkg.testbed.qkv(B, Sq, H, D, seqlen_kv=Skv, seed=7)
+    if keys == "climbing":      # weights beyond the fp16 range: the loop that follows the running max
+        k, v = climbing_keys(k, ramp=4.0, spike=4.0), v / 4
+    q, k, v = (x.astype(np.float16) for x in (q, k, v))
+    if keys == "masked":        # whole units without a finite score
+        q[..., 0], k[..., 0] = 1.0, 0.0
+        k[:, 64:Skv - 96, :, 0] = -np.inf
+    dev = [to_dev(x) for x in (q, k, v)]
+    assert "16p<" in f.fmha_forward_kernel(f.CFK_FP16, B, H, Sq, Skv, D)
+    call = pkg.fmha_forward(*dev, prepare=True)
+    assert call._ws_bytes > 0, "query blocks of this problem are meant to be cut"
+    o = pkg.fmha_forward(*dev)
+    whole = torch.empty_like(o)
+    p = f.make_params(f.CFK_FP16, B, H, Sq, Skv, D, *(t.data_ptr() for t in dev), whole.data_ptr())
+    assert pkg.lib().cfk_fmha_forward(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    row_max, row_sum = (torch.zeros((B, H, Sq), dtype=torch.float32, device="cuda:0") for _ in range(2))
+    tapped = pkg.fmha_forward(*dev, row_max=row_max, row_sum=row_sum)
+    torch.cuda.synchronize()
+    # both are within the gate of the exact result
+    assert max_abs(o.float().cpu().numpy(), whole.float().cpu().numpy()) <= 2 * TOL_FP16
+    for b, h in {(0, 0), (B - 1, H - 1)}:
+        qf, kf, vf = (x[b:b + 1, :, h:h + 1].astype(np.float32) for x in (q, k, v))
+        if keys == "masked":
+            kf, vf = (np.concatenate([x[:, :64], x[:, Skv - 96:]], 1) for x in (kf, vf))
+        want = oracle.attention_f32(qf, kf, vf)["O"]
+        for got in (o, tapped):
+            assert max_abs(got[b:b + 1, :, h:h + 1].float().cpu().numpy(), want) <= TOL_FP16, (b, h)
+        s = (qf[0, :, 0] @ kf[0, :, 0].T) * (np.log2(np.e) / np.sqrt(D))
+        np.testing.assert_allclose(row_max[b, h].cpu().numpy(), s.max(-1), rtol=1e-4, atol=1e-3)
+        np.testing.assert_allclose(row_sum[b, h].cpu().numpy(), np.exp2(s - s.max(-1, keepdims=True)).sum(-1), rtol=2e-3)

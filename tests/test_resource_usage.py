@@ -89,6 +89,13 @@ def test_auto_picked_kernels_stay_within_their_spill_allowance(kernels):
     assert k["occupancy"] == 2 and k["vgprs"] + k["agprs"] <= 256 and k["scratch"] == 0
 
 
+def test_split_builds_stay_within_their_spill_allowance(kernels):
+    # (which unit of which item it is, kept across the loop for the epilogue: once per unit)
+    for name, allowed in {"128,64,8,2": 2, "128,64,4,1": 0, "64,64,8,2": 0, "64,64,4,1": 0, "256,32,4,1": 22}.items():
+        k = kernels["fmha_fwd_kernel16p<%s,0,0,0,0,2,0,1,1>/split" % name]
+        assert k["vgpr_spill"] <= allowed, (name, k)
+
+
 def test_no_kernel_spills_more_than_the_table_says(kernels):
     # every kernel, picked automatically or only through CFK_FMHA_TILE: the committed table is the ceiling
     table = open(os.path.join(ROOT, "profiles", "kernel_resource_usage.md")).read()
