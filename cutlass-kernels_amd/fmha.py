@@ -62,6 +62,15 @@ class GemmParams(ctypes.Structure):
 # The same two blocks for the launch path: packing bytes takes a fraction of the time of filling a ctypes structure.
 _FMHA_BLOCK = struct.Struct("=8i4Q4f3Q")
 _GEMM_BLOCK = struct.Struct("=6i2f4Q")
+
+
+def _pack(block, *args):
+    try:
+        return block.pack(*args)
+    except OverflowError:   # a factor beyond float32: infinite there, as the field of a ctypes structure makes it
+        return block.pack(*(ctypes.c_float(x).value if isinstance(x, float) else x for x in args))
+
+
 assert _FMHA_BLOCK.size == ctypes.sizeof(FmhaFwdParams) and _GEMM_BLOCK.size == ctypes.sizeof(GemmParams)
 
 
@@ -250,7 +259,7 @@ def fmha_forward(q, k, v, o=None, softmax_scale=None, q_descale=1.0, k_descale=1
                                or not scores.is_contiguous()):
         raise ValueError("scores must be contiguous float32 [B,H,Sq,Skv]")
     scale = 1.0 / math.sqrt(D) if softmax_scale is None else softmax_scale
-    block = _FMHA_BLOCK.pack(dtype, v_dtype, B, H, Sq, Skv, D, v_layout, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+    block = _pack(_FMHA_BLOCK, dtype, v_dtype, B, H, Sq, Skv, D, v_layout, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                              scale, q_descale, k_descale, v_descale, *(0 if t is None else t.data_ptr() for t in (scores, row_max, row_sum)))
     if prepare:
         return PreparedForward(FmhaFwdParams.from_buffer_copy(block), (q, k, v, o, row_max, row_sum, scores), stream)
@@ -343,7 +352,7 @@ def gemm(a, b, c=None, alpha=1.0, beta=0.0, out=None, layout=CFK_GEMM_TN, stream
     for t in (c, out):
         if t is not None and (t.dtype != dt or t.shape != shape or not t.is_contiguous() or not t.is_cuda):
             raise ValueError("c / out must be contiguous device tensors of a's dtype and shape " + str(tuple(shape)))
-    rc = launch(_GEMM_BLOCK.pack(CFK_FP16 if dt == _torch.float16 else CFK_FP32, layout, M, N, K, lead[0] if lead else 1, alpha, beta,
+    rc = launch(_pack(_GEMM_BLOCK, CFK_FP16 if dt == _torch.float16 else CFK_FP32, layout, M, N, K, lead[0] if lead else 1, alpha, beta,
                                  a.data_ptr(), b.data_ptr(), 0 if c is None else c.data_ptr(), out.data_ptr()), _stream_ptr(stream))
     if rc != 0:
         _check(rc)
