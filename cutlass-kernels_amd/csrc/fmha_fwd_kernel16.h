@@ -1,4 +1,4 @@
-// The fp16 FMHA forward kernel on 16x16x32 MFMAs (v_mfma_f32_16x16x32_f16).  Same algorithm, LDS staging, pipeline
+// The FMHA forward kernel on 16x16 MFMAs (v_mfma_f32_16x16x32_f16) for fp16 P and V, with fp16 or e4m3 Q and K.  Same algorithm, LDS staging, pipeline
 // (one or two key tiles per barrier) and epilogue as fmha_fwd_kernel.h, which it takes its configuration struct and
 // host-side plumbing from; what differs is the MFMA shape, with it every register layout, and how the softmax notices
 // that its reference point has to move: not by a row max per tile but by the row sum it needs anyway (softmax_tile
@@ -47,11 +47,13 @@ __device__ __forceinline__ int swz_v16n(int row) {
 template <class C>
 __global__ void __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
 fmha_fwd_kernel16(const FmhaArgs a) {
-  static_assert(!C::QK8 && !C::PV8 && !C::VT && !C::TAP_S, "fp16 operands only, no score tap");
+  static_assert(!C::PV8 && !C::VT && !C::TAP_S, "fp16 P and V, no score tap");
   constexpr int D = C::D, BN = C::BN;
+  constexpr bool QK8 = C::QK8;
+  constexpr int QES = QK8 ? 1 : 2;
   constexpr int QB = 2;        // 16-query blocks per wave
   constexpr int KB = BN / 16;  // 16-key blocks per tile (M blocks of S^T)
-  constexpr int KS = D / 32;   // K-steps of S^T
+  constexpr int KF = D * QES / 64;  // 16-byte fragments of a K row per lane (fp16: one K-step of S^T each)
   constexpr int DB = D / 16;   // 16-row blocks of O^T
   constexpr int PS = BN / 32;  // K-steps of O^T
   const float kTau = a.tau;    // deferred-rescale threshold above the running max (log2 domain)
@@ -62,29 +64,32 @@ fmha_fwd_kernel16(const FmhaArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
 
-  const int q_blocks = a.Sq / C::BM;
+  const int q_blocks = (a.Sq + C::BM - 1) / C::BM;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   const int bh = tile / q_blocks;
   const int qblk = tile - bh * q_blocks;
   const int b = bh / a.H, h = bh - b * a.H;
   const int64_t ld = (int64_t)a.H * D;  // row stride in elements
-  const char *Qp = (const char *)a.q + (((int64_t)b * a.Sq * a.H + h) * D) * 2;
-  const char *Kp = (const char *)a.k + (((int64_t)b * a.Skv * a.H + h) * D) * 2;
+  const char *Qp = (const char *)a.q + (((int64_t)b * a.Sq * a.H + h) * D) * QES;
+  const char *Kp = (const char *)a.k + (((int64_t)b * a.Skv * a.H + h) * D) * QES;
   const char *Vp = (const char *)a.v + (((int64_t)b * a.Skv * a.H + h) * D) * 2;
   _Float16 *Op = (_Float16 *)a.o + ((int64_t)b * a.Sq * a.H + h) * D;
-  const int q0 = qblk * C::BM + wave * 32;
+  // (waves behind the last query row of a partly filled tile copy and meet the barriers like the others, compute the last
+  // rows a second time and store nothing)
+  const int q0 = qblk * C::BM + wave * 32, q0_in = q0 < a.Sq ? q0 : a.Sq - 32;
   const int n_tiles = a.Skv / BN;
   const float c_log2 = a.scale_log2;
-  const uint32_t k_ld = (uint32_t)(ld * 2), v_ld = k_ld;  // global row pitch in bytes
+  const uint32_t k_ld = (uint32_t)(ld * QES), v_ld = (uint32_t)(ld * 2);  // global row pitch in bytes
 
   // ---- global -> LDS copies, as in fmha_fwd_kernel.h: copy i of wave w covers tile rows (i*NWAVES + w)*RPI .. +RPI;
   // lane l writes LDS slot (row l / CPR, chunk position l % CPR) and fetches chunk position ^ swz(row) of that row.
+  auto swz_k = [](int row) { return QK8 ? swz_row<C::K_PITCH>(row) : swz_k16n<C::K_PITCH>(row); };
   uint32_t goff_k[C::K_IPW], goff_v[C::V_IPW];
 #pragma unroll
   for (int i = 0; i < C::K_IPW; ++i) {
     constexpr int CPR = C::K_PITCH / 16;
     const int row = (i * C::NWAVES + wave) * C::K_RPI + lane / CPR;
-    goff_k[i] = (uint32_t)row * k_ld + (uint32_t)(((lane % CPR) ^ swz_k16n<C::K_PITCH>(row)) * 16);
+    goff_k[i] = (uint32_t)row * k_ld + (uint32_t)(((lane % CPR) ^ swz_k(row)) * 16);
   }
 #pragma unroll
   for (int i = 0; i < C::V_IPW; ++i) {
@@ -107,18 +112,19 @@ fmha_fwd_kernel16(const FmhaArgs a) {
       lds_dma16(gt, goff_v[i], lds_wave, C::V_ST0 + stage * C::V_TILE + i * C::NWAVES * 1024);
   };
 
-  // ---- Q: B operand of S^T, resident in VGPRs: lane (c, g), query block qb, K-step s holds Q[q0+16qb+c][32s+8g .. +8)
-  half8 qreg[QB][KS];
+  // ---- Q: B operand of S^T, resident in VGPRs: lane (c, g), query block qb, fragment f holds the 16 bytes 64f+16g of row
+  // q0+16qb+c (fp16: d = 32f+8g .. +8)
+  int4v qreg[QB][KF];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qreg[qb][s] = *(const half8 *)(Qp + ((int64_t)(q0 + 16 * qb + c) * ld + 32 * s + 8 * g) * 2);
+    for (int f = 0; f < KF; ++f) qreg[qb][f] = *(const int4v *)(Qp + (int64_t)(q0_in + 16 * qb + c) * k_ld + 64 * f + 16 * g);
 
   // ---- per-lane LDS read addresses (absolute LDS byte addresses of slot 0; slots and blocks are immediates: the
   // swizzles only depend on the row within its 16- or 8-row group)
-  uint32_t k_rd[KS];  // K operand, K-step s: row c (+16 kb), chunk 4s+g
+  uint32_t k_rd[KF];  // K operand, fragment f: row c (+16 kb), chunk 4f+g
 #pragma unroll
-  for (int s = 0; s < KS; ++s) k_rd[s] = lds_base + C::K_ST0 + c * C::K_PITCH + (((4 * s + g) ^ swz_k16n<C::K_PITCH>(c)) * 16);
+  for (int f = 0; f < KF; ++f) k_rd[f] = lds_base + C::K_ST0 + c * C::K_PITCH + (((4 * f + g) ^ swz_k(c)) * 16);
   // V operand: within its block of 16 lanes, lane L hands the transpose read the address of (key L/4, columns
   // 4(L%4) .. +3) and receives keys 0..3 of column L; the block g reads keys 4g .. 4g+3 (+16 for the second read)
   uint32_t v_rd[DB];
@@ -150,18 +156,49 @@ fmha_fwd_kernel16(const FmhaArgs a) {
   const float sum_cap = __builtin_amdgcn_exp2f(kTau);
   const bool want_taps = a.row_max != nullptr || a.row_sum != nullptr;
   const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-  // S^T = K . Q^T for the K tile in LDS slot `stage`
+  // S^T = K . Q^T, with frag(f, kb) = fragment f of 16-key block kb.  e4m3: two fragments are one 128-deep multiply
+  // (v_mfma_f32_16x16x128_f8f6f4, twice the rate of fp16; which slot means which d is free as long as K and Q agree);
+  // head dim 64, half as deep, takes the 32-deep form at the fp16 rate
+  auto multiply_qk = [&](auto frag, f32x4 (&sacc)[KB][QB]) __attribute__((always_inline)) {
+    if constexpr (QK8 && KF >= 2) {
+#pragma unroll
+      for (int f = 0; f < KF; f += 2)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          const int4v lo = frag(f, kb), hi = frag(f + 1, kb);
+          const int8v ka = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb) {
+            const int4v ql = qreg[qb][f], qh = qreg[qb][f + 1];
+            const int8v qv = {ql[0], ql[1], ql[2], ql[3], qh[0], qh[1], qh[2], qh[3]};
+            sacc[kb][qb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ka, qv, f == 0 ? zero4 : sacc[kb][qb], 0, 0, 0, 0, 0, 0);
+          }
+        }
+    } else {
+#pragma unroll
+      for (int f = 0; f < KF; ++f)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          const int4v ka = frag(f, kb);
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb) {
+            f32x4 acc = f == 0 ? zero4 : sacc[kb][qb];
+            if constexpr (QK8) {
+              auto as_long = [](int lo, int hi) { return (long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo); };
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(as_long(ka[0], ka[1]), as_long(qreg[qb][f][0], qreg[qb][f][1]), acc, 0, 0, 0);
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(as_long(ka[2], ka[3]), as_long(qreg[qb][f][2], qreg[qb][f][3]), acc, 0, 0, 0);
+            } else {
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, ka), __builtin_bit_cast(half8, qreg[qb][f]), acc, 0, 0, 0);
+            }
+            sacc[kb][qb] = acc;
+          }
+        }
+    }
+  };
+  // ... for the K tile in LDS slot `stage`
   auto qk = [&](int stage, f32x4 (&sacc)[KB][QB]) __attribute__((always_inline)) {
     const uint32_t kt = stage * C::K_TILE;
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const half8 ka = *LDS_AT(half8, kt + k_rd[s] + kb * 16 * C::K_PITCH);
-#pragma unroll
-        for (int qb = 0; qb < QB; ++qb)
-          sacc[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qreg[qb][s], s == 0 ? zero4 : sacc[kb][qb], 0, 0, 0);
-      }
+    multiply_qk([&](int f, int kb) __attribute__((always_inline)) { return *LDS_AT(int4v, kt + k_rd[f] + kb * 16 * C::K_PITCH); }, sacc);
   };
   // this lane's max over its quarter of the keys of query block qb: a chain of three-operand maxima
   auto lane_max = [&](const f32x4 (&sacc)[KB][QB], int qb) __attribute__((always_inline)) -> float {
@@ -232,16 +269,15 @@ fmha_fwd_kernel16(const FmhaArgs a) {
       // occupy ten registers for all of the kernel)
       int cc = c, gg = g;
       asm volatile("" : "+v"(cc), "+v"(gg));
-      const char *kt = Kp + (size_t)jt * ((size_t)BN * k_ld) + (size_t)cc * k_ld + 16 * gg;
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          const half8 ka = *(const half8 *)(kt + (size_t)(16 * kb) * k_ld + 64 * s);
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb)
-            sr[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qreg[qb][s], s == 0 ? zero4 : sr[kb][qb], 0, 0, 0);
-        }
+      const char *kt = Kp + (size_t)jt * ((size_t)BN * k_ld);
+      const uint32_t lane_off = (uint32_t)cc * k_ld + 16 * gg;
+      // (which half of the address holds the block's rows is a matter of spilled registers: 13 against 20 in the 256-row build with
+      // one key tile per barrier, while scalar ones spill in the other builds)
+      constexpr bool SCALAR_ROWS = C::NWAVES == 8 && C::SUB == 1;
+      multiply_qk([&](int f, int kb) __attribute__((always_inline)) {
+        return SCALAR_ROWS ? *(const int4v *)(kt + (size_t)(16 * kb) * k_ld + 64 * f + lane_off)
+                           : *(const int4v *)(kt + (lane_off + (uint32_t)(16 * kb) * k_ld + 64 * f));
+      }, sr);
       rebase(sr);
       exp_and_sum(sr, pb, rsum);
     }
@@ -387,10 +423,10 @@ fmha_fwd_kernel16(const FmhaArgs a) {
     for (int pass = 0; pass < 32 / RPP; ++pass) {
       const int row = pass * RPP + orow_l;
       const int4v val = *(const int4v *)(ot + row * C::O_PITCH + ochunk * 16);
-      *(int4v *)(Op + (int64_t)(q0 + row) * ld + ochunk * 8) = val;
+      if (q0 < a.Sq) *(int4v *)(Op + (int64_t)(q0 + row) * ld + ochunk * 8) = val;
     }
   }
-  if (want_taps) {
+  if (q0 < a.Sq && want_taps) {
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       float m_true = fmaxf(m_lane[qb], __shfl_xor(m_lane[qb], 16, 64));
