@@ -32,6 +32,10 @@ using K128T = KsCfg8<128, 8, true, true>;
 using K256T = KsCfg8<256, 4, true, true>;
 
 // V pre-transposed to [B,D,H,S] (the reference's offline transpose, src/fmha-pipeline/fmha_forward.cu:514-532)
+// Head dim 64: three waves per SIMD once there are more than two workgroups for every CU (B=8 H=16 S=1024 36.7 -> 34.5 us, B=4
+// H=16 S=4096 180 -> 173, 8 x 32 heads of 544 rows, 384 keys 20.3 -> 18.8; up to 512 workgroups a tie, 31.3 at B=2 H=16 S=2048;
+// two key tiles per barrier at two waves 36.3, 174 and 20.0).
+using C64T3 = FmhaCfg<64, 64, 4, 3, true, true, true>;
 using C64T = FmhaCfg<64, 64, 4, 2, true, true, true>;
 using C128T = FmhaCfg<128, 64, 4, 2, true, true, true>;
 using C256T = FmhaCfg<256, 64, 4, 1, true, true, true>;
@@ -61,7 +65,10 @@ bool dispatch(int head_dim, int sq, int skv, int bh, int v_layout, bool tap_s, F
   }
   if (v_layout == 1) {
     switch (head_dim) {
-      case 64: select_tile<CfgList<C64T>, CfgList<K64T, C64T>, C64T>(sq, skv, bh, f); return true;
+      case 64: 
+      if ((long long)bh * ((sq + 127) / 128) > 512) select_tile<CfgList<C64T3>, CfgList<K64T, C64T3>, C64T3>(sq, skv, bh, f);
+      else select_tile<CfgList<C64T>, CfgList<K64T, C64T>, C64T>(sq, skv, bh, f);
+      return true;
       case 128: select_tile<CfgList<C128T>, CfgList<K128T, C128T>, C128T>(sq, skv, bh, f); return true;
       case 256: select_tile<CfgList<C256T>, CfgList<K256T, C256T>, C256T>(sq, skv, bh, f); return true;
       default: return false;
@@ -94,7 +101,7 @@ hipError_t prepare_fmha_fp8() {
   if (e == hipSuccess) e = prepare_all(All128{});
   if (e == hipSuccess) e = prepare_all(All256{});
   if (e == hipSuccess) e = prepare_all(CfgList<K64, K128, K256, K64T, K128T, K256T>{});
-  if (e == hipSuccess) e = prepare_all(CfgList<C64T, C128T, C256T, C64Tap, C128Tap, C256Tap, C64TTap, C128TTap, C256TTap>{});
+  if (e == hipSuccess) e = prepare_all(CfgList<C64T, C64T3, C128T, C256T, C64Tap, C128Tap, C256Tap, C64TTap, C128TTap, C256TTap>{});
   return e;
 }
 

@@ -21,6 +21,7 @@ CASES = [
     ("hybrid", (1, 8), 16384, 128, "fmha_fwd_kernel16<128,64,8,2,1,0,0,0,1,", (64, 128, 192, 1024)),
     ("hybrid", (1, 8), 16384, 128, "fmha_fwd_kernel16<128,64,8,2,1,0,0,0,2,", (3072, 3200)),  # an even and an odd number of steps
     ("hybrid", (1, 8), 16384, 64, "fmha_fwd_kernel16<64,64,4,3,1,", (1024, 1088)),
+    ("e4m3-bdhs", (2, 8), 4256, 64, "fmha_fwd_kernel<64,64,4,3,1,1,1,", (64, 128, 192)),
 ]
 
 
