@@ -214,3 +214,10 @@ def test_predictable_latency_option_changes_the_choice_of_kernel_without_gpu():
     assert f.fmha_forward_kernel(f.CFK_FP8_E4M3, 4, 16, 4096, 4096, 128) == "fmha_fwd_kernel8p<128,64,8,2,1,1,0,0,2,0,0,1>"
     with pytest.raises(pkg.CfkError):
         f.set_option(99, 1)
+
+
+def test_a_factor_beyond_float32_is_infinite():
+    f = pkg.fmha
+    block = f._pack(f._GEMM_BLOCK, f.CFK_FP16, 0, 256, 256, 64, 1, 1e40, -1e40, 0, 0, 0, 0)
+    p = f.GemmParams.from_buffer_copy(block)
+    assert (p.alpha, p.beta, p.m) == (float("inf"), float("-inf"), 256)
