@@ -263,24 +263,29 @@ def fmha_forward(q, k, v, o=None, softmax_scale=None, q_descale=1.0, k_descale=1
                              scale, q_descale, k_descale, v_descale, *(0 if t is None else t.data_ptr() for t in (scores, row_max, row_sum)))
     if prepare:
         return PreparedForward(FmhaFwdParams.from_buffer_copy(block), (q, k, v, o, row_max, row_sum, scores), stream)
-    rc = launch(block, _stream_ptr(stream))
+    stream = _stream_ptr(stream)
+    rc = launch(block, stream)
     if rc > 0:   # the call is not made yet: it can use this much scratch memory
         try:
-            ws = _workspace(rc, q.device, stream)
+            ws = _workspace(rc, stream)
         except _torch.OutOfMemoryError:   # no room: the call without it
             ws, rc = None, 0
-        rc = launch_ws(block, 0 if ws is None else ws.data_ptr(), rc, _stream_ptr(stream))
+        rc = launch_ws(block, 0 if ws is None else ws.data_ptr(), rc, stream)
     if rc != 0:
         _check(rc)
     return o
 
 
-def _workspace(n, device, stream):
-    """n bytes of scratch memory for one call, from torch's allocator for the stream that the call runs on: free again when the
-    caller drops it, reused only by later work of that stream (or of the graph being captured)."""
-    if stream is None:
+def _workspace(n, stream):
+    """n bytes of scratch memory for one call, from torch's allocator for the stream that the call runs on (a hipStream_t of the
+    current device): free again when the caller drops it, reused only by later work of that stream (or of the graph being
+    captured)."""
+    dev = _torch._C._cuda_getDevice()
+    device = _torch.device("cuda", dev)
+    if stream == _torch._C._cuda_getCurrentRawStream(dev):
         return _torch.empty(n, dtype=_torch.uint8, device=device)
-    with _torch.cuda.stream(_torch.cuda.ExternalStream(stream, device=device) if isinstance(stream, int) else stream):
+    # (0 is the default stream; to torch.cuda.ExternalStream it is "none given", and its answer a stream of torch's pool)
+    with _torch.cuda.stream(_torch.cuda.ExternalStream(stream, device=device) if stream else _torch.cuda.default_stream(device)):
         return _torch.empty(n, dtype=_torch.uint8, device=device)
 
 
@@ -294,11 +299,12 @@ class PreparedForward:
         self.params, self.tensors = params, tensors   # (the tensors are held so that their memory stays alive)
         self.o = tensors[3]
         self._ref = ctypes.byref(params)
-        self._stream = ctypes.c_void_p(_stream_ptr(stream))
+        stream = _stream_ptr(stream)
+        self._stream = ctypes.c_void_p(stream)
         self._fn = lib().cfk_fmha_forward_ws
         self._ws_bytes = lib().cfk_fmha_forward_workspace(self._ref)
         # (kept: the calls run one after the other on one stream)
-        self._ws = _workspace(self._ws_bytes, tensors[0].device, stream) if self._ws_bytes else None
+        self._ws = _workspace(self._ws_bytes, stream) if self._ws_bytes else None
         self._ws_ptr = self._ws.data_ptr() if self._ws_bytes else None
 
     def __call__(self):
