@@ -1,8 +1,7 @@
 // FMHA forward, hybrid precision: Q, K e4m3 (GEMM-I on the fp8 MFMA), P and V fp16 (GEMM-II on the fp16 MFMA) --
 // what the reference's --prec-type=2 computes when built without -DGEMM2FP8 (src/fmha-pipeline/fmha_forward.cu:
-// 446-450).  Tile shapes and dispatch; the kernels are in fmha_fwd_kernel.h and, on 16x16
-// MFMAs, fmha_fwd_kernel16.h.
-#include "fmha_fwd_kernel16.h"
+// 446-450).  Tile shapes and dispatch; the kernel is in fmha_fwd_kernel.h.
+#include "fmha_fwd_kernel.h"
 #include "fmha_fwd_kernel_ks.h"
 
 namespace cfk {
@@ -15,14 +14,9 @@ using C128_128x64 = FmhaCfg<128, 64, 4, 2, true, false>;
 using C128_256x64 = FmhaCfg<128, 64, 8, 2, true, false>;
 using C128_256x128 = FmhaCfg<128, 64, 8, 2, true, false, false, false, 2>;
 using C256_128x32 = FmhaCfg<256, 32, 4, 1, true, false>;
-// Big problems: the 16x16 builds of fmha_fwd_kernel16.h (S on v_mfma_f32_16x16x128_f8f6f4), which find the reference point by
-// the row sum instead of a row max per tile.  us, 32x32 build -> this one, N(0,1): B=4 H=16 S=4096 D=128 387 -> 372 (1478
-// TFLOP/s; one key tile per barrier 379), B=8 H=16 S=1024 D=128 58.9 -> 56.9; head dim 64, S=4096 249 -> 245, B=8 H=16 S=1024
-// 37.6 -> 36.3.  Not built: 128 rows at head dim 128 (3 x 17 heads of 1696 rows, 3520 keys 130.4 -> 135.0 with one key tile per
-// barrier; with two, B=4 H=16 S=4096 387 -> 528).  The line to the 32x32 builds: first_fit in fmha_fwd_kernel.h.
-using N64_128x64 = FmhaCfg<64, 64, 4, 3, true, false, false, false, 1, 0, true>;
-using N128_256x64 = FmhaCfg<128, 64, 8, 2, true, false, false, false, 1, 0, true>;
-using N128_256x128 = FmhaCfg<128, 64, 8, 2, true, false, false, false, 2, 0, true>;
+// (No 16x16-MFMA build for this mode: with S on v_mfma_f32_16x16x128_f8f6f4 and the reference point found by the row sum, as in
+// fmha_fwd_kernel16.h, 725 drawn calls at head dim 128 took 4..5 % longer in the median once the clock had settled, at every key
+// length from 192 to 8192, head dim 64 2..4 % longer, and B=4 H=16 S=4096 D=128 684 us against 406 where the scores climb along the keys.)
 
 // few query rows: the waves of a workgroup split the keys (fmha_fwd_kernel_ks.h; not by wish)
 using K64 = KsCfg8<64, 8, false, false>;
@@ -49,8 +43,8 @@ bool dispatch(int head_dim, int sq, int skv, int bh, bool tap_s, F &&f) {
     }
   }
   switch (head_dim) {
-    case 64: select_tile<All64, CfgList<K64, N64_128x64, C64_128x64>, C64_128x64>(sq, skv, bh, f); return true;
-    case 128: select_tile<All128, CfgList<K128, N128_256x128, N128_256x64, C128_256x64, C128_128x64>, C128_128x64>(sq, skv, bh, f); return true;
+    case 64: select_tile<All64, CfgList<K64, C64_128x64>, C64_128x64>(sq, skv, bh, f); return true;
+    case 128: select_tile<All128, CfgList<K128, C128_256x64, C128_128x64>, C128_128x64>(sq, skv, bh, f); return true;
     case 256: select_tile<All256, CfgList<K256, C256_128x32>, C256_128x32>(sq, skv, bh, f); return true;
     default: return false;
   }
@@ -72,7 +66,7 @@ hipError_t prepare_fmha_hybrid() {
   hipError_t e = prepare_all(All64{});
   if (e == hipSuccess) e = prepare_all(All128{});
   if (e == hipSuccess) e = prepare_all(All256{});
-  if (e == hipSuccess) e = prepare_all(CfgList<K64, K128, K256, N64_128x64, N128_256x64, N128_256x128>{});
+  if (e == hipSuccess) e = prepare_all(CfgList<K64, K128, K256>{});
   if (e == hipSuccess) e = prepare_all(CfgList<C64Tap, C128Tap, C256Tap>{});
   return e;
 }

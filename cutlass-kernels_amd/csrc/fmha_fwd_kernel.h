@@ -1030,17 +1030,11 @@ bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish
     // build.  Head dim 64, by 128-row items: 1120 (1696 rows, 3520 keys) 157.2 -> 147.0, 952 (896, 3520) 129.6 -> 121.3, 680 (992,
     // 1728) 48.7 -> 47.5, 640 (416, 2240) 60.0 -> 59.0, but 576 (1056, 192) 9.1 -> 9.7, 540 (1440, 1088) 30.1 -> 30.3, 320 (2016, 448)
     // 11.3 -> 11.7.  Head dim 128, lengths that leave the last tile partly filled: 1120 (1696, 3520) 271.6 -> 264.0, 1280 (544, 384)
-    // 42.7 -> 42.0, but 528 (1312, 832) 43.2 -> 44.9; 192 keys 22.9 -> 25.7.  Few keys: 192 at head dim 64 10.1 -> 10.7, 256 a tie.
-    // Hybrid: 512 items of 256 rows at head dim 128 26.5 -> 24.8 with 256 keys, 38.6 -> 36.9 with 512, but 160 items 15.8 -> 16.6;
-    // head dim 64, 1024 items of 128 rows: 1024 keys 37.6 -> 36.3, but 22.8 -> 23.0 with 512 and 14.9 -> 15.2 with 256)
+    // 42.7 -> 42.0, but 528 (1312, 832) 43.2 -> 44.9; 192 keys 22.9 -> 25.7.  Few keys: 192 at head dim 64 10.1 -> 10.7, 256 a tie)
     const long long items128 = bh * ((sq + 127) / 128);
-    const bool m16_pays = C::QK8 ? size == 2 && (C::D != 64 || skv >= 1024)
-                                   : size == 2 || (C::BM == 128 && skv >= 384 && (C::D == 64 ? items128 >= 640 : sq % 128 != 0 && items128 >= 1024));
-    // (e4m3 Q and K on 16x16 MFMAs: two key tiles per barrier, 2 % at 4096 keys and 1 % at 1024, from 3072 keys on; the plan of 2048
-    // keys is held by tests/test_fmha_fp8.py)
-    if (C::M16 && C::QK8 && C::SUB == 2 && skv < 3072) return;
+    const bool m16_pays = size == 2 || (C::BM == 128 && skv >= 384 && (C::D == 64 ? items128 >= 640 : sq % 128 != 0 && items128 >= 1024));
     const bool by_size = C::ASM ? tight && stacked_ok && hand_loop_pays<C>(bh * ((sq + C::BM - 1) / C::BM), skv)
-                                : (C::QK8 && C::BM > 128 && !C::M16 ? fills256 : C::M16 ? m16_pays && (!C::QK8 || C::BM == 128 || fills256) : !(C::BM > 128 && size != 2)) &&
+                                : (C::QK8 && C::BM > 128 ? fills256 : C::M16 ? m16_pays : !(C::BM > 128 && size != 2)) &&
                                       !(C::BM > 128 && skv < (C::PV8 ? 2048 : C::QK8 ? 0 : 1152));
     if (C::KSPLIT ? (w.bm ? C::BM != w.bm : !key_split_pays<C>(bh * ((sq + 31) / 32), sq, skv)) : (w.bm ? C::BM != w.bm : !by_size)) return;
     if (w.bn && C::BN * C::SUB != w.bn) return;

@@ -1,4 +1,4 @@
-// The FMHA forward kernel on 16x16 MFMAs (v_mfma_f32_16x16x32_f16) for fp16 P and V, with fp16 or e4m3 Q and K.  Same algorithm, LDS staging, pipeline
+// The fp16 FMHA forward kernel on 16x16x32 MFMAs (v_mfma_f32_16x16x32_f16).  Same algorithm, LDS staging, pipeline
 // (one or two key tiles per barrier) and epilogue as fmha_fwd_kernel.h, which it takes its configuration struct and
 // host-side plumbing from; what differs is the MFMA shape, with it every register layout, and how the softmax notices
 // that its reference point has to move: not by a row max per tile but by the row sum it needs anyway (softmax_tile
@@ -47,13 +47,11 @@ __device__ __forceinline__ int swz_v16n(int row) {
 template <class C>
 __global__ void __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
 fmha_fwd_kernel16(const FmhaArgs a) {
-  static_assert(!C::PV8 && !C::VT && !C::TAP_S, "fp16 P and V, no score tap");
+  static_assert(!C::QK8 && !C::PV8 && !C::VT && !C::TAP_S, "fp16 operands only, no score tap");
   constexpr int D = C::D, BN = C::BN;
-  constexpr bool QK8 = C::QK8;
-  constexpr int QES = QK8 ? 1 : 2;
   constexpr int QB = 2;        // 16-query blocks per wave
   constexpr int KB = BN / 16;  // 16-key blocks per tile (M blocks of S^T)
-  constexpr int KF = D * QES / 64;  // 16-byte fragments of a K row per lane (fp16: one K-step of S^T each)
+  constexpr int KF = D / 32;   // K-steps of S^T: one 16-byte fragment of a K row per lane each
   constexpr int DB = D / 16;   // 16-row blocks of O^T
   constexpr int PS = BN / 32;  // K-steps of O^T
   const float kTau = a.tau;    // deferred-rescale threshold above the running max (log2 domain)
@@ -70,8 +68,8 @@ fmha_fwd_kernel16(const FmhaArgs a) {
   const int qblk = tile - bh * q_blocks;
   const int b = bh / a.H, h = bh - b * a.H;
   const int64_t ld = (int64_t)a.H * D;  // row stride in elements
-  const char *Qp = (const char *)a.q + (((int64_t)b * a.Sq * a.H + h) * D) * QES;
-  const char *Kp = (const char *)a.k + (((int64_t)b * a.Skv * a.H + h) * D) * QES;
+  const char *Qp = (const char *)a.q + (((int64_t)b * a.Sq * a.H + h) * D) * 2;
+  const char *Kp = (const char *)a.k + (((int64_t)b * a.Skv * a.H + h) * D) * 2;
   const char *Vp = (const char *)a.v + (((int64_t)b * a.Skv * a.H + h) * D) * 2;
   _Float16 *Op = (_Float16 *)a.o + ((int64_t)b * a.Sq * a.H + h) * D;
   // (waves behind the last query row of a partly filled tile copy and meet the barriers like the others, compute the last
@@ -79,17 +77,16 @@ fmha_fwd_kernel16(const FmhaArgs a) {
   const int q0 = qblk * C::BM + wave * 32, q0_in = q0 < a.Sq ? q0 : a.Sq - 32;
   const int n_tiles = a.Skv / BN;
   const float c_log2 = a.scale_log2;
-  const uint32_t k_ld = (uint32_t)(ld * QES), v_ld = (uint32_t)(ld * 2);  // global row pitch in bytes
+  const uint32_t k_ld = (uint32_t)(ld * 2), v_ld = k_ld;  // global row pitch in bytes
 
   // ---- global -> LDS copies, as in fmha_fwd_kernel.h: copy i of wave w covers tile rows (i*NWAVES + w)*RPI .. +RPI;
   // lane l writes LDS slot (row l / CPR, chunk position l % CPR) and fetches chunk position ^ swz(row) of that row.
-  auto swz_k = [](int row) { return QK8 ? swz_row<C::K_PITCH>(row) : swz_k16n<C::K_PITCH>(row); };
   uint32_t goff_k[C::K_IPW], goff_v[C::V_IPW];
 #pragma unroll
   for (int i = 0; i < C::K_IPW; ++i) {
     constexpr int CPR = C::K_PITCH / 16;
     const int row = (i * C::NWAVES + wave) * C::K_RPI + lane / CPR;
-    goff_k[i] = (uint32_t)row * k_ld + (uint32_t)(((lane % CPR) ^ swz_k(row)) * 16);
+    goff_k[i] = (uint32_t)row * k_ld + (uint32_t)(((lane % CPR) ^ swz_k16n<C::K_PITCH>(row)) * 16);
   }
 #pragma unroll
   for (int i = 0; i < C::V_IPW; ++i) {
@@ -112,8 +109,7 @@ fmha_fwd_kernel16(const FmhaArgs a) {
       lds_dma16(gt, goff_v[i], lds_wave, C::V_ST0 + stage * C::V_TILE + i * C::NWAVES * 1024);
   };
 
-  // ---- Q: B operand of S^T, resident in VGPRs: lane (c, g), query block qb, fragment f holds the 16 bytes 64f+16g of row
-  // q0+16qb+c (fp16: d = 32f+8g .. +8)
+  // ---- Q: B operand of S^T, resident in VGPRs: lane (c, g), query block qb, K-step f holds Q[q0_in+16qb+c][32f+8g .. +8)
   int4v qreg[QB][KF];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb)
@@ -122,9 +118,9 @@ fmha_fwd_kernel16(const FmhaArgs a) {
 
   // ---- per-lane LDS read addresses (absolute LDS byte addresses of slot 0; slots and blocks are immediates: the
   // swizzles only depend on the row within its 16- or 8-row group)
-  uint32_t k_rd[KF];  // K operand, fragment f: row c (+16 kb), chunk 4f+g
+  uint32_t k_rd[KF];  // K operand, K-step f: row c (+16 kb), chunk 4f+g
 #pragma unroll
-  for (int f = 0; f < KF; ++f) k_rd[f] = lds_base + C::K_ST0 + c * C::K_PITCH + (((4 * f + g) ^ swz_k(c)) * 16);
+  for (int f = 0; f < KF; ++f) k_rd[f] = lds_base + C::K_ST0 + c * C::K_PITCH + (((4 * f + g) ^ swz_k16n<C::K_PITCH>(c)) * 16);
   // V operand: within its block of 16 lanes, lane L hands the transpose read the address of (key L/4, columns
   // 4(L%4) .. +3) and receives keys 0..3 of column L; the block g reads keys 4g .. 4g+3 (+16 for the second read)
   uint32_t v_rd[DB];
@@ -156,44 +152,17 @@ fmha_fwd_kernel16(const FmhaArgs a) {
   const float sum_cap = __builtin_amdgcn_exp2f(kTau);
   const bool want_taps = a.row_max != nullptr || a.row_sum != nullptr;
   const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-  // S^T = K . Q^T, with frag(f, kb) = fragment f of 16-key block kb.  e4m3: two fragments are one 128-deep multiply
-  // (v_mfma_f32_16x16x128_f8f6f4, twice the rate of fp16; which slot means which d is free as long as K and Q agree);
-  // head dim 64, half as deep, takes the 32-deep form at the fp16 rate
+  // S^T = K . Q^T, with frag(f, kb) = K-step f of 16-key block kb
   auto multiply_qk = [&](auto frag, f32x4 (&sacc)[KB][QB]) __attribute__((always_inline)) {
-    if constexpr (QK8 && KF >= 2) {
 #pragma unroll
-      for (int f = 0; f < KF; f += 2)
+    for (int f = 0; f < KF; ++f)
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          const int4v lo = frag(f, kb), hi = frag(f + 1, kb);
-          const int8v ka = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      for (int kb = 0; kb < KB; ++kb) {
+        const half8 ka = __builtin_bit_cast(half8, frag(f, kb));
 #pragma unroll
-          for (int qb = 0; qb < QB; ++qb) {
-            const int4v ql = qreg[qb][f], qh = qreg[qb][f + 1];
-            const int8v qv = {ql[0], ql[1], ql[2], ql[3], qh[0], qh[1], qh[2], qh[3]};
-            sacc[kb][qb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ka, qv, f == 0 ? zero4 : sacc[kb][qb], 0, 0, 0, 0, 0, 0);
-          }
-        }
-    } else {
-#pragma unroll
-      for (int f = 0; f < KF; ++f)
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          const int4v ka = frag(f, kb);
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb) {
-            f32x4 acc = f == 0 ? zero4 : sacc[kb][qb];
-            if constexpr (QK8) {
-              auto as_long = [](int lo, int hi) { return (long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo); };
-              acc = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(as_long(ka[0], ka[1]), as_long(qreg[qb][f][0], qreg[qb][f][1]), acc, 0, 0, 0);
-              acc = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(as_long(ka[2], ka[3]), as_long(qreg[qb][f][2], qreg[qb][f][3]), acc, 0, 0, 0);
-            } else {
-              acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, ka), __builtin_bit_cast(half8, qreg[qb][f]), acc, 0, 0, 0);
-            }
-            sacc[kb][qb] = acc;
-          }
-        }
-    }
+        for (int qb = 0; qb < QB; ++qb)
+          sacc[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, __builtin_bit_cast(half8, qreg[qb][f]), f == 0 ? zero4 : sacc[kb][qb], 0, 0, 0);
+      }
   };
   // ... for the K tile in LDS slot `stage`
   auto qk = [&](int stage, f32x4 (&sacc)[KB][QB]) __attribute__((always_inline)) {

@@ -131,6 +131,21 @@ def test_python_binding_refuses_cpu_tensors():
         pkg.fmha_forward(x, x, x)
 
 
+@pytest.mark.parametrize("option", [0, 1])
+def test_hybrid_calls_run_kernels_whose_time_does_not_depend_on_the_scores(option):
+    # (fmha_fwd_kernel without e4m3 P and the key-split kernel follow the running max on every tile; fmha_fwd_kernel16 repeats a tile's
+    # scores where the row sum calls for a new reference point)
+    f = pkg.fmha
+    f.set_option(f.CFK_OPT_PREDICTABLE_LATENCY, option)
+    try:
+        for B, H, Sq, Skv, D in [(4, 16, 4096, 4096, 128), (8, 16, 1024, 1024, 128), (8, 32, 1024, 512, 128), (1, 8, 16384, 64, 128),
+                                 (8, 16, 1024, 1024, 64), (4, 16, 4096, 4096, 64), (2, 8, 8192, 4096, 256), (2, 2, 64, 4096, 128)]:
+            name = f.fmha_forward_kernel(f.CFK_FP8_E4M3, B, H, Sq, Skv, D, v_dtype=f.CFK_FP16)
+            assert name.startswith(("fmha_fwd_kernel<", "fmha_fwd_kernel_ks<")), name
+    finally:
+        f.set_option(f.CFK_OPT_PREDICTABLE_LATENCY, 0)
+
+
 def test_predictable_latency_option_changes_the_choice_of_kernel_without_gpu():
     # big fp16 problems at head dim 128 run the two-pass build with the hand-scheduled loop (160 KB of LDS); with the option
     # set the choice falls on the one-pass build (128 KB); unknown options are refused

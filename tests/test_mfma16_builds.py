@@ -1,6 +1,6 @@
 """GPU parity of the compiler-scheduled 16x16-MFMA builds (fmha_fwd_kernel16) where the automatic choice takes them: last query
-tiles of one to four waves, one key tile to a few, e4m3 Q and K, and rows whose scores climb over the keys, which sends waves through
-the slow path of the row-sum test; and of the e4m3 build with pre-transposed V that runs three waves per SIMD.  Gates as in the
+tiles of one to four waves, a few key tiles, and rows whose scores climb over the keys, which sends waves through the slow path of the
+row-sum test; of hybrid calls of the same sizes; and of the e4m3 build with pre-transposed V that runs three waves per SIMD.  Gates as in the
 other parity tests (max-abs error against fp32 attention, src/fmha-pipeline/fmha_forward.cu:599-683)."""
 import math
 
@@ -18,9 +18,10 @@ CASES = [
     ("fp16", (2, 8), 5152, 64, "fmha_fwd_kernel16<64,64,4,3,0,", (384, 448, 704)),         # a last tile with one wave
     ("fp16", (2, 8), 5216, 64, "fmha_fwd_kernel16<64,64,4,3,0,", (448,)),                  # ... with three
     ("fp16", (2, 8), 8128, 128, "fmha_fwd_kernel16<128,64,4,2,0,", (384, 576)),            # ... with two
-    ("hybrid", (1, 8), 16384, 128, "fmha_fwd_kernel16<128,64,8,2,1,0,0,0,1,", (64, 128, 192, 1024)),
-    ("hybrid", (1, 8), 16384, 128, "fmha_fwd_kernel16<128,64,8,2,1,0,0,0,2,", (3072, 3200)),  # an even and an odd number of steps
-    ("hybrid", (1, 8), 16384, 64, "fmha_fwd_kernel16<64,64,4,3,1,", (1024, 1088)),
+    # hybrid calls of many items run the 32x32 build, whose time does not depend on the scores
+    ("hybrid", (1, 8), 16384, 128, "fmha_fwd_kernel<128,64,8,2,1,0,0,0,1,", (64, 128, 192, 1024)),
+    ("hybrid", (1, 8), 16384, 128, "fmha_fwd_kernel<128,64,8,2,1,0,0,0,1,", (3072, 3200)),  # an even and an odd number of steps
+    ("hybrid", (1, 8), 16384, 64, "fmha_fwd_kernel<64,64,4,3,1,", (1024, 1088)),
     ("e4m3-bdhs", (2, 8), 4256, 64, "fmha_fwd_kernel<64,64,4,3,1,1,1,", (64, 128, 192)),
 ]
 
