@@ -289,9 +289,16 @@ def _workspace(n, stream):
         return _torch.empty(n, dtype=_torch.uint8, device=device)
 
 
+def _is_capturing(stream):
+    """Whether a graph is being captured from ``stream`` (a c_void_p; the null stream cannot be captured)."""
+    status = ctypes.c_int(0)
+    return bool(stream.value) and lib().hipStreamIsCapturing(stream, ctypes.byref(status)) == 0 and status.value != 0
+
+
 class PreparedForward:
     """One ``cfk_fmha_forward`` call with its parameter block filled in once (``fmha_forward(..., prepare=True)``): calling
     the object launches it again on the stream given at preparation (torch's current stream then, if none was given).
+    Captured through ``torch.cuda.graph`` the call belongs to the graph, which needs q, k, v, o and not this object.
     What a C++ caller's launch loop does (src/fmha-pipeline/fmha_forward.cu:578-592): the checks and the ctypes
     marshalling of ``fmha_forward`` cost several microseconds per call, as much as a small problem's kernel."""
 
@@ -308,7 +315,21 @@ class PreparedForward:
         self._ws_ptr = self._ws.data_ptr() if self._ws_bytes else None
 
     def __call__(self):
+        if self._ws_bytes and _is_capturing(self._stream):
+            return self._captured()
         rc = self._fn(self._ref, self._ws_ptr, self._ws_bytes, self._stream)
+        if rc != 0:
+            _check(rc)
+        return self.o
+
+    def _captured(self):
+        """The call as part of a graph: its replays may come after this object's scratch memory is gone, so they get their own."""
+        n = self._ws_bytes
+        try:
+            ws = _workspace(n, self._stream.value or 0)
+        except _torch.OutOfMemoryError:   # no room: the call without it
+            ws, n = None, 0
+        rc = self._fn(self._ref, None if ws is None else ws.data_ptr(), n, self._stream)
         if rc != 0:
             _check(rc)
         return self.o

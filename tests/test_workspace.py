@@ -38,7 +38,8 @@ class FakeTorch:
 
     def empty(self, n, dtype, device):
         self.allocated.append((n, self.current))
-        return types.SimpleNamespace(data_ptr=lambda: 0x1000, n=n)
+        address = 0x1000 * len(self.allocated)
+        return types.SimpleNamespace(data_ptr=lambda: address, n=n)
 
 
 @pytest.mark.parametrize("current", [0, 7])
@@ -48,6 +49,33 @@ def test_workspace_belongs_to_the_stream_of_the_call(monkeypatch, current, strea
     monkeypatch.setattr(f, "_torch", fake)
     f._workspace(64, stream)
     assert fake.allocated == [(64, stream)] and fake.current == current
+
+
+def _prepared(monkeypatch, fake, stream):
+    """A prepared split call of the real library's plan on a stand-in torch, and the (workspace, bytes) of its launches."""
+    launches = []
+    monkeypatch.setattr(f, "_torch", fake)
+    B, H, Sq, Skv, D = SPLIT
+    call = f.PreparedForward(f.make_params(f.CFK_FP16, B, H, Sq, Skv, D), (None,) * 7, stream)
+    call._fn = lambda ref, ws, n, stream: launches.append((ws, n)) or 0
+    return call, launches
+
+
+def test_captured_prepared_call_has_scratch_memory_of_the_graph(monkeypatch):
+    # (what the object keeps dies with it, while the graph can still be replayed)
+    fake, capturing = FakeTorch(), []
+    monkeypatch.setattr(f, "_is_capturing", lambda stream: bool(capturing), raising=False)
+    call, launches = _prepared(monkeypatch, fake, 7)
+    call()
+    kept = list(fake.allocated)
+    capturing.append(True)
+    call(), call()
+    capturing.clear()
+    call()
+    need = kept[0][0]
+    assert kept == [(need, 7)] and fake.allocated == [(need, 7)] * 3
+    addresses = [ws for ws, _ in launches]
+    assert addresses[0] == addresses[3] and len(set(addresses)) == 3 and all(n == need for _, n in launches)
 
 
 class _NotingTorch:
@@ -91,3 +119,31 @@ def test_workspace_belongs_to_the_stream_of_the_call_gpu(monkeypatch):
     assert noting.streams == [s for s in expect for _ in range(2)]
     for o in outs:
         assert max_abs(o.float().cpu().numpy(), want) <= TOL_FP16
+
+
+@pytest.mark.gpu
+def test_graph_outlives_the_prepared_call_that_it_captured():
+    import torch
+    dev, want = _operands()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    o = torch.zeros_like(dev[0])
+    call = pkg.fmha_forward(*dev, o=o, stream=side, prepare=True)
+    need = call._ws_bytes
+    assert need > 0
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        assert f._is_capturing(call._stream)
+        call()
+    assert not f._is_capturing(call._stream)
+    torch.cuda.synchronize()
+    del call
+    for rep in range(3):
+        with torch.cuda.stream(side):      # what the object kept is free: other tensors of its stream
+            others = [torch.full((need,), 77, dtype=torch.uint8, device="cuda:0") for _ in range(4)]
+        o.fill_(-1.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert max_abs(o.float().cpu().numpy(), want) <= TOL_FP16, rep
+        assert all(bool((x == 77).all()) for x in others), rep
