@@ -266,11 +266,8 @@ def fmha_forward(q, k, v, o=None, softmax_scale=None, q_descale=1.0, k_descale=1
     stream = _stream_ptr(stream)
     rc = launch(block, stream)
     if rc > 0:   # the call is not made yet: it can use this much scratch memory
-        try:
-            ws = _workspace(rc, stream)
-        except _torch.OutOfMemoryError:   # no room: the call without it
-            ws, rc = None, 0
-        rc = launch_ws(block, 0 if ws is None else ws.data_ptr(), rc, stream)
+        ws = _workspace_or_none(rc, stream)
+        rc = launch_ws(block, None if ws is None else ws.data_ptr(), rc, stream)
     if rc != 0:
         _check(rc)
     return o
@@ -287,6 +284,14 @@ def _workspace(n, stream):
     # (0 is the default stream; to torch.cuda.ExternalStream it is "none given", and its answer a stream of torch's pool)
     with _torch.cuda.stream(_torch.cuda.ExternalStream(stream, device=device) if stream else _torch.cuda.default_stream(device)):
         return _torch.empty(n, dtype=_torch.uint8, device=device)
+
+
+def _workspace_or_none(n, stream):
+    """``_workspace``; None if there is no room: the call runs without it."""
+    try:
+        return _workspace(n, stream)
+    except _torch.OutOfMemoryError:
+        return None
 
 
 def _is_capturing(stream):
@@ -311,25 +316,15 @@ class PreparedForward:
         self._fn = lib().cfk_fmha_forward_ws
         self._ws_bytes = lib().cfk_fmha_forward_workspace(self._ref)
         # (kept: the calls run one after the other on one stream)
-        self._ws = _workspace(self._ws_bytes, stream) if self._ws_bytes else None
-        self._ws_ptr = self._ws.data_ptr() if self._ws_bytes else None
+        self._ws = _workspace_or_none(self._ws_bytes, stream) if self._ws_bytes else None
+        self._ws_ptr = None if self._ws is None else self._ws.data_ptr()
 
     def __call__(self):
-        if self._ws_bytes and _is_capturing(self._stream):
-            return self._captured()
-        rc = self._fn(self._ref, self._ws_ptr, self._ws_bytes, self._stream)
-        if rc != 0:
-            _check(rc)
-        return self.o
-
-    def _captured(self):
-        """The call as part of a graph: its replays may come after this object's scratch memory is gone, so they get their own."""
-        n = self._ws_bytes
-        try:
-            ws = _workspace(n, self._stream.value or 0)
-        except _torch.OutOfMemoryError:   # no room: the call without it
-            ws, n = None, 0
-        rc = self._fn(self._ref, None if ws is None else ws.data_ptr(), n, self._stream)
+        ws = self._ws_ptr
+        if self._ws_bytes and _is_capturing(self._stream):   # (replays may come when what this object keeps is gone)
+            graphs = _workspace_or_none(self._ws_bytes, self._stream.value)
+            ws = None if graphs is None else graphs.data_ptr()
+        rc = self._fn(self._ref, ws, self._ws_bytes, self._stream)
         if rc != 0:
             _check(rc)
         return self.o

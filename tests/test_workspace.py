@@ -78,6 +78,19 @@ def test_captured_prepared_call_has_scratch_memory_of_the_graph(monkeypatch):
     assert addresses[0] == addresses[3] and len(set(addresses)) == 3 and all(n == need for _, n in launches)
 
 
+@pytest.mark.parametrize("capturing", [False, True])
+def test_prepared_call_without_room_for_scratch_memory_runs_without_it(monkeypatch, capturing):
+    fake = FakeTorch()
+
+    def empty(*args, **kw):
+        raise FakeTorch.OutOfMemoryError
+    fake.empty = empty
+    monkeypatch.setattr(f, "_is_capturing", lambda stream: capturing)
+    call, launches = _prepared(monkeypatch, fake, 7)
+    call()
+    assert [ws for ws, _ in launches] == [None]
+
+
 class _NotingTorch:
     """torch, noting on which stream ``empty`` is called for bytes."""
 
