@@ -67,8 +67,8 @@ _GEMM_BLOCK = struct.Struct("=6i2f4Q")
 def _pack(block, *args):
     try:
         return block.pack(*args)
-    except OverflowError:   # a factor beyond float32: infinite there, as the field of a ctypes structure makes it
-        return block.pack(*(ctypes.c_float(x).value if isinstance(x, float) else x for x in args))
+    except (OverflowError, struct.error):   # a factor beyond float32, of whatever type: infinite, as the field of a ctypes structure and native mode make it
+        return struct.pack(block.format.replace("=", "@"), *args)
 
 
 assert _FMHA_BLOCK.size == ctypes.sizeof(FmhaFwdParams) and _GEMM_BLOCK.size == ctypes.sizeof(GemmParams)

@@ -236,3 +236,12 @@ def test_a_factor_beyond_float32_is_infinite():
     block = f._pack(f._GEMM_BLOCK, f.CFK_FP16, 0, 256, 256, 64, 1, 1e40, -1e40, 0, 0, 0, 0)
     p = f.GemmParams.from_buffer_copy(block)
     assert (p.alpha, p.beta, p.m) == (float("inf"), float("-inf"), 256)
+
+
+def test_a_whole_number_or_tensor_beyond_float32_is_infinite():
+    import torch
+    f = pkg.fmha
+    for big in (10**39, torch.tensor(1e39, dtype=torch.float64)):
+        p = f.FmhaFwdParams.from_buffer_copy(f._pack(f._FMHA_BLOCK, 1, 1, 1, 1, 64, 64, 64, 0, 0, 0, 0, 2**64 - 1, 1.0, big, -big, 0.5, 0, 0, 7))
+        assert (p.softmax_scale, p.q_descale, p.k_descale, p.v_descale) == (1.0, float("inf"), float("-inf"), 0.5)
+        assert (p.dtype, p.head_dim, p.o, p.dbg_row_sum) == (1, 64, 2**64 - 1, 7)
