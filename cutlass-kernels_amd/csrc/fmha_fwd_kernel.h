@@ -1032,7 +1032,10 @@ bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish
     // 11.3 -> 11.7.  Head dim 128, lengths that leave the last tile partly filled: 1120 (1696, 3520) 271.6 -> 264.0, 1280 (544, 384)
     // 42.7 -> 42.0, but 528 (1312, 832) 43.2 -> 44.9; 192 keys 22.9 -> 25.7.  Few keys: 192 at head dim 64 10.1 -> 10.7, 256 a tie)
     const long long items128 = bh * ((sq + 127) / 128);
-    const bool m16_pays = size == 2 || (C::BM == 128 && skv >= 384 && (C::D == 64 ? items128 >= 640 : sq % 128 != 0 && items128 >= 1024));
+    // (but not for callers that asked for a run time independent of the data, where the rule was size 2 all along: where the scores
+    // climb these builds take far longer than the 32x32 builds -- 5 x 16 heads of 1696 rows, 3520 keys, head dim 64 162 -> 222 us,
+    // 4 x 20 of 1184, 1728 keys 68 -> 113, 8 x 32 of 544, 1024 keys, head dim 128 100 -> 185)
+    const bool m16_pays = size == 2 || (!predictable_latency() && C::BM == 128 && skv >= 384 && (C::D == 64 ? items128 >= 640 : sq % 128 != 0 && items128 >= 1024));
     const bool by_size = C::ASM ? tight && stacked_ok && hand_loop_pays<C>(bh * ((sq + C::BM - 1) / C::BM), skv)
                                 : (C::QK8 && C::BM > 128 ? fills256 : C::M16 ? m16_pays : !(C::BM > 128 && size != 2)) &&
                                       !(C::BM > 128 && skv < (C::PV8 ? 2048 : C::QK8 ? 0 : 1152));

@@ -174,8 +174,11 @@ typedef enum cfk_option {
    * tile (no row max per tile) and, only if some weight left the range of P's type, walk them again tracking the running
    * max as the reference does on every tile (online_softmax.h:123-165): e4m3 P from 3072 keys on, and fp16 problems
    * with more work items than half the CUs.  On scores that climb along the key axis that costs up to twice the time.  With this option
-   * every call takes the max-tracking path from the start: the same results to rounding, a run time that does not
-   * depend on the data (a few per cent slower on ordinary data).  0 (default): two passes where they pay. */
+   * no call takes such a pass: the same results to rounding (a few per cent slower on ordinary data).  The run time
+   * then does not depend on the data, with one exception: fp16 at head dims 64 and 128, query lengths that are multiples of 256 and
+   * at least 512 tiles of 256 rows, whose 16x16-MFMA build tests the row sum in place of a row max and repeats the scores of a tile
+   * that calls for a new reference point (1.3 to 2.3 times the time on scores that climb along the key axis).
+   * 0 (default): two passes where they pay. */
   CFK_OPT_PREDICTABLE_LATENCY = 1,
   /* 1: e4m3 weights without an exponential.  In the first of the two passes above, kernels with e4m3 P (head dims 64
    * and 128) then build the e4m3 code of a weight directly: read as an integer, the code of a positive e4m3 number is

@@ -146,6 +146,20 @@ def test_hybrid_calls_run_kernels_whose_time_does_not_depend_on_the_scores(optio
         f.set_option(f.CFK_OPT_PREDICTABLE_LATENCY, 0)
 
 
+def test_predictable_latency_keeps_smaller_fp16_calls_on_builds_that_track_the_max():
+    # (the 16x16-MFMA builds repeat a tile's scores where the row sum calls for a new reference point)
+    f = pkg.fmha
+    calls = [(5, 16, 1696, 3520, 64), (4, 20, 1184, 1728, 64), (8, 32, 544, 1024, 64), (8, 10, 1696, 3520, 128), (8, 32, 544, 1024, 128),
+             (8, 16, 1312, 832, 128)]
+    f.set_option(f.CFK_OPT_PREDICTABLE_LATENCY, 1)
+    try:
+        for c in calls:
+            assert f.fmha_forward_kernel(f.CFK_FP16, *c).startswith("fmha_fwd_kernel<"), c
+    finally:
+        f.set_option(f.CFK_OPT_PREDICTABLE_LATENCY, 0)
+    assert f.fmha_forward_kernel(f.CFK_FP16, *calls[0]) == "fmha_fwd_kernel16<64,64,4,3,0,0,0,0,1,0,1,0>"
+
+
 def test_predictable_latency_option_changes_the_choice_of_kernel_without_gpu():
     # big fp16 problems at head dim 128 run the two-pass build with the hand-scheduled loop (160 KB of LDS); with the option
     # set the choice falls on the one-pass build (128 KB); unknown options are refused
