@@ -1026,16 +1026,16 @@ bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish
     // 768 0..+4 %: taken while their rounds of 256 workgroups fill)
     const long long items256 = bh * ((sq + 255) / 256), rounds256 = (items256 + 255) / 256;
     const bool fills256 = sq % 256 == 0 && items256 >= 160 && (rounds256 == 1 || items256 * 5 >= rounds256 * 256 * 4);
-    // (the fp16 128-row 16x16x32 builds also for other query lengths, and at head dim 64 for fewer items; us, 32x32 build -> 16x16x32
-    // build.  Head dim 64, by 128-row items: 1120 (1696 rows, 3520 keys) 157.2 -> 147.0, 952 (896, 3520) 129.6 -> 121.3, 680 (992,
-    // 1728) 48.7 -> 47.5, 640 (416, 2240) 60.0 -> 59.0, but 576 (1056, 192) 9.1 -> 9.7, 540 (1440, 1088) 30.1 -> 30.3, 320 (2016, 448)
-    // 11.3 -> 11.7.  Head dim 128, lengths that leave the last tile partly filled: 1120 (1696, 3520) 271.6 -> 264.0, 1280 (544, 384)
-    // 42.7 -> 42.0, but 528 (1312, 832) 43.2 -> 44.9; 192 keys 22.9 -> 25.7.  Few keys: 192 at head dim 64 10.1 -> 10.7, 256 a tie)
+    // (the fp16 16x16x32 build of head dim 64 also for other query lengths and fewer items, from 768 keys on.  Time relative to the
+    // 32x32 build, geometric means of 2330 drawn calls of 640 to 3000 items of 128 rows: 384 and 448 keys 1.015, 512 to 704 1.007, 768 to
+    // 960 0.995, 1024 to 1408 0.985, more 0.974; by items 0.96..0.99 with no trend.  Some shapes: 1120 items (1696 rows, 3520 keys) 157.2
+    // -> 147.0 us, 680 (992, 1728) 48.7 -> 47.5, but 576 (1056, 192) 9.1 -> 9.7, 540 (1440, 1088) 30.1 -> 30.3.  Not the 128-row build of
+    // head dim 128: where it leaves the last tile partly filled, 727 calls of 1024 items and more took 1.042 of the 32x32 build's time
+    // at 384 to 511 keys, 1.030 and 1.024 up to 1023, 1.011 up to 1447, 0.998 beyond, the worst 1.11.
+    // And not for callers that asked for a run time independent of the data: where the scores climb, 5 x 16 heads of 1696 rows, 3520
+    // keys take 222 us against 162, 4 x 20 of 1184, 1728 keys 113 against 68)
     const long long items128 = bh * ((sq + 127) / 128);
-    // (but not for callers that asked for a run time independent of the data, where the rule was size 2 all along: where the scores
-    // climb these builds take far longer than the 32x32 builds -- 5 x 16 heads of 1696 rows, 3520 keys, head dim 64 162 -> 222 us,
-    // 4 x 20 of 1184, 1728 keys 68 -> 113, 8 x 32 of 544, 1024 keys, head dim 128 100 -> 185)
-    const bool m16_pays = size == 2 || (!predictable_latency() && C::BM == 128 && skv >= 384 && (C::D == 64 ? items128 >= 640 : sq % 128 != 0 && items128 >= 1024));
+    const bool m16_pays = size == 2 || (C::D == 64 && skv >= 768 && items128 >= 640 && !predictable_latency());
     const bool by_size = C::ASM ? tight && stacked_ok && hand_loop_pays<C>(bh * ((sq + C::BM - 1) / C::BM), skv)
                                 : (C::QK8 && C::BM > 128 ? fills256 : C::M16 ? m16_pays : !(C::BM > 128 && size != 2)) &&
                                       !(C::BM > 128 && skv < (C::PV8 ? 2048 : C::QK8 ? 0 : 1152));
