@@ -272,3 +272,18 @@ def test_a_whole_number_or_tensor_beyond_float32_is_infinite():
         p = f.FmhaFwdParams.from_buffer_copy(f._pack(f._FMHA_BLOCK, 1, 1, 1, 1, 64, 64, 64, 0, 0, 0, 0, 2**64 - 1, 1.0, big, -big, 0.5, 0, 0, 7))
         assert (p.softmax_scale, p.q_descale, p.k_descale, p.v_descale) == (1.0, float("inf"), float("-inf"), 0.5)
         assert (p.dtype, p.head_dim, p.o, p.dbg_row_sum) == (1, 64, 2**64 - 1, 7)
+
+
+def test_short_calls_are_not_cut_along_the_keys():
+    # where the merge costs what the shorter walks save: slower cut than whole, by 1.36 down to 1.04
+    f = pkg.fmha
+
+    def workspace(bh, Sq, Skv, D):
+        p = f.make_params(f.CFK_FP16, 1, bh, Sq, Skv, D)
+        return pkg.lib().cfk_fmha_forward_workspace(ctypes.byref(p))
+    for call in [(8, 1472, 2048, 64), (40, 256, 2048, 64), (11, 992, 2112, 64), (24, 480, 2624, 64), (6, 1344, 1024, 256), (85, 128, 1408, 256),
+                 (70, 128, 1152, 256), (8, 1024, 1024, 256)]:
+        assert "kernel16p<" in f.fmha_forward_kernel(f.CFK_FP16, 1, *call) and workspace(*call) == 0, call
+    for call in [(36, 256, 10176, 128), (16, 1024, 8192, 128), (20, 6528, 6144, 128), (16, 4512, 6976, 64), (160, 1216, 4864, 64),
+                 (36, 256, 8192, 256), (15, 2976, 4096, 256), (8, 1024, 2048, 256)]:
+        assert workspace(*call) > 0, call
