@@ -102,6 +102,22 @@ def test_macro_tiles_integer_inputs_bit_exact(L, M, N, K, dtype, layout):
         assert np.array_equal(got[i], want), i
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("K", [192, 256])
+def test_last_round_whole_or_in_tiles_bit_exact(K, layout):
+    # 384 blocks of 256 x 256: the 128 behind the first round of the CUs stay whole below K = 256 and are 256 x 128 tiles from there on
+    import torch
+    M, N = 6144, 4096
+    rng = np.random.default_rng(K)
+    a = rng.integers(-8, 9, (M, K)).astype(np.float32)
+    b = rng.integers(-8, 9, (N, K)).astype(np.float32)
+    got = pkg.gemm(to_dev(a.astype(np.float16)), to_dev((b if layout == 0 else np.ascontiguousarray(b.T)).astype(np.float16)), layout=layout)
+    torch.cuda.synchronize()
+    rows = np.arange(3, M, 61, dtype=np.int32)      # four of every row of blocks
+    want = oracle.gemm_f32(a, b, rows=rows).astype(np.float16)
+    assert np.array_equal(got.cpu().numpy()[rows], want)
+
+
 def test_fp32_uniform_inputs():
     # the CuTe example's type 1 (float operands, gemm.cu:677-684), U(-1,1) data (:482-485).  Both sides accumulate in
     # fp32 in different orders: |error| <~ sqrt(K) * 2^-24 * |terms|
