@@ -281,7 +281,7 @@ def test_short_calls_are_not_cut_along_the_keys():
     def workspace(bh, Sq, Skv, D):
         p = f.make_params(f.CFK_FP16, 1, bh, Sq, Skv, D)
         return pkg.lib().cfk_fmha_forward_workspace(ctypes.byref(p))
-    for call in [(8, 1472, 2048, 64), (40, 256, 2048, 64), (11, 992, 2112, 64), (24, 480, 2624, 64), (6, 1344, 1024, 256), (85, 128, 1408, 256),
+    for call in [(8, 1472, 2048, 64), (40, 256, 2048, 64), (11, 992, 2112, 64), (24, 480, 2624, 64), (8, 1760, 3072, 64), (11, 928, 2560, 64), (6, 1344, 1024, 256), (85, 128, 1408, 256),
                  (70, 128, 1152, 256), (8, 1024, 1024, 256)]:
         assert "kernel16p<" in f.fmha_forward_kernel(f.CFK_FP16, 1, *call) and workspace(*call) == 0, call
     for call in [(36, 256, 10176, 128), (16, 1024, 8192, 128), (20, 6528, 6144, 128), (16, 4512, 6976, 64), (160, 1216, 4864, 64),

@@ -88,8 +88,6 @@ def test_macro_tiles_integer_inputs_bit_exact(L, M, N, K, dtype, layout):
     # a tile for, and whole turns.  Integers: every sum is exact in fp32 in any order.
     import torch
     rng = np.random.default_rng(L + M + N + K)
-    if L > 4 and K > 64:
-        K = 64 if L > 100 else K                         # (the oracle's time)
     a = rng.integers(-8, 9, (L, M, K)).astype(np.float32)
     b = rng.integers(-8, 9, (L, N, K)).astype(np.float32)
     c = rng.integers(-8, 9, (L, M, N)).astype(np.float32)
@@ -100,6 +98,23 @@ def test_macro_tiles_integer_inputs_bit_exact(L, M, N, K, dtype, layout):
     for i in sorted({0, L // 2, L - 1}):
         want = (0.5 * oracle.gemm_f32(a[i], b[i]) - c[i]).astype(dtype)
         assert np.array_equal(got[i], want), i
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("M,N", [(512, 512), (1024, 1024), (1024, 2048), (2048, 2048), (4096, 2048)])
+def test_main_loop_of_every_tile_size_bit_exact(M, N, layout):
+    # 33 K tiles of 64, one, two or four of them per turn and two to four turns in the LDS: every tile size (32 x 32, 64 x 64, 128 x 64,
+    # 128 x 128, 256 x 128) refills each of its slots more than once while others multiply, and the last turn has a tile for one wave
+    # group only
+    import torch
+    K = 2112
+    rng = np.random.default_rng(M + N)
+    a = rng.integers(-8, 9, (M, K)).astype(np.float32)
+    b = rng.integers(-8, 9, (N, K)).astype(np.float32)
+    want = oracle.gemm_f32(a, b).astype(np.float16)
+    got = pkg.gemm(to_dev(a.astype(np.float16)), to_dev((b if layout == 0 else np.ascontiguousarray(b.T)).astype(np.float16)), layout=layout)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy(), want)
 
 
 @pytest.mark.parametrize("layout", [0, 1])
