@@ -980,8 +980,11 @@ constexpr bool hand_loop_pays(long long items, int skv) {
 // below a loss.  128 keys: e4m3 Q and K lose there (4.2 -> 4.7).  e4m3 Q and K at head dim 64, where the tiles are small (with
 // e4m3 V two of these workgroups share a CU), up to 512 workgroups from
 // 1024 keys: 2048 keys e4m3 21.2 -> 16.5, hybrid 22.6 -> 18.4; at head dims 128 and 256 a tie there.
-// fp16 at head dim 256 (1024 keys, 256 workgroups 31.4 -> 23.1) stays on the hand-scheduled build from 1024 query rows and
-// keys on: tests/test_abi.py holds the choice of kernel there.
+// fp16 at head dim 256 stays on the hand-scheduled build (whose items are cut along the keys where there is scratch memory) from 1024
+// query rows and keys on.  The times cross elsewhere: us at 1024, 2048, 4096, 8192 keys, hand-scheduled / key-split, 256 workgroups
+// 30.7 / 23.3, 40.0 / 38.0, 52.8 / 66.5, 80.3 / 126.7; 128 workgroups 32.0 / 22.0, 35.7 / 29.0, 41.1 / 43.6, 54.4 / 72; 64 workgroups
+// 26.5 / 18.7, 33.0 / 22.9, 35.2 / 29.6, 46.4 / 45.3.  So the line is right from 2048 keys on at more than 128 workgroups and from 3072 at
+// 65 to 128, and costs up to three tenths below; tests/test_abi.py pins the kernel of 64 workgroups at 1024 keys, on the costly side.
 template <class C>
 constexpr bool key_split_pays(long long wgs, int sq, int skv) {
   if (skv < (C::QK8 && C::D <= 128 ? 192 : 128)) return false;
@@ -1036,10 +1039,16 @@ bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish
     // keys take 222 us against 162, 4 x 20 of 1184, 1728 keys 113 against 68)
     const long long items128 = bh * ((sq + 127) / 128);
     const bool m16_pays = size == 2 || (C::D == 64 && skv >= 768 && items128 >= 640 && !predictable_latency());
-    const bool by_size = C::ASM ? tight && stacked_ok && hand_loop_pays<C>(bh * ((sq + C::BM - 1) / C::BM), skv)
-                                : (C::QK8 && C::BM > 128 ? fills256 : C::M16 ? m16_pays : !(C::BM > 128 && size != 2)) &&
-                                      !(C::BM > 128 && skv < (C::PV8 ? 2048 : C::QK8 ? 0 : 1152));
-    if (C::KSPLIT ? (w.bm ? C::BM != w.bm : !key_split_pays<C>(bh * ((sq + 31) / 32), sq, skv)) : (w.bm ? C::BM != w.bm : !by_size)) return;
+    const auto pays = [&] {
+      if (C::KSPLIT) return key_split_pays<C>(bh * ((sq + 31) / 32), sq, skv);
+      if (C::ASM) return tight && stacked_ok && hand_loop_pays<C>(bh * ((sq + C::BM - 1) / C::BM), skv);
+      if (C::M16 && !m16_pays) return false;
+      if (C::BM <= 128) return true;
+      // (256-row tiles need key length to pay: figures above)
+      if (C::QK8) return fills256 && (!C::PV8 || skv >= 2048);
+      return size == 2 && skv >= 1152;
+    };
+    if (w.bm ? C::BM != w.bm : !pays()) return;
     if (w.bn && C::BN * C::SUB != w.bn) return;
     if (w.mfma && (C::M16 ? 16 : 32) != w.mfma) return;
     if (w.hand && C::ASM != (w.hand > 0)) return;
