@@ -1029,16 +1029,17 @@ bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish
     // 768 0..+4 %: taken while their rounds of 256 workgroups fill)
     const long long items256 = bh * ((sq + 255) / 256), rounds256 = (items256 + 255) / 256;
     const bool fills256 = sq % 256 == 0 && items256 >= 160 && (rounds256 == 1 || items256 * 5 >= rounds256 * 256 * 4);
-    // (the fp16 16x16x32 build of head dim 64 also for other query lengths and fewer items, from 768 keys on.  Time relative to the
-    // 32x32 build, geometric means of 2330 drawn calls of 640 to 3000 items of 128 rows: 384 and 448 keys 1.015, 512 to 704 1.007, 768 to
-    // 960 0.995, 1024 to 1408 0.985, more 0.974; by items 0.96..0.99 with no trend.  Some shapes: 1120 items (1696 rows, 3520 keys) 157.2
-    // -> 147.0 us, 680 (992, 1728) 48.7 -> 47.5, but 576 (1056, 192) 9.1 -> 9.7, 540 (1440, 1088) 30.1 -> 30.3.  Not the 128-row build of
-    // head dim 128: where it leaves the last tile partly filled, 727 calls of 1024 items and more took 1.042 of the 32x32 build's time
-    // at 384 to 511 keys, 1.030 and 1.024 up to 1023, 1.011 up to 1447, 0.998 beyond, the worst 1.11.
-    // And not for callers that asked for a run time independent of the data: where the scores climb, 5 x 16 heads of 1696 rows, 3520
-    // keys take 222 us against 162, 4 x 20 of 1184, 1728 keys 113 against 68)
+    // (the fp16 128-row 16x16x32 builds also for other query lengths, and at head dim 64 for fewer items.  Time relative to the 32x32
+    // build, medians of drawn calls, each side 0.1 s at a time in turn: head dim 64 from 640 items of 128 rows (314 calls) 0.965 at 384 to
+    // 723 keys, 0.960 to 1023, 0.94..0.95 beyond; below 640 items 576 (1056 rows, 192 keys) 9.1 -> 9.7 us, 540 (1440, 1088) 30.1 -> 30.3.
+    // Head dim 128 with a partly filled last tile from 1024 items (104 calls): 1.000 at 384 to 511 keys, 0.997 to 723, 0.985 to 1023,
+    // 0.97..0.98 beyond; 528 items (1312, 832) 43.2 -> 44.9.  Fewer keys: 192 at head dim 64 10.1 -> 10.7, at 128 22.9 -> 25.7.  In turns
+    // of 2.5 ms, where each side runs on the clock that the other leaves, the same calls show 0.97..1.04: too short to tell.
+    // Not for callers that asked for a run time independent of the data, where the rule was size 2 all along: where the scores climb,
+    // 5 x 16 heads of 1696 rows, 3520 keys, head dim 64 take 222 us against 162, 4 x 20 of 1184, 1728 keys 113 against 68, 8 x 32 of 544,
+    // 1024 keys, head dim 128 185 against 100)
     const long long items128 = bh * ((sq + 127) / 128);
-    const bool m16_pays = size == 2 || (C::D == 64 && skv >= 768 && items128 >= 640 && !predictable_latency());
+    const bool m16_pays = size == 2 || (!predictable_latency() && C::BM == 128 && skv >= 384 && (C::D == 64 ? items128 >= 640 : sq % 128 != 0 && items128 >= 1024));
     const auto pays = [&] {
       if (C::KSPLIT) return key_split_pays<C>(bh * ((sq + 31) / 32), sq, skv);
       if (C::ASM) return tight && stacked_ok && hand_loop_pays<C>(bh * ((sq + C::BM - 1) / C::BM), skv);

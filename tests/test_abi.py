@@ -160,19 +160,6 @@ def test_predictable_latency_keeps_smaller_fp16_calls_on_builds_that_track_the_m
     assert f.fmha_forward_kernel(f.CFK_FP16, *calls[0]) == "fmha_fwd_kernel16<64,64,4,3,0,0,0,0,1,0,1,0>"
 
 
-def test_16x16_builds_only_where_they_are_faster_than_the_32x32_builds():
-    # partly filled query tiles: head dim 64 from 768 keys on, head dim 128 not at all
-    f = pkg.fmha
-    for Skv in (384, 512, 704):
-        assert f.fmha_forward_kernel(f.CFK_FP16, 2, 8, 5152, Skv, 64) == "fmha_fwd_kernel<64,64,4,3,0,0,0,0,1,0,0,0>", Skv
-    assert f.fmha_forward_kernel(f.CFK_FP16, 2, 8, 5152, 832, 64) == "fmha_fwd_kernel16<64,64,4,3,0,0,0,0,1,0,1,0>"
-    for Skv in (384, 576, 832, 1088, 1728):
-        assert f.fmha_forward_kernel(f.CFK_FP16, 8, 16, 1184, Skv, 128).startswith("fmha_fwd_kernel<128,64,4,2,0,"), Skv
-    # whole tiles of 256 rows, enough of them to fill the CUs twice: as ever
-    assert f.fmha_forward_kernel(f.CFK_FP16, 1, 8, 16384, 448, 64) == "fmha_fwd_kernel16<64,64,4,3,0,0,0,0,1,0,1,0>"
-    assert f.fmha_forward_kernel(f.CFK_FP16, 1, 8, 16384, 448, 128) == "fmha_fwd_kernel16<128,64,4,2,0,0,0,0,1,0,1,0>"
-
-
 def test_predictable_latency_option_changes_the_choice_of_kernel_without_gpu():
     # big fp16 problems at head dim 128 run the two-pass build with the hand-scheduled loop (160 KB of LDS); with the option
     # set the choice falls on the one-pass build (128 KB); unknown options are refused
