@@ -671,15 +671,14 @@ constexpr int kCus = 256;
 // 256 x 256 blocks (85 us at K=4096): 256 x 128 0.70, 128 x 128 0.47, 128 x 64 0.26, 64 x 64 0.17, 32 x 32 0.10; a tile size
 // down costs two rounds of its own.  Measured, us (TN), against 256 x 256 blocks alone: M=N=K=1024 8.4 / 25.1, M=N=512 K=4096
 // 8.7 / 75.4, M=N=2048 K=4096 39.5 / 79.5, 5120 x 4096 x 4096 (256 blocks, then 64 in 128 x 128 tiles) 144 / 175 and with C 155 / 199.
-// Behind whole rounds the tiles are a second launch.  Short K, time relative to whole blocks: 1 to 64 blocks behind a round 0.77..0.91 at
-// K=64, 65 to 104 behind one to four rounds 0.92..0.99 at K=64 and 256; 105 to 128, which make 256 x 128 tiles, 0.97..1.03 at K=64,
-// 0.95..1.02 at 256, 0.92..0.98 at 512 (384 blocks, M=6144 N=4096: 19.4 / 20.1 us at K=64, 26.7 / 27.3 at 256, 37.6 / 36.6 at 512):
-// these stay whole below 256.
+// Behind whole rounds the tiles are a second launch, which pays down to the shortest K.  Time relative to whole blocks, behind one and
+// three rounds, at K=64, 128, 256, 512 (means of TN and NN, each side 60 ms at a time in turn): 8 blocks left 0.78, 0.77, 0.76, 0.74 and
+// 0.89, 0.88, 0.87, 0.85; 40 0.87, 0.86, 0.88, 0.85 and 0.94, 0.93, 0.93, 0.92; 72 0.92, 0.94, 0.93, 0.92 and 0.97, 0.97, 0.97, 0.94;
+// 104 0.96, 0.97, 0.96, 0.94 and 0.99, 0.98, 0.97, 0.95; 120 0.97, 0.97, 0.96, 0.95 and 1.00, 0.99, 0.98, 0.95; 128 0.98, 0.99, 0.98, 0.97
+// and 1.01, 1.00, 0.99, 0.96.  Worst found: M=6144 N=4096 (128 left) 1.03, 1.03, 1.00, 0.99, 19.4 -> 20.0 us at K=64.
 template <bool NN>
 hipError_t launch_f16(const GemmArgs &g, hipStream_t s, int blocks) {
-  const int left = blocks % kCus;
-  const bool keep = left > kCus / 2 || (left > 104 && blocks > kCus && g.K < 256);
-  const int whole = keep ? blocks : blocks - left;
+  const int left = blocks % kCus, whole = left > kCus / 2 ? blocks : blocks - left;
   if (whole) {
     const hipError_t e = launch_blocks<NN>(g, s, whole);
     if (e != hipSuccess || whole == blocks) return e;

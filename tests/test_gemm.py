@@ -119,8 +119,8 @@ def test_main_loop_of_every_tile_size_bit_exact(M, N, layout):
 
 @pytest.mark.parametrize("layout", [0, 1])
 @pytest.mark.parametrize("K", [192, 256])
-def test_last_round_whole_or_in_tiles_bit_exact(K, layout):
-    # 384 blocks of 256 x 256: the 128 behind the first round of the CUs stay whole below K = 256 and are 256 x 128 tiles from there on
+def test_last_round_in_tiles_bit_exact(K, layout):
+    # 384 blocks of 256 x 256: the 128 behind the first round of the CUs are 256 x 128 tiles, with as many K tiles as stages and one more
     import torch
     M, N = 6144, 4096
     rng = np.random.default_rng(K)
