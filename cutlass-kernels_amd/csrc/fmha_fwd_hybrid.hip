@@ -14,9 +14,11 @@ using C128_128x64 = FmhaCfg<128, 64, 4, 2, true, false>;
 using C128_256x64 = FmhaCfg<128, 64, 8, 2, true, false>;
 using C128_256x128 = FmhaCfg<128, 64, 8, 2, true, false, false, false, 2>;
 using C256_128x32 = FmhaCfg<256, 32, 4, 1, true, false>;
-// (No 16x16-MFMA build for this mode: with S on v_mfma_f32_16x16x128_f8f6f4 and the reference point found by the row sum, as in
-// fmha_fwd_kernel16.h, 725 drawn calls at head dim 128 took 4..5 % longer in the median once the clock had settled, at every key
-// length from 192 to 8192, head dim 64 2..4 % longer, and B=4 H=16 S=4096 D=128 684 us against 406 where the scores climb along the keys.)
+// (No 16x16-MFMA build for this mode.  With S on v_mfma_f32_16x16x128_f8f6f4 and the reference point found by the row sum, as in
+// fmha_fwd_kernel16.h, its time depends on the scores, which that of a hybrid call is not to do: B=4 H=16 S=4096 D=128 684 us against
+// 406 where they climb along the keys.  On N(0,1) data, time relative to this build, medians of 420 drawn calls, each side 0.1 s at a
+// time in turn: head dim 128 1.09 at 192 keys, 1.05 at 256 to 361, 1.03 to 511, 0.97..0.98 at 512 to 1447, 0.99..1.00 beyond
+// (B=4 H=16 S=4096 398 us here, 383 there); head dim 64 1.01..1.02.)
 
 // few query rows: the waves of a workgroup split the keys (fmha_fwd_kernel_ks.h; not by wish)
 using K64 = KsCfg8<64, 8, false, false>;
