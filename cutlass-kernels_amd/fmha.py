@@ -218,7 +218,8 @@ def fmha_forward(q, k, v, o=None, softmax_scale=None, q_descale=1.0, k_descale=1
     q,k,v: torch CUDA tensors, float16, or float8_e4m3fn / uint8 holding e4m3 codes (v may be float16 with e4m3
     q,k: hybrid mode).  ``v`` is [B,D,H,S] when
     ``v_layout == CFK_V_BDHS``.  ``row_max`` / ``row_sum`` / ``scores`` are the optional debug taps.  Returns ``o`` (float16 [B,Sq,H,D]); launches asynchronously on ``stream``
-    (default: torch's current stream)."""
+    (default: torch's current stream).  A call whose keys are split takes scratch memory from torch's allocator; capture it through
+    ``torch.cuda.graph``, which keeps that memory for the replays."""
     launch, launch_ws, _ = _launch or _launchers()
     f16 = _torch.float16
     if not (q.is_cuda and k.is_cuda and v.is_cuda):

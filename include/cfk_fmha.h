@@ -98,7 +98,8 @@ int cfk_fmha_forward(const cfk_fmha_fwd_params *params, void *stream);
  * round leaves most of them idle, the keys of those blocks are split over several workgroups, whose partial results (fp32 O, reference point and row sum per query row) meet in
  * `workspace` -- device memory of at least cfk_fmha_forward_workspace(params) bytes, 16-byte aligned, that nothing else uses
  * until the call has run on `stream`; its content does not matter before and after.  With workspace = NULL, or one that is
- * too small, this is cfk_fmha_forward.  Two launches per call where the keys are split.  No counterpart in the reference,
+ * too small, this is cfk_fmha_forward.  Two launches per call where the keys are split.  A captured call uses the workspace at every
+ * replay.  No counterpart in the reference,
  * which walks a query block's keys in one thread block (src/fmha-pipeline/fmha_forward.cu:361-372). */
 int cfk_fmha_forward_ws(const cfk_fmha_fwd_params *params, void *workspace, int64_t workspace_bytes, void *stream);
 
@@ -110,7 +111,7 @@ int64_t cfk_fmha_forward_or_workspace(const cfk_fmha_fwd_params *params, void *s
 int64_t cfk_fmha_forward_workspace(const cfk_fmha_fwd_params *params);
 
 /* Bytes of LDS and the tile shape the library would pick for `params` (query rows per workgroup, keys per
- * tile); the reference fixes these at compile time (src/fmha-pipeline/shared_storage.h:4-22).  Any of the
+ * tile) without a workspace, as the two queries below (with one, calls whose keys are split may run another row tile); the reference fixes these at compile time (src/fmha-pipeline/shared_storage.h:4-22).  Any of the
  * out-pointers may be NULL.  Does not touch the GPU. */
 int cfk_fmha_forward_plan(const cfk_fmha_fwd_params *params, int32_t *block_m, int32_t *block_n,
                           int32_t *lds_bytes, int32_t *threads);
