@@ -89,12 +89,11 @@ hipError_t launch_fmha_f16(const FmhaArgs &a, int head_dim, hipStream_t s) {
 // for; the call is cut if that is less than its time otherwise by a twentieth.  Times, us, by head dim: a key tile of a unit while
 // all CUs work and while at most half do (the clock is higher then), a unit's start and end, tiles behind the last group of four
 // as two and a half, the merge 5 and 4 TB/s for the partial results.  That is short of what a cut costs where the whole call is
-// short, so a call stays whole unless a second sum says less time as well: with 6 us for a cut of 128-row items, of 256-row items
-// 11.5, or 13 where a head has more than two of them, 5 behind whole rounds, and 12.5 and 10 TB/s at head dim 256.  (Drawn calls
-// that the first sum alone would cut, whole -> cut: head dim 64 55 of 1732 slower by more than a hundredth, up to 1.36 -- 8 heads of
-// 1472 rows, 2048 keys 18.9 -> 25.8 us --, head dim 256 24 of 618, up to 1.15; with both one in a hundred and one in three hundred,
-// up to 1.1.  The calls that the second sum keeps whole took
-// 1.05 and 1.03 of the time cut, in the geometric mean.)  Measured, N(0,1), us before -> after: D=128, 36 heads of 256
+// short, so a call stays whole unless a second sum says less time as well: with 5 us for a cut behind whole rounds, else 6 for one of
+// 128-row items, 13.5 at head dim 256, and of 256-row items 10.5, or 12.5 where a head has more than two of them.  (1442 drawn calls that
+// the first sum alone would cut, each side 0.1 s at a time in turn, whole -> cut: head dim 64 52 of 1102 slower by more than a hundredth, up
+// to 1.37 -- 25 heads of 512 rows, 2048 keys 19.0 -> 26.0 us --, head dim 128 1 of 168, head dim 256 8 of 172, up to 1.06.  With both 9 of
+// 1041, 0 of 167 and 3 of 156; of the 78 calls that the second sum keeps whole 14 would gain more than three hundredths cut.)  Measured, N(0,1), us before -> after: D=128, 36 heads of 256
 // rows, 10176 keys 127.6 -> 65.5 (3 units); 16 heads of 1024 rows, 8192 keys 99.2 -> 71.0; 20 heads of 6528 rows, 6144 keys (520
 // items of 256 rows) 399 -> 334; D=64, 16 heads of 4512 rows, 6976 keys 174.0 -> 132.4; 160 heads of 1216 rows, 4864 keys 259 -> 234;
 // D=256, 36 heads of 256 rows, 8192 keys 225.8 -> 114.4; 15 heads of 2976 rows, 4096 keys 202.1 -> 181.7.  No gain, and the rule
@@ -124,11 +123,10 @@ bool plan_fmha_f16_split(int head_dim, int sq, int skv, int bh, const FmhaPlan &
     const int items = bh * ((sq + b.bm - 1) / b.bm), from = items / kCus * kCus, cut = items - from;
     const float whole_us = rounds_us(b, from);
     for (int n = 2; n * cut <= kCus && 2 * n <= groups && cut; ++n) {
-      const float partial_bytes = (float)n * cut * b.bm * head_dim * 4.f;
       const float units_us = whole_us + round_us(b, n * cut, 4 * ((groups + n - 1) / n), left);
-      const float us = units_us + 5.f + partial_bytes / 4e6f;
+      const float us = units_us + 5.f + (float)n * cut * b.bm * head_dim * 4.f / 4e6f;
       if (us >= best_us) continue;
-      const float cut_us = head_dim == 256 ? 12.5f + partial_bytes / 10e6f : from ? 5.f : b.bm == 128 ? 6.f : sq <= 512 ? 11.5f : 13.f;
+      const float cut_us = from ? 5.f : head_dim == 256 ? 13.5f : b.bm == 128 ? 6.f : sq <= 512 ? 10.5f : 12.5f;
       best_us = us, best = KeySplit{n, b.bm, from}, pays = units_us + cut_us < call_us;
     }
   }
