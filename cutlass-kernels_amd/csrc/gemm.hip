@@ -10,12 +10,12 @@
 // read with ds_read_b64_tr_b16 exactly as V is in the attention kernel.  The reference writes C column-major
 // (:386-389); C and D are row-major here.  gfx950 has no tf32/xf32 MFMA: fp32 operands multiply in full fp32.
 //
-// Two kernels.  gemm_kernel16 (fp16): 4 waves, one per SIMD, on a 256 x 256 macro tile, for as many of those as fill the CUs
-// in whole rounds; wave (wm, wn) of a 2 x 2 grid owns 128 x 128 of C, its 256 accumulator registers in the AGPR half of the
-// register file, 8 x 8 blocks of 16x16x32 MFMAs (the power-efficient shape on this board).  K tiles are 128 bytes deep and go
+// Two kernels.  gemm_kernel16 (fp16): 8 waves, two per SIMD, on a 256 x 256 macro tile, for as many of those as fill the CUs
+// in whole rounds; wave (wm, wn) of a 2 x 4 grid owns 128 x 64 of C, its 128 accumulator registers in the AGPR half of the
+// register file, 8 x 4 blocks of 16x16x32 MFMAs (the power-efficient shape on this board).  K tiles are 128 bytes deep and go
 // global -> registers -> LDS: 16-byte buffer loads a tile ahead (scalar resource + 32-bit lane offset, no vector address
 // arithmetic), parked in one of two 64 KB LDS stages by ds_write_b128 while the other stage multiplies, one barrier per tile;
-// every multiply is followed by at most one fragment read or one store/load pair, see the pipeline comment in the kernel.
+// every multiply is followed by at most one fragment read or one store/load pair, see the pipeline comment at BlockCfg.
 // (Global -> LDS copy instructions instead of the register path, through a ring of four 32-deep stages and spread the
 // same way, measured 1.57 against 1.94 PFLOP/s on constant operands: with one wave per SIMD an LDS-destination load
 // holds up the issuing wave and with it the MFMA pipe.)
@@ -49,43 +49,105 @@ constexpr int BM = 256, BN = 256;
 template <int PITCH>
 __device__ __forceinline__ int swz_k(int row) { return PITCH == 128 ? (row >> 1) & 7 : (row >> 2) & 3; }
 
-// 512-byte rows read with ds_read_b64_tr_b16 in the 16x16x32 lane map: a 32-lane half of the wave touches rows
-// 8g .. 8g+3 of two k groups g x 32 contiguous bytes; bit 0 stays clear so the 32 bytes stay contiguous
-__device__ __forceinline__ int swz512n(int row) { return ((row & 3) | (((row >> 3) & 1) << 2)) << 1; }
+// B rows [k][n] of PITCH bytes read with ds_read_b64_tr_b16 in the 16x16x32 lane map: a 32-lane half of the wave touches rows 8g .. 8g+3
+// of two k groups g x 32 contiguous bytes, which spread over the 256-byte bank period (of which 256/PITCH rows share one); bit 0 stays
+// clear so that the 32 bytes stay contiguous
+template <int PITCH>
+__device__ __forceinline__ int swz_bn(int row) {
+  if (PITCH % 256 == 0) return ((row & 3) | (((row >> 3) & 1) << 2)) << 1;
+  if (PITCH % 128 == 0) return (((row >> 1) & 1) | (((row >> 3) & 1) << 1)) << 1;
+  return ((row >> 3) & 1) << 1;
+}
 
-// The fp16 kernel on 16x16x32 MFMAs (v_mfma_f32_16x16x32_f16): the wave's 128 x 128 of C as 8 x 8 blocks (NWAVES = 4; NWAVES = 8 runs two waves per SIMD on
-// 128 x 64 each and measured the same).  Measured, 8192^3 TN, same session: 1401 TFLOP/s on U(-1,1) operands against
-// 1309 for the same kernel on 32x32x16 MFMAs (8 waves: 1390); on constant operands 1837 against 2048 (LDS writes between the
-// short multiplies hold the MFMA pipe up for about 20 cycles each).  On U(-1,1) operands this board is
-// power-limited and the deeper, narrower MFMA moves half the accumulator bits per FLOP: a register-only loop sustains
-// 1.90 PFLOP/s with it against 1.69 with 32x32x16.  Lane (c = lane % 16, g = lane / 16) holds, of an operand fragment,
-// row c and contraction slots 8g .. 8g+7 (16 bytes), and of an accumulator block column c, rows 4g .. 4g+3.  The MFMA
-// computes the transposed block (rows = n, columns = m), so a lane owns 4 consecutive n of one row m of C.
-template <bool NN, int NWAVES>
-__global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(NWAVES / 4, NWAVES / 4)))
-gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
-              _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta) {
+// The fp16 kernel on 16x16x32 MFMAs (v_mfma_f32_16x16x32_f16).  8 waves, two per SIMD, in a 2 x 4 grid; a wave owns MB x NB blocks of
+// 16 x 16 of C (8 x 4: 128 x 64 of a 256 x 256 macro tile).  Measured, 8192^3 TN, one session, 4 waves of 128 x 128: 1401 TFLOP/s on
+// U(-1,1) operands against 1309 for the same kernel on 32x32x16 MFMAs; on constant operands 1837 against 2048 (LDS writes between the
+// short multiplies hold the MFMA pipe up for about 20 cycles each).  On U(-1,1) operands this board is power-limited and the deeper,
+// narrower MFMA moves half the accumulator bits per FLOP: a register-only loop sustains 1.90 PFLOP/s with it against 1.69 with 32x32x16.
+// 8 waves read a half more from the LDS than 4 waves of 128 x 128, but with two on a SIMD one multiplies while the other waits for
+// memory, which shows wherever the time is not all main loop (us, 4 -> 8 waves, one session): M=N=4096 with K=64 12.5 -> 10.3, K=192 and
+// C 24.1 -> 18.9, K=1024 33.6 -> 31.6, NN and C 43.3 -> 39.6; 8192^3 819.6 -> 808.5.  (The same tile by 8 waves in two groups half a step
+// apart, copies straight into the LDS through a ring of five 32 KB slots: 812.7, with K=192 and C 19.7; without those copies 691, so
+// what is left at large K is the 64 KB that every 8.4 MFLOP take from L2.)
+// Lane (c = lane % 16, g = lane / 16) holds, of an operand fragment, row c and contraction slots 8g .. 8g+7 (16 bytes), and of an
+// accumulator block column c, rows 4g .. 4g+3.  The MFMA computes the transposed block (rows = n, columns = m), so a lane owns 4
+// consecutive n of one row m of C.
+//
+// Pipeline: two LDS stages and one K tile in registers.  While tile kt multiplies out of stage kt % 2, the registers (tile kt+1, loaded a
+// tile ago) are written to the other stage -- whose readers passed the barrier that opened this tile -- and refilled with tile kt+2, all
+// before the tile's one barrier.  A run of LDS and memory instructions between two multiplies stalls the MFMA pipe, so a tile is laid
+// out as slots of one multiply each (K-step major, then m block, then n block) with at most one piece of other work behind each, pinned
+// in that order.  The n-side fragments of a K-step are live throughout it and double-buffered; the m-side fragments, needed for NB
+// multiplies only, live in a ring of four and are read LOOK blocks ahead; a load is issued two staging pieces behind the store that frees
+// its register (right behind it, it waits for that store to have read it).
+template <int MB, int NB>
+struct BlockCfg {
+  static constexpr int BMT = 32 * MB, BNT = 64 * NB, S = MB * NB;
+  static constexpr int A_PPW = MB / 2, CPT = MB / 2 + NB;   // 16-byte pieces per lane of an A tile, of both
+  static constexpr int A_TILE = BMT * 128, STAGE = (BMT + BNT) * 128;
+  static constexpr int LOOK = NB >= 4 ? 2 : 3;              // m-side fragments are read so many blocks ahead
+  static constexpr int E_PITCH = NB * 64 + 16;
+  static constexpr int LDS_BYTES = 2 * STAGE > 8 * 16 * E_PITCH ? 2 * STAGE : 8 * 16 * E_PITCH;
+  static_assert(MB % 2 == 0 && LDS_BYTES <= 160 * 1024, "pieces, stages");
+  static constexpr int LD_LAG = 2;
+  // Per slot of a tile (two K-steps of S): the m-side fragment (its block, counted through both K-steps), the n-side fragment of K-step 1,
+  // the staging piece to store and the one to load that lie behind its multiply, or -1.  From `barrier` on the slots carry the first
+  // fragments of the next tile: every read of this tile's stage and every store of the next one's is in front of it.
+  struct Slots {
+    int m_frag[2 * S], n_frag[2 * S], store[2 * S], load[2 * S], barrier;
+    bool fits;
+  };
+  static constexpr Slots slots() {
+    Slots r{};
+    bool used[2 * S] = {};
+    for (int i = 0; i < 2 * S; ++i) r.m_frag[i] = r.n_frag[i] = r.store[i] = r.load[i] = -1;
+    r.barrier = S + (MB - 2) * NB;
+    r.fits = (2 * MB - 1 - LOOK) * NB < r.barrier && NB + LOOK <= 2 * NB;
+    for (int x = 0; x < 2 * MB - LOOK; ++x) {
+      r.m_frag[x * NB] = x + LOOK;
+      used[x * NB] = true;
+    }
+    for (int j = 0; j < NB; ++j) {
+      int i = j * (S - 2) / NB + NB / 2;
+      while (used[i]) ++i;
+      r.n_frag[i] = j;
+      used[i] = true;
+      r.fits = r.fits && i < S - 2;
+    }
+    for (int q = 0, last = 0; q < CPT + LD_LAG; ++q) {
+      int i = q * S / CPT + 1;
+      while (i < r.barrier && (used[i] || i <= last)) ++i;
+      if (i >= r.barrier) {
+        r.fits = false;
+        break;
+      }
+      if (q < CPT) r.store[i] = q;
+      if (q >= LD_LAG) r.load[i] = q - LD_LAG;
+      used[i] = true;
+      last = i;
+    }
+    return r;
+  }
+};
+
+template <bool NN, int MB, int NB>
+__device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
+                                           _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta) {
   using T = _Float16;
-  constexpr int ES = 2, PITCH = 128, BK = PITCH / ES;  // 64-deep K tiles: two K-steps of 32
+  using C = BlockCfg<MB, NB>;
+  constexpr int PITCH = 128, BK = PITCH / 2, S = C::S, CPT = C::CPT, A_PPW = C::A_PPW, A_TILE = C::A_TILE, STAGE = C::STAGE;
+  constexpr int BPITCH = C::BNT * 2;   // NN: bytes of a k row of the B tile
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  constexpr int WN = NWAVES / 2;       // waves along n: the wave tile is 128 x 256/WN
-  constexpr int NB = 8;                // 16-row blocks per wave
-  constexpr int NBN = BN / WN / 16;    // 16-column blocks per wave
-  constexpr int A_TILE = BM * PITCH;   // TN: B tile likewise (n rows); NN: BK rows (k) of 512 B
-  constexpr int STAGE = 2 * A_TILE;
-  constexpr int CPW = A_TILE / 1024 / NWAVES;  // 16-byte pieces per lane and operand tile
-  constexpr int RPC = 1024 / PITCH;    // rows per wave-wide 1 KB piece
-  constexpr int KS = PITCH / 64;       // K-steps per tile: 64 bytes of a row (four 16-byte fragments, one per g) each
-  const int wm = wave / WN, wn = wave % WN;
+  const int wm = wave / 4, wn = wave % 4;
 
   // tile order: groups of 8 tile rows, column-major inside a group, so concurrently running workgroups share A and
   // B panels in L2; workgroup ids are first remapped so that each XCD owns a contiguous range of that order (the problems
   // of a batch one after the other)
-  const int tiles_n = N / BN, tiles_m = M / BM;
+  const int tiles_n = (N + C::BNT - 1) / C::BNT, tiles_m = (M + C::BMT - 1) / C::BMT;
   int t = xcd_remap(blockIdx.x, gridDim.x);
   const int64_t batch = t / (tiles_m * tiles_n);  // packed strides M*K, N*K, M*N (reference: gemm.cu:519-521)
   t -= (int)batch * tiles_m * tiles_n;
@@ -95,9 +157,9 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
   const int first_m = grp * GROUP;
   const int rows_in_group = tiles_m - first_m < GROUP ? tiles_m - first_m : GROUP;
   const int in_grp = t - grp * per_group;
-  const int tm = first_m + in_grp % rows_in_group;
-  const int tn = in_grp / rows_in_group;
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m_own = (first_m + in_grp % rows_in_group) * C::BMT, n_own = in_grp / rows_in_group * C::BNT;
+  // a last tile that would reach beyond the edge lies against it instead, and leaves out what its neighbour stores
+  const int m0 = m_own + C::BMT <= M ? m_own : M - C::BMT, n0 = n_own + C::BNT <= N ? n_own : N - C::BNT;
 
   A += batch * M * K;
   B += batch * N * K;
@@ -106,28 +168,30 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
   const char *Ap = (const char *)(A + (int64_t)m0 * K);
   const char *Bp = NN ? (const char *)(B + n0) : (const char *)(B + (int64_t)n0 * K);
 
-  // ---- global -> register -> LDS staging, 16 B per lane and piece.  Piece i of wave w covers tile rows
-  // (i*NWAVES + w)*RPC .. +RPC; lane l owns LDS slot (row l / CPR, chunk position l % CPR) of the piece and fetches
-  // chunk position ^ swz(row) of that row: the XOR swizzle is applied on the global side, LDS writes are linear.
-  // The loads are ordinary loads into registers (compiler-tracked), issued a tile ahead of the ds_write that parks
-  // them in LDS: unlike LDS-destination loads they do not hold up the issuing wave, which with one wave per SIMD
-  // would hold up the MFMA pipe.
-  uint32_t goff_a[CPW], goff_b[CPW];
+  // ---- global -> register -> LDS staging, 16 B per lane and piece.  Piece i of wave w covers the 8 tile rows from (8 i + w) * 8 on;
+  // lane l owns LDS slot (row l / 8, chunk position l % 8) of the piece and fetches chunk position ^ swz(row) of that row: the
+  // XOR swizzle is applied on the global side, LDS writes are linear.  (NN: the B tile is 64 k rows of BPITCH bytes, cut into
+  // pieces of 1 KB.)  The pieces lie 64 rows apart, but one lane offset plus a scalar offset per piece is slower than a lane
+  // offset for each: 8192^3 797.0 us against 787.5.  The loads are ordinary loads into registers
+  // (compiler-tracked), issued a tile ahead of the ds_write that parks them in LDS.
+  constexpr int KP = NN || A_PPW > NB ? A_PPW : NB;
+  uint32_t goff_k[KP];
 #pragma unroll
-  for (int i = 0; i < CPW; ++i) {
-    const int row = (i * NWAVES + wave) * RPC + lane / (PITCH / 16);
-    const int cp = lane % (PITCH / 16);
-    goff_a[i] = (uint32_t)row * (uint32_t)(K * ES) + (uint32_t)((cp ^ swz_k<PITCH>(row)) * 16);
-    if (!NN) {
-      goff_b[i] = goff_a[i];
-    } else {  // B tile is BK rows (k) of 512 B (256 n): 2 rows per piece
-      const int krow = (i * NWAVES + wave) * 2 + (lane >> 5);
-      const int cpb = lane & 31;
-      goff_b[i] = (uint32_t)krow * (uint32_t)(N * 2) + (uint32_t)((cpb ^ swz512n(krow)) * 16);
+  for (int i = 0; i < KP; ++i) {
+    const int row = (i * 8 + wave) * 8 + lane / 8;
+    goff_k[i] = (uint32_t)row * (uint32_t)(K * 2) + (uint32_t)(((lane % 8) ^ swz_k<PITCH>(row)) * 16);
+  }
+  uint32_t goff_b[NB];
+  if constexpr (NN) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      constexpr int CPR = BPITCH / 16;
+      const int idx = (i * 8 + wave) * 64 + lane, krow = idx / CPR;
+      goff_b[i] = (uint32_t)krow * (uint32_t)(N * 2) + (uint32_t)(((idx % CPR) ^ swz_bn<BPITCH>(krow)) * 16);
     }
   }
   const uint32_t st_off = wave * 1024 + lane * 16;
-  int4v stg[2 * CPW];
+  int4v stg[CPT];
   using Rsrc = __amdgpu_buffer_rsrc_t;
   auto tile_ptrs = [&](int kt, Rsrc &ga, Rsrc &gb) {
     const char *pa = Ap + (size_t)kt * PITCH;
@@ -136,43 +200,46 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
     gb = __builtin_amdgcn_make_buffer_rsrc((void *)pb, 0, -1, 0x00020000);
   };
   auto load_piece = [&](Rsrc ga, Rsrc gb, int p) {
-    const u32x4 x = p < CPW ? __builtin_amdgcn_raw_buffer_load_b128(ga, (int)goff_a[p], 0, 0)
-                            : __builtin_amdgcn_raw_buffer_load_b128(gb, (int)goff_b[p - CPW], 0, 0);
+    u32x4 x;
+    if (p < A_PPW) x = __builtin_amdgcn_raw_buffer_load_b128(ga, (int)goff_k[p], 0, 0);
+    else if (NN) x = __builtin_amdgcn_raw_buffer_load_b128(gb, (int)goff_b[p - A_PPW], 0, 0);
+    else x = __builtin_amdgcn_raw_buffer_load_b128(gb, (int)goff_k[p - A_PPW], 0, 0);
     stg[p] = __builtin_bit_cast(int4v, x);
   };
   auto store_piece = [&](int stage, int p) {
-    char *dst = smem + stage * STAGE + st_off + (p < CPW ? p * NWAVES * 1024 : A_TILE + (p - CPW) * NWAVES * 1024);
+    char *dst = smem + stage * STAGE + st_off + (p < A_PPW ? p * 8192 : A_TILE + (p - A_PPW) * 8192);
     *(int4v *)dst = stg[p];
   };
 
   // ---- LDS read addresses.  K-step s: lane (c, g) needs bytes 64s + 16g .. +16 of its row (k = 32s + 8g .. +8).
   // swz_k<128> depends on the row within its group of 16 only, so blocks are immediates.
-  int a_rd[KS], b_rd[KS];
+  int a_rd[2], b_rd[2];
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    a_rd[s] = (wm * 128 + c) * PITCH + (((4 * s + g) ^ swz_k<PITCH>(c)) * 16);                // + 16 rows per m block
-    b_rd[s] = A_TILE + (wn * NBN * 16 + c) * PITCH + (((4 * s + g) ^ swz_k<PITCH>(c)) * 16);       // + 16 rows per n block (TN)
+  for (int s = 0; s < 2; ++s) {
+    a_rd[s] = (wm * MB * 16 + c) * PITCH + (((4 * s + g) ^ swz_k<PITCH>(c)) * 16);
+    b_rd[s] = A_TILE + (wn * NB * 16 + c) * PITCH + (((4 * s + g) ^ swz_k<PITCH>(c)) * 16);
   }
   // NN: the n-side operand via two ds_read_b64_tr_b16 from [k][n] rows: within its block of 16 lanes, lane L hands
   // the read the address of (k row L/4, columns 4(L%4) .. +3) and receives k rows 0..3 of column L; block g reads k
   // rows 8g .. 8g+3, the second read 4 further
   const int bk_row = 8 * g + (c >> 2);          // + 32 s (+ 4)
   const int cg = c & 3;
-  int bt_rd[NBN];
+  int bt_rd[NB];
+  if constexpr (NN) {
 #pragma unroll
-  for (int nb = 0; nb < NBN; ++nb) {
-    const int chunk = (wn * NBN * 16 + 16 * nb) / 8 + (cg >> 1);  // 16-byte chunk of the 512-byte row
-    bt_rd[nb] = A_TILE + bk_row * 512 + ((chunk ^ swz512n(bk_row)) * 16) + (cg & 1) * 8;
+    for (int nb = 0; nb < NB; ++nb) {
+      const int chunk = (wn * NB * 16 + 16 * nb) / 8 + (cg >> 1);
+      bt_rd[nb] = A_TILE + bk_row * BPITCH + ((chunk ^ swz_bn<BPITCH>(bk_row)) * 16) + (cg & 1) * 8;
+    }
   }
 
-  f32x4 acc[NB][NBN];  // [m block][n block]
+  f32x4 acc[MB][NB];  // [m block][n block]
 #pragma unroll
-  for (int mb = 0; mb < NB; ++mb)
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-    for (int nb = 0; nb < NBN; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int k_tiles = K / BK;
-  // operand fragments of K-step s of the tile in LDS stage `st`: m block blk, n block blk
   auto fetch_a = [&](const char *st, int s, int blk) -> half8 { return *(const half8 *)(st + a_rd[s] + blk * 16 * PITCH); };
   auto fetch_b = [&](const char *st, int s, int blk) -> half8 {
     if constexpr (!NN) {
@@ -182,40 +249,20 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
         struct { short4v lo, hi; } p;
         half8 h;
       } u;
-      const char *bp = st + bt_rd[blk] + s * 32 * 512;
+      const char *bp = st + bt_rd[blk] + s * 32 * BPITCH;
       u.p.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4v, bp));
-      u.p.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4v, bp + 4 * 512));
+      u.p.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(short4v, bp + 4 * BPITCH));
       return u.h;
     }
   };
-
-  // Pipeline: two LDS stages and one tile in registers.  While tile kt multiplies out of stage kt % 2, the registers
-  // (tile kt+1, loaded a tile ago) are written to the other stage -- whose readers passed the barrier that opened
-  // this tile -- and refilled with tile kt+2, all before the tile's one barrier.  With one wave per SIMD nothing but
-  // this wave's own instruction stream keeps the MFMA pipe fed: a run of LDS and memory instructions between two
-  // multiplies stalls it.  So a tile is laid out as slots of one multiply each (K-step major, then m block, then n block;
-  // SPM = NBN slots per m block) with at most one piece of other work behind each multiply, pinned in that order; a load is
-  // issued LD_LAG pieces behind the store that frees its register (right behind it, it waits for that store to have read it).  Fragment registers: the n-side fragments of a K-step
-  // are live throughout it and double-buffered (bop[K-step parity]); the m-side fragment of block mb is only needed
-  // for its NBN multiplies and lives in a ring of four (aop[mb % 4]), read two blocks ahead.
-  //   K-step 0:  first slot of m block mb: m fragment mb+2 (the last two: blocks 0, 1 of K-step 1);  slot SPM/2 of
-  //              m blocks 0 .. NBN-1: n fragment mb of K-step 1;  the CPT slots i % (NB*NBN/CPT) == 1: ds_write of a
-  //              staging piece of tile kt+1 and, LD_LAG pieces behind it, the load of the same piece of tile kt+2
-  //   K-step 1:  first slot of m blocks 0..5: m fragment mb+2;  first slot of m block 6: the barrier (every read of
-  //              this tile's stage and every write of the next tile's is in front of it), then one per slot the first
-  //              fragments of the next tile (n 0 .. NBN-1 and m 0, 1 of its K-step 0) in the order they are needed
-  constexpr int CPT = 2 * CPW;
-  constexpr int LD_LAG = 2;
-  constexpr int SPM = NBN;                    // slots per m block
-  constexpr int ST_EVERY = NB * NBN / CPT;    // a staging piece every so many slots of K-step 0
-  static_assert(KS == 2 && ST_EVERY >= 2 && NB * NBN % CPT == 0, "slot layout");
-  // The multiplies are asm statements with "+a" accumulators: the compiler's hazard recognizer does not see the
+  constexpr typename C::Slots sl = C::slots();
+  static_assert(sl.fits, "slot layout");
+  // The multiplies are asm statements with in-place accumulators: the compiler's hazard recognizer does not see the
   // matrix-pipe write -> accumulate-read dependency between two of them, so the distance between two multiplies into
-  // one accumulator is this layout's business.  Every accumulator block is used once per K-step: NB * NBN multiplies
-  // lie between two uses (64), each holding the pipe for the 4 passes of v_mfma_f32_16x16x32_f16; back-to-back
-  // dependent MFMAs of this shape need 4 passes + 2 wait states.  Fewer blocks per wave than that (or a reordering that
-  // revisits a block within one K-step) would need nops here.
-  static_assert(NB * NBN >= 8, "distance between two multiplies into one accumulator: at least the MFMA's passes plus its wait states");
+  // one accumulator is this layout's business.  Every accumulator block is used once per K-step: MB * NB multiplies
+  // lie between two uses, each holding the pipe for the 4 passes of v_mfma_f32_16x16x32_f16; back-to-back
+  // dependent MFMAs of this shape need 4 passes + 2 wait states.
+  static_assert(S >= 8, "distance between two multiplies into one accumulator: at least the MFMA's passes plus its wait states");
   Rsrc ga, gb;
   tile_ptrs(0, ga, gb);
 #pragma unroll
@@ -226,11 +273,11 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
 #pragma unroll
   for (int p = 0; p < CPT; ++p) load_piece(ga, gb, p);
   __syncthreads();
-  half8 aop[4], bop[2][NBN];
+  half8 aop[4], bop[2][NB];
 #pragma unroll
-  for (int nb = 0; nb < NBN; ++nb) bop[0][nb] = fetch_b(smem, 0, nb);
-  aop[0] = fetch_a(smem, 0, 0);
-  aop[1] = fetch_a(smem, 0, 1);
+  for (int nb = 0; nb < NB; ++nb) bop[0][nb] = fetch_b(smem, 0, nb);
+#pragma unroll
+  for (int x = 0; x < C::LOOK; ++x) aop[x] = fetch_a(smem, 0, x);
   int stage = 0;
   for (int kt = 0; kt < k_tiles; ++kt) {
     const char *st = smem + stage * STAGE;
@@ -238,34 +285,27 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
     const int nstage = stage ^ 1;
     tile_ptrs(kt + 2 < k_tiles ? kt + 2 : k_tiles - 1, ga, gb);  // clamped at the end: a surplus tile is loaded and dropped
 #pragma unroll
-    for (int s2 = 0; s2 < KS; ++s2) {
-#pragma unroll
-      for (int i = 0; i < NB * NBN; ++i) {
-        const int mb = i / SPM, nb = i % SPM;
-        if (s2 == 1 && i == 6 * SPM) __syncthreads();
-        // written out so that the accumulator is updated in place in the AGPR half: through the builtin the register
-        // allocator moves the small accumulators between the two halves (280 copies per tile).  Nothing but these
-        // multiplies touches the accumulators inside the loop, so no hazard is hidden from the compiler here.
-        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[mb][nb]) : "v"(bop[s2][nb]), "v"(aop[mb % 4]));
-        if (nb == 0 && (s2 == 0 || mb <= 5)) {
-          const int blk = mb + 2;
-          aop[blk % 4] = blk < NB ? fetch_a(st, s2, blk) : fetch_a(st, 1, blk - NB);
+    for (int i = 0; i < 2 * S; ++i) {
+      const int x = i / NB, nb = i % NB, s2 = i / S, mb = x % MB;   // x: the m block, counted through both K-steps
+      if (i == sl.barrier) __syncthreads();
+      // written out so that the accumulator is updated in place: through the builtin the register allocator moves the small
+      // accumulators between the two halves of the register file.  Nothing but these multiplies touches the accumulators inside the
+      // loop, so no hazard is hidden from the compiler here.  (The compiler gives a wave 128 AGPRs: 32 blocks.)
+      if (mb * NB + nb < 32) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[mb][nb]) : "v"(bop[s2][nb]), "v"(aop[x % 4]));
+      else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[mb][nb]) : "v"(bop[s2][nb]), "v"(aop[x % 4]));
+      if (sl.m_frag[i] >= 0) aop[sl.m_frag[i] % 4] = fetch_a(st, sl.m_frag[i] / MB, sl.m_frag[i] % MB);
+      if (sl.n_frag[i] >= 0) bop[1][sl.n_frag[i]] = fetch_b(st, 1, sl.n_frag[i]);
+      if (i >= sl.barrier) {
+        const int j = i - sl.barrier;   // n 0, m 0, n 1, m 1, .., then the rest of the n side
+        if (j < 2 * C::LOOK && j % 2 == 1) aop[j / 2] = fetch_a(nx, 0, j / 2);
+        else if (j < NB + C::LOOK) {
+          const int n = j < 2 * C::LOOK ? j / 2 : j - C::LOOK;
+          bop[0][n] = fetch_b(nx, 0, n);
         }
-        if (s2 == 0 && nb == SPM / 2 && mb < NBN) bop[1][mb] = fetch_b(st, 1, mb);
-        if (s2 == 1 && i >= 6 * SPM && i < 6 * SPM + NBN + 2) {
-          // n 0, m 0, n 1, m 1, n 2 ...
-          const int j = i - 6 * SPM;
-          if (j == 1) aop[0] = fetch_a(nx, 0, 0);
-          else if (j == 3) aop[1] = fetch_a(nx, 0, 1);
-          else bop[0][j == 0 ? 0 : j == 2 ? 1 : j - 2] = fetch_b(nx, 0, j == 0 ? 0 : j == 2 ? 1 : j - 2);
-        }
-        if (i % ST_EVERY == 1) {
-          const int q = (s2 * NB * NBN + i) / ST_EVERY;  // staging slot number within the tile
-          if (q < CPT) store_piece(nstage, q);
-          if (q >= LD_LAG && q - LD_LAG < CPT) load_piece(ga, gb, q - LD_LAG);
-        }
-        __builtin_amdgcn_sched_barrier(0);
       }
+      if (sl.store[i] >= 0) store_piece(nstage, sl.store[i]);
+      if (sl.load[i] >= 0) load_piece(ga, gb, sl.load[i]);
+      __builtin_amdgcn_sched_barrier(0);
     }
     stage = nstage;
   }
@@ -273,30 +313,28 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
   // the last multiplies have left the pipe before the epilogue reads their accumulators (the compiler does not see
   // the dependency through the asm statements)
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
-  // ---- epilogue: D = alpha * acc + beta * C in fp32, each 16 x 128 row of blocks staged through the wave's own LDS
-  // region and stored as whole rows, 16 bytes per lane
-  constexpr int E_PITCH = 128 * 4 + 16;
-  constexpr int EPL = 8;                          // halves per lane and store
-  constexpr int WCOLS = NBN * 16;                   // columns of the wave tile
-  constexpr int LPR = WCOLS / EPL, RPP = 64 / LPR;  // lanes per row, rows per wave-wide store
+  // ---- epilogue: D = alpha * acc + beta * C in fp32, each row of blocks staged through the wave's own LDS region and stored as
+  // whole rows, 16 bytes per lane
+  constexpr int EPL = 8, LPR = NB * 2, CHUNKS = 16 * LPR;   // halves per lane and store, lanes per row
   const bool with_c = Cin != nullptr && beta != 0.f;
-  char *et = smem + wave * (16 * E_PITCH);
-  const int e_row = lane / LPR, e_col = (lane % LPR) * EPL;
+  char *et = smem + wave * (16 * C::E_PITCH);
 #pragma unroll
-  for (int mb = 0; mb < NB; ++mb) {
+  for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
-    for (int nb = 0; nb < NBN; ++nb) *(f32x4 *)(et + c * E_PITCH + (nb * 16 + 4 * g) * 4) = acc[mb][nb];
+    for (int nb = 0; nb < NB; ++nb) *(f32x4 *)(et + c * C::E_PITCH + (nb * 16 + 4 * g) * 4) = acc[mb][nb];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int pass = 0; pass < 16 / RPP; ++pass) {
-      const int row = pass * RPP + e_row;
-      const int64_t off = (int64_t)(m0 + wm * 128 + mb * 16 + row) * N + n0 + wn * WCOLS + e_col;
+    for (int pass = 0; pass < (CHUNKS + 63) / 64; ++pass) {
+      const int idx = pass * 64 + lane, row = idx / LPR, col = idx % LPR * EPL;
+      const int gm = m0 + (wm * MB + mb) * 16 + row, gn = n0 + wn * NB * 16 + col;
+      if ((CHUNKS % 64 != 0 && idx >= CHUNKS) || gm < m_own || gn < n_own) continue;
+      const int64_t off = (int64_t)gm * N + gn;
       float v[EPL];
 #pragma unroll
       for (int q = 0; q < EPL / 4; ++q) {
-        const f32x4 x = *(const f32x4 *)(et + row * E_PITCH + (e_col + 4 * q) * 4);
+        const f32x4 x = *(const f32x4 *)(et + row * C::E_PITCH + (col + 4 * q) * 4);
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[4 * q + j] = alpha * x[j];
       }
@@ -314,6 +352,13 @@ gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, co
     __builtin_amdgcn_wave_barrier();  // the region is rewritten by the next row of blocks
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
+}
+
+template <bool NN, int NB>   // 256 rows
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
+              _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta) {
+  gemm_block<NN, 8, NB>(A, B, Cin, D, M, N, K, alpha, beta);
 }
 
 // ---- Smaller macro tiles (which of them a call takes: launch_f16 and launch_f32 below).
@@ -339,15 +384,6 @@ struct TileCfg {
   static_assert(A_PPW * WPG * 8 == BMT && PPW * WPG * 8 == BMT + BNT, "whole 1 KB copies per wave");
   static_assert(LDS_BYTES <= 160 * 1024 && ST >= 2, "stages");
 };
-
-// B rows [k][n] of PITCH bytes read with ds_read_b64_tr_b16 in the 16x16x32 lane map (see swz512n): rows 8g .. 8g+3 of
-// two k groups g x 32 contiguous bytes spread over the 256-byte bank period, of which 256/PITCH rows share one
-template <int PITCH>
-__device__ __forceinline__ int swz_bn(int row) {
-  if (PITCH >= 256) return ((row & 3) | (((row >> 3) & 1) << 2)) << 1;
-  if (PITCH == 128) return (((row >> 1) & 1) | (((row >> 3) & 1) << 1)) << 1;
-  return ((row >> 3) & 1) << 1;
-}
 
 template <class C>
 __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, const typename C::T *__restrict__ B,
@@ -623,9 +659,6 @@ gemm_kernel_f32(const float *__restrict__ A, const float *__restrict__ B, const 
   gemm_tile<FTile<EDGE>>(A, B, Cin, D, M, N, K, alpha, beta, block0);
 }
 
-constexpr int kWaves16 = 4;                          // waves of gemm_kernel16
-constexpr int kLds16 = 2 * 2 * BM * 128;             // two stages of an A and a B tile, 128 bytes deep
-
 // one-time set-up of a kernel (its dynamic-LDS limit), thread-safe and callable ahead of any launch
 template <auto Kern, int Lds>
 hipError_t prepare_kernel() {
@@ -638,9 +671,10 @@ hipError_t prepare_kernel() {
 // the 256 x 256 blocks 0 .. blocks-1 of the batch
 template <bool NN>
 hipError_t launch_blocks(const GemmArgs &g, hipStream_t s, int blocks) {
-  const hipError_t e = prepare_kernel<gemm_kernel16<NN, kWaves16>, kLds16>();
+  using C = BlockCfg<8, 4>;
+  const hipError_t e = prepare_kernel<gemm_kernel16<NN, 4>, C::LDS_BYTES>();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((gemm_kernel16<NN, kWaves16>), dim3(blocks), dim3(kWaves16 * 64), kLds16, s, (const _Float16 *)g.A, (const _Float16 *)g.B,
+  hipLaunchKernelGGL((gemm_kernel16<NN, 4>), dim3(blocks), dim3(512), C::LDS_BYTES, s, (const _Float16 *)g.A, (const _Float16 *)g.B,
                      (const _Float16 *)g.C, (_Float16 *)g.D, g.M, g.N, g.K, g.alpha, g.beta);
   return hipGetLastError();
 }
@@ -704,7 +738,7 @@ hipError_t launch_f32(const GemmArgs &g, hipStream_t s, int blocks) {
 
 template <bool NN>
 hipError_t prepare_f16() {
-  const hipError_t e[] = {prepare_kernel<gemm_kernel16<NN, kWaves16>, kLds16>(),
+  const hipError_t e[] = {prepare_kernel<gemm_kernel16<NN, 4>, BlockCfg<8, 4>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 256, 128>, HTile<NN, 256, 128>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 128, 128>, HTile<NN, 128, 128>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 128, 64>, HTile<NN, 128, 64>::LDS_BYTES>(),
