@@ -181,10 +181,14 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
     const int row = (i * 8 + wave) * 8 + lane / 8;
     goff_k[i] = (uint32_t)row * (uint32_t)(K * 2) + (uint32_t)(((lane % 8) ^ swz_k<PITCH>(row)) * 16);
   }
-  uint32_t goff_b[NB];
+  // (320 rows NN: registers for one lane offset of B only, which serves all pieces, 16 k rows apart, with a scalar offset)
+  constexpr bool ONE_B = NN && MB > 8;
+  static_assert(!ONE_B || BPITCH == 512, "pieces a multiple of 16 rows apart");
+  constexpr int BPN = ONE_B ? 1 : NB;
+  uint32_t goff_b[BPN];
   if constexpr (NN) {
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
+    for (int i = 0; i < BPN; ++i) {
       constexpr int CPR = BPITCH / 16;
       const int idx = (i * 8 + wave) * 64 + lane, krow = idx / CPR;
       goff_b[i] = (uint32_t)krow * (uint32_t)(N * 2) + (uint32_t)(((idx % CPR) ^ swz_bn<BPITCH>(krow)) * 16);
@@ -202,7 +206,7 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
   auto load_piece = [&](Rsrc ga, Rsrc gb, int p) {
     u32x4 x;
     if (p < A_PPW) x = __builtin_amdgcn_raw_buffer_load_b128(ga, (int)goff_k[p], 0, 0);
-    else if (NN) x = __builtin_amdgcn_raw_buffer_load_b128(gb, (int)goff_b[p - A_PPW], 0, 0);
+    else if (NN) x = __builtin_amdgcn_raw_buffer_load_b128(gb, (int)goff_b[ONE_B ? 0 : p - A_PPW], ONE_B ? (int)(32u * (uint32_t)N * (uint32_t)(p - A_PPW)) : 0, 0);
     else x = __builtin_amdgcn_raw_buffer_load_b128(gb, (int)goff_k[p - A_PPW], 0, 0);
     stg[p] = __builtin_bit_cast(int4v, x);
   };
@@ -378,6 +382,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 gemm_kernel16(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
               _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta) {
   gemm_block<NN, 8, NB>(A, B, Cin, D, M, N, K, alpha, beta);
+}
+template <bool NN, int MB, int NB>   // 32 MB rows
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+gemm_kernel16_rows(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
+                   _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta) {
+  gemm_block<NN, MB, NB>(A, B, Cin, D, M, N, K, alpha, beta);
 }
 
 // ---- Smaller macro tiles (which of them a call takes: launch_f16 and launch_f32 below).
@@ -687,14 +697,20 @@ hipError_t prepare_kernel() {
   return status;
 }
 
-// the 256 x 256 blocks 0 .. blocks-1 of the batch
-template <bool NN>
-hipError_t launch_blocks(const GemmArgs &g, hipStream_t s, int blocks) {
-  using C = BlockCfg<8, 4>;
-  const hipError_t e = prepare_kernel<gemm_kernel16<NN, 4>, C::LDS_BYTES>();
+template <bool NN, int MB, int NB>
+constexpr auto block_kernel() {
+  if constexpr (MB == 8) return &gemm_kernel16<NN, NB>;
+  else return &gemm_kernel16_rows<NN, MB, NB>;
+}
+// the macro tiles 0 .. tiles-1 of the batch
+template <bool NN, int MB, int NB>
+hipError_t launch_blocks(const GemmArgs &g, hipStream_t s, int tiles) {
+  using C = BlockCfg<MB, NB>;
+  constexpr auto kern = block_kernel<NN, MB, NB>();
+  const hipError_t e = prepare_kernel<kern, C::LDS_BYTES>();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((gemm_kernel16<NN, 4>), dim3(blocks), dim3(512), C::LDS_BYTES, s, (const _Float16 *)g.A, (const _Float16 *)g.B,
-                     (const _Float16 *)g.C, (_Float16 *)g.D, g.M, g.N, g.K, g.alpha, g.beta);
+  hipLaunchKernelGGL(kern, dim3(tiles), dim3(512), C::LDS_BYTES, s, (const _Float16 *)g.A, (const _Float16 *)g.B, (const _Float16 *)g.C,
+                     (_Float16 *)g.D, g.M, g.N, g.K, g.alpha, g.beta);
   return hipGetLastError();
 }
 
@@ -730,10 +746,10 @@ constexpr int kCus = 256;
 // 104 0.96, 0.97, 0.96, 0.94 and 0.99, 0.98, 0.97, 0.95; 120 0.97, 0.97, 0.96, 0.95 and 1.00, 0.99, 0.98, 0.95; 128 0.98, 0.99, 0.98, 0.97
 // and 1.01, 1.00, 0.99, 0.96.  Worst found: M=6144 N=4096 (128 left) 1.03, 1.03, 1.00, 0.99, 19.4 -> 20.0 us at K=64.
 template <bool NN>
-hipError_t launch_f16(const GemmArgs &g, hipStream_t s, int blocks) {
+hipError_t launch_blocks_and_tiles(const GemmArgs &g, hipStream_t s, int blocks) {
   const int left = blocks % kCus, whole = left > kCus / 2 ? blocks : blocks - left;
   if (whole) {
-    const hipError_t e = launch_blocks<NN>(g, s, whole);
+    const hipError_t e = launch_blocks<NN, 8, 4>(g, s, whole);
     if (e != hipSuccess || whole == blocks) return e;
   }
   if (left * HTile<NN, 32, 32>::SUB <= kCus) return launch_tiles16<NN, 32, 32>(g, s, whole, left);
@@ -741,6 +757,46 @@ hipError_t launch_f16(const GemmArgs &g, hipStream_t s, int blocks) {
   if (left * HTile<NN, 128, 64>::SUB <= kCus) return launch_tiles16<NN, 128, 64>(g, s, whole, left);
   if (left * HTile<NN, 128, 128>::SUB <= kCus) return launch_tiles16<NN, 128, 128>(g, s, whole, left);
   return launch_tiles16<NN, 256, 128>(g, s, whole, left);
+}
+
+// fp16, more than half a round of 256 x 256 blocks: rounds of other macro tiles where these waste less of the chip.  Times in rounds of
+// 256 x 256 tiles (106 us at K=4096): a full one of 192 x 256 tiles 0.772, 256 x 192 0.792, 192 x 192 0.622, 320 x 256 1.192; one of which a
+// share f is filled takes (1 + f)/2 of that, because the idle CUs leave the others their power; the smaller tiles behind whole rounds
+// (launch_blocks_and_tiles) 0.06, 0.14, 0.22, 0.40 and 0.55 of a round by size when they fill it.  231 drawn products of 129 to 1100 blocks,
+// K from 192, TN and NN, with and without C: 0.945 of the time in the geometric mean (the best choice for each: 0.943), worst 1.04.
+// us, 256 x 256 and small tiles -> the rule: 5120 x 4096 x 4096 TN 146 -> 129 and with C NN 177 -> 145 (256 tiles of 320 x 256); M=N=3072 K=4096
+// 81 -> 68 (256 of 192 x 192), K=512 18.6 -> 14.7; 3072 x 4096 x 4096 89 -> 84 (192 x 256).  Not built: 320 x 192 and 192 x 320 (103.6 against
+// 102.7 and 100.7 against 102.0 for 240 blocks), 256 x 128 and less by this kernel (64.3 against 61.8 for a round of 256 x 128).
+template <bool NN>
+hipError_t launch_f16(const GemmArgs &g, hipStream_t s, int blocks) {
+  if (blocks <= kCus / 2) return launch_blocks_and_tiles<NN>(g, s, blocks);
+  const auto rounds = [](long long tiles) {
+    const int part = (int)(tiles % kCus);
+    return (double)(tiles / kCus) + (part ? 0.5 + 0.5 * part / kCus : 0.0);
+  };
+  const int left = blocks % kCus;
+  double best = rounds(blocks);
+  if (left > 0 && left <= kCus / 2) {
+    const int sub = left <= 4 ? 64 : left <= 16 ? 16 : left <= 32 ? 8 : left <= 64 ? 4 : 2;
+    const double full = sub == 64 ? 0.06 : sub == 16 ? 0.14 : sub == 8 ? 0.22 : sub == 4 ? 0.40 : 0.55;
+    best = blocks / kCus + full * (0.6 + 0.4 * left * sub / kCus) + 0.03;
+  }
+  int rows = 256, cols = 256, tiles = 0;
+  const auto offer = [&](int r, int c, double round) {
+    // (a tile against the edge needs a whole one; 32-bit byte offsets within a tile's rows)
+    if (g.M < r || g.N < c || (long long)r * g.K * 2 >= (1LL << 32)) return;
+    const long long n = (long long)((g.M + r - 1) / r) * ((g.N + c - 1) / c) * g.batch;
+    const double t = round * rounds(n);
+    if (t < best) best = t, rows = r, cols = c, tiles = (int)n;
+  };
+  offer(192, 256, 0.772);
+  offer(256, 192, 0.792);
+  offer(192, 192, 0.622);
+  offer(320, 256, 1.192);
+  if (!tiles) return launch_blocks_and_tiles<NN>(g, s, blocks);
+  if (rows == 320) return launch_blocks<NN, 10, 4>(g, s, tiles);
+  if (rows == 256) return launch_blocks<NN, 8, 3>(g, s, tiles);
+  return cols == 256 ? launch_blocks<NN, 6, 4>(g, s, tiles) : launch_blocks<NN, 6, 3>(g, s, tiles);
 }
 
 // fp32: the multiplies bound every tile size, so what counts is how full the last round of the CUs is: the tile whose rounds,
@@ -757,7 +813,11 @@ hipError_t launch_f32(const GemmArgs &g, hipStream_t s, int blocks) {
 
 template <bool NN>
 hipError_t prepare_f16() {
-  const hipError_t e[] = {prepare_kernel<gemm_kernel16<NN, 4>, BlockCfg<8, 4>::LDS_BYTES>(),
+  const hipError_t e[] = {prepare_kernel<block_kernel<NN, 8, 4>(), BlockCfg<8, 4>::LDS_BYTES>(),
+                          prepare_kernel<block_kernel<NN, 8, 3>(), BlockCfg<8, 3>::LDS_BYTES>(),
+                          prepare_kernel<block_kernel<NN, 6, 4>(), BlockCfg<6, 4>::LDS_BYTES>(),
+                          prepare_kernel<block_kernel<NN, 6, 3>(), BlockCfg<6, 3>::LDS_BYTES>(),
+                          prepare_kernel<block_kernel<NN, 10, 4>(), BlockCfg<10, 4>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 256, 128>, HTile<NN, 256, 128>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 128, 128>, HTile<NN, 128, 128>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 128, 64>, HTile<NN, 128, 64>::LDS_BYTES>(),

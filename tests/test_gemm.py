@@ -133,6 +133,35 @@ def test_last_round_in_tiles_bit_exact(K, layout):
     assert np.array_equal(got.cpu().numpy()[rows], want)
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("L,M,N", [
+    (1, 3072, 3072),     # 192 x 192 tiles, 256 of them
+    (2, 1280, 3328),     # ... the last ones of two problems against both edges
+    (1, 3072, 4096),     # 192 x 256
+    (1, 1280, 7168),     # ... the last row of tiles against the edge
+    (1, 4096, 3072),     # 256 x 192
+    (1, 1792, 5888),     # ... the last column of tiles against the edge
+    (1, 2560, 6656),     # 320 x 256
+    (1, 2816, 6144)])    # ... the last row of tiles against the edge
+@pytest.mark.parametrize("K", [64, 192, 448])
+def test_macro_tiles_beyond_half_a_round_bit_exact(L, M, N, K, layout):
+    # one, three and seven K tiles; D over C: what two tiles at an edge both cover is read and stored once
+    import torch
+    rng = np.random.default_rng(M + N + K)
+    a = rng.integers(-8, 9, (L, M, K)).astype(np.float32)
+    b = rng.integers(-8, 9, (L, N, K)).astype(np.float32)
+    c = rng.integers(-8, 9, (L, M, N)).astype(np.float32)
+    bt = b if layout == 0 else np.ascontiguousarray(b.transpose(0, 2, 1))
+    d = to_dev(c.astype(np.float16))
+    pkg.gemm(to_dev(a.astype(np.float16)), to_dev(bt.astype(np.float16)), c=d, alpha=0.5, beta=-1.0, layout=layout, out=d)
+    torch.cuda.synchronize()
+    rows = np.unique(np.concatenate([np.arange(3, M, 61), np.arange(M - 70, M)])).astype(np.int32)
+    got = d.cpu().numpy()
+    for i in range(L):
+        want = (0.5 * oracle.gemm_f32(a[i], b[i], rows=rows) - c[i][rows]).astype(np.float16)
+        assert np.array_equal(got[i][rows], want), i
+
+
 def test_fp32_uniform_inputs():
     # the CuTe example's type 1 (float operands, gemm.cu:677-684), U(-1,1) data (:482-485).  Both sides accumulate in
     # fp32 in different orders: |error| <~ sqrt(K) * 2^-24 * |terms|
