@@ -318,7 +318,10 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
   // the dependency through the asm statements)
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
   // ---- epilogue: D = alpha * acc + beta * C in fp32, each row of blocks staged through the wave's own LDS region and stored as
-  // whole rows, 16 bytes per lane
+  // whole rows, 16 bytes per lane, through the L2 to memory: a round of tiles writes as much as the L2s hold, and left there as dirty
+  // lines it has to be written out before the operands of the next round find room (us, left in the L2 / through it: 8192 x 8192
+  // with K=320 80.8 / 62.5, K=512 84.7 / 78.9, K=768 104.4 / 102.7, K=64 36.4 / 36.5; 4096 x 4096 x 320 17.5 / 16.4; 4 waves, whose stores
+  // came out more slowly, 67.8 with K=320).
   constexpr int EPL = 8, LPR = NB * 2, CHUNKS = 16 * LPR;   // halves per lane and store, lanes per row
   const bool with_c = Cin != nullptr && beta != 0.f;
   char *et = smem + wave * (16 * C::E_PITCH);
@@ -369,7 +372,7 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
       half8 o;
 #pragma unroll
       for (int j = 0; j < EPL; ++j) o[j] = (T)v[j];
-      *(half8 *)(D + off) = o;
+      store16_through(D + off, o);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();  // the region is rewritten by the next row of blocks
@@ -655,7 +658,7 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
     OutV o;
 #pragma unroll
     for (int x = 0; x < EPL; ++x) o[x] = (T)v[x];
-    *(OutV *)(D + off) = o;
+    store16_through(D + off, o);
   }
 }
 
