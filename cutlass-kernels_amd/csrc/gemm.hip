@@ -150,6 +150,7 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
   const int tiles_n = (N + C::BNT - 1) / C::BNT, tiles_m = (M + C::BMT - 1) / C::BMT;
   int t = xcd_remap(blockIdx.x, gridDim.x);
   const int64_t batch = t / (tiles_m * tiles_n);  // packed strides M*K, N*K, M*N (reference: gemm.cu:519-521)
+  const int batches = ((int)gridDim.x + tiles_m * tiles_n - 1) / (tiles_m * tiles_n);
   t -= (int)batch * tiles_m * tiles_n;
   constexpr int GROUP = 8;
   const int per_group = GROUP * tiles_n;
@@ -335,16 +336,27 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
   };
   // All of C that this wave needs is asked for at once, into the registers that the main loop has left: a load per store had its latency
   // in every pass (us: M=N=4096 K=192 20.1 -> 18.3; two of 4096 x 2048 x 512 NN 28.0 -> 26.4; 8192 x 8192 x 2048 286.0 -> 271.0).
+  // From 64 MB on it is read past the caches, where a C of that size is not anyway and its lines would take the place of others; smaller
+  // ones often lie in the 256 MB behind the L2s, written by the call before.  us, past the caches / through them, K=512, three sets of
+  // operands in turn: 33 MB 27.6 / 25.1, 50 MB 43.2 / 36.6, 67 MB 54.5 / 55.3, 101 MB 74.5 / 81.1, 134 MB 101.5 / 123.3.
+  const bool big_c = (int64_t)M * N * batches * 2 >= (64 << 20);
   half8 cv[MB][PASSES];
-  if (with_c) {
+  const auto read_c = [&](auto &&load) __attribute__((always_inline)) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int pass = 0; pass < PASSES; ++pass) {
         int row, col;
         int64_t off;
-        if (place(mb, pass, row, col, off)) cv[mb][pass] = *(const half8 *)(Cin + off);
+        if (place(mb, pass, row, col, off)) cv[mb][pass] = load((const half8 *)(Cin + off));
       }
+  };
+  if (with_c && big_c) {
+    asm volatile("; C past the caches");   // (or the compiler makes one branch of the two)
+    read_c([](const half8 *p) __attribute__((always_inline)) { return __builtin_nontemporal_load(p); });
+    asm volatile("; C past the caches");
+  } else if (with_c) {
+    read_c([](const half8 *p) __attribute__((always_inline)) { return *p; });
   }
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
