@@ -131,12 +131,13 @@ __device__ __forceinline__ void lds_dma16(const void *base, uint32_t lane_off, u
 #pragma clang diagnostic pop
 __device__ __forceinline__ void wait_lds_dma() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// A 16-byte store that goes through the L2 to memory (sc1) instead of staying there as a dirty line.  (The data registers must not be
-// written in the next wait state, which the compiler cannot know of a store inside an asm statement: hence the s_nop.)
+// A 16-byte store that goes through the L2 to memory (sc1) instead of staying there as a dirty line.  (The data registers of a
+// store of more than 8 bytes must not be written by a vector instruction in the next two wait states; the compiler does not look for that
+// behind an asm statement: hence the s_nop.)
 template <class V>
 __device__ __forceinline__ void store16_through(void *p, const V &v) {
   static_assert(sizeof(V) == 16, "four dwords");
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 
 // The lane number, computed on the spot (two v_mbcnt) from an operand the compiler cannot see through: neither kept in a
