@@ -739,7 +739,7 @@ fmha_fwd_kernel(const FmhaArgs a) {
     for (int pass = 0; pass < 32 / RPP; ++pass) {
       const int row = pass * RPP + orow_l;
       const int4v val = *(const int4v *)(ot + row * C::O_PITCH + ochunk * 16);
-      if (live) *(int4v *)(Op + (int64_t)(q0 + row) * ld + ochunk * 8) = val;
+      if (live) store16_through(Op + (int64_t)(q0 + row) * ld + ochunk * 8, val);
     }
   }
   if (live && (a.row_max || a.row_sum)) {

@@ -392,7 +392,7 @@ fmha_fwd_kernel16(const FmhaArgs a) {
     for (int pass = 0; pass < 32 / RPP; ++pass) {
       const int row = pass * RPP + orow_l;
       const int4v val = *(const int4v *)(ot + row * C::O_PITCH + ochunk * 16);
-      if (q0 < a.Sq) *(int4v *)(Op + (int64_t)(q0 + row) * ld + ochunk * 8) = val;
+      if (q0 < a.Sq) store16_through(Op + (int64_t)(q0 + row) * ld + ochunk * 8, val);
     }
   }
   if (q0 < a.Sq && want_taps) {
