@@ -291,7 +291,10 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
     tile_ptrs(kt + 2 < k_tiles ? kt + 2 : k_tiles - 1, ga, gb);  // clamped at the end: a surplus tile is loaded and dropped
 #pragma unroll
     for (int i = 0; i < 2 * S; ++i) {
-      const int x = i / NB, nb = i % NB, s2 = i / S, mb = x % MB;   // x: the m block, counted through both K-steps
+      // x: the m block, counted through both K-steps.  The n blocks are walked there and back, so that from one multiply to the next only
+      // one operand changes: an operand that stays costs less power (register-only loops on U(-1,1) operands: 1893 TFLOP/s with one
+      // operand changing, 1815 with both; 8192^3 819.0 -> 815.9 us, 8192 x 8192 x 4096 NN 436.4 -> 431.4).
+      const int x = i / NB, nb = x & 1 ? NB - 1 - i % NB : i % NB, s2 = i / S, mb = x % MB;
       if (i == sl.barrier) __syncthreads();
       // written out so that the accumulator is updated in place: through the builtin the register allocator moves the small
       // accumulators between the two halves of the register file.  Nothing but these multiplies touches the accumulators inside the
