@@ -428,11 +428,15 @@ struct TileCfg {
   static constexpr int E_PITCH = BNT * 4 + 16, E_BYTES = KG * BMT * E_PITCH;  // epilogue: fp32 sums, rows padded
   static constexpr int LDS_BYTES = ST * STAGE > E_BYTES ? ST * STAGE : E_BYTES;
   static constexpr int FB = ES == 2 ? 16 : 32;                                // block edge of the MFMA
+  static constexpr int RPP = THREADS * (16 / ES) / BNT, PASSES = (BMT + RPP - 1) / RPP;   // epilogue: rows per pass
   static_assert(A_PPW * WPG * 8 == BMT && PPW * WPG * 8 == BMT + BNT, "whole 1 KB copies per wave");
   static_assert(LDS_BYTES <= 160 * 1024 && ST >= 2, "stages");
 };
 
-template <class C>
+// AHEAD: there is a C, and all of it that a lane needs is asked for before the sums meet, not pass by pass (us: 2048 x 2048 x 512 NN 11.1 ->
+// 9.4, 2048 x 4096 x 512 15.4 -> 13.0, fp32 4096 x 4096 x 512 140.2 -> 131.5; in front of the main loop 10.3, 15.0 and 133.4).  For tiles
+// of several passes, in kernels of their own: with both epilogues in one kernel a call without C takes 1 % longer.
+template <class C, bool AHEAD = false>
 __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, const typename C::T *__restrict__ B,
                                           const typename C::T *__restrict__ Cin, typename C::T *__restrict__ D, int M, int N, int K,
                                           float alpha, float beta, int block0) {
@@ -632,6 +636,14 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
 
   // ---- epilogue: every group leaves its fp32 sums in the LDS as rows of C; they are added up, scaled and rounded once on
   // the way out, 16 bytes per lane of whole tile rows
+  constexpr int PASSES = C::PASSES;
+  std::conditional_t<F16, half8, f32x4> c_ahead[AHEAD ? PASSES : 1];
+  if constexpr (AHEAD) {
+    constexpr int EPL = 16 / ES, LPR = C::BNT / EPL, RPP = C::THREADS / LPR;
+#pragma unroll
+    for (int pass = 0; pass < PASSES; ++pass)
+      c_ahead[pass] = *(const decltype(&c_ahead[0]))(Cin + (int64_t)(m0 + pass * RPP + tid / LPR) * N + n0 + (tid % LPR) * EPL);
+  }
   __syncthreads();
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
@@ -648,11 +660,11 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   __syncthreads();
   constexpr int EPL = 16 / ES, LPR = C::BNT / EPL, RPP = C::THREADS / LPR;
   using OutV = std::conditional_t<F16, half8, f32x4>;
-  const bool with_c = Cin != nullptr && beta != 0.f;
+  const bool with_c = AHEAD || (Cin != nullptr && beta != 0.f);
   const int e_row = tid / LPR, e_col = (tid % LPR) * EPL;
   static_assert(C::BMT % RPP == 0 || RPP > C::BMT, "whole passes");
 #pragma unroll
-  for (int pass = 0; pass < (C::BMT + RPP - 1) / RPP; ++pass) {
+  for (int pass = 0; pass < PASSES; ++pass) {
     const int row = pass * RPP + e_row;
     if (RPP > C::BMT && row >= C::BMT) break;
     const int64_t off = (int64_t)(m0 + row) * N + n0 + e_col;
@@ -666,7 +678,7 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
       for (int x2 = 0; x2 < 4; ++x2) v[4 * q + x2] = alpha * x[x2];
     }
     if (with_c) {
-      const OutV cv = *(const OutV *)(Cin + off);
+      const OutV cv = AHEAD ? c_ahead[AHEAD ? pass : 0] : *(const OutV *)(Cin + off);
 #pragma unroll
       for (int x = 0; x < EPL; ++x) v[x] += beta * (float)cv[x];
     }
@@ -697,6 +709,20 @@ __global__ void __launch_bounds__((HTile<NN, ROWS, COLS>::THREADS))
 gemm_kernel16_tile(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
                    _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta, int block0) {
   gemm_tile<HTile<NN, ROWS, COLS>>(A, B, Cin, D, M, N, K, alpha, beta, block0);
+}
+
+template <bool NN, int ROWS, int COLS>
+__global__ void __launch_bounds__((HTile<NN, ROWS, COLS>::THREADS))
+gemm_kernel16_tile_c(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
+                     _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta, int block0) {
+  gemm_tile<HTile<NN, ROWS, COLS>, true>(A, B, Cin, D, M, N, K, alpha, beta, block0);
+}
+
+template <int EDGE>
+__global__ void __launch_bounds__(FTile<EDGE>::THREADS)
+gemm_kernel_f32_c(const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ Cin, float *__restrict__ D,
+                  int M, int N, int K, float alpha, float beta, int block0) {
+  gemm_tile<FTile<EDGE>, true>(A, B, Cin, D, M, N, K, alpha, beta, block0);
 }
 
 template <int EDGE>
@@ -744,11 +770,19 @@ hipError_t launch_tiles(const GemmArgs &g, hipStream_t s, int block0, int blocks
 }
 template <bool NN, int ROWS, int COLS>
 hipError_t launch_tiles16(const GemmArgs &g, hipStream_t s, int block0, int blocks) {
-  return launch_tiles<HTile<NN, ROWS, COLS>, gemm_kernel16_tile<NN, ROWS, COLS>>(g, s, block0, blocks);
+  using C = HTile<NN, ROWS, COLS>;
+  if constexpr (C::PASSES > 1) {
+    if (g.C && g.beta != 0.f) return launch_tiles<C, gemm_kernel16_tile_c<NN, ROWS, COLS>>(g, s, block0, blocks);
+  }
+  return launch_tiles<C, gemm_kernel16_tile<NN, ROWS, COLS>>(g, s, block0, blocks);
 }
 template <int EDGE>
 hipError_t launch_tiles32(const GemmArgs &g, hipStream_t s, int blocks) {
-  return launch_tiles<FTile<EDGE>, gemm_kernel_f32<EDGE>>(g, s, 0, blocks);
+  using C = FTile<EDGE>;
+  if constexpr (C::PASSES > 1) {
+    if (g.C && g.beta != 0.f) return launch_tiles<C, gemm_kernel_f32_c<EDGE>>(g, s, 0, blocks);
+  }
+  return launch_tiles<C, gemm_kernel_f32<EDGE>>(g, s, 0, blocks);
 }
 
 constexpr int kCus = 256;
@@ -839,6 +873,9 @@ hipError_t prepare_f16() {
                           prepare_kernel<gemm_kernel16_tile<NN, 256, 128>, HTile<NN, 256, 128>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 128, 128>, HTile<NN, 128, 128>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 128, 64>, HTile<NN, 128, 64>::LDS_BYTES>(),
+                          prepare_kernel<gemm_kernel16_tile_c<NN, 256, 128>, HTile<NN, 256, 128>::LDS_BYTES>(),
+                          prepare_kernel<gemm_kernel16_tile_c<NN, 128, 128>, HTile<NN, 128, 128>::LDS_BYTES>(),
+                          prepare_kernel<gemm_kernel16_tile_c<NN, 128, 64>, HTile<NN, 128, 64>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 64, 64>, HTile<NN, 64, 64>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 32, 32>, HTile<NN, 32, 32>::LDS_BYTES>()};
   for (hipError_t x : e)
@@ -860,6 +897,8 @@ hipError_t prepare_gemm() {
   if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32<128>, FTile<128>::LDS_BYTES>();
   if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32<64>, FTile<64>::LDS_BYTES>();
   if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32<32>, FTile<32>::LDS_BYTES>();
+  if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32_c<128>, FTile<128>::LDS_BYTES>();
+  if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32_c<64>, FTile<64>::LDS_BYTES>();
   return e;
 }
 
