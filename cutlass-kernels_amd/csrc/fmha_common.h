@@ -134,7 +134,8 @@ __device__ __forceinline__ void wait_lds_dma() { asm volatile("s_waitcnt vmcnt(0
 // A 16-byte store that goes through the L2 to memory (sc1) instead of staying there as a dirty line: the end of a kernel then has
 // nothing to write out, and the operands of later workgroups find room.  523 drawn attention calls 0.984 of the time (geometric mean), the
 // shortest keys most (us: hybrid 8 x 7776 rows x 256 keys 11.7 -> 9.9, fp16 65 x 640 x 192 11.7 -> 10.3, e4m3 90 x 640 x 128 8.4 -> 7.3).  Not in
-// the key-split kernel, where it gained nothing and cost up to 2.6 % (36 x 160 x 6976: 44.9 -> 46.1), nor for its partial results, which
+// the persistent kernels, whose next item waits for its copies behind the stores (fp16 B=8 H=16 S=2048 D=128 220.9 -> 222.2, e4m3 B=4 H=16
+// S=4096 256.6 -> 258.0), in the key-split kernel, where it gained nothing and cost up to 2.6 % (36 x 160 x 6976: 44.9 -> 46.1), nor for its partial results, which
 // fmha_combine reads back (16.2 -> 16.5).  (The data registers of a
 // store of more than 8 bytes must not be written by a vector instruction in the next two wait states; the compiler does not look for that
 // behind an asm statement: hence the s_nop.)
