@@ -10,15 +10,14 @@
 // read with ds_read_b64_tr_b16 exactly as V is in the attention kernel.  The reference writes C column-major
 // (:386-389); C and D are row-major here.  gfx950 has no tf32/xf32 MFMA: fp32 operands multiply in full fp32.
 //
-// Two kernels.  gemm_kernel16 (fp16): 8 waves, two per SIMD, on a 256 x 256 macro tile, for as many of those as fill the CUs
+// gemm_kernel16 (fp16): 8 waves, two per SIMD, on a 256 x 256 macro tile, for as many of those as fill the CUs
 // in whole rounds; wave (wm, wn) of a 2 x 4 grid owns 128 x 64 of C, its 128 accumulator registers in the AGPR half of the
 // register file, 8 x 4 blocks of 16x16x32 MFMAs (the power-efficient shape on this board).  K tiles are 128 bytes deep and go
 // global -> registers -> LDS: 16-byte buffer loads a tile ahead (scalar resource + 32-bit lane offset, no vector address
 // arithmetic), parked in one of two 64 KB LDS stages by ds_write_b128 while the other stage multiplies, one barrier per tile;
 // every multiply is followed by at most one fragment read or one store/load pair, see the pipeline comment at BlockCfg.
-// (Global -> LDS copy instructions instead of the register path, through a ring of four 32-deep stages and spread the
-// same way, measured 1.57 against 1.94 PFLOP/s on constant operands: with one wave per SIMD an LDS-destination load
-// holds up the issuing wave and with it the MFMA pipe.)
+// gemm_kernel16_rows, gemm_kernel16<NN, 3>: the same kernel on 192 x 192, 192 x 256, 256 x 192 and 320 x 256 macro tiles, for products whose
+// rounds these fill better (launch_f16).
 // gemm_tile (gemm_kernel16_tile, gemm_kernel_f32): the smaller macro tiles, for what 256 x 256 blocks leave over and for all
 // fp32 products (v_mfma_f32_32x32x2_f32), whose 16 times slower multiplies any tile can feed.
 // The MFMA computes the TRANSPOSED block (rows = n, columns = m); the epilogue stages blocks through LDS and stores whole
