@@ -135,14 +135,16 @@ __device__ __forceinline__ void wait_lds_dma() { asm volatile("s_waitcnt vmcnt(0
 // nothing to write out, and the operands of later workgroups find room.  523 drawn attention calls 0.984 of the time (geometric mean), the
 // shortest keys most (us: hybrid 8 x 7776 rows x 256 keys 11.7 -> 9.9, fp16 65 x 640 x 192 11.7 -> 10.3, e4m3 90 x 640 x 128 8.4 -> 7.3).  Not in
 // the persistent kernels, whose next item waits for its copies behind the stores (fp16 B=8 H=16 S=2048 D=128 220.9 -> 222.2, e4m3 B=4 H=16
-// S=4096 256.6 -> 258.0), in the key-split kernel, where it gained nothing and cost up to 2.6 % (36 x 160 x 6976: 44.9 -> 46.1), nor for its partial results, which
-// fmha_combine reads back (16.2 -> 16.5).  (The data registers of a
-// store of more than 8 bytes must not be written by a vector instruction in the next two wait states; the compiler does not look for that
-// behind an asm statement: hence the s_nop.)
+// S=4096 256.6 -> 258.0), in the key-split kernel, where it gained nothing and cost up to 2.6 % (36 x 160 x 6976: 44.9 -> 46.1), nor for its
+// partial results, which fmha_combine reads back (16.2 -> 16.5).
+// The builtin and not an asm statement: the compiler then counts the store, so that a wait for a load does not become one for the stores
+// behind it (2048 x 4096 x 512 with C 14.0 -> 13.7), and keeps the two wait states in which no vector instruction may write the data
+// registers of a store of more than 8 bytes (with one of them rows came out wrong).
 template <class V>
 __device__ __forceinline__ void store16_through(void *p, const V &v) {
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   static_assert(sizeof(V) == 16, "four dwords");
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+  __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) u32x4 *)p, __builtin_bit_cast(u32x4, v), "agent");
 }
 
 // The lane number, computed on the spot (two v_mbcnt) from an operand the compiler cannot see through: neither kept in a

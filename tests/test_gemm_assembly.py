@@ -1,0 +1,43 @@
+"""What the GEMM kernels' gfx950 assembly has to look like, read from a compile of gemm.hip with the library's flags (no GPU): where a
+matrix instruction is an asm statement, or a wait stands between two stores, the sources alone do not show it."""
+import os
+import re
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cutlass-kernels_amd", "csrc")
+FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+         "-Wno-unused-command-line-argument", "-fno-gpu-rdc", "--offload-device-only"]
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """name -> its instructions, in the order of the text"""
+    out = str(tmp_path_factory.mktemp("asm") / "gemm.s")
+    subprocess.run(["/opt/rocm/bin/hipcc"] + FLAGS + ["-S", "-o", out, "gemm.hip"], cwd=CSRC, check=True, capture_output=True)
+    found = {}
+    for m in re.finditer(r"^(_ZN3cfk12_GLOBAL__N_1\d+(gemm_kernel\w*?)I(\S*?)EEv\S*):.*?\n(.*?)\.Lfunc_end", open(out).read(), re.S | re.M):
+        name = m.group(2) + "<" + ",".join(re.findall(r"L[bi](\d+)", m.group(3))) + ">"
+        lines = [x.strip() for x in m.group(4).splitlines()]
+        found[name] = [x for x in lines if x and x[0] not in ";."]
+    return found
+
+
+def _through(ins):
+    return [i for i, x in enumerate(ins) if x.startswith("global_store_dwordx4") and x.endswith("sc1")]
+
+
+def _waits(ins):
+    """(index, n) of every wait for all but n vector memory instructions"""
+    return [(i, int(m.group(1))) for i, x in enumerate(ins) if (m := re.search(r"s_waitcnt.*vmcnt\((\d+)\)", x))]
+
+
+@pytest.mark.parametrize("name", ["gemm_kernel16_tile_c<%d,%s>" % (nn, t) for nn in (0, 1) for t in ("256,128", "128,128", "128,64")] +
+                         ["gemm_kernel_f32_c<128>", "gemm_kernel_f32_c<64>"])
+def test_tiles_over_c_do_not_wait_for_their_stores(kernels, name):
+    ins = kernels[name]
+    st = _through(ins)
+    assert len(st) >= 2
+    # all of C is asked for in front of the first store, so the last piece of it lies behind none of them
+    assert min([n for i, n in _waits(ins) if st[0] < i < st[-1]], default=len(st)) >= len(st) - 1, name
