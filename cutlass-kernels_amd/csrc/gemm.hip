@@ -326,72 +326,92 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
   // with K=320 80.8 / 62.5, K=512 84.7 / 78.9, K=768 104.4 / 102.7, K=64 36.4 / 36.5; 4096 x 4096 x 320 17.5 / 16.4; 4 waves, whose stores
   // came out more slowly, 67.8 with K=320).
   constexpr int EPL = 8, LPR = NB * 2, CHUNKS = 16 * LPR;   // halves per lane and store, lanes per row
-  const bool with_c = Cin != nullptr && beta != 0.f;
-  char *et = smem + wave * (16 * C::E_PITCH);
   constexpr int PASSES = (CHUNKS + 63) / 64;
-  const auto place = [&](int mb, int pass, int &row, int &col, int64_t &off) __attribute__((always_inline)) {
-    const int idx = pass * 64 + lane;
-    row = idx / LPR, col = idx % LPR * EPL;
-    const int gm = m0 + (wm * MB + mb) * 16 + row, gn = n0 + wn * NB * 16 + col;
-    off = (int64_t)gm * N + gn;
-    return !((CHUNKS % 64 != 0 && idx >= CHUNKS) || gm < m_own || gn < n_own);
+  char *et = smem + wave * (16 * C::E_PITCH);
+  const int el = fresh_lane();   // (no register is kept for it across the main loop: 320 rows NN have none)
+  // Three forms, so that a call without C meets no wait for it.
+  enum { NO_C, C_CACHED, C_STREAMED };
+  // C is asked for in front of the first store, into the registers that the main loop has left: a load per store had its latency in every
+  // pass (us: M=N=4096 K=192 20.1 -> 18.3; two of 4096 x 2048 x 512 NN 28.0 -> 26.4; 8192 x 8192 x 2048 286.0 -> 271.0).  Up to 256 rows all of
+  // it, and waited for once: between the stores the waits would in the end be waits for stores, which may be left out at an edge and so
+  // don't count (M=N=4096 K=192 17.5 -> 16.9).  With 320 rows 160 accumulators leave no room for its 80 registers: five rows of blocks ahead of
+  // the one that is stored (5 or 6: the same; all of it, through scratch: two of 4352 x 4096 x 192 50.2 -> 41.3, 5120 x 4096 x 512 36.5 -> 32.1,
+  // x 4096 138.5 -> 135.6).
+  constexpr int C_AHEAD = MB > 8 ? 5 : MB;
+  half8 cv[C_AHEAD][PASSES];
+  const auto read_c = [&](auto form, int mb, int pass) __attribute__((always_inline)) {
+    int idx = pass * 64 + el;
+    if (CHUNKS % 64 != 0) idx = idx < CHUNKS ? idx : CHUNKS - 1;
+    int gm = m0 + (wm * MB + mb) * 16 + idx / LPR, gn = n0 + wn * NB * 16 + idx % LPR * EPL;
+    gm = gm < m_own ? m_own : gm;   // (what a neighbour stores is not used: some line that is read anyway)
+    gn = gn < n_own ? n_own : gn;
+    const half8 *p = (const half8 *)(Cin + (int64_t)gm * N + gn);
+    cv[mb % C_AHEAD][pass] = form.value == C_STREAMED ? __builtin_nontemporal_load(p) : *p;
   };
-  // All of C that this wave needs is asked for at once, into the registers that the main loop has left: a load per store had its latency
-  // in every pass (us: M=N=4096 K=192 20.1 -> 18.3; two of 4096 x 2048 x 512 NN 28.0 -> 26.4; 8192 x 8192 x 2048 286.0 -> 271.0).
-  // From 64 MB on it is read past the caches, where a C of that size is not anyway and its lines would take the place of others; smaller
-  // ones often lie in the 256 MB behind the L2s, written by the call before.  us, past the caches / through them, K=512, three sets of
-  // operands in turn: 33 MB 27.6 / 25.1, 50 MB 43.2 / 36.6, 67 MB 54.5 / 55.3, 101 MB 74.5 / 81.1, 134 MB 101.5 / 123.3.
-  const bool big_c = (int64_t)M * N * batches * 2 >= (64 << 20);
-  half8 cv[MB][PASSES];
-  const auto read_c = [&](auto &&load) __attribute__((always_inline)) {
+  const auto epilogue = [&](auto form) __attribute__((always_inline)) {
+    constexpr bool WITH_C = form.value != NO_C;
+    if constexpr (WITH_C) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+      for (int mb = 0; mb < C_AHEAD; ++mb)
+#pragma unroll
+        for (int pass = 0; pass < PASSES; ++pass) read_c(form, mb, pass);
+      if constexpr (C_AHEAD == MB) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) *(f32x4 *)(et + (el & 15) * C::E_PITCH + (nb * 16 + 4 * (el >> 4)) * 4) = acc[mb][nb];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
       for (int pass = 0; pass < PASSES; ++pass) {
-        int row, col;
-        int64_t off;
-        if (place(mb, pass, row, col, off)) cv[mb][pass] = load((const half8 *)(Cin + off));
+        half8 cm{};
+        if constexpr (WITH_C) {
+          cm = cv[mb % C_AHEAD][pass];
+          if (mb + C_AHEAD < MB) read_c(form, mb + C_AHEAD, pass);
+        }
+        const int idx = pass * 64 + el, row = idx / LPR, col = idx % LPR * EPL;
+        const int gm = m0 + (wm * MB + mb) * 16 + row, gn = n0 + wn * NB * 16 + col;
+        if ((CHUNKS % 64 != 0 && idx >= CHUNKS) || gm < m_own || gn < n_own) continue;
+        float v[EPL];
+#pragma unroll
+        for (int q = 0; q < EPL / 4; ++q) {
+          const f32x4 x = *(const f32x4 *)(et + row * C::E_PITCH + (col + 4 * q) * 4);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[4 * q + j] = alpha * x[j];
+        }
+        if constexpr (WITH_C) {
+#pragma unroll
+          for (int j = 0; j < EPL; ++j) v[j] += beta * (float)cm[j];
+        }
+        half8 o;
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) o[j] = (T)v[j];
+        store16_through(D + (int64_t)gm * N + gn, o);
       }
-  };
-  if (with_c && big_c) {
-    asm volatile("; C past the caches");   // (or the compiler makes one branch of the two)
-    read_c([](const half8 *p) __attribute__((always_inline)) { return __builtin_nontemporal_load(p); });
-    asm volatile("; C past the caches");
-  } else if (with_c) {
-    read_c([](const half8 *p) __attribute__((always_inline)) { return *p; });
-  }
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) *(f32x4 *)(et + c * C::E_PITCH + (nb * 16 + 4 * g) * 4) = acc[mb][nb];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int pass = 0; pass < PASSES; ++pass) {
-      int row, col;
-      int64_t off;
-      if (!place(mb, pass, row, col, off)) continue;
-      float v[EPL];
-#pragma unroll
-      for (int q = 0; q < EPL / 4; ++q) {
-        const f32x4 x = *(const f32x4 *)(et + row * C::E_PITCH + (col + 4 * q) * 4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[4 * q + j] = alpha * x[j];
-      }
-      if (with_c) {
-#pragma unroll
-        for (int j = 0; j < EPL; ++j) v[j] += beta * (float)cv[mb][pass][j];
-      }
-      half8 o;
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) o[j] = (T)v[j];
-      store16_through(D + off, o);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();  // the region is rewritten by the next row of blocks
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();  // the region is rewritten by the next row of blocks
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  // From 64 MB on C is read past the caches, where a C of that size is not anyway and its lines would take the place of others; smaller
+  // ones often lie in the 256 MB behind the L2s, written by the call before.  us, past the caches / through them, K=512, three sets of
+  // operands in turn: 33 MB 27.6 / 25.1, 50 MB 43.2 / 36.6, 67 MB 54.5 / 55.3, 101 MB 74.5 / 81.1, 134 MB 101.5 / 123.3.  (64 MB are two rounds of
+  // 256 x 256 blocks.  A call of more than that whose last ones run as small tiles has two whole rounds here, and one of less has not.)
+  const bool big_c = (int64_t)M * N * batches * 2 >= (64 << 20);
+  if (Cin == nullptr || beta == 0.f) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // the surplus tile, whose registers are used anew (asked for a tile ago: it is there)
+    epilogue(std::integral_constant<int, NO_C>{});
+    return;
   }
+  if (big_c) {
+    asm volatile("; C past the caches");   // (or the compiler makes one branch of the two)
+    epilogue(std::integral_constant<int, C_STREAMED>{});
+    asm volatile("; C past the caches");
+    return;
+  }
+  epilogue(std::integral_constant<int, C_CACHED>{});
 }
 
 template <bool NN, int NB>   // 256 rows

@@ -162,6 +162,45 @@ def test_macro_tiles_beyond_half_a_round_bit_exact(L, M, N, K, layout):
         assert np.array_equal(got[i][rows], want), i
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("L,M,N", [
+    (1, 8192, 8192),     # 256 x 256 blocks, 134 MB of C
+    (2, 4352, 4096)])    # 320 x 256, the last row of tiles of both problems against the edge, 71 MB
+def test_c_of_64_mb_and_more_bit_exact(L, M, N, layout):
+    # such a C is read past the caches; D over C
+    import torch
+    K = 192
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    a, b, c = (torch.randint(-8, 9, shape, generator=gen, device="cuda").half() for shape in ((L, M, K), (L, N, K), (L, M, N)))
+    d = c.clone()
+    pkg.gemm(a, b if layout == 0 else b.transpose(1, 2).contiguous(), c=d, alpha=0.5, beta=-1.0, layout=layout, out=d)
+    torch.cuda.synchronize()
+    rows = np.unique(np.concatenate([np.arange(5, M, 173), np.arange(M - 70, M, 3)])).astype(np.int32)
+    for i in range(L):
+        want = (0.5 * oracle.gemm_f32(*(x[i].float().cpu().numpy() for x in (a, b)), rows=rows) - c[i].float().cpu().numpy()[rows]).astype(np.float16)
+        assert np.array_equal(d[i].cpu().numpy()[rows], want), i
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("L,M,N", [
+    (2, 1280, 3328),     # 192 x 192 tiles, the last ones of two problems against both edges
+    (1, 1280, 7168),     # 192 x 256, the last row of tiles against the edge
+    (1, 2816, 6144)])    # 320 x 256, likewise
+def test_macro_tiles_at_an_edge_without_c_bit_exact(L, M, N, layout):
+    import torch
+    K = 192
+    rng = np.random.default_rng(M + N)
+    a = rng.integers(-8, 9, (L, M, K)).astype(np.float32)
+    b = rng.integers(-8, 9, (L, N, K)).astype(np.float32)
+    bt = b if layout == 0 else np.ascontiguousarray(b.transpose(0, 2, 1))
+    got = pkg.gemm(to_dev(a.astype(np.float16)), to_dev(bt.astype(np.float16)), layout=layout)
+    torch.cuda.synchronize()
+    rows = np.unique(np.concatenate([np.arange(3, M, 61), np.arange(M - 70, M)])).astype(np.int32)
+    got = got.cpu().numpy()
+    for i in range(L):
+        assert np.array_equal(got[i][rows], oracle.gemm_f32(a[i], b[i], rows=rows).astype(np.float16)), i
+
+
 def test_fp32_uniform_inputs():
     # the CuTe example's type 1 (float operands, gemm.cu:677-684), U(-1,1) data (:482-485).  Both sides accumulate in
     # fp32 in different orders: |error| <~ sqrt(K) * 2^-24 * |terms|

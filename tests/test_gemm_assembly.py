@@ -41,3 +41,30 @@ def test_tiles_over_c_do_not_wait_for_their_stores(kernels, name):
     assert len(st) >= 2
     # all of C is asked for in front of the first store, so the last piece of it lies behind none of them
     assert min([n for i, n in _waits(ins) if st[0] < i < st[-1]], default=len(st)) >= len(st) - 1, name
+
+
+BLOCK_KERNELS = [("gemm_kernel16%s" % (k % nn), rows // 16 // 2, cols) for nn in (0, 1)
+                 for k, rows, cols in (("<%d,4>", 256, 256), ("<%d,3>", 256, 192), ("_rows<%d,6,4>", 192, 256), ("_rows<%d,6,3>", 192, 192),
+                                       ("_rows<%d,10,4>", 320, 256))]
+
+
+@pytest.mark.parametrize("name", [k[0] for k in BLOCK_KERNELS])
+def test_nothing_touches_the_accumulators_between_the_asm_multiplies(kernels, name):
+    # the multiplies of these kernels are asm statements, whose latency the compiler does not see: a copy or a spill of an
+    # accumulator between them, or of an operand right in front of one, would read or write it too early
+    ins = kernels[name]
+    at = [i for i, x in enumerate(ins) if x.startswith("v_mfma")]
+    other = {x.split()[0] for x in ins[at[0]:at[-1] + 1] if not x.startswith(("v_mfma", "s_", "ds_", "buffer_load_dwordx4"))}
+    assert other <= {"v_add_u32_e32", "v_add3_u32"}, (name, other)   # LDS and scalar-offset addresses
+
+
+@pytest.mark.parametrize("name,blocks,cols", BLOCK_KERNELS)
+def test_blocks_without_c_wait_for_nothing_between_their_stores(kernels, name, blocks, cols):
+    ins = kernels[name]
+    waits = {i for i, _ in _waits(ins)}
+    run = longest = 0
+    for i, x in enumerate(ins):
+        if i in waits: run = 0
+        elif x.startswith("global_store_dwordx4") and x.endswith("sc1"): run += 1
+        longest = max(longest, run)
+    assert longest >= blocks * 2, (name, longest)   # two stores for each row of blocks of a wave

@@ -53,10 +53,12 @@ AUTO_PICKED = {
     "fmha_fwd_kernel<128,64,8,2,1,0,0,0,1,0,0,0>": (0, ""),
     "fmha_fwd_kernel<128,64,4,2,1,0,0,0,1,0,0,0>": (0, ""),
     "fmha_fwd_kernel<256,32,4,1,1,0,0,0,1,0,0,0>": (0, ""),
-    # GEMM
-    "gemm_kernel16<0,4>": (0, ""),
-    "gemm_kernel16<1,4>": (0, ""),
-    "gemm_kernel_f32<128>": (0, ""),
+    # GEMM: 256 x 256, 256 x 192, 192 x 256, 192 x 192 and 320 x 256 macro tiles, TN and NN; the smaller ones without and over C
+    **{k % nn: (0, "") for nn in (0, 1) for k in ("gemm_kernel16<%d,4>", "gemm_kernel16<%d,3>", "gemm_kernel16_rows<%d,6,4>",
+                                                  "gemm_kernel16_rows<%d,6,3>", "gemm_kernel16_rows<%d,10,4>")},
+    **{"gemm_kernel16_tile%s<%d,%s>" % (c, nn, t): (0, "") for nn in (0, 1) for c in ("", "_c") for t in ("256,128", "128,128", "128,64")},
+    **{"gemm_kernel16_tile<%d,%s>" % (nn, t): (0, "") for nn in (0, 1) for t in ("64,64", "32,32")},
+    **{"gemm_kernel_f32%s" % t: (0, "") for t in ("<128>", "<64>", "<32>", "_c<128>", "_c<64>")},
 }
 
 
