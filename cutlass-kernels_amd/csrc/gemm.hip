@@ -332,30 +332,35 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
   // Three forms, so that a call without C meets no wait for it.
   enum { NO_C, C_CACHED, C_STREAMED };
   // C is asked for in front of the first store, into the registers that the main loop has left: a load per store had its latency in every
-  // pass (us: M=N=4096 K=192 20.1 -> 18.3; two of 4096 x 2048 x 512 NN 28.0 -> 26.4; 8192 x 8192 x 2048 286.0 -> 271.0).  Up to 256 rows all of
-  // it, and waited for once: between the stores the waits would in the end be waits for stores, which may be left out at an edge and so
-  // don't count (M=N=4096 K=192 17.5 -> 16.9).  With 320 rows 160 accumulators leave no room for its 80 registers: five rows of blocks ahead of
-  // the one that is stored (5 or 6: the same; all of it, through scratch: two of 4352 x 4096 x 192 50.2 -> 41.3, 5120 x 4096 x 512 36.5 -> 32.1,
-  // x 4096 138.5 -> 135.6).
+  // pass (us: M=N=4096 K=192 20.1 -> 18.3; two of 4096 x 2048 x 512 NN 28.0 -> 26.4; 8192 x 8192 x 2048 286.0 -> 271.0).  Up to 256 rows all of it.
+  // With 320 rows 160 accumulators leave no room for its 80 registers: five rows of blocks ahead of the one that is stored (5 or 6: the same;
+  // all of it, through scratch memory: two of 4352 x 4096 x 192 50.2 -> 41.3, 5120 x 4096 x 512 36.5 -> 32.1, x 4096 138.5 -> 135.6).
   constexpr int C_AHEAD = MB > 8 ? 5 : MB;
   half8 cv[C_AHEAD][PASSES];
   const auto read_c = [&](auto form, int mb, int pass) __attribute__((always_inline)) {
     int idx = pass * 64 + el;
-    if (CHUNKS % 64 != 0) idx = idx < CHUNKS ? idx : CHUNKS - 1;
     int gm = m0 + (wm * MB + mb) * 16 + idx / LPR, gn = n0 + wn * NB * 16 + idx % LPR * EPL;
-    gm = gm < m_own ? m_own : gm;   // (what a neighbour stores is not used: some line that is read anyway)
-    gn = gn < n_own ? n_own : gn;
+    if constexpr (C_AHEAD == MB) {
+      // (asked for by the lanes that use it, behind a branch each: without, the compiler moves the first piece into the branch around its
+      // store, behind the wait for the others, or, kept from that, calls of one round take longer: 4096 x 4096 x 192 17.0 -> 17.7)
+      if ((CHUNKS % 64 != 0 && idx >= CHUNKS) || gm < m_own || gn < n_own) return;
+    } else {
+      // (by every lane, so that the compiler can count what is on its way: some line that is read anyway instead of what a neighbour stores)
+      static_assert(CHUNKS % 64 == 0, "no lane beyond the row of blocks");
+      gm = gm < m_own ? m_own : gm;
+      gn = gn < n_own ? n_own : gn;
+    }
     const half8 *p = (const half8 *)(Cin + (int64_t)gm * N + gn);
     cv[mb % C_AHEAD][pass] = form.value == C_STREAMED ? __builtin_nontemporal_load(p) : *p;
   };
   const auto epilogue = [&](auto form) __attribute__((always_inline)) {
     constexpr bool WITH_C = form.value != NO_C;
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the surplus tile, whose registers are used anew (asked for a tile ago: it is there)
     if constexpr (WITH_C) {
 #pragma unroll
       for (int mb = 0; mb < C_AHEAD; ++mb)
 #pragma unroll
         for (int pass = 0; pass < PASSES; ++pass) read_c(form, mb, pass);
-      if constexpr (C_AHEAD == MB) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
     }
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
@@ -401,7 +406,6 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
   // 256 x 256 blocks.  A call of more than that whose last ones run as small tiles has two whole rounds here, and one of less has not.)
   const bool big_c = (int64_t)M * N * batches * 2 >= (64 << 20);
   if (Cin == nullptr || beta == 0.f) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // the surplus tile, whose registers are used anew (asked for a tile ago: it is there)
     epilogue(std::integral_constant<int, NO_C>{});
     return;
   }

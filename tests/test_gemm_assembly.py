@@ -68,3 +68,20 @@ def test_blocks_without_c_wait_for_nothing_between_their_stores(kernels, name, b
         elif x.startswith("global_store_dwordx4") and x.endswith("sc1"): run += 1
         longest = max(longest, run)
     assert longest >= blocks * 2, (name, longest)   # two stores for each row of blocks of a wave
+
+
+@pytest.mark.parametrize("name,blocks", [k[:2] for k in BLOCK_KERNELS if k[1] <= 8])
+def test_blocks_over_c_ask_for_all_of_it_before_their_first_store(kernels, name, blocks):
+    # two forms (through the caches and past them), two pieces for each row of blocks of a wave, none of them asked for behind a wait for
+    # the others or behind a store: the compiler likes to move the first one into the branch around its store
+    ins = kernels[name]
+    start = [i for i, x in enumerate(ins) if x.startswith("v_mfma")][-1]
+    waits = {i for i, n in _waits(ins) if n == 0}
+    runs, run, waited = [], 0, False
+    for i in range(start, len(ins)):
+        if i in waits: waited = run > 0
+        elif ins[i].startswith("global_load_dwordx4"):
+            assert not waited, (name, i - start)
+            run += 1
+        elif ins[i].startswith("global_store") and run: runs, run, waited = runs + [run], 0, False
+    assert runs == [2 * blocks] * 2, (name, runs)
