@@ -17,7 +17,7 @@
 // arithmetic), parked in one of two 64 KB LDS stages by ds_write_b128 while the other stage multiplies, one barrier per tile;
 // every multiply is followed by at most one fragment read or one store/load pair, see the pipeline comment at BlockCfg.
 // gemm_kernel16_rows, gemm_kernel16<NN, 3>: the same kernel on 192 x 192, 192 x 256, 256 x 192 and 320 x 256 macro tiles, for products whose
-// rounds these fill better (launch_f16).
+// rounds these fill better (choose_gemm_f16).
 // gemm_tile (gemm_kernel16_tile, gemm_kernel_f32): the smaller macro tiles, for what 256 x 256 blocks leave over and for all
 // fp32 products (v_mfma_f32_32x32x2_f32), whose 16 times slower multiplies any tile can feed.
 // The MFMA computes the TRANSPOSED block (rows = n, columns = m); the epilogue stages blocks through LDS and stores whole
@@ -29,6 +29,7 @@
 #include <mutex>
 
 #include "fmha_common.h"
+#include "gemm_choice.h"
 
 namespace cfk {
 namespace {
@@ -431,7 +432,7 @@ gemm_kernel16_rows(const _Float16 *__restrict__ A, const _Float16 *__restrict__ 
   gemm_block<NN, MB, NB>(A, B, Cin, D, M, N, K, alpha, beta);
 }
 
-// ---- Smaller macro tiles (which of them a call takes: launch_f16 and launch_f32 below).
+// ---- Smaller macro tiles (which of them a call takes: gemm_choice.h).
 // 8 waves (two per SIMD) or 4: WM x WN of them share a tile of K, each with TM x TN of C, and KG such groups take the
 // 128-byte deep K tiles in turn; their partial sums meet in the LDS.  Splitting the waves over K instead of over C keeps
 // the wave tile large -- an operand fragment feeds TM/16 or TN/16 multiplies -- where the macro tile is small, and puts KG
@@ -811,82 +812,28 @@ hipError_t launch_tiles32(const GemmArgs &g, hipStream_t s, int blocks) {
   return launch_tiles<C, gemm_kernel_f32<EDGE>>(g, s, 0, blocks);
 }
 
-constexpr int kCus = 256;
-
-// fp16: 256 x 256 blocks run in whole rounds of the CUs, one to a CU; the blocks of a last round that at most half fills the
-// CUs are cut into the smallest tiles that still go round the CUs once.  The time of such a round over K, relative to one of
-// 256 x 256 blocks (85 us at K=4096): 256 x 128 0.70, 128 x 128 0.47, 128 x 64 0.26, 64 x 64 0.17, 32 x 32 0.10; a tile size
-// down costs two rounds of its own.  Measured, us (TN), against 256 x 256 blocks alone: M=N=K=1024 8.4 / 25.1, M=N=512 K=4096
-// 8.7 / 75.4, M=N=2048 K=4096 39.5 / 79.5, 5120 x 4096 x 4096 (256 blocks, then 64 in 128 x 128 tiles) 144 / 175 and with C 155 / 199.
-// Behind whole rounds the tiles are a second launch, which pays down to the shortest K.  Time relative to whole blocks, behind one and
-// three rounds, at K=64, 128, 256, 512 (means of TN and NN, each side 60 ms at a time in turn): 8 blocks left 0.78, 0.77, 0.76, 0.74 and
-// 0.89, 0.88, 0.87, 0.85; 40 0.87, 0.86, 0.88, 0.85 and 0.94, 0.93, 0.93, 0.92; 72 0.92, 0.94, 0.93, 0.92 and 0.97, 0.97, 0.97, 0.94;
-// 104 0.96, 0.97, 0.96, 0.94 and 0.99, 0.98, 0.97, 0.95; 120 0.97, 0.97, 0.96, 0.95 and 1.00, 0.99, 0.98, 0.95; 128 0.98, 0.99, 0.98, 0.97
-// and 1.01, 1.00, 0.99, 0.96.  Worst found: M=6144 N=4096 (128 left) 1.03, 1.03, 1.00, 0.99, 19.4 -> 20.0 us at K=64.
+// What the choice names (gemm_choice.h).
 template <bool NN>
-hipError_t launch_blocks_and_tiles(const GemmArgs &g, hipStream_t s, int blocks) {
-  const int left = blocks % kCus, whole = left > kCus / 2 ? blocks : blocks - left;
-  if (whole) {
-    const hipError_t e = launch_blocks<NN, 8, 4>(g, s, whole);
-    if (e != hipSuccess || whole == blocks) return e;
-  }
-  if (left * HTile<NN, 32, 32>::SUB <= kCus) return launch_tiles16<NN, 32, 32>(g, s, whole, left);
-  if (left * HTile<NN, 64, 64>::SUB <= kCus) return launch_tiles16<NN, 64, 64>(g, s, whole, left);
-  if (left * HTile<NN, 128, 64>::SUB <= kCus) return launch_tiles16<NN, 128, 64>(g, s, whole, left);
-  if (left * HTile<NN, 128, 128>::SUB <= kCus) return launch_tiles16<NN, 128, 128>(g, s, whole, left);
-  return launch_tiles16<NN, 256, 128>(g, s, whole, left);
+hipError_t launch_f16(const GemmArgs &g, hipStream_t s) {
+  const GemmChoice c = choose_gemm_f16(g.M, g.N, g.K, g.batch);
+  hipError_t e = hipSuccess;
+  if (c.rows == 256 && c.cols == 256) e = launch_blocks<NN, 8, 4>(g, s, c.tiles);
+  else if (c.rows == 256) e = launch_blocks<NN, 8, 3>(g, s, c.tiles);
+  else if (c.rows == 320) e = launch_blocks<NN, 10, 4>(g, s, c.tiles);
+  else if (c.cols == 256) e = launch_blocks<NN, 6, 4>(g, s, c.tiles);
+  else if (c.rows == 192) e = launch_blocks<NN, 6, 3>(g, s, c.tiles);
+  if (e != hipSuccess || !c.tail_blocks) return e;
+  const int from = c.tiles, left = c.tail_blocks;
+  if (c.tail_rows == 32) return launch_tiles16<NN, 32, 32>(g, s, from, left);
+  if (c.tail_rows == 64) return launch_tiles16<NN, 64, 64>(g, s, from, left);
+  if (c.tail_rows == 256) return launch_tiles16<NN, 256, 128>(g, s, from, left);
+  return c.tail_cols == 64 ? launch_tiles16<NN, 128, 64>(g, s, from, left) : launch_tiles16<NN, 128, 128>(g, s, from, left);
 }
 
-// fp16, more than half a round of 256 x 256 blocks: rounds of other macro tiles where these waste less of the chip.  Times in rounds of
-// 256 x 256 tiles (106 us at K=4096): a full one of 192 x 256 tiles 0.772, 256 x 192 0.792, 192 x 192 0.622, 320 x 256 1.192; one of which a
-// share f is filled takes (1 + f)/2 of that, because the idle CUs leave the others their power; the smaller tiles behind whole rounds
-// (launch_blocks_and_tiles) 0.06, 0.14, 0.22, 0.40 and 0.55 of a round by size when they fill it.  231 drawn products of 129 to 1100 blocks,
-// K from 192, TN and NN, with and without C: 0.945 of the time in the geometric mean (the best choice for each: 0.943), worst 1.04.
-// us, 256 x 256 and small tiles -> the rule: 5120 x 4096 x 4096 TN 146 -> 129 and with C NN 177 -> 145 (256 tiles of 320 x 256); M=N=3072 K=4096
-// 81 -> 68 (256 of 192 x 192), K=512 18.6 -> 14.7; 3072 x 4096 x 4096 89 -> 84 (192 x 256).  Not built: 320 x 192 and 192 x 320 (103.6 against
-// 102.7 and 100.7 against 102.0 for 240 blocks), 256 x 128 and less by this kernel (64.3 against 61.8 for a round of 256 x 128).
-template <bool NN>
-hipError_t launch_f16(const GemmArgs &g, hipStream_t s, int blocks) {
-  if (blocks <= kCus / 2) return launch_blocks_and_tiles<NN>(g, s, blocks);
-  const auto rounds = [](long long tiles) {
-    const int part = (int)(tiles % kCus);
-    return (double)(tiles / kCus) + (part ? 0.5 + 0.5 * part / kCus : 0.0);
-  };
-  const int left = blocks % kCus;
-  double best = rounds(blocks);
-  if (left > 0 && left <= kCus / 2) {
-    const int sub = left <= 4 ? 64 : left <= 16 ? 16 : left <= 32 ? 8 : left <= 64 ? 4 : 2;
-    const double full = sub == 64 ? 0.06 : sub == 16 ? 0.14 : sub == 8 ? 0.22 : sub == 4 ? 0.40 : 0.55;
-    best = blocks / kCus + full * (0.6 + 0.4 * left * sub / kCus) + 0.03;
-  }
-  int rows = 256, cols = 256, tiles = 0;
-  const auto offer = [&](int r, int c, double round) {
-    // (a tile against the edge needs a whole one; 32-bit byte offsets within a tile's rows)
-    if (g.M < r || g.N < c || (long long)r * g.K * 2 >= (1LL << 32)) return;
-    const long long n = (long long)((g.M + r - 1) / r) * ((g.N + c - 1) / c) * g.batch;
-    const double t = round * rounds(n);
-    if (t < best) best = t, rows = r, cols = c, tiles = (int)n;
-  };
-  offer(192, 256, 0.772);
-  offer(256, 192, 0.792);
-  offer(192, 192, 0.622);
-  offer(320, 256, 1.192);
-  if (!tiles) return launch_blocks_and_tiles<NN>(g, s, blocks);
-  if (rows == 320) return launch_blocks<NN, 10, 4>(g, s, tiles);
-  if (rows == 256) return launch_blocks<NN, 8, 3>(g, s, tiles);
-  return cols == 256 ? launch_blocks<NN, 6, 4>(g, s, tiles) : launch_blocks<NN, 6, 3>(g, s, tiles);
-}
-
-// fp32: the multiplies bound every tile size, so what counts is how full the last round of the CUs is: the tile whose rounds,
-// at their measured times relative to 128 x 128 (66 us per 1024 of K), add up to least.  Three problems of M=1024 N=768 K=1536
-// (576 tiles of 64 x 64, 2304 of 32 x 32) 64.6 us by 32 x 32 against 76.3 and 97; M=N=5120 K=4096 1532 us by 64 x 64 against
-// 1615 and 1717; M=N=K=8192 7.31 ms by 128 x 128.  (256 x 256 blocks, 4 waves of 128 x 128 with registers between global memory
-// and LDS: 345 us, 1989 us and 7.89 ms for the three.)
-hipError_t launch_f32(const GemmArgs &g, hipStream_t s, int blocks) {
-  const auto rounds = [&](int sub) { return (double)(((long long)blocks * sub + kCus - 1) / kCus); };
-  const double t128 = rounds(FTile<128>::SUB), t64 = 0.267 * rounds(FTile<64>::SUB), t32 = 0.072 * rounds(FTile<32>::SUB);
-  if (t128 <= t64 && t128 <= t32) return launch_tiles32<128>(g, s, blocks);
-  return t64 <= t32 ? launch_tiles32<64>(g, s, blocks) : launch_tiles32<32>(g, s, blocks);
+hipError_t launch_f32(const GemmArgs &g, hipStream_t s) {
+  const int blocks = (g.M / BM) * (g.N / BN) * g.batch, edge = choose_gemm_f32(blocks);
+  if (edge == 128) return launch_tiles32<128>(g, s, blocks);
+  return edge == 64 ? launch_tiles32<64>(g, s, blocks) : launch_tiles32<32>(g, s, blocks);
 }
 
 template <bool NN>
@@ -912,9 +859,8 @@ hipError_t prepare_f16() {
 }  // namespace
 
 hipError_t launch_gemm(const GemmArgs &g, hipStream_t s) {
-  const int blocks = (g.M / BM) * (g.N / BN) * g.batch;
-  if (g.f32) return g.layout == 0 ? launch_f32(g, s, blocks) : hipErrorNotSupported;
-  return g.layout == 0 ? launch_f16<false>(g, s, blocks) : launch_f16<true>(g, s, blocks);
+  if (g.f32) return g.layout == 0 ? launch_f32(g, s) : hipErrorNotSupported;
+  return g.layout == 0 ? launch_f16<false>(g, s) : launch_f16<true>(g, s);
 }
 
 hipError_t prepare_gemm() {

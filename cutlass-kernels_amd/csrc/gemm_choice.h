@@ -1,0 +1,89 @@
+// Which macro tiles a product of cfk_gemm runs in.  Host code without HIP: gemm.hip launches what stands here, and
+// tests/test_gemm_choice.py asks it which kernels a shape takes.
+#pragma once
+
+namespace cfk {
+
+constexpr int kCus = 256;
+
+// A first launch of `tiles` macro tiles of rows x cols, and a second one of `tail_blocks` blocks of 256 x 256, the last ones of the batch, in
+// tiles of tail_rows x tail_cols; either may be missing (0).
+struct GemmChoice {
+  int rows, cols, tiles, tail_rows, tail_cols, tail_blocks;
+};
+
+// 256 x 256 blocks run in whole rounds of the CUs, one to a CU; the blocks of a last round that at most half fills the CUs are cut into the
+// smallest tiles that still go round the CUs once.  Such a round takes, at K=4096 (1024), of one of 256 x 256 blocks, 105 (32.4) us: 256 x 128
+// 0.58 (0.61), 128 x 128 0.38 (0.41), 128 x 64 0.22 (0.26), 64 x 64 0.14 (0.19), 32 x 32 0.08 (0.17).
+// Behind whole rounds the tiles are a second launch.  Time relative to whole blocks alone, batches of 256 x 256 problems, with and without
+// C, TN and NN (range of the four; three sets of operands and results in turn), behind one and behind three rounds:
+//   K=64    8 left 0.81..0.91, 0.95..0.97    40 0.90, 0.98..1.00        72 0.94..0.95, 0.98..1.02  104 0.96..0.98, 1.01..1.03  128 0.96..1.00, 1.03..1.04
+//   K=256          0.83..0.88, 0.94..0.96       0.91, 0.96..0.99           0.94..0.97, 0.98..1.01      0.95..1.01, 0.99..1.01      1.05..1.11, 1.05..1.08
+//   K=512          0.82..0.87, 0.92..0.93       0.91..0.97, 0.94..0.98     0.94..0.97, 0.96..0.99      0.96..1.01, 0.96..0.98      0.97..1.01, 0.97..1.00
+//   K=2048         0.80..0.83, 0.91..0.92       0.91..0.95, 0.95..0.98     0.95..0.99, 0.98..1.01      0.97..1.01, 0.98..1.04      1.00..1.03, 0.99..1.06
+inline GemmChoice gemm_blocks_and_tiles(int blocks) {
+  const int left = blocks % kCus, whole = left > kCus / 2 ? blocks : blocks - left;
+  GemmChoice c{};
+  if (whole) c.rows = c.cols = 256, c.tiles = whole;
+  if (whole == blocks) return c;
+  c.tail_blocks = left;
+  if (left * 64 <= kCus) c.tail_rows = c.tail_cols = 32;
+  else if (left * 16 <= kCus) c.tail_rows = c.tail_cols = 64;
+  else if (left * 8 <= kCus) c.tail_rows = 128, c.tail_cols = 64;
+  else if (left * 4 <= kCus) c.tail_rows = c.tail_cols = 128;
+  else c.tail_rows = 256, c.tail_cols = 128;
+  return c;
+}
+
+// fp16.  From half a round of 256 x 256 blocks on: rounds of other macro tiles where these waste less of the chip.  Times in rounds of 256 x 256
+// tiles; one of which a share f is filled takes (1 + f)/2, because the idle CUs leave the others their power.
+// Measured, every tile for 842 drawn products of 129 to 1040 blocks, TN and NN, with and without C, D the same and three in turn; a full round,
+// relative to 256 x 256: 192 x 256 0.77 at K=192 to 0.82 from 768 on, with C 0.78 to 0.82; 192 x 192 0.66 to 0.69; 320 x 256 1.12 to 1.23, with C
+// 1.19 to 1.21; 256 x 192 0.89 up to K=1536 and 0.84 from 3072 on, with C 0.86 and 0.85.  (The 192-column tiles write rows of 96 bytes, parts of lines.)
+// The choice is 1.001 of the best tile for each in the geometric mean, and 0.950 of 256 x 256 blocks with small tiles behind them; worst 1.04 of
+// those (5632 x 3840 x 2880 NN: 121 -> 126).  With 0.792 for 256 x 192 at every K and 0.622 for 192 x 192, 30 of them went to these two at 1.05 of the
+// time that they take now: 7 x 1024 x 5120 x 640 60 -> 76 us, 6 x 512 x 7168 x 1024 53 -> 61, 4 x 768 x 6144 x 1856 NN with C 79 -> 84.
+// us, blocks and small tiles / the choice: 5120 x 4096 x 4096 TN 149 / 128 and with C 158 / 135 (256 tiles of 320 x 256); M=N=3072 K=512 15.3 / 13.7 (256 of
+// 192 x 192).  Not built: 320 x 192 and 192 x 320 (103.6 against 102.7 and 100.7 against 102.0 for 240 blocks), 256 x 128 and less by the block kernel
+// (64.3 against 61.8 for a round of 256 x 128).
+inline GemmChoice choose_gemm_f16(int M, int N, int K, int batch) {
+  const int blocks = (M / 256) * (N / 256) * batch;
+  GemmChoice choice = gemm_blocks_and_tiles(blocks);
+  if (blocks <= kCus / 2) return choice;
+  const auto rounds = [](long long tiles) {
+    const int part = (int)(tiles % kCus);
+    return (double)(tiles / kCus) + (part ? 0.5 + 0.5 * part / kCus : 0.0);
+  };
+  double best = rounds(blocks);
+  if (choice.tail_blocks) {
+    const int sub = 256 / choice.tail_rows * (256 / choice.tail_cols);
+    const double full = sub == 64 ? 0.06 : sub == 16 ? 0.14 : sub == 8 ? 0.22 : sub == 4 ? 0.40 : 0.55;
+    best = blocks / kCus + full * (0.6 + 0.4 * choice.tail_blocks * sub / kCus) + 0.03;
+  }
+  const auto offer = [&](int r, int c, double round) {
+    // (a tile against the edge needs a whole one; 32-bit byte offsets within a tile's rows)
+    if (M < r || N < c || (long long)r * K * 2 >= (1LL << 32)) return;
+    const long long n = (long long)((M + r - 1) / r) * ((N + c - 1) / c) * batch;
+    const double t = round * rounds(n);
+    if (t < best) best = t, choice = GemmChoice{r, c, (int)n, 0, 0, 0};
+  };
+  offer(192, 256, 0.772);
+  offer(256, 192, 0.85 + 40.0 / K);
+  offer(192, 192, 0.65);
+  offer(320, 256, 1.192);
+  return choice;
+}
+
+// fp32, the edge of the square tiles: the multiplies bound every tile size, so what counts is how full the last round of the CUs is: the tile
+// whose rounds, at their measured times relative to 128 x 128 (66 us per 1024 of K), add up to least.  Three problems of M=1024 N=768 K=1536
+// (576 tiles of 64 x 64, 2304 of 32 x 32) 64.6 us by 32 x 32 against 76.3 and 97; M=N=5120 K=4096 1532 us by 64 x 64 against
+// 1615 and 1717; M=N=K=8192 7.31 ms by 128 x 128.  (256 x 256 blocks, 4 waves of 128 x 128 with registers between global memory
+// and LDS: 345 us, 1989 us and 7.89 ms for the three.)
+inline int choose_gemm_f32(int blocks) {
+  const auto rounds = [&](int sub) { return (double)(((long long)blocks * sub + kCus - 1) / kCus); };
+  const double t128 = rounds(4), t64 = 0.267 * rounds(16), t32 = 0.072 * rounds(64);
+  if (t128 <= t64 && t128 <= t32) return 128;
+  return t64 <= t32 ? 64 : 32;
+}
+
+}  // namespace cfk
