@@ -684,7 +684,7 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   __syncthreads();
   constexpr int EPL = 16 / ES, LPR = C::BNT / EPL, RPP = C::THREADS / LPR;
   using OutV = std::conditional_t<F16, half8, f32x4>;
-  const bool with_c = AHEAD || (Cin != nullptr && beta != 0.f);
+  const bool with_c = AHEAD || (PASSES == 1 && Cin != nullptr && beta != 0.f);   // (several passes meet a C in the AHEAD kernels only)
   const int e_row = tid / LPR, e_col = (tid % LPR) * EPL;
   static_assert(C::BMT % RPP == 0 || RPP > C::BMT, "whole passes");
 #pragma unroll

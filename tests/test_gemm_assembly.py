@@ -43,6 +43,16 @@ def test_tiles_over_c_do_not_wait_for_their_stores(kernels, name):
     assert min([n for i, n in _waits(ins) if st[0] < i < st[-1]], default=len(st)) >= len(st) - 1, name
 
 
+@pytest.mark.parametrize("name", ["gemm_kernel16_tile<%d,%s>" % (nn, t) for nn in (0, 1) for t in ("256,128", "128,128", "128,64")] +
+                         ["gemm_kernel_f32<128>", "gemm_kernel_f32<64>"])
+def test_tiles_without_c_carry_no_code_for_it(kernels, name):
+    # (calls with C take the kernels above)
+    ins = kernels[name]
+    st = _through(ins)
+    assert len(st) >= 2 and not [x for x in ins if x.startswith("global_load_dwordx4")], name
+    assert not [i for i, _ in _waits(ins) if st[0] < i < st[-1]], name
+
+
 BLOCK_KERNELS = [("gemm_kernel16%s" % (k % nn), rows // 16 // 2, cols) for nn in (0, 1)
                  for k, rows, cols in (("<%d,4>", 256, 256), ("<%d,3>", 256, 192), ("_rows<%d,6,4>", 192, 256), ("_rows<%d,6,3>", 192, 192),
                                        ("_rows<%d,10,4>", 320, 256))]
