@@ -120,7 +120,7 @@ def test_main_loop_of_every_tile_size_bit_exact(M, N, layout):
 @pytest.mark.parametrize("layout", [0, 1])
 @pytest.mark.parametrize("K", [192, 256])
 def test_last_round_in_tiles_bit_exact(K, layout):
-    # 384 blocks of 256 x 256: the 128 behind the first round of the CUs are 256 x 128 tiles, with as many K tiles as stages and one more
+    # 384 blocks of 256 x 256, which run as 512 tiles of 192 x 256: two whole rounds of the CUs
     import torch
     M, N = 6144, 4096
     rng = np.random.default_rng(K)
@@ -133,14 +133,33 @@ def test_last_round_in_tiles_bit_exact(K, layout):
     assert np.array_equal(got.cpu().numpy()[rows], want)
 
 
+@pytest.mark.parametrize("with_c", [False, True])
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("L", [264, 280, 310, 384])
+@pytest.mark.parametrize("K", [192, 256])
+def test_tiles_behind_a_whole_round_bit_exact(L, K, layout, with_c):
+    # the 8, 24, 54 and 128 blocks behind the first round of the CUs are tiles of 64 x 64, 128 x 64, 128 x 128 and 256 x 128
+    # (test_gemm_choice.py asks for that), with as many K tiles as the largest has stages and one more
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(L + K)
+    a, b, c = (torch.randint(-8, 9, shape, generator=gen, device="cuda").half() for shape in ((L, 256, K), (L, 256, K), (L, 256, 256)))
+    kw = dict(c=c, alpha=0.5, beta=-1.0) if with_c else {}
+    got = pkg.gemm(a, b if layout == 0 else b.transpose(1, 2).contiguous(), layout=layout, **kw)
+    torch.cuda.synchronize()
+    for i in (0, 255, 256, 257, (256 + L) // 2, L - 1):
+        want = oracle.gemm_f32(a[i].float().cpu().numpy(), b[i].float().cpu().numpy())
+        if with_c: want = 0.5 * want - c[i].float().cpu().numpy()
+        assert np.array_equal(got[i].cpu().numpy(), want.astype(np.float16)), i
+
+
 @pytest.mark.parametrize("layout", [0, 1])
 @pytest.mark.parametrize("L,M,N", [
     (1, 3072, 3072),     # 192 x 192 tiles, 256 of them
     (2, 1280, 3328),     # ... the last ones of two problems against both edges
     (1, 3072, 4096),     # 192 x 256
     (1, 1280, 7168),     # ... the last row of tiles against the edge
-    (1, 4096, 3072),     # 256 x 192
-    (1, 1792, 5888),     # ... the last column of tiles against the edge
+    (1, 4096, 3072),     # 256 x 256
+    (1, 1792, 5888),     # 192 x 256, the last row of tiles against the edge
     (1, 2560, 6656),     # 320 x 256
     (1, 2816, 6144)])    # ... the last row of tiles against the edge
 @pytest.mark.parametrize("K", [64, 192, 448])
@@ -199,6 +218,25 @@ def test_macro_tiles_at_an_edge_without_c_bit_exact(L, M, N, layout):
     got = got.cpu().numpy()
     for i in range(L):
         assert np.array_equal(got[i][rows], oracle.gemm_f32(a[i], b[i], rows=rows).astype(np.float16)), i
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("L,M,N", [(1, 4096, 3072), (5, 256, 7168)])   # (the second: the last column of tiles of each problem against the edge)
+@pytest.mark.parametrize("K", [1664, 2112])
+def test_256_x_192_tiles_bit_exact(L, M, N, K, layout):
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, b, c = (torch.randint(-8, 9, shape, generator=gen, device="cuda").half() for shape in ((L, M, K), (L, N, K), (L, M, N)))
+    bt = b if layout == 0 else b.transpose(1, 2).contiguous()
+    plain = pkg.gemm(a, bt, layout=layout)
+    d = c.clone()
+    pkg.gemm(a, bt, c=d, alpha=0.5, beta=-1.0, layout=layout, out=d)
+    torch.cuda.synchronize()
+    rows = np.arange(3, M, 61).astype(np.int32)
+    for i in range(L):
+        want = oracle.gemm_f32(*(x[i].float().cpu().numpy() for x in (a, b)), rows=rows)
+        assert np.array_equal(plain[i].cpu().numpy()[rows], want.astype(np.float16)), i
+        assert np.array_equal(d[i].cpu().numpy()[rows], (0.5 * want - c[i].float().cpu().numpy()[rows]).astype(np.float16)), i
 
 
 def test_fp32_uniform_inputs():

@@ -32,7 +32,7 @@ def _f16(lib, L, M, N, K):
     return tuple(out)
 
 
-BLOCKS, SMALL = (256, 256), {4: (32, 32), 16: (64, 64), 32: (128, 64), 64: (128, 128), 128: (256, 128)}
+BLOCKS = (256, 256)
 
 
 @pytest.mark.parametrize("L,M,N,first,tail", [
@@ -41,10 +41,13 @@ BLOCKS, SMALL = (256, 256), {4: (32, 32), 16: (64, 64), 32: (128, 64), 64: (128,
     (17, 256, 256, None, (128, 64)), (1, 1024, 2048, None, (128, 64)), (2, 1024, 1024, None, (128, 64)), (1, 256, 8448, None, (128, 128)),
     (4, 1024, 1024, None, (128, 128)), (1, 2048, 2048, None, (128, 128)), (65, 256, 256, None, (256, 128)), (1, 4096, 2048, None, (256, 128)),
     (129, 256, 256, BLOCKS, None), (257, 256, 256, BLOCKS, (32, 32)),
+    # test_tiles_behind_a_whole_round_bit_exact
+    (264, 256, 256, BLOCKS, (64, 64)), (280, 256, 256, BLOCKS, (128, 64)), (310, 256, 256, BLOCKS, (128, 128)), (384, 256, 256, BLOCKS, (256, 128)),
     # test_last_round_in_tiles_bit_exact
     (1, 6144, 4096, (192, 256), None),
     # test_macro_tiles_beyond_half_a_round_bit_exact, test_macro_tiles_at_an_edge_without_c_bit_exact
     (1, 3072, 3072, (192, 192), None), (2, 1280, 3328, (192, 192), None), (1, 3072, 4096, (192, 256), None), (1, 1280, 7168, (192, 256), None),
+    (1, 4096, 3072, BLOCKS, None), (1, 1792, 5888, (192, 256), None),
     (1, 2560, 6656, (320, 256), None), (1, 2816, 6144, (320, 256), None),
     # test_c_of_64_mb_and_more_bit_exact
     (1, 8192, 8192, BLOCKS, None), (2, 4352, 4096, (320, 256), None)])
@@ -66,10 +69,11 @@ def test_near_ties_stay_in_blocks(lib, L, M, N, K):
     assert _f16(lib, L, M, N, K)[:2] == BLOCKS
 
 
-@pytest.mark.parametrize("K", [2048, 4096, 8192])
-def test_256_x_192_where_it_is_the_faster_one(lib, K):
-    # 256 tiles in one round against 192 blocks: 83 against 87 us at K=4096
-    assert _f16(lib, 1, 4096, 3072, K) == (256, 192, 256, 0, 0, 0)
+@pytest.mark.parametrize("K", [1664, 2112, 4096, 8192])
+@pytest.mark.parametrize("L,M,N,tiles", [(1, 4096, 3072, 256), (5, 256, 7168, 190)])
+def test_256_x_192_where_it_is_the_faster_one(lib, L, M, N, tiles, K):
+    # (test_256_x_192_tiles_bit_exact; 256 tiles in one round against 192 blocks: 83 against 87 us at K=4096)
+    assert _f16(lib, L, M, N, K) == (256, 192, tiles, 0, 0, 0)
 
 
 def test_limits(lib):
