@@ -59,6 +59,15 @@ __device__ __forceinline__ int swz_bn(int row) {
   return ((row >> 3) & 1) << 1;
 }
 
+// beta * C + alpha * acc, the latter as rounded to fp32, rounded to fp32 once: left to itself the compiler rounds some elements of a row to fp16
+// right away (v_fma_mixlo_f16) and others not, by kernel, and a result would depend on the tile that it lies in.
+template <class T>
+__device__ __forceinline__ float add_c(float x, float beta, T c) {
+  x = __builtin_fmaf(beta, (float)c, x);
+  asm("" : "+v"(x));
+  return x;
+}
+
 // The fp16 kernel on 16x16x32 MFMAs (v_mfma_f32_16x16x32_f16).  8 waves, two per SIMD, in a 2 x 4 grid; a wave owns MB x NB blocks of
 // 16 x 16 of C (8 x 4: 128 x 64 of a 256 x 256 macro tile).  Measured, 8192^3 TN, one session, 4 waves of 128 x 128: 1401 TFLOP/s on
 // U(-1,1) operands against 1309 for the same kernel on 32x32x16 MFMAs; on constant operands 1837 against 2048 (LDS writes between the
@@ -389,7 +398,7 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
         }
         if constexpr (WITH_C) {
 #pragma unroll
-          for (int j = 0; j < EPL; ++j) v[j] += beta * (float)cm[j];
+          for (int j = 0; j < EPL; ++j) v[j] = add_c(v[j], beta, cm[j]);
         }
         half8 o;
 #pragma unroll
@@ -704,7 +713,7 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
     if (with_c) {
       const OutV cv = AHEAD ? c_ahead[AHEAD ? pass : 0] : *(const OutV *)(Cin + off);
 #pragma unroll
-      for (int x = 0; x < EPL; ++x) v[x] += beta * (float)cv[x];
+      for (int x = 0; x < EPL; ++x) v[x] = add_c(v[x], beta, cv[x]);
     }
     OutV o;
 #pragma unroll

@@ -239,6 +239,22 @@ def test_256_x_192_tiles_bit_exact(L, M, N, K, layout):
         assert np.array_equal(d[i].cpu().numpy()[rows], (0.5 * want - c[i].float().cpu().numpy()[rows]).astype(np.float16)), i
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+def test_an_element_does_not_depend_on_the_tile_it_lies_in(layout):
+    # corners of one product over C, each by another macro tile (32 x 32 to 256 x 128, 192 x 192, 192 x 256, 320 x 256; the whole in 256 x 256
+    # blocks), with factors that round: one K tile, so that all add up the same products in the same order, and the same bits come out
+    import torch
+    K = 64
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    a, b, c = ((torch.rand(shape, generator=gen, device="cuda") * 2 - 1).half() for shape in ((8192, K), (8192, K), (8192, 8192)))
+    def product(m, n):
+        bt = b[:n] if layout == 0 else b[:n].t().contiguous()
+        return pkg.gemm(a[:m], bt, c=c[:m, :n].contiguous(), alpha=1.9, beta=0.707, layout=layout)
+    whole = product(8192, 8192)
+    for m, n in [(512, 512), (1024, 1024), (1024, 2048), (2048, 2048), (4096, 2048), (3072, 3072), (3072, 4096), (2560, 6656)]:
+        assert torch.equal(product(m, n), whole[:m, :n]), (m, n)
+
+
 def test_fp32_uniform_inputs():
     # the CuTe example's type 1 (float operands, gemm.cu:677-684), U(-1,1) data (:482-485).  Both sides accumulate in
     # fp32 in different orders: |error| <~ sqrt(K) * 2^-24 * |terms|
