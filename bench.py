@@ -36,7 +36,7 @@ TRAFFIC_SOURCE = {
                  fetch_kib=172627, write_kib=65536),
     "cfg4": dict(profile="profiles/fmha_fwd_fp8_B4_H16_S4096_D128.md", kernel="fmha_fwd_kernel8p<128,64,8,2,1,1,0,0,2,0,0,1>",
                  fetch_kib=53713, write_kib=65536),
-    "cfg5": dict(profile="profiles/gemm_M8192_N8192_K8192.md", kernel="gemm_kernel16<0,4>", fetch_kib=787158, write_kib=131072),
+    "cfg5": dict(profile="profiles/gemm_M8192_N8192_K8192.md", kernel="gemm_kernel16<0,4>", fetch_kib=786509, write_kib=131072),
 }
 
 

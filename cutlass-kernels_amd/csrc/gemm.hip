@@ -22,7 +22,7 @@
 // fp32 products (v_mfma_f32_32x32x2_f32), whose 16 times slower multiplies any tile can feed.
 // The MFMA computes the TRANSPOSED block (rows = n, columns = m); the epilogue stages blocks through LDS and stores whole
 // rows, 16 bytes per lane.
-// Measured on MI355X, M=N=K=8192 fp16 TN: 1.34-1.40 PFLOP/s on U(-1,1) operands, where the board is power-limited
+// Measured on MI355X, M=N=K=8192 fp16 TN: 1.33-1.42 PFLOP/s by box on U(-1,1) operands, where the board is power-limited
 // (the vendor library's kernel for this shape, also on 16x16x32 MFMAs: 1.55); fp32: 150 TFLOP/s.
 #include <type_traits>
 
@@ -74,9 +74,10 @@ __device__ __forceinline__ float add_c(float x, float beta, T c) {
 // short multiplies hold the MFMA pipe up for about 20 cycles each).  On U(-1,1) operands this board is power-limited and the deeper,
 // narrower MFMA moves half the accumulator bits per FLOP: a register-only loop sustains 1.90 PFLOP/s with it against 1.69 with 32x32x16.
 // 8 waves read a half more from the LDS than 4 waves of 128 x 128, but with two on a SIMD one multiplies while the other waits for
-// memory, which shows wherever the time is not all main loop (us, 4 -> 8 waves, one session): M=N=4096 with K=64 12.5 -> 10.3, K=192 and
-// C 24.1 -> 18.9, K=1024 33.6 -> 31.6, NN and C 43.3 -> 39.6; 8192^3 819.6 -> 808.5.  (The same tile by 8 waves in two groups half a step
-// apart, copies straight into the LDS through a ring of five 32 KB slots: 812.7, with K=192 and C 19.7; without those copies 691, so
+// memory, which shows wherever the time is not all main loop (us, 4 -> 8 waves, one session, three sets of operands and results in turn):
+// M=N=4096 with K=64 12.4 -> 10.8, K=192 and C 24.6 -> 20.4, K=1024 33.8 -> 32.5, K=4096 108.1 -> 105.5; two of 4096 x 2048 x 512 NN and C 31.6 ->
+// 27.5; 8192^3 the same (816 and 820).  (The same tile by 8 waves in two groups half a step
+// apart, copies straight into the LDS through a ring of five 32 KB slots: 812.7 beside 808.5, with K=192 and C 19.7; without those copies 691, so
 // what is left at large K is the 64 KB that every 8.4 MFLOP take from L2.)
 // Lane (c = lane % 16, g = lane / 16) holds, of an operand fragment, row c and contraction slots 8g .. 8g+7 (16 bytes), and of an
 // accumulator block column c, rows 4g .. 4g+3.  The MFMA computes the transposed block (rows = n, columns = m), so a lane owns 4
@@ -332,9 +333,11 @@ __device__ __forceinline__ void gemm_block(const _Float16 *__restrict__ A, const
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
   // ---- epilogue: D = alpha * acc + beta * C in fp32, each row of blocks staged through the wave's own LDS region and stored as
   // whole rows, 16 bytes per lane, through the L2 to memory: a round of tiles writes as much as the L2s hold, and left there as dirty
-  // lines it has to be written out before the operands of the next round find room (us, left in the L2 / through it: 8192 x 8192
-  // with K=320 80.8 / 62.5, K=512 84.7 / 78.9, K=768 104.4 / 102.7, K=64 36.4 / 36.5; 4096 x 4096 x 320 17.5 / 16.4; 4 waves, whose stores
-  // came out more slowly, 67.8 with K=320).
+  // lines it has to be written out before the operands of the next round find room.  us, left in the L2 / through it, where D is the same in
+  // every call, and where three take turns: 8192 x 4096 x 320 38.2 / 31.4, 37.9 / 31.4; 4096 x 4096 x 512 20.6 / 19.3, the same; 7936 x 7936 x 320
+  // 66.1 / 55.9, 62.6 / 59.7; 8192 x 8192 with K=320 73.8 / 60.2, 71.9 / 77.2, NN 68.9 / 61.2, 72.1 / 72.9, with K=512 84.1 / 76.9, 87.5 / 89.8.  (The last
+  // are the largest: three D of 134 MB do not fit the 256 MB behind the L2s.  Past the caches they take 70.5, 70.6 with K=320 and 60.6, 60.1 with
+  // K=192, where through the L2 they take 54.9, 77.0; 4096 x 8192 x 320 36.4, 36.3, where 32.5, 32.0.)
   constexpr int EPL = 8, LPR = NB * 2, CHUNKS = 16 * LPR;   // halves per lane and store, lanes per row
   constexpr int PASSES = (CHUNKS + 63) / 64;
   char *et = smem + wave * (16 * C::E_PITCH);
