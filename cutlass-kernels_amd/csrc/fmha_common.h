@@ -25,6 +25,7 @@ struct FmhaArgs {
   int32_t n_split;     // units of work that share a query block's keys (1: no workspace is touched) ...
   int32_t split_bm;    // ... of so many rows; 32: the key-split kernel, else a SplitCfg build
   int32_t split_from;  // ... from this query block on, in the order [B,H,query block]
+  int32_t split_tiles;  // ... key tiles of a unit, rounded down (SplitCfg builds: set at their launch)
   float *part_o;       // their partial results [n_split][query blocks from split_from on][split_bm]: O not divided by the row sum,
   float *part_ml;      // and (reference point, row sum) pairs
   int32_t direct_p;    // first pass with e4m3 P: codes without an exponential (cfk_set_option(CFK_OPT_FAST_E4M3_WEIGHTS, 1))
@@ -44,6 +45,7 @@ struct FmhaPlan {
   float split_turn_us;
   int32_t mfma;  // 32: 32x32 MFMA build, 16: 16x16x32 build
   bool hand;     // a build with a hand-scheduled main loop
+  bool fma;      // ... and a multiply-add per score (fmha_fwd_kernel.h: FmaCfg)
   bool want_name;   // set by a caller that wants the next field
   char kernel[80];  // the instantiation, as profilers print it without namespaces: fmha_fwd_kernel16p<128,64,8,2,0,0,0,0,2,0,1,1>
 };

@@ -21,10 +21,13 @@ using C256_128x64 = FmhaCfg<256, 64, 4, 1, false, false>;
 // The hand-scheduled persistent build on 16x16x32 MFMAs (fmha_fwd_kernel16p.h; key length a multiple of 128, at least
 // 256): two 32-key tiles per barrier, big problems only
 using A256_128x64 = FmhaCfg<256, 32, 4, 1, false, false, false, false, 2, 0, true, true>;
+// ... with a multiply-add per score: every key length above 512 that the former does not take (145 drawn calls, time relative to the
+// compiler-scheduled build: 512 to 1023 keys 0.84 to 1.01, from 1024 on 0.79 to 0.94, with the keys of some items cut 0.34 to 0.94)
+using F256_128x64 = FmaCfg<A256_128x64>;
 // few query rows: the waves of a workgroup split the keys (not by wish)
 using K256_32x32 = KsCfg<256, 4>;
-using All256 = CfgList<C256_128x32P, C256_128x32, C256_128x64, A256_128x64>;
-using Auto256 = CfgList<K256_32x32, A256_128x64, C256_128x32P, C256_128x32>;
+using All256 = CfgList<C256_128x32P, C256_128x32, C256_128x64, A256_128x64, F256_128x64>;
+using Auto256 = CfgList<K256_32x32, A256_128x64, F256_128x64, C256_128x32P, C256_128x32>;
 
 template <class F>
 void dispatch(int sq, int skv, int bh, F &&f) {
@@ -38,8 +41,13 @@ void plan_fmha_f16_d256(int sq, int skv, int bh, FmhaPlan *p) {
 }
 
 hipError_t launch_fmha_f16_d256(const FmhaArgs &a, hipStream_t s) {
-  if (a.n_split > 1 && a.split_bm == 128) return launch_fmha_split<A256_128x64>(a, s);
   hipError_t e = hipErrorInvalidValue;
+  if (a.n_split > 1 && a.split_bm == 128) {
+    dispatch(a.Sq, a.Skv, a.B * a.H, [&](auto cfg) {
+      if constexpr (decltype(cfg)::ASM) e = launch_fmha_split<decltype(cfg)>(a, s);
+    });
+    return e;
+  }
   dispatch(a.Sq, a.Skv, a.B * a.H, [&](auto cfg) { e = launch_fmha_cfg<decltype(cfg)>(a, s); });
   return e;
 }
@@ -47,7 +55,8 @@ hipError_t launch_fmha_f16_d256(const FmhaArgs &a, hipStream_t s) {
 hipError_t prepare_fmha_f16_d256() {
   hipError_t e = prepare_all(All256{});
   if (e == hipSuccess) e = prepare_all(CfgList<K256_32x32>{});
-  return e != hipSuccess ? e : prepare_fmha_split<A256_128x64>();
+  if (e == hipSuccess) e = prepare_fmha_split<A256_128x64>();
+  return e != hipSuccess ? e : prepare_fmha_split<F256_128x64>();
 }
 
 }  // namespace cfk

@@ -93,6 +93,7 @@ struct FmhaCfg {
   static constexpr bool QK8 = QK8_, PV8 = PV8_;                 // e4m3 (true) or fp16 (false) operands of GEMM-I / II
   static constexpr bool DIRECT = false;                         // (DirectCfg below)
   static constexpr bool SPLIT = false;                          // (SplitCfg below)
+  static constexpr bool FMA = false;                            // (FmaCfg below)
   static constexpr bool VT = VT_;                               // V given pre-transposed, [B,D,H,S] (e4m3 only)
   static constexpr bool TAP_S = TAP_S_;                         // also write the pre-softmax scores (debug build)
   static constexpr int T = NWAVES * 64;
@@ -760,6 +761,8 @@ __global__ void __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(C::WP
 template <class C>
 __global__ void __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(2, 2))) fmha_fwd_kernel16p(const FmhaArgs a);
 template <class C>
+__global__ void __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(2, 2))) fmha_fwd_kernel16f(const FmhaArgs a);
+template <class C>
 __global__ void __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(2, 2))) fmha_fwd_kernel8p(const FmhaArgs a);
 template <class C>
 __global__ void __launch_bounds__(C::T) fmha_fwd_kernel_ks(const FmhaArgs a);
@@ -776,6 +779,11 @@ template <class C>
 struct SplitCfg : C {
   static constexpr bool SPLIT = true;
 };
+// The hand-scheduled fp16 build with a multiply-add per score instead of a scale folded into Q (fmha_fwd_kernel16p.h: kFold).
+template <class C>
+struct FmaCfg : C {
+  static constexpr bool FMA = true;
+};
 template <class C>
 constexpr bool has_direct_build = C::PV8 && C::D <= 128 && !C::TAP_S && !C::KSPLIT;
 
@@ -788,6 +796,7 @@ template <class C>
 constexpr auto fmha_kernel_of() {
   if constexpr (C::KSPLIT) return &fmha_fwd_kernel_ks<C>;
   else if constexpr (C::ASM && C::QK8) return &fmha_fwd_kernel8p<C>;
+  else if constexpr (C::FMA) return &fmha_fwd_kernel16f<C>;
   else if constexpr (C::ASM) return &fmha_fwd_kernel16p<C>;
   else if constexpr (C::M16) return &fmha_fwd_kernel16<C>;
   else return &fmha_fwd_kernel<C>;
@@ -850,7 +859,9 @@ hipError_t launch_fmha_split(const FmhaArgs &a, hipStream_t s) {
   const hipError_t e = prepare_fmha_split<C>();
   if (e != hipSuccess) return e;
   const int items = a.B * a.H * ((a.Sq + C::BM - 1) / C::BM), units = a.split_from + (items - a.split_from) * a.n_split;
-  hipLaunchKernelGGL(fmha_kernel_of<SplitCfg<C>>(), dim3(persistent_grid(units)), dim3(C::T), C::LDS_BYTES, s, a);
+  FmhaArgs with_tiles = a;
+  with_tiles.split_tiles = a.Skv / C::BN / a.n_split;
+  hipLaunchKernelGGL(fmha_kernel_of<SplitCfg<C>>(), dim3(persistent_grid(units)), dim3(C::T), C::LDS_BYTES, s, with_tiles);
   return hipGetLastError();
 }
 
@@ -858,7 +869,7 @@ template <class C>
 void fill_fmha_plan(int sq, int skv, int bh, FmhaPlan *p) {
   p->block_m = C::BM;
   p->block_n = C::BN * C::SUB;
-  p->kv_multiple = C::ASM && C::D != 256 ? C::BN : C::BN * C::SUB;
+  p->kv_multiple = C::ASM ? C::BN : C::BN * C::SUB;
   p->q_multiple = kQMultiple;
   p->mfma = C::M16 ? 16 : 32;
   p->lds_bytes = C::LDS_BYTES;
@@ -866,6 +877,7 @@ void fill_fmha_plan(int sq, int skv, int bh, FmhaPlan *p) {
   p->grid = bh * ((sq + C::BM - 1) / C::BM);
   p->split_tiles = p->split_waves = 0;
   p->hand = C::ASM;
+  p->fma = C::FMA;
   if constexpr (C::KSPLIT) {
     p->split_tiles = skv / C::TK;
     p->split_waves = C::NWAVES;
@@ -877,7 +889,7 @@ void fill_fmha_plan(int sq, int skv, int bh, FmhaPlan *p) {
   }
   if (!p->want_name) return;
   snprintf(p->kernel, sizeof p->kernel, "%s<%d,%d,%d,%d,%d,%d,%d,%d,%d,%d,%d,%d>",
-           C::ASM ? (C::QK8 ? "fmha_fwd_kernel8p" : "fmha_fwd_kernel16p") : C::M16 ? "fmha_fwd_kernel16" : "fmha_fwd_kernel", C::D, C::BN, C::NWAVES, C::WPE,
+           C::ASM ? (C::QK8 ? "fmha_fwd_kernel8p" : C::FMA ? "fmha_fwd_kernel16f" : "fmha_fwd_kernel16p") : C::M16 ? "fmha_fwd_kernel16" : "fmha_fwd_kernel", C::D, C::BN, C::NWAVES, C::WPE,
            (int)C::QK8, (int)C::PV8, (int)C::VT, (int)C::TAP_S, C::SUB, C::KPRE, (int)C::M16, (int)C::ASM);
   if constexpr (has_direct_build<C>) {
     if (fast_e4m3_weights()) strncat(p->kernel, "/direct", sizeof p->kernel - strlen(p->kernel) - 1);   // the DirectCfg build
@@ -886,14 +898,15 @@ void fill_fmha_plan(int sq, int skv, int bh, FmhaPlan *p) {
 
 // ---- tile selection.  The reference fixes its tile at compile time (-DQBLKSIZE / -DKBLKSIZE,
 // src/fmha-pipeline/shared_storage.h:4-15, swept by compile_run_all_config.sh:3-6); here every shape is built and one is
-// picked per call.  CFK_FMHA_TILE=<query rows>x<keys>[/16|/16h|/32|/32h] (e.g. 256x128, or 256x64/16 for the build on
-// 16x16x32 MFMAs, 256x128/16h and 256x128/32h for the fp16 / e4m3 ones with the hand-scheduled main loop, 32x64 for the
+// picked per call.  CFK_FMHA_TILE=<query rows>x<keys>[/16|/16h|/16f|/32|/32h] (e.g. 256x128, or 256x64/16 for the build on
+// 16x16x32 MFMAs, 256x128/16h and 256x128/32h for the fp16 / e4m3 ones with the hand-scheduled main loop, 256x128/16f for the fp16 one
+// with a multiply-add per score, 32x64 for the
 // key-split build), or small | large for the query rows alone, states a wish; a wish no instantiation can serve for the given shape is ignored.  CFK_FMHA_HANDLOOP=0 keeps
 // the automatic choice off the hand-scheduled builds (for A/B measurements).
 struct TileWish {
   int bm, bn;  // 0 = no wish
   int mfma;    // 16 or 32: the MFMA shape of the build (fp16 kernels come in both); 0 = no wish
-  int hand;    // +1: the build with the hand-scheduled loop, -1: a compiler-scheduled build, 0 = no wish
+  int hand;    // +1: the build with the hand-scheduled loop, +2: the one with a multiply-add per score, -1: a compiler-scheduled build, 0 = no wish
 };
 inline TileWish tile_wish() {
   static const TileWish w = [] {
@@ -908,7 +921,7 @@ inline TileWish tile_wish() {
       const int n = sscanf(e, "%dx%d/%d%c", &bm, &bn, &mfma, &suffix);
       if (n >= 2) {
         const bool shape = n >= 3 && (mfma == 16 || mfma == 32);
-        t = TileWish{bm, bn, shape ? mfma : 0, !shape ? 0 : (n == 4 && suffix == 'h') ? 1 : -1};
+        t = TileWish{bm, bn, shape ? mfma : 0, !shape ? 0 : n != 4 ? -1 : suffix == 'h' ? 1 : suffix == 'f' ? 2 : -1};
       }
     }
     return t;
@@ -920,13 +933,11 @@ template <class... Cs>
 struct CfgList {};
 
 // the shapes an instantiation can run: whole query tiles (fmha_fwd_kernel: whole waves), whole key steps (four key tiles per loop turn with the K
-// fragment prefetch and in the e4m3 hand-scheduled loop; the hand-scheduled loops need eight tiles to fill and drain;
-// two tiles with the two-tile step)
+// fragment prefetch; the hand-scheduled loops take any number of tiles from eight on, to fill and drain; the one at head dim 256 with the scale folded into Q
+// whole groups of four, as ever -- other lengths there are calls of its FmaCfg build --; two tiles with the two-tile step)
 template <class C>
 constexpr bool fits(int sq, int skv) {
-  // (the hand-scheduled builds at head dims 64 and 128 take up to three tiles behind the last group of four outside
-  // their loop)
-  return sq % kQMultiple == 0 && skv % (C::BN * (C::ASM && C::D != 256 ? 1 : C::KPRE || C::ASM ? 4 : C::SUB)) == 0 &&
+  return sq % kQMultiple == 0 && skv % (C::BN * (C::ASM ? (C::D == 256 && !C::FMA ? 4 : 1) : C::KPRE ? 4 : C::SUB)) == 0 &&
          (!C::ASM || skv >= 8 * C::BN);
 }
 
@@ -948,10 +959,11 @@ constexpr bool fits(int sq, int skv) {
 template <class C>
 constexpr bool hand_loop_pays(long long items, int skv) {
   if (!C::QK8) {
+    // (the other head dims: fmha_fwd_f16.hip.  The tests pin the kernels of 512 keys, where this one is no faster, and of 8160)
+    if (C::FMA) return C::D == 256 && skv > 512 && skv % 64 == 0;
     if (C::D == 256) return skv >= 1024;
-    // (key tiles behind the last group of four run outside the generated loop, at three to four times a tile's time in it:
-    // worth it from 2048 keys on and while they are few -- 2112 keys +9 %, 3008 keys with three of them 0..+27 %, 704 keys
-    // with three -15 %, 1088 keys with one -9 %)
+    // (which calls fold the scale into Q is a matter of exactness -- fmha_fwd_kernel16p.h: kFold -- and drawn where these loops took whole
+    // groups of four tiles only: from 2048 keys on with few tiles behind the last one; what is left is for the FmaCfg builds)
     const int n_tiles = skv / C::BN, n_left = n_tiles & 3;
     if (n_left != 0 && (n_tiles < 32 || n_left * 10 > n_tiles)) return false;
     return C::BM == 128 ? items <= 256 && skv >= 1024 : items > 128;
@@ -1052,7 +1064,8 @@ bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish
     if (w.bm ? C::BM != w.bm : !pays()) return;
     if (w.bn && C::BN * C::SUB != w.bn) return;
     if (w.mfma && (C::M16 ? 16 : 32) != w.mfma) return;
-    if (w.hand && C::ASM != (w.hand > 0)) return;
+    if (w.hand && (C::ASM != (w.hand > 0) || (C::ASM && C::FMA != (w.hand > 1)))) return;
+    if (w.bm && !w.hand && C::FMA) return;   // (a wish for a tile alone names the other hand-scheduled build)
     f(c);
     done = true;
   };
@@ -1062,16 +1075,24 @@ bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish
 
 // wish first (over every instantiation), then the automatic order, then -- for shapes nothing fits -- the fallback,
 // whose tile the caller's divisibility check then names in its error
+inline int problem_size(int sq, int bh) { return sq % 256 == 0 && (long long)bh * (sq / 256) >= 512 ? 2 : 1; }
+template <class All, class F>
+bool tile_by_wish(int sq, int skv, int bh, F &&f) {
+  const TileWish w = tile_wish();
+  return (w.bm || w.bn) && first_fit(All{}, sq, skv, bh, problem_size(sq, bh), w, f);
+}
+// (the hand-scheduled build is a two-pass kernel: not for callers that asked for a data-independent run time)
+inline bool hand_loops_allowed() {
+  static const bool no_hand = [] { const char *e = getenv("CFK_FMHA_HANDLOOP"); return e && e[0] == '0'; }();
+  return !no_hand && !predictable_latency();
+}
+template <class Auto, class Fallback, class F>
+void tile_by_rule(int sq, int skv, int bh, F &&f) {
+  if (!first_fit(Auto{}, sq, skv, bh, problem_size(sq, bh), TileWish{0, 0, 0, hand_loops_allowed() ? 0 : -1}, f)) f(Fallback{});
+}
 template <class All, class Auto, class Fallback, class F>
 void select_tile(int sq, int skv, int bh, F &&f) {
-  const bool big = sq % 256 == 0 && (long long)bh * (sq / 256) >= 512;
-  const int size = big ? 2 : 1;
-  const TileWish w = tile_wish();
-  if ((w.bm || w.bn) && first_fit(All{}, sq, skv, bh, size, w, f)) return;
-  static const bool no_hand = [] { const char *e = getenv("CFK_FMHA_HANDLOOP"); return e && e[0] == '0'; }();
-  // (the hand-scheduled build is a two-pass kernel: not for callers that asked for a data-independent run time)
-  if (first_fit(Auto{}, sq, skv, bh, size, TileWish{0, 0, 0, no_hand || predictable_latency() ? -1 : 0}, f)) return;
-  f(Fallback{});
+  if (!tile_by_wish<All>(sq, skv, bh, f)) tile_by_rule<Auto, Fallback>(sq, skv, bh, f);
 }
 
 template <class... Cs>

@@ -29,7 +29,7 @@ namespace cfk {
 template <int D_, int NWAVES_, bool QK8_, bool PV8_, bool VT_, int TK_, int BN_>
 struct KsTiles {
   static constexpr int D = D_, NWAVES = NWAVES_, TK = TK_, BN = BN_, BM = 32, T = NWAVES * 64, WPE = 1, SUB = 1, KPRE = 0;
-  static constexpr bool QK8 = QK8_, PV8 = PV8_, VT = VT_, TAP_S = false, M16 = true, ASM = false, DIRECT = false, KSPLIT = true;
+  static constexpr bool QK8 = QK8_, PV8 = PV8_, VT = VT_, TAP_S = false, M16 = true, ASM = false, FMA = false, DIRECT = false, KSPLIT = true;
   static constexpr int K_PITCH = D * (QK8 ? 1 : 2), V_PITCH = VT ? TK : D * (PV8 ? 1 : 2);
   static constexpr int K_BYTES = TK * K_PITCH, V_BYTES = (VT ? D : TK) * V_PITCH, WAVE_BYTES = K_BYTES + V_BYTES;
   static constexpr int K_IPW = K_BYTES / 1024, V_IPW = V_BYTES / 1024;   // 1 KB copies of a tile, all by the wave that owns it

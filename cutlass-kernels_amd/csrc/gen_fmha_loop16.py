@@ -11,7 +11,7 @@ FmhaCfg::ASM), in three shapes:
         are 192 registers per lane; O lives in the accumulation registers a[0:127])
 d128 and d256 have the same timeline (64 MFMA slots and 16 KB of K and of V per tile); the text below describes d128.
 
-    python3 gen_fmha_loop16.py            # rewrites fmha_fwd_loop16_{d128,d128w4,d256,d64,d64w4}.inc beside this file
+    python3 gen_fmha_loop16.py            # rewrites fmha_fwd_loop16_{d128,d128w4,d256,d64,d64w4}{,_fma}.inc beside this file
     python3 gen_fmha_loop16.py --check    # exit status 1 if those files are not what the generator produces
 
 Why a generator: the loop is one inline-asm statement of ~2800 instructions with every register assigned by hand.
@@ -77,7 +77,8 @@ K_ST0 = 0                               # LDS map: K slots, then V slots (the re
 ROWSUM = "add"
 # FOLD: Q arrives multiplied by the softmax scale c and S = K.Q^T starts from -m (the C operand of the first K-step is
 # a register quad that holds -m) instead of from zero: the scores leave the matrix pipe as c S - m and the softmax has
-# no multiply-add per score.  The caller subtracts m from S(0) itself.  (Not with ROWSUM = "dot".)
+# no multiply-add per score.  The caller subtracts m from S(0) itself.  (Not with ROWSUM = "dot".)  Without it every score takes a
+# v_fma_f32 in fp32: 2.5 to 9 % more time, and no second rounding of Q.  Both forms are built (..._fma.inc: FmaCfg).
 FOLD = True
 RING = 8
 LOOKAHEAD = 7      # fragments requested ahead of use
@@ -94,13 +95,13 @@ def configure():
     if SHAPE == "d128":
         g.update(D=128, BN=64, NWAVES=8, O_ACC=False, O0=192, SA0=128, SB0=160, Q0=96, P0=80, RING0=48, KRD0=24, VRD0=28, GOK0=36, GOV0=38)
     elif SHAPE == "d128w4":   # the same loop for 128 query rows: 4 waves, one per SIMD, four copies per wave and tile, O in a[0:63]
-        assert ROWSUM == "add" and FOLD
+        assert ROWSUM == "add"
         g.update(D=128, BN=64, NWAVES=4, O_ACC=True, O0=0, SA0=128, SB0=160, Q0=96, P0=80, RING0=48, KRD0=24, VRD0=28, GOK0=192, GOV0=196)
     elif SHAPE == "d64":
         assert ROWSUM == "mfma"
         g.update(D=64, BN=64, NWAVES=8, O_ACC=False, O0=224, SA0=160, SB0=192, Q0=144, P0=128, RING0=96, KRD0=82, VRD0=78, GOK0=77, GOV0=76)
     elif SHAPE == "d64w4":    # ... and the head-dim-64 loop for 128 query rows: 4 waves, two copies per wave and tile, O in a[0:31]
-        assert ROWSUM == "mfma" and FOLD
+        assert ROWSUM == "mfma"
         g.update(D=64, BN=64, NWAVES=4, O_ACC=True, O0=0, SA0=160, SB0=192, Q0=144, P0=128, RING0=96, KRD0=82, VRD0=78, GOK0=224, GOV0=226)
     else:
         assert ROWSUM == "add"
@@ -221,12 +222,16 @@ def copy_ops(kind, slot):
 
 
 def schedule(n_tiles):
-    """straight-line program for n_tiles key tiles (a multiple of 4, at least 8), as a list of segments, one per
-    super-step; a segment ends with its barrier (the last one has none)"""
-    assert n_tiles % 4 == 0 and n_tiles >= 8
+    """straight-line program for n_tiles key tiles (at least 7), as a list of segments, one per super-step; a segment
+    ends with its barrier (the last one has none)"""
+    assert n_tiles >= 7
     n_slots = T * n_tiles
-    n_steps = n_tiles // 2
-    SS = 2 * T   # slots per super-step
+    left = n_tiles % 4
+    # super-steps of two tiles, behind the last group of four tiles of one (their first tiles; the barrier between the last two
+    # says that every wave is done with K tile n-1 and V tile n-2)
+    steps = list(range(0, n_tiles - 2, 2)) + [n_tiles - 2] + ([n_tiles - 1] if left == 2 else []) if n_tiles % 2 == 0 else list(range(0, n_tiles, 2))
+    n_steps = len(steps)
+    barrier_after = {T * t - HOLD: J for J, t in enumerate(steps) if J}   # slot -> the super-step that starts behind it
     # ---- MFMA slots: slot -> (fragment, qb) or ("L", ps, qb)
     slot_item = [None] * n_slots
     frags = []
@@ -254,26 +259,37 @@ def schedule(n_tiles):
         # the tile's sums join l a few instructions into the next tile's softmax (or right after, for the last tile)
         for txt, cost in tile_sum_ops():
             valu_at.setdefault(max(int(start + cum / V_RATE) + 2, -1), []).append(txt)
-    # ---- copies: super-step J, one copy instruction group every fourth slot from its second slot on
+    # ---- copies: the super-step of tiles 2J, 2J+1, one copy instruction group every fourth slot from its second slot on
     copies_at = {}
-    for J in range(n_steps):
+    for J in range(n_tiles // 2):
         todo = [('K', 2 * J + 3), ('K', 2 * J + 4), ('V', 2 * J + 2), ('V', 2 * J + 3)]
         groups = []
         for kind, t in todo:
             if t < n_tiles: groups += copy_ops(kind, t % NSLOT)
-        for i, grp in enumerate(groups): copies_at[SS * J + 1 + 4 * i] = grp
+        for i, grp in enumerate(groups): copies_at[2 * T * J + 1 + 4 * i] = grp
     # ---- the workgroup's next work item (persistent workgroups): in the last super-step, whose K slots 0-2 and V slots
     # 0-1 are free, copy that item's first three K and two V tiles into them and, once the last S = K.Q^T has been
-    # issued, load its Q into the Q registers; both are waited for at the end of the statement
-    Z = SS * (n_steps - 1)
+    # issued, load its Q into the Q registers; both are waited for at the end of the statement.  With tiles behind the last
+    # group of four the last super-step is one tile without a K.Q^T: all K slots are free, but of V slots 0 and 1 the one that
+    # tile n-1 lies in (one tile: 0, two: 1, three: neither).  What goes there, and behind it, waits for a barrier of its own
+    # behind the last operand read.
+    Z = T * steps[-1]
     copies_at.setdefault(Z, [])
     copies_at[Z] = ["s_mov_b64 s[40:41], %[kn]", "s_mov_b64 s[42:43], %[vn]"]
-    groups = []
-    for kind, slot in (('K', 0), ('K', 1), ('K', 2), ('V', 0), ('V', 1)): groups += copy_ops(kind, slot)
-    for i, grp in enumerate(groups): copies_at[Z + 1 + 4 * i] = grp
+    late_v = {0: 2, 1: 0, 2: 1, 3: 2}[left]   # V slots from here on are copied last
+    groups, late_groups = [], []
+    for kind, slot in (('K', 0), ('K', 1), ('K', 2), ('V', 0), ('V', 1)):
+        (late_groups if kind == 'V' and slot >= late_v else groups).extend(copy_ops(kind, slot))
+    if left:
+        room = T - 2 * LOOKAHEAD - 2
+        for i, grp in enumerate(groups): copies_at.setdefault(Z + 1 + i * room // len(groups), []).extend(grp)
+    else:
+        for i, grp in enumerate(groups): copies_at[Z + 1 + 4 * i] = grp
+    late_slot = n_slots - 2 * LOOKAHEAD + 2 if late_groups else None   # the barrier stands in front of this slot
+    for i, grp in enumerate(late_groups): copies_at.setdefault(late_slot + 1 + i, []).extend(grp)
     for i in range(QB * KS):
         qb, ks = i // KS, i % KS
-        copies_at.setdefault(Z + QKS + 1 + 3 * i, []).append("global_load_dwordx4 %s, v%d, %%[qn] offset:%d" % (vr(q_reg(qb, ks)), QOFF0 + qb, 64 * ks))
+        copies_at.setdefault(Z + (2 + 2 * i if left else QKS + 1 + 3 * i), []).append("global_load_dwordx4 %s, v%d, %%[qn] offset:%d" % (vr(q_reg(qb, ks)), QOFF0 + qb, 64 * ks))
     # ---- emission
     segs, cur = [], []
     nread = 0             # LDS read instructions issued so far
@@ -284,8 +300,7 @@ def schedule(n_tiles):
     def barrier_passed_for(f, slot):
         # a K fragment of tile t >= 2 (first read in super-step (t-1)/2) needs the barrier of the super-step before
         if f.kind != 'K' or f.t < 2: return True
-        J = (f.t - 1) // 2
-        return slot > SS * J - HOLD   # `slot` is the slot after the MFMA just issued
+        return slot > 2 * T * ((f.t - 1) // 2) - HOLD   # `slot` is the slot after the MFMA just issued
     def request(slot, limit):
         nonlocal next_frag, nread
         n = 0
@@ -318,8 +333,12 @@ def schedule(n_tiles):
     request(0, LOOKAHEAD)
     for txt in valu_at.get(-1, []): cur.append(txt)
     for slot in range(n_slots):
-        J = slot // SS
-        if slot % SS == SS - HOLD and J < n_steps - 1:
+        if slot == late_slot:
+            assert next_frag == len(frags)
+            cur.append("s_waitcnt lgkmcnt(0)")   # (the copies under way are waited for at the end)
+            cur.append("s_barrier")
+            done_reads = nread
+        if slot in barrier_after:
             cur.append("s_waitcnt lgkmcnt(0)" if "vmwait" in ABLATE else "s_waitcnt vmcnt(0) lgkmcnt(0)")
             if "barrier" not in ABLATE: cur.append("s_barrier")
             done_reads = nread
@@ -352,7 +371,7 @@ def schedule(n_tiles):
 
 
 def folded():
-    """(head, loop body, tail): head = super-steps 0,1; body = 2,3 (repeated); tail = the last two"""
+    """(head, loop body, tail) of whole groups of four tiles: head = super-steps 0,1; body = 2,3 (repeated); tail = the last two"""
     segs = schedule(16)
     assert segs[2] + segs[3] == segs[4] + segs[5], "the schedule is not periodic"
     # the same schedule for other lengths must be made of the same pieces
@@ -363,10 +382,32 @@ def folded():
     return segs[0] + segs[1], segs[2] + segs[3], segs[6] + segs[7]
 
 
+def tails():
+    """what follows head and loop body, by the number of tiles behind the last group of four: the last 4, 5, 6 or 3 tiles (the body's
+    copies run up to three tiles ahead of it, so that three tiles at least have to follow)"""
+    head, body, tail = folded()
+    out = [tail]
+    for left in (1, 2, 3):
+        rest = left if left == 3 else 4 + left
+        for n in (4 + rest, 8 + rest, 16 + rest):
+            segs = schedule(n)
+            assert segs[0] + segs[1] == head
+            for j in range(2, 2 + (n - 4 - rest) // 2, 2): assert segs[j] + segs[j + 1] == body
+            end = sum(segs[2 + (n - 4 - rest) // 2:], [])
+            if n == 4 + rest: out.append(end)
+            assert end == out[left]
+    return out
+
+
 def program(n_tiles):
     """the instruction sequence a wave executes for n_tiles key tiles (loop unrolled): what the checker walks"""
-    head, body, tail = folded()
-    return head + body * ((n_tiles // 2 - 4) // 2) + tail
+    head, body, _ = folded()
+    return head + body * loop_turns(n_tiles) + tails()[n_tiles % 4]
+
+
+def loop_turns(n_tiles):
+    """... and how often it goes through the loop body: (n_tiles - 7) / 4, as the caller computes it"""
+    return (n_tiles - 7) // 4
 
 
 def render():
@@ -374,12 +415,14 @@ def render():
     in scope: bool sum_is_complete (out: the flag), f32x16 o0, o1, .. (out: the O accumulators, 16 registers each, in register order), sa0, .. (in, clobbered:
     S(0)), q0, .. (in: this item's Q; out: the next item's); float l0, l1 (out); uint64_t kptr, vptr (in: this item's K
     tile 3 / V tile 2; out: the same of the next item), kn, vn, qn (the next item's K, V and this wave's Q rows);
-    uint32_t nloop, k_rd[KS], v_rd[DB], goff_k[IPW], goff_v[IPW], qoff[2], lds_wave, tile_stride; float m_ref[2], c_log2
+    uint32_t nloop (four times the turns of the loop plus the tiles behind the last group of four), k_rd[KS], v_rd[DB], goff_k[IPW], goff_v[IPW], qoff[2], lds_wave, tile_stride; float m_ref[2], c_log2
     (FOLD: float m_neg[2] instead of those two); constexpr bool kFold."""
-    head, body, tail = folded()
+    head, body, _ = folded()
+    tail = tails()
     L = []
     L.append("// GENERATED by gen_fmha_loop16.py -- do not edit.  The hand-scheduled main loop of fmha_fwd_kernel16p (FmhaCfg::ASM: head")
-    L.append("// dim %d, %d x %d): %d + %d (loop) + %d instructions, row sum by \"%s\"." % (D, 32 * NWAVES, 2 * BN, len(head), len(body), len(tail), ROWSUM))
+    L.append("// dim %d, %d x %d): %d + %d (loop) + %s instructions (by the tiles behind the last group of four)," % (D, 32 * NWAVES, 2 * BN, len(head), len(body), " / ".join(str(len(t)) for t in tail)))
+    L.append("// row sum by \"%s\"." % ROWSUM)
     L.append("// l0 / l1 hold the complete row sum of the lane's query in every lane (true) or the lane's share of it (false)")
     L.append("sum_is_complete = %s;" % ("true" if L_TOTAL else "false"))
     L.append("// Q is expected multiplied by the softmax scale, S(0) with the reference point taken off, m_neg[] = minus that point (true);")
@@ -388,15 +431,25 @@ def render():
     L.append("asm volatile(")
     def emit(ins): L.append('    "%s\\n"' % ins)
     for i in head: emit(i)
-    emit("s_cmp_eq_u32 %[nloop], 0")
+    emit("s_cmp_lt_u32 %[nloop], 4")
     emit("s_cbranch_scc1 2f")
     emit("1:")
     for i in body: emit(i)
-    emit("s_sub_u32 %[nloop], %[nloop], 1")
-    emit("s_cmp_lg_u32 %[nloop], 0")
+    emit("s_sub_u32 %[nloop], %[nloop], 4")
+    emit("s_cmp_ge_u32 %[nloop], 4")
     emit("s_cbranch_scc1 1b")
     emit("2:")
-    for i in tail: emit(i)
+    emit("s_cmp_eq_u32 %[nloop], 1")
+    emit("s_cbranch_scc1 3f")
+    emit("s_cmp_eq_u32 %[nloop], 2")
+    emit("s_cbranch_scc1 4f")
+    emit("s_cmp_eq_u32 %[nloop], 3")
+    emit("s_cbranch_scc1 5f")
+    for left, label in ((0, None), (1, 3), (2, 4), (3, 5)):
+        if label: emit("%d:" % label)
+        for i in tail[left]: emit(i)
+        if left < 3: emit("s_branch 6f")
+    emit("6:")
     def vec16(base, name, n, kind="v", mode="="):
         return ['"%s{%s[%d:%d]}"(%s%d)' % (mode, kind, base + 16 * i, base + 16 * i + 15, name, i) for i in range(n)]
     n_o, n_s, n_q = 4 * DB * QB // 16, 4 * KB * QB // 16, 4 * KS * QB // 16
@@ -422,7 +475,7 @@ def render():
     # (vector registers the loop never names stay the compiler's: values it keeps across the statement need not be spilled)
     import re
     named = set()
-    for ins in head + body + tail:
+    for ins in head + body + sum(tail, []):
         for m in re.finditer(r"\bv\[(\d+):(\d+)\]|\bv(\d+)\b", ins):
             named |= set(range(int(m.group(1)), int(m.group(2)) + 1)) if m.group(1) else {int(m.group(3))}
     clob = ['"memory"', '"scc"', '"m0"'] + ['"v%d"' % r for r in range(LOW, 256) if r not in used and r in named]
@@ -436,12 +489,13 @@ if __name__ == "__main__":
     stale = False
     defaults = {k: globals()[k] for k in overrides}
     for shape, rowsum in (("d128", "add"), ("d128w4", "add"), ("d256", "add"), ("d64", "mfma"), ("d64w4", "mfma")):
-        SHAPE, ROWSUM = shape, rowsum
+      for fold in (True, False):
+        SHAPE, ROWSUM, FOLD = shape, rowsum, fold
         for k, v in overrides.items():
             if isinstance(v, dict): v = v.get(shape, rowsum if k == "ROWSUM" else defaults[k])   # {"ROWSUM": {"d128": "mfma"}}: one shape only
             globals()[k] = v
         configure()
-        out = os.path.join(os.path.dirname(os.path.abspath(__file__)), "fmha_fwd_loop16_%s.inc" % shape)
+        out = os.path.join(os.path.dirname(os.path.abspath(__file__)), "fmha_fwd_loop16_%s%s.inc" % (shape, "" if fold else "_fma"))
         txt = render()
         if "--check" in sys.argv:
             stale = stale or not (os.path.exists(out) and open(out).read() == txt)

@@ -36,7 +36,7 @@ def short_name(d):
     d = re.sub(r"\(.*\)$", "", d)
     direct = "DirectCfg<" in d     # the build with e4m3 weights written as codes: shown as <...>/direct
     split = "SplitCfg<" in d       # ... and with some items' keys cut into units: <...>/split
-    d = d.replace("cfk::", "").replace("DirectCfg<", "").replace("SplitCfg<", "").replace("FmhaCfg<", "").replace("KsCfg<", "").replace("KsCfg8<", "").replace(">>", ">").replace(">>", ">")
+    d = d.replace("cfk::", "").replace("DirectCfg<", "").replace("SplitCfg<", "").replace("FmaCfg<", "").replace("FmhaCfg<", "").replace("KsCfg<", "").replace("KsCfg8<", "").replace(">>", ">").replace(">>", ">")
     d = d.replace("false", "0").replace("true", "1").replace(" ", "")
     return re.sub(r">+$", ">", d) + ("/direct" if direct else "/split" if split else "")
 
