@@ -451,7 +451,9 @@ gemm_kernel16_rows(const _Float16 *__restrict__ A, const _Float16 *__restrict__ 
 // times the bytes in flight.  Tiles go global -> LDS by copy instructions (1 KB a wave, whole 128-byte row pieces: a
 // lane-per-row load of operand fragments straight into registers runs at 16 bytes per clock and CU, a quarter of this)
 // through ST stages, waited for by count.
-template <class T_, bool NN_, int WM_, int WN_, int TM_, int TN_, int KG_, int ST_>
+// FB: block edge of the MFMA (fp32: 32 or 16).  SETS (fp32): accumulators of a block that its multiplies take in turn, added up at the end: as
+// many partial sums as SETS groups over K would make, without the groups.
+template <class T_, bool NN_, int WM_, int WN_, int TM_, int TN_, int KG_, int ST_, int FB_ = sizeof(T_) == 2 ? 16 : 32, int SETS_ = 1>
 struct TileCfg {
   using T = T_;
   static constexpr bool NN = NN_;
@@ -463,7 +465,8 @@ struct TileCfg {
   static constexpr int A_PPW = BMT / 8 / WPG, PPW = (BMT + BNT) / 8 / WPG;   // 1 KB copies per wave and stage
   static constexpr int E_PITCH = BNT * 4 + 16, E_BYTES = KG * BMT * E_PITCH;  // epilogue: fp32 sums, rows padded
   static constexpr int LDS_BYTES = ST * STAGE > E_BYTES ? ST * STAGE : E_BYTES;
-  static constexpr int FB = ES == 2 ? 16 : 32;                                // block edge of the MFMA
+  static constexpr int SETS = SETS_;
+  static constexpr int FB = FB_;                                              // block edge of the MFMA
   static constexpr int RPP = THREADS * (16 / ES) / BNT, PASSES = (BMT + RPP - 1) / RPP;   // epilogue: rows per pass
   static_assert(A_PPW * WPG * 8 == BMT && PPW * WPG * 8 == BMT + BNT, "whole 1 KB copies per wave");
   static_assert(LDS_BYTES <= 160 * 1024 && ST >= 2, "stages");
@@ -475,7 +478,7 @@ struct TileCfg {
 template <class C, bool AHEAD = false>
 __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, const typename C::T *__restrict__ B,
                                           const typename C::T *__restrict__ Cin, typename C::T *__restrict__ D, int M, int N, int K,
-                                          float alpha, float beta, int block0) {
+                                          float alpha, float beta, int block0, int wg, int wgs) {
   using T = typename C::T;
   constexpr bool F16 = C::ES == 2, NN = C::NN;
   constexpr int ES = C::ES, FB = C::FB, MB = C::TM / FB, NB = C::TN / FB;
@@ -489,7 +492,7 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   // tile order: the 256 x 256 blocks in the order of the kernels above (from block0 on, the batch's problems one after the
   // other), the tiles of a block next to each other
   const int tiles_n = N / BN, tiles_m = M / BM;
-  const int w = xcd_remap(blockIdx.x, gridDim.x);
+  const int w = xcd_remap(wg, wgs);
   int t = block0 + w / C::SUB;
   const int s_idx = w % C::SUB;
   const int64_t batch = t / (tiles_m * tiles_n);
@@ -541,8 +544,8 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   // ---- LDS read addresses, relative to the group's part of a stage (see gemm_kernel16; fp32: lane (c, g) needs bytes
   // 32s + 16g .. +16 of its row, k = 8s + 4g .. +4, used one element per 32x32x2 MFMA: which contraction slot means which k
   // is free as long as A and B agree)
-  constexpr int KS = F16 ? 2 : 4;                  // K-steps (one 16-byte fragment per operand block) of a tile
-  constexpr int FPS = F16 ? 4 : 2;                 // fragments of a row in a K-step
+  constexpr int KS = FB == 16 ? 2 : 4;             // K-steps (one 16-byte fragment per operand block) of a tile
+  constexpr int FPS = FB == 16 ? 4 : 2;            // fragments of a row in a K-step
   int a_rd[KS], b_rd[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
@@ -559,15 +562,18 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
     }
   }
   using Frag = std::conditional_t<F16, half8, f32x4>;
-  using Acc = std::conditional_t<F16, f32x4, f32x16>;
-  constexpr int AV = F16 ? 4 : 16;
-  Acc acc[MB][NB];
+  using Acc = std::conditional_t<FB == 16, f32x4, f32x16>;
+  constexpr int AV = FB == 16 ? 4 : 16;
+  Acc accs[C::SETS][MB][NB];
+  auto &acc = accs[0];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
+  for (int x = 0; x < C::SETS; ++x)
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int v = 0; v < AV; ++v) acc[mb][nb][v] = 0.f;
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int v = 0; v < AV; ++v) accs[x][mb][nb][v] = 0.f;
 
   Frag af[2][MB], bf[2][NB];
   // fragment i of K-step s of the stage in `slot`, in the order the multiplies want them: B 0, A 0, B 1 .., A 1 ..
@@ -596,9 +602,12 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   auto multiply_block = [&](int mb, int nb, const Frag (&fa)[MB], const Frag (&fb)[NB]) __attribute__((always_inline)) {
     if constexpr (F16) {
       acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[nb], fa[mb], acc[mb][nb], 0, 0, 0);
+    } else if constexpr (FB == 16) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) accs[e % C::SETS][mb][nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[nb][e], fa[mb][e], accs[e % C::SETS][mb][nb], 0, 0, 0);
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[nb][e], fa[mb][e], acc[mb][nb], 0, 0, 0);
+      for (int e = 0; e < 4; ++e) accs[e % C::SETS][mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[nb][e], fa[mb][e], accs[e % C::SETS][mb][nb], 0, 0, 0);
     }
   };
   // The multiplies of one K-step with the other work (fragment reads of the next, copies).  Where all waves work on one tile
@@ -670,6 +679,14 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
     }
   }
 
+#pragma unroll
+  for (int x = 1; x < C::SETS; x *= 2)
+#pragma unroll
+    for (int y = 0; y < C::SETS; y += 2 * x)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) accs[y][mb][nb] += accs[y + x][mb][nb];
   // ---- epilogue: every group leaves its fp32 sums in the LDS as rows of C; they are added up, scaled and rounded once on
   // the way out, 16 bytes per lane of whole tile rows
   constexpr int PASSES = C::PASSES;
@@ -739,6 +756,9 @@ template <bool NN> struct HTile<NN, 128, 64> : TileCfg<_Float16, NN, 2, 2, 64, 3
 template <bool NN> struct HTile<NN, 64, 64> : TileCfg<_Float16, NN, 2, 2, 32, 32, 2, 4> {};
 template <bool NN> struct HTile<NN, 32, 32> : TileCfg<_Float16, NN, 1, 1, 32, 32, 4, 4> {};
 template <int EDGE> struct FTile;
+// ... and the two tiles of gemm_kernel_f32_mix, 32 KB of LDS each: 4 waves of 32 x 32 and of 16 x 16
+template <int SETS> struct FMix64 : TileCfg<float, false, 2, 2, 32, 32, 1, 2, 32, SETS> {};
+template <int SETS> struct FMix32 : TileCfg<float, false, 2, 2, 16, 16, 1, 4, 16, SETS> {};
 template <> struct FTile<128> : TileCfg<float, false, 2, 2, 64, 64, 1, 2> {};
 template <> struct FTile<64> : TileCfg<float, false, 2, 2, 32, 32, 2, 2> {};
 template <> struct FTile<32> : TileCfg<float, false, 1, 1, 32, 32, 4, 2> {};
@@ -747,28 +767,53 @@ template <bool NN, int ROWS, int COLS>
 __global__ void __launch_bounds__((HTile<NN, ROWS, COLS>::THREADS))
 gemm_kernel16_tile(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
                    _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta, int block0) {
-  gemm_tile<HTile<NN, ROWS, COLS>>(A, B, Cin, D, M, N, K, alpha, beta, block0);
+  gemm_tile<HTile<NN, ROWS, COLS>>(A, B, Cin, D, M, N, K, alpha, beta, block0, blockIdx.x, gridDim.x);
 }
 
 template <bool NN, int ROWS, int COLS>
 __global__ void __launch_bounds__((HTile<NN, ROWS, COLS>::THREADS))
 gemm_kernel16_tile_c(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
                      _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta, int block0) {
-  gemm_tile<HTile<NN, ROWS, COLS>, true>(A, B, Cin, D, M, N, K, alpha, beta, block0);
+  gemm_tile<HTile<NN, ROWS, COLS>, true>(A, B, Cin, D, M, N, K, alpha, beta, block0, blockIdx.x, gridDim.x);
 }
 
 template <int EDGE>
 __global__ void __launch_bounds__(FTile<EDGE>::THREADS)
 gemm_kernel_f32_c(const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ Cin, float *__restrict__ D,
                   int M, int N, int K, float alpha, float beta, int block0) {
-  gemm_tile<FTile<EDGE>, true>(A, B, Cin, D, M, N, K, alpha, beta, block0);
+  gemm_tile<FTile<EDGE>, true>(A, B, Cin, D, M, N, K, alpha, beta, block0, blockIdx.x, gridDim.x);
 }
 
 template <int EDGE>
 __global__ void __launch_bounds__(FTile<EDGE>::THREADS)
 gemm_kernel_f32(const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ Cin, float *__restrict__ D,
                 int M, int N, int K, float alpha, float beta, int block0) {
-  gemm_tile<FTile<EDGE>>(A, B, Cin, D, M, N, K, alpha, beta, block0);
+  gemm_tile<FTile<EDGE>>(A, B, Cin, D, M, N, K, alpha, beta, block0, blockIdx.x, gridDim.x);
+}
+
+// Tiles of 64 x 64 for the first blocks64 blocks and of 32 x 32 for the others, in one launch of workgroups of 4 waves, five of which share a
+// CU.  What bounds fp32 products is how evenly the multiplies go round the CUs and what of a workgroup's life is not multiplies (first
+// copies, sums through the LDS, stores: some 4 us): in whole rounds of one tile size three problems of 1024 x 768 x 1536 took nine 32 x 32
+// tiles on each CU, two at a time, 63.1 us -- now two of 64 x 64 and one of 32 x 32 beside each other 56.6; without the small ones, where some CUs
+// have three of 64 x 64, 73.4; the small ones first 57.2; three stages, so that three share a CU, 55.9, but 2304 x 768 x 3072 101.1 instead of 87.0.
+template <int SETS, bool AHEAD>
+__device__ __forceinline__ void gemm_f32_mix(const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ Cin, float *__restrict__ D,
+                                             int M, int N, int K, float alpha, float beta, int blocks64) {
+  const int n64 = blocks64 * FMix64<SETS>::SUB, wg = blockIdx.x;
+  if (wg < n64) gemm_tile<FMix64<SETS>, AHEAD>(A, B, Cin, D, M, N, K, alpha, beta, 0, wg, n64);
+  else gemm_tile<FMix32<SETS>>(A, B, Cin, D, M, N, K, alpha, beta, blocks64, wg - n64, (int)gridDim.x - n64);
+}
+template <int SETS>
+__global__ void __launch_bounds__(256)
+gemm_kernel_f32_mix(const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ Cin, float *__restrict__ D, int M, int N,
+                    int K, float alpha, float beta, int blocks64) {
+  gemm_f32_mix<SETS, false>(A, B, Cin, D, M, N, K, alpha, beta, blocks64);
+}
+template <int SETS>
+__global__ void __launch_bounds__(256)
+gemm_kernel_f32_mix_c(const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ Cin, float *__restrict__ D, int M, int N,
+                      int K, float alpha, float beta, int blocks64) {
+  gemm_f32_mix<SETS, true>(A, B, Cin, D, M, N, K, alpha, beta, blocks64);
 }
 
 // one-time set-up of a kernel (its dynamic-LDS limit), thread-safe and callable ahead of any launch
@@ -842,8 +887,24 @@ hipError_t launch_f16(const GemmArgs &g, hipStream_t s) {
   return c.tail_cols == 64 ? launch_tiles16<NN, 128, 64>(g, s, from, left) : launch_tiles16<NN, 128, 128>(g, s, from, left);
 }
 
+template <int SETS> constexpr int kMixLds = FMix64<SETS>::LDS_BYTES > FMix32<SETS>::LDS_BYTES ? FMix64<SETS>::LDS_BYTES : FMix32<SETS>::LDS_BYTES;
+template <int SETS>
+hipError_t launch_mix(const GemmArgs &g, hipStream_t s, int blocks, int blocks64) {
+  const bool with_c = g.C && g.beta != 0.f;
+  const hipError_t e = with_c ? prepare_kernel<gemm_kernel_f32_mix_c<SETS>, kMixLds<SETS>>() : prepare_kernel<gemm_kernel_f32_mix<SETS>, kMixLds<SETS>>();
+  if (e != hipSuccess) return e;
+  const int tiles = blocks64 * FMix64<SETS>::SUB + (blocks - blocks64) * FMix32<SETS>::SUB;
+  hipLaunchKernelGGL(with_c ? &gemm_kernel_f32_mix_c<SETS> : &gemm_kernel_f32_mix<SETS>, dim3(tiles), dim3(256), kMixLds<SETS>, s, (const float *)g.A, (const float *)g.B,
+                     (const float *)g.C, (float *)g.D, g.M, g.N, g.K, g.alpha, g.beta, blocks64);
+  return hipGetLastError();
+}
+
 hipError_t launch_f32(const GemmArgs &g, hipStream_t s) {
   const int blocks = (g.M / BM) * (g.N / BN) * g.batch, edge = choose_gemm_f32(blocks);
+  const GemmMix mix = choose_gemm_f32_mix(blocks, g.K);
+  if (mix.sums == 1) return launch_mix<1>(g, s, blocks, mix.blocks64);
+  if (mix.sums == 2) return launch_mix<2>(g, s, blocks, mix.blocks64);
+  if (mix.sums == 4) return launch_mix<4>(g, s, blocks, mix.blocks64);
   if (edge == 128) return launch_tiles32<128>(g, s, blocks);
   return edge == 64 ? launch_tiles32<64>(g, s, blocks) : launch_tiles32<32>(g, s, blocks);
 }
@@ -883,6 +944,11 @@ hipError_t prepare_gemm() {
   if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32<32>, FTile<32>::LDS_BYTES>();
   if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32_c<128>, FTile<128>::LDS_BYTES>();
   if (e == hipSuccess) e = prepare_kernel<gemm_kernel_f32_c<64>, FTile<64>::LDS_BYTES>();
+  const hipError_t mix[] = {prepare_kernel<gemm_kernel_f32_mix<1>, kMixLds<1>>(), prepare_kernel<gemm_kernel_f32_mix_c<1>, kMixLds<1>>(),
+                            prepare_kernel<gemm_kernel_f32_mix<2>, kMixLds<2>>(), prepare_kernel<gemm_kernel_f32_mix_c<2>, kMixLds<2>>(),
+                            prepare_kernel<gemm_kernel_f32_mix<4>, kMixLds<4>>(), prepare_kernel<gemm_kernel_f32_mix_c<4>, kMixLds<4>>()};
+  for (hipError_t x : mix)
+    if (e == hipSuccess) e = x;
   return e;
 }
 

@@ -86,4 +86,22 @@ inline int choose_gemm_f32(int blocks) {
   return t64 <= t32 ? 64 : 32;
 }
 
+// ... or, where sums > 0, tiles of 64 x 64 for the first blocks64 blocks, whole rounds of the CUs, and of 32 x 32 for the others beside them in one
+// launch (gemm_kernel_f32_mix).  An element is added up from as many partial sums as in the tile above, `sums`: with fewer it would be
+// further off, with more the time is up to 4 % longer (1, 2 and 4 at 3072 x 3328 x 384: 0.954, 0.978 and 0.995 of it).
+// Time relative to the tile above, one problem, K=256 to 4096: 17 to 28 blocks 0.78 to 0.98, 33 to 44 0.70 to 0.96, 49 to 60 0.81 to 0.98, 66 to 168
+// 0.84 to 0.99; with more than 12 blocks behind whole rounds, which would be a whole round themselves, 1.05 to 1.15; whole rounds
+// alone 1.01 up to 64 blocks and 0.98 to 0.99 beyond; 124 of two rounds of 64 blocks 1.00, 120 0.99, 561 of nine 1.025.  9 to 12 blocks in 32 x 32 tiles
+// alone: 0.92 at K=256, 0.95 at 768, 1.00 at 2048; fewer 1.03 to 1.28.
+struct GemmMix {
+  int blocks64, sums;
+};
+inline GemmMix choose_gemm_f32_mix(int blocks, int K) {
+  const int edge = choose_gemm_f32(blocks), left = blocks % 16, sums = edge == 128 ? 1 : edge == 64 ? 2 : 4;
+  if (blocks <= 16) return GemmMix{0, blocks >= 9 && blocks <= 12 && K <= 1024 ? 4 : 0};
+  if (left > 12 || (left == 0 && blocks <= 64)) return GemmMix{0, 0};
+  if (edge == 128 && blocks > 61 * ((blocks + 63) / 64)) return GemmMix{0, 0};   // (its rounds nearly full)
+  return GemmMix{blocks - left, sums};
+}
+
 }  // namespace cfk
