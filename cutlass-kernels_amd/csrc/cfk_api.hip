@@ -94,7 +94,13 @@ int query_blocks(const cfk_fmha_fwd_params *p, int bm) { return p->batch * p->he
 
 KeySplit plan_key_split(const cfk_fmha_fwd_params *p, const cfk::FmhaPlan &plan) {
   KeySplit k{key_splits(plan), 32, 0};
-  if (p->dtype == CFK_FP16 && !p->dbg_s) cfk::plan_fmha_f16_split(p->head_dim, p->seqlen_q, p->seqlen_kv, p->batch * p->heads, plan, &k);
+  if (p->dbg_s) return k;
+  if (p->dtype == CFK_FP16) cfk::plan_fmha_f16_split(p->head_dim, p->seqlen_q, p->seqlen_kv, p->batch * p->heads, plan, &k);
+  // (the taps are against the row max, which the partial results of fmha_fwd_kernel are not)
+  else if (!p->dbg_row_max && !p->dbg_row_sum) {
+    const bool hybrid = p->v_dtype == CFK_FP16;
+    (hybrid ? cfk::plan_fmha_hybrid_split : cfk::plan_fmha_fp8_split)(p->head_dim, p->seqlen_q, p->seqlen_kv, p->batch * p->heads, plan, &k);
+  }
   return k;
 }
 // one partial result: fp32 O and a (reference point, row sum) pair per query row

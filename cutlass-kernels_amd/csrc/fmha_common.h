@@ -56,6 +56,9 @@ struct KeySplit {
 };
 // For a fp16 call that would launch `plan`: whether cutting query blocks of a hand-scheduled build pays, and how.
 bool plan_fmha_f16_split(int head_dim, int sq, int skv, int bh, const FmhaPlan &plan, KeySplit *out);
+// ... and for one with e4m3 Q and K, of the compiler-scheduled builds; *out: how the call would share keys out otherwise.
+bool plan_fmha_fp8_split(int head_dim, int sq, int skv, int bh, const FmhaPlan &plan, KeySplit *out);
+bool plan_fmha_hybrid_split(int head_dim, int sq, int skv, int bh, const FmhaPlan &plan, KeySplit *out);
 
 // Each launcher validates nothing: the C-ABI layer has already checked shapes against the plan.
 // `tap_s` (plan) / a.s_tap (launch) selects the build of the kernel that also writes the score tap.

@@ -1,9 +1,8 @@
 // FMHA forward, fp16 operands: tile shapes and dispatch.  The kernels are in fmha_fwd_kernel.h (32x32 MFMAs) and
 // fmha_fwd_kernel16.h (16x16x32 MFMAs).
-#include <cmath>
-
 #include "fmha_fwd_kernel16p.h"
 #include "fmha_fwd_kernel_ks.h"
+#include "fmha_split_choice.h"
 
 namespace cfk {
 namespace {
@@ -66,10 +65,6 @@ using All128 = CfgList<C128_128x64, N128_128x64, C128_256x64P, C128_256x64, N128
 // time of the compiler-scheduled builds (geometric mean; the best choice for each 0.940), worst 1.04.  us, compiler-scheduled -> chosen:
 // head dim 64, 80 heads of 1696 rows, 3520 keys 144.9 -> 135.1; 161 of 192, 6400 keys 113.4 -> 94.5; head dim 128, 108 of 2560, 1856 keys
 // 277.5 -> 243.3; 168 of 704, 1664 keys 125.2 -> 107.8; 36 of 2016, 3200 keys 146.4 -> 117.3 (last round cut along the keys).
-float either(float a, float b) {   // about the larger of two times that overlap: the sixth root of the sum of their sixth powers
-  a *= a * a, b *= b * b;
-  return cbrtf(sqrtf(a * a + b * b));
-}
 struct Call {
   int head_dim, sq, skv, bh;
   int items(int bm) const { return bh * ((sq + bm - 1) / bm); }

@@ -3,6 +3,7 @@
 #include "fmha_fwd_kernel.h"
 #include "fmha_fwd_kernel8p.h"
 #include "fmha_fwd_kernel_ks.h"
+#include "fmha_split_choice.h"
 
 namespace cfk {
 namespace {
@@ -84,14 +85,40 @@ bool dispatch(int head_dim, int sq, int skv, int bh, int v_layout, bool tap_s, F
   }
 }
 
+// the SplitCfg build of a call: compiler-scheduled, 128 rows
+template <class F>
+void split_build(int head_dim, int skv, int v_layout, int units, F &&f) {
+  if (head_dim == 64) return v_layout != 1 ? f(C64_128x64{}) : units > 512 ? f(C64T3{}) : f(C64T{});
+  if (head_dim == 128) return v_layout != 1 ? f(C128_128x64{}) : f(C128T{});
+  return v_layout == 1 ? f(C256T{}) : skv % 128 == 0 ? f(C256_128x128{}) : f(C256_128x64{});
+}
+
 }  // namespace
 
 bool plan_fmha_fp8(int head_dim, int sq, int skv, int bh, int v_layout, bool tap_s, FmhaPlan *p) {
   return dispatch(head_dim, sq, skv, bh, v_layout, tap_s, [&](auto cfg) { fill_fmha_plan<decltype(cfg)>(sq, skv, bh, p); });
 }
 
+// The pass that tracks the row max (key lengths below 3072; cfk_api.hip) is slower in a way of its own.
+bool plan_fmha_fp8_split(int head_dim, int sq, int skv, int bh, const FmhaPlan &plan, KeySplit *out) {
+  const TileWish w = tile_wish();
+  const bool first_pass = skv >= 3072 && !predictable_latency();
+  if (plan.split_tiles || w.bm || w.bn || fast_e4m3_weights() || (!first_pass && head_dim != 256)) return false;
+  static constexpr CutTimes k64{3, {0.234f, 0.393f, 0.662f, 0.827f}, 8.67f, 1.06f, 0.f, 2.52f}, k128{2, {0.424f, 0.491f, 0.935f}, 0.f, 11.f, 1.95f, 4.43f},
+      k256{1, {0.895f, 1.023f}, 0.f, 2.84f, 0.f, 1.92f}, k256_tracked{1, {1.665f, 1.782f}, 4.66f, 0.83f, 6.07f, 4.32f};
+  const CutTimes &c = head_dim == 64 ? k64 : head_dim == 128 ? k128 : first_pass ? k256 : k256_tracked;
+  const float mbytes = 1e-6f * bh * head_dim * (3.f * sq + 2.f * skv);
+  return choose_cut(c, bh * ((sq + 127) / 128), skv, head_dim == 256 && skv % 128 == 0 ? 128 : 64, mbytes,
+                    head_dim, plan, out);
+}
+
 hipError_t launch_fmha_fp8(const FmhaArgs &a, int head_dim, hipStream_t s) {
   hipError_t e = hipErrorNotSupported;
+  if (a.n_split > 1 && a.split_bm == 128) {
+    const int items = a.B * a.H * ((a.Sq + 127) / 128);
+    split_build(head_dim, a.Skv, a.v_layout, a.split_from + (items - a.split_from) * a.n_split, [&](auto cfg) { e = launch_fmha_split<decltype(cfg)>(a, s); });
+    return e;
+  }
   dispatch(head_dim, a.Sq, a.Skv, a.B * a.H, a.v_layout, a.s_tap != nullptr, [&](auto cfg) { e = launch_fmha_cfg<decltype(cfg)>(a, s); });
   return e;
 }
@@ -101,6 +128,10 @@ hipError_t prepare_fmha_fp8() {
   if (e == hipSuccess) e = prepare_all(All128{});
   if (e == hipSuccess) e = prepare_all(All256{});
   if (e == hipSuccess) e = prepare_all(CfgList<K64, K128, K256, K64T, K128T, K256T>{});
+  const hipError_t split[] = {prepare_fmha_split<C64_128x64>(), prepare_fmha_split<C64T3>(), prepare_fmha_split<C64T>(), prepare_fmha_split<C128_128x64>(),
+                              prepare_fmha_split<C128T>(), prepare_fmha_split<C256T>(), prepare_fmha_split<C256_128x128>(), prepare_fmha_split<C256_128x64>()};
+  for (hipError_t x : split)
+    if (e == hipSuccess) e = x;
   if (e == hipSuccess) e = prepare_all(CfgList<C64T, C64T3, C128T, C256T, C64Tap, C128Tap, C256Tap, C64TTap, C128TTap, C256TTap>{});
   return e;
 }

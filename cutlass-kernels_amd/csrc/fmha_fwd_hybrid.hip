@@ -3,6 +3,7 @@
 // 446-450).  Tile shapes and dispatch; the kernel is in fmha_fwd_kernel.h.
 #include "fmha_fwd_kernel.h"
 #include "fmha_fwd_kernel_ks.h"
+#include "fmha_split_choice.h"
 
 namespace cfk {
 namespace {
@@ -58,8 +59,19 @@ bool plan_fmha_hybrid(int head_dim, int sq, int skv, int bh, bool tap_s, FmhaPla
   return dispatch(head_dim, sq, skv, bh, tap_s, [&](auto cfg) { fill_fmha_plan<decltype(cfg)>(sq, skv, bh, p); });
 }
 
+bool plan_fmha_hybrid_split(int head_dim, int sq, int skv, int bh, const FmhaPlan &plan, KeySplit *out) {
+  const TileWish w = tile_wish();
+  if (plan.split_tiles || w.bm || w.bn) return false;
+  static constexpr CutTimes k64{3, {0.404f, 0.609f, 1.039f, 1.314f}, 1.3f, 3.61f, 2.42f, 2.44f}, k128{2, {0.606f, 0.841f, 1.51f}, 2.74f, 2.1f, 3.65f, 3.16f},
+      k256{1, {1.207f, 1.481f}, 5.35f, 0.75f, 0.f, 2.31f};
+  const float mbytes = 1e-6f * bh * head_dim * 3.f * ((float)sq + skv);
+  return choose_cut(head_dim == 64 ? k64 : head_dim == 128 ? k128 : k256, bh * ((sq + 127) / 128), skv,
+                    head_dim == 256 ? 32 : 64, mbytes, head_dim, plan, out);
+}
+
 hipError_t launch_fmha_hybrid(const FmhaArgs &a, int head_dim, hipStream_t s) {
   hipError_t e = hipErrorNotSupported;
+  if (a.n_split > 1 && a.split_bm == 128) return head_dim == 64 ? launch_fmha_split<C64_128x64>(a, s) : head_dim == 128 ? launch_fmha_split<C128_128x64>(a, s) : launch_fmha_split<C256_128x32>(a, s);
   dispatch(head_dim, a.Sq, a.Skv, a.B * a.H, a.s_tap != nullptr, [&](auto cfg) { e = launch_fmha_cfg<decltype(cfg)>(a, s); });
   return e;
 }
@@ -69,6 +81,9 @@ hipError_t prepare_fmha_hybrid() {
   if (e == hipSuccess) e = prepare_all(All128{});
   if (e == hipSuccess) e = prepare_all(All256{});
   if (e == hipSuccess) e = prepare_all(CfgList<K64, K128, K256>{});
+  const hipError_t split[] = {prepare_fmha_split<C64_128x64>(), prepare_fmha_split<C128_128x64>(), prepare_fmha_split<C256_128x32>()};
+  for (hipError_t x : split)
+    if (e == hipSuccess) e = x;
   if (e == hipSuccess) e = prepare_all(CfgList<C64Tap, C128Tap, C256Tap>{});
   return e;
 }

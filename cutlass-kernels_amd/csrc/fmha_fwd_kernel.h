@@ -182,7 +182,25 @@ fmha_fwd_kernel(const FmhaArgs a) {
   const int r = lane & 31, g = lane >> 5;
 
   const int q_blocks = (a.Sq + C::BM - 1) / C::BM;   // the last query tile may be partly filled: whole waves of 32 rows
-  const int tile = xcd_remap(blockIdx.x, gridDim.x);
+  // SplitCfg: items from a.split_from on are n_split workgroups each, with a share of the item's key tiles (whole steps of SUB)
+  int tile, first_tile = 0, n_tiles = a.Skv / BN;
+  int64_t part_row = -1;   // index of the wave's first row in the partial results, -1: a whole item
+  if constexpr (C::SPLIT) {
+    const int n_cut = (int)(gridDim.x - a.split_from) / a.n_split;
+    if ((int)blockIdx.x < a.split_from) {
+      tile = xcd_remap(blockIdx.x, a.split_from);
+    } else {
+      const int unit = xcd_remap((int)blockIdx.x - a.split_from, n_cut * a.n_split);   // (an item's units next to each other)
+      const int x = unit / a.n_split, split = unit - x * a.n_split;
+      const int more = n_tiles / C::SUB - a.split_tiles * a.n_split;   // (the first units take a step more)
+      tile = a.split_from + x;
+      first_tile = C::SUB * (split * a.split_tiles + (split < more ? split : more));
+      n_tiles = C::SUB * (a.split_tiles + (split < more));
+      part_row = ((int64_t)split * n_cut + x) * C::BM + wave * 32;
+    }
+  } else {
+    tile = xcd_remap(blockIdx.x, gridDim.x);
+  }
   const int bh = tile / q_blocks;
   const int qb = tile - bh * q_blocks;
   const int b = bh / a.H, h = bh - b * a.H;
@@ -198,10 +216,13 @@ fmha_fwd_kernel(const FmhaArgs a) {
   // the last 32 rows (loads stay in bounds) and stores nothing.
   const bool live = qb * C::BM + wave * 32 < a.Sq;
   const int q0 = live ? qb * C::BM + wave * 32 : a.Sq - 32;
-  const int n_tiles = a.Skv / BN;
   const float c_log2 = a.scale_log2;
   // global row pitch in bytes
   const uint32_t k_ld = (uint32_t)(ld * QES), v_ld = C::VT ? (uint32_t)a.H * (uint32_t)a.Skv : (uint32_t)(ld * VES);
+  if constexpr (C::SPLIT) {
+    Kp += (size_t)first_tile * ((size_t)BN * k_ld);
+    Vp += C::VT ? (size_t)first_tile * BN : (size_t)first_tile * ((size_t)BN * v_ld);
+  }
 
   // ---- global -> LDS copies.  Copy i of wave w covers tile rows (i*NWAVES + w)*RPI .. +RPI; lane l writes LDS slot
   // (row l / CPR, chunk position l % CPR) and fetches chunk position ^ swz(row) of that row.
@@ -714,6 +735,18 @@ fmha_fwd_kernel(const FmhaArgs a) {
 
   // ---- epilogue: O = out_scale * O / l (online_softmax.h:59-85), fp16, [B,S,H,D]; a lane holds 4 consecutive d
   const float l_tot = MFMA_SUM ? l_acc[0] : l_run + __shfl_xor(l_run, 32, 64);
+  if constexpr (C::SPLIT) {
+    if (part_row >= 0) {   // fp32, as the accumulators hold it
+      if (!live) return;
+      float *po = a.part_o + (part_row + r) * D, *ml = a.part_ml + (part_row + r) * 2;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *(f32x4 *)(po + db * 32 + 8 * i + 4 * g) = f32x4{oacc[db][4 * i], oacc[db][4 * i + 1], oacc[db][4 * i + 2], oacc[db][4 * i + 3]};
+      if (g == 0) ml[0] = m_ref, ml[1] = l_tot;
+      return;
+    }
+  }
   const float inv = a.out_scale / l_tot;
   const int qrow = q0 + r;
   // The accumulator layout gives a lane 4 consecutive d of ONE row: stored directly, a wave-wide store would touch
@@ -774,7 +807,7 @@ template <class C>
 struct DirectCfg : C {
   static constexpr bool DIRECT = true;
 };
-// The hand-scheduled persistent build with the keys of some items cut into units of work of their own (FmhaArgs::n_split).
+// The same build with the keys of some items cut into units of work of their own (FmhaArgs::n_split): fmha_fwd_kernel and the hand-scheduled fp16 ones.
 template <class C>
 struct SplitCfg : C {
   static constexpr bool SPLIT = true;
@@ -860,8 +893,8 @@ hipError_t launch_fmha_split(const FmhaArgs &a, hipStream_t s) {
   if (e != hipSuccess) return e;
   const int items = a.B * a.H * ((a.Sq + C::BM - 1) / C::BM), units = a.split_from + (items - a.split_from) * a.n_split;
   FmhaArgs with_tiles = a;
-  with_tiles.split_tiles = a.Skv / C::BN / a.n_split;
-  hipLaunchKernelGGL(fmha_kernel_of<SplitCfg<C>>(), dim3(persistent_grid(units)), dim3(C::T), C::LDS_BYTES, s, with_tiles);
+  with_tiles.split_tiles = a.Skv / (C::ASM ? C::BN : C::BN * C::SUB) / a.n_split;
+  hipLaunchKernelGGL(fmha_kernel_of<SplitCfg<C>>(), dim3(C::ASM ? persistent_grid(units) : units), dim3(C::T), C::LDS_BYTES, s, with_tiles);
   return hipGetLastError();
 }
 
