@@ -7,6 +7,8 @@ and streams; all compute happens in ``libcfk_fmha.so``.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import math
 import os
 import struct
@@ -16,6 +18,8 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_HERE, "libcfk_fmha.so")
 _lib = None
 _launch = None   # (fmha, fmha with workspace, gemm): the launching entry points taking their parameter block as bytes
+_BINDING_PATH = os.path.join(_HERE, "cfk_torch.so")
+_native = None   # csrc/cfk_torch.cpp: plain calls without the interpreter between their steps
 _torch = None
 
 CFK_FP16 = 1
@@ -189,13 +193,24 @@ def fmha_forward_kernel(dtype, batch, heads, seqlen_q, seqlen_kv, head_dim, v_la
     return buf.value.decode()
 
 
+def _load_native(l):
+    if not os.path.exists(_BINDING_PATH):
+        raise RuntimeError(f"{_BINDING_PATH} is missing: build it first (make -C {os.path.join(_HERE, 'csrc')})")
+    loader = importlib.machinery.ExtensionFileLoader("cfk_torch", _BINDING_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("cfk_torch", loader))
+    loader.exec_module(module)
+    module.setup(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (l.cfk_fmha_forward_or_workspace, l.cfk_fmha_forward_ws, l.cfk_gemm)))
+    return module
+
+
 def _launchers():
     """torch and the launching entry points, looked up once."""
-    global _torch, _launch
+    global _torch, _launch, _native
     if _launch is None:
         import torch
         l = lib()
         _torch = torch
+        _native = _load_native(l)
         _launch = (ctypes.CFUNCTYPE(ctypes.c_int64, ctypes.c_char_p, ctypes.c_void_p)(("cfk_fmha_forward_or_workspace", l)),
                    ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_char_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p)(("cfk_fmha_forward_ws", l)),
                    ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_char_p, ctypes.c_void_p)(("cfk_gemm", l)))
@@ -220,6 +235,10 @@ def fmha_forward(q, k, v, o=None, softmax_scale=None, q_descale=1.0, k_descale=1
     ``v_layout == CFK_V_BDHS``.  ``row_max`` / ``row_sum`` / ``scores`` are the optional debug taps.  Returns ``o`` (float16 [B,Sq,H,D]); launches asynchronously on ``stream``
     (default: torch's current stream).  A call whose keys are split takes scratch memory from torch's allocator; capture it through
     ``torch.cuda.graph``, which keeps that memory for the replays."""
+    if _native is not None and stream is None and row_max is None and row_sum is None and scores is None and not prepare:
+        done = _native.fmha(q, k, v, o, softmax_scale, q_descale, k_descale, v_descale, v_layout, _workspace_or_none)
+        if done is not None:   # (None: not a plain call)
+            return done if type(done) is not int else _check(done)
     launch, launch_ws, _ = _launch or _launchers()
     f16 = _torch.float16
     if not (q.is_cuda and k.is_cuda and v.is_cuda):
@@ -355,6 +374,10 @@ def gemm(a, b, c=None, alpha=1.0, beta=0.0, out=None, layout=CFK_GEMM_TN, stream
     [K,N] (NN, fp16 only), with the same leading batch dimension; ``c`` / ``out`` are [M,N] or [L,M,N].  float16 or
     float32 device tensors, all of one dtype (the reference's types 3 and 1, gemm.cu:677-684).
     """
+    if _native is not None and stream is None:
+        done = _native.gemm(a, b, c, alpha, beta, out, layout)
+        if done is not None:   # (None: not a plain call)
+            return done if type(done) is not int else _check(done)
     _, _, launch = _launch or _launchers()
     dt = a.dtype
     if dt not in (_torch.float16, _torch.float32) or b.dtype != dt or not (a.is_cuda and b.is_cuda):
