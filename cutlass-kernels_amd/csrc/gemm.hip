@@ -453,7 +453,9 @@ gemm_kernel16_rows(const _Float16 *__restrict__ A, const _Float16 *__restrict__ 
 // through ST stages, waited for by count.
 // FB: block edge of the MFMA (fp32: 32 or 16).  SETS (fp32): accumulators of a block that its multiplies take in turn, added up at the end: as
 // many partial sums as SETS groups over K would make, without the groups.
-template <class T_, bool NN_, int WM_, int WN_, int TM_, int TN_, int KG_, int ST_, int FB_ = sizeof(T_) == 2 ? 16 : 32, int SETS_ = 1>
+// SHARE: the two groups take the two K-steps of one K tile instead of a K tile each.  All waves fill a stage, half the size, so twice as
+// many of them are in flight, for a barrier every K-step (which tiles: gemm_choice.h; M=N=2048 K=4096 TN 39.4 -> 36.9 us).
+template <class T_, bool NN_, int WM_, int WN_, int TM_, int TN_, int KG_, int ST_, int FB_ = sizeof(T_) == 2 ? 16 : 32, int SETS_ = 1, bool SHARE_ = false>
 struct TileCfg {
   using T = T_;
   static constexpr bool NN = NN_;
@@ -461,14 +463,21 @@ struct TileCfg {
   static constexpr int BMT = WM * TM, BNT = WN * TN, SUB = (BM / BMT) * (BN / BNT);  // tiles of a 256 x 256 block
   static constexpr int WPG = WM * WN, NW = WPG * KG, THREADS = NW * 64;
   static constexpr int BK = 128 / ES;
-  static constexpr int A_BYTES = BMT * 128, G_BYTES = (BMT + BNT) * 128, STAGE = KG * G_BYTES;
-  static constexpr int A_PPW = BMT / 8 / WPG, PPW = (BMT + BNT) / 8 / WPG;   // 1 KB copies per wave and stage
+  static constexpr bool SHARE = SHARE_;
+  static constexpr int A_BYTES = BMT * 128, G_BYTES = (BMT + BNT) * 128, STAGE = (SHARE ? 1 : KG) * G_BYTES;
+  static constexpr int CW = SHARE ? NW : WPG;                                 // waves that fill a group's part of a stage
+  static constexpr int A_PIECES = BMT / 8, PIECES = (BMT + BNT) / 8, PPW = (PIECES + CW - 1) / CW;   // 1 KB copies of a stage, per wave
   static constexpr int E_PITCH = BNT * 4 + 16, E_BYTES = KG * BMT * E_PITCH;  // epilogue: fp32 sums, rows padded
   static constexpr int LDS_BYTES = ST * STAGE > E_BYTES ? ST * STAGE : E_BYTES;
   static constexpr int SETS = SETS_;
   static constexpr int FB = FB_;                                              // block edge of the MFMA
-  static constexpr int RPP = THREADS * (16 / ES) / BNT, PASSES = (BMT + RPP - 1) / RPP;   // epilogue: rows per pass
-  static_assert(A_PPW * WPG * 8 == BMT && PPW * WPG * 8 == BMT + BNT, "whole 1 KB copies per wave");
+  static constexpr bool EDGES = BM % BMT || BN % BNT;                          // tiles of M x N instead of a 256 x 256 block's
+  static constexpr int RPP = THREADS / (BNT * ES / 16), PASSES = (BMT + RPP - 1) / RPP;   // epilogue: rows per pass
+  // what piece i of a wave copies: a part of A, a part of B, or the one or the other by wave, some of them a part that another wave copies too
+  static constexpr int A_PART = 0, B_PART = 1, BY_WAVE = 2;
+  static constexpr int part(int i) { return (i + 1) * CW <= A_PIECES ? A_PART : i * CW >= A_PIECES && (i + 1) * CW <= PIECES ? B_PART : BY_WAVE; }
+  static_assert(A_PIECES * 8 == BMT && PIECES * 8 == BMT + BNT && (SHARE || PIECES % CW == 0), "whole 1 KB copies");
+  static_assert(!SHARE || (ES == 2 && KG == 2), "two groups, two K-steps");
   static_assert(LDS_BYTES <= 160 * 1024 && ST >= 2, "stages");
 };
 
@@ -490,11 +499,12 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   const int c = lane % FB, g = lane / FB;
 
   // tile order: the 256 x 256 blocks in the order of the kernels above (from block0 on, the batch's problems one after the
-  // other), the tiles of a block next to each other
-  const int tiles_n = N / BN, tiles_m = M / BM;
+  // other), the tiles of a block next to each other; EDGES: the tiles themselves in that order, and a last one that would reach beyond the edge
+  // lies against it instead and leaves out what its neighbour stores
+  const int tiles_n = C::EDGES ? (N + C::BNT - 1) / C::BNT : N / BN, tiles_m = C::EDGES ? (M + C::BMT - 1) / C::BMT : M / BM;
   const int w = xcd_remap(wg, wgs);
-  int t = block0 + w / C::SUB;
-  const int s_idx = w % C::SUB;
+  int t = C::EDGES ? w : block0 + w / C::SUB;
+  const int s_idx = C::EDGES ? 0 : w % C::SUB;
   const int64_t batch = t / (tiles_m * tiles_n);
   t -= (int)batch * tiles_m * tiles_n;
   constexpr int GROUP = 8;
@@ -503,8 +513,9 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   const int first_m = grp * GROUP;
   const int rows_in_group = tiles_m - first_m < GROUP ? tiles_m - first_m : GROUP;
   const int in_grp = t - grp * per_group;
-  const int m0 = (first_m + in_grp % rows_in_group) * BM + s_idx / (BN / C::BNT) * C::BMT;
-  const int n0 = in_grp / rows_in_group * BN + s_idx % (BN / C::BNT) * C::BNT;
+  const int m_own = (first_m + in_grp % rows_in_group) * (C::EDGES ? C::BMT : BM) + (C::EDGES ? 0 : s_idx / (BN / C::BNT) * C::BMT);
+  const int n_own = in_grp / rows_in_group * (C::EDGES ? C::BNT : BN) + (C::EDGES ? 0 : s_idx % (BN / C::BNT) * C::BNT);
+  const int m0 = !C::EDGES || m_own + C::BMT <= M ? m_own : M - C::BMT, n0 = !C::EDGES || n_own + C::BNT <= N ? n_own : N - C::BNT;
   A += batch * M * K;
   B += batch * N * K;
   D += batch * M * N;
@@ -513,28 +524,33 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   const char *Bp = NN ? (const char *)(B + n0) : (const char *)(B + (int64_t)n0 * K);
 
   // ---- copies: group kg fills its own part of a stage; piece i of a wave is 8 rows of A or B (NN: 1 KB of k rows of B)
+  const int ci = C::SHARE ? wave : wi;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)LDS_PTR(char, smem);
+  const uint32_t lds_wave = lds_base + (C::SHARE ? 0 : kg * C::G_BYTES) + ci * 1024;
   uint32_t goff[C::PPW];
+  bool of_a[C::PPW], again[C::PPW];
 #pragma unroll
   for (int i = 0; i < C::PPW; ++i) {
-    const int p = i < C::A_PPW ? i * C::WPG + wi : (i - C::A_PPW) * C::WPG + wi;
-    if (!NN || i < C::A_PPW) {
+    int q = i * C::CW + ci;
+    again[i] = C::part(i) == C::BY_WAVE && q >= C::PIECES;
+    if (again[i]) q -= C::PIECES;
+    of_a[i] = C::part(i) == C::BY_WAVE ? q < C::A_PIECES : C::part(i) == C::A_PART;
+    const int p = of_a[i] ? q : q - C::A_PIECES;
+    if (!NN || of_a[i]) {
       const int row = p * 8 + lane / 8;
       goff[i] = (uint32_t)row * (uint32_t)(K * ES) + (uint32_t)(((lane % 8) ^ swz_k<128>(row)) * 16);
     } else {
       constexpr int CPR = BPITCH / 16;
-      const int krow = p * (64 / CPR) + lane / CPR;
-      goff[i] = (uint32_t)krow * (uint32_t)(N * 2) + (uint32_t)(((lane % CPR) ^ swz_bn<BPITCH>(krow)) * 16);
+      const int idx = p * 64 + lane, krow = idx / CPR;
+      goff[i] = (uint32_t)krow * (uint32_t)(N * 2) + (uint32_t)(((idx % CPR) ^ swz_bn<BPITCH>(krow)) * 16);
     }
   }
-  const uint32_t lds_base = (uint32_t)(uintptr_t)LDS_PTR(char, smem);
-  const uint32_t lds_wave = lds_base + kg * C::G_BYTES + wi * 1024;
-  const int chunks = K / C::BK, n_st = (chunks + C::KG - 1) / C::KG;
+  const int chunks = K / C::BK, n_st = C::SHARE ? chunks : (chunks + C::KG - 1) / C::KG;
   auto load_piece = [&](int j, int slot, int i) __attribute__((always_inline)) {
-    int ch = j * C::KG + kg;
+    int ch = C::SHARE ? j : j * C::KG + kg;
     ch = ch < chunks ? ch : chunks - 1;   // (a group without a tile in the last turn copies one it does not multiply)
-    const bool is_a = i < C::A_PPW;
-    const char *gp = is_a ? Ap + (size_t)ch * 128 : NN ? Bp + (size_t)ch * ((size_t)C::BK * N * 2) : Bp + (size_t)ch * 128;
-    lds_dma16(gp, goff[i], lds_wave + slot * C::STAGE, is_a ? i * C::WPG * 1024 : C::A_BYTES + (i - C::A_PPW) * C::WPG * 1024);
+    const char *gp = of_a[i] ? Ap + (size_t)ch * 128 : NN ? Bp + (size_t)ch * ((size_t)C::BK * N * 2) : Bp + (size_t)ch * 128;
+    lds_dma16(gp, goff[i], lds_wave + slot * C::STAGE, (uint32_t)(i * C::CW - (again[i] ? C::PIECES : 0)) * 1024u);
   };
   auto load_stage = [&](int j, int slot) __attribute__((always_inline)) {
 #pragma unroll
@@ -544,13 +560,14 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   // ---- LDS read addresses, relative to the group's part of a stage (see gemm_kernel16; fp32: lane (c, g) needs bytes
   // 32s + 16g .. +16 of its row, k = 8s + 4g .. +4, used one element per 32x32x2 MFMA: which contraction slot means which k
   // is free as long as A and B agree)
-  constexpr int KS = FB == 16 ? 2 : 4;             // K-steps (one 16-byte fragment per operand block) of a tile
+  constexpr int KS = C::SHARE ? 1 : FB == 16 ? 2 : 4;   // K-steps (one 16-byte fragment per operand block) of a tile
   constexpr int FPS = FB == 16 ? 4 : 2;            // fragments of a row in a K-step
   int a_rd[KS], b_rd[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
-    a_rd[s] = (wm * C::TM + c) * 128 + (((FPS * s + g) ^ swz_k<128>(c)) * 16);
-    b_rd[s] = C::A_BYTES + (wn * C::TN + c) * 128 + (((FPS * s + g) ^ swz_k<128>(c)) * 16);
+    const int ks = C::SHARE ? kg : s;
+    a_rd[s] = (wm * C::TM + c) * 128 + (((FPS * ks + g) ^ swz_k<128>(c)) * 16);
+    b_rd[s] = C::A_BYTES + (wn * C::TN + c) * 128 + (((FPS * ks + g) ^ swz_k<128>(c)) * 16);
   }
   int bt_rd[NB];
   if constexpr (NN) {
@@ -558,7 +575,7 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       const int chunk = (wn * C::TN + 16 * nb) / 8 + (cg >> 1);
-      bt_rd[nb] = C::A_BYTES + bk_row * BPITCH + ((chunk ^ swz_bn<BPITCH>(bk_row)) * 16) + (cg & 1) * 8;
+      bt_rd[nb] = C::A_BYTES + (C::SHARE ? kg * 32 * BPITCH : 0) + bk_row * BPITCH + ((chunk ^ swz_bn<BPITCH>(bk_row)) * 16) + (cg & 1) * 8;
     }
   }
   using Frag = std::conditional_t<F16, half8, f32x4>;
@@ -579,7 +596,7 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   // fragment i of K-step s of the stage in `slot`, in the order the multiplies want them: B 0, A 0, B 1 .., A 1 ..
   constexpr int FRAGS = MB + NB;
   auto fetch_piece = [&](int slot, int s, int i, Frag (&fa)[MB], Frag (&fb)[NB]) __attribute__((always_inline)) {
-    const char *st = smem + slot * C::STAGE + kg * C::G_BYTES;
+    const char *st = smem + slot * C::STAGE + (C::SHARE ? 0 : kg * C::G_BYTES);
     if (i == 1 || i > NB) {
       const int mb = i == 1 ? 0 : i - NB;
       fa[mb] = *(const Frag *)(st + a_rd[s] + mb * FB * 128);
@@ -633,8 +650,12 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   };
   // Waits until all but this wave's copies of the `behind` newest stages have landed and its LDS reads have returned, and
   // meets the others: then everybody's copies have, and a slot whose reads lie in front of the barrier is free.
+  static_assert(C::ST <= 8 && (C::ST - 1) * C::PPW < 64, "copies that can be waited for by count");
   auto arrive = [&](int behind) __attribute__((always_inline)) {
-    if (C::ST >= 5 && behind >= 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(3 * C::PPW) : "memory");
+    if (C::ST >= 8 && behind >= 6) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::ST >= 8 ? 6 * C::PPW : 0) : "memory");
+    else if (C::ST >= 7 && behind >= 5) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::ST >= 7 ? 5 * C::PPW : 0) : "memory");
+    else if (C::ST >= 6 && behind >= 4) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::ST >= 6 ? 4 * C::PPW : 0) : "memory");
+    else if (C::ST >= 5 && behind >= 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(3 * C::PPW) : "memory");
     else if (C::ST >= 4 && behind >= 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * C::PPW) : "memory");
     else if (C::ST >= 3 && behind >= 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::PPW) : "memory");
     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -650,32 +671,54 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   for (int i = 0; i < FRAGS; ++i) fetch_piece(0, 0, i, af[0], bf[0]);
   using std::integral_constant;
   int slot = 0;
-  for (int j = 0; j + 1 < n_st; ++j) {
-    const int next = slot == C::ST - 1 ? 0 : slot + 1;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      if (s + 1 < KS) {
-        multiply_with(af[s & 1], bf[s & 1], integral_constant<int, FRAGS>{},
-                      [&](int k) __attribute__((always_inline)) { fetch_piece(slot, s + 1, k, af[(s + 1) & 1], bf[(s + 1) & 1]); });
-      } else {
-        const int behind = n_st - 2 - j;
-        arrive(behind < C::ST - 2 ? behind : C::ST - 2);
-        const bool more = j + C::ST < n_st;
-        multiply_with(af[s & 1], bf[s & 1], integral_constant<int, FRAGS + C::PPW>{}, [&](int k) __attribute__((always_inline)) {
-          if (k < FRAGS) fetch_piece(next, 0, k, af[0], bf[0]);
-          else if (more) load_piece(j + C::ST, slot, k - FRAGS);
-        });
-      }
+  if constexpr (C::SHARE) {
+    auto step = [&](auto parity, int j) __attribute__((always_inline)) {   // one K-step of a stage: the fragments change places every stage
+      constexpr int P = decltype(parity)::value;
+      const int next = slot == C::ST - 1 ? 0 : slot + 1, behind = n_st - 2 - j;
+      arrive(behind < C::ST - 2 ? behind : C::ST - 2);
+      const bool more = j + C::ST < n_st;
+      multiply_with(af[P], bf[P], integral_constant<int, FRAGS + C::PPW>{}, [&](int k) __attribute__((always_inline)) {
+        if (k < FRAGS) fetch_piece(next, 0, k, af[P ^ 1], bf[P ^ 1]);
+        else if (more) load_piece(j + C::ST, slot, k - FRAGS);
+      });
+      slot = next;
+    };
+    int j = 0;
+    for (; j + 2 < n_st; j += 2) {
+      step(integral_constant<int, 0>{}, j);
+      step(integral_constant<int, 1>{}, j + 1);
     }
-    slot = next;
-  }
-  if (C::KG == 1 || (n_st - 1) * C::KG + kg < chunks) {
+    if (j + 1 < n_st) step(integral_constant<int, 0>{}, j);
+    if (n_st % 2 == 0) multiply_with(af[1], bf[1], integral_constant<int, 0>{}, [](int) {});
+    else multiply_with(af[0], bf[0], integral_constant<int, 0>{}, [](int) {});
+  } else {
+    for (int j = 0; j + 1 < n_st; ++j) {
+      const int next = slot == C::ST - 1 ? 0 : slot + 1;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      if (s + 1 < KS)
-        multiply_with(af[s & 1], bf[s & 1], integral_constant<int, FRAGS>{},
-                      [&](int k) __attribute__((always_inline)) { fetch_piece(slot, s + 1, k, af[(s + 1) & 1], bf[(s + 1) & 1]); });
-      else multiply_with(af[s & 1], bf[s & 1], integral_constant<int, 0>{}, [](int) {});
+      for (int s = 0; s < KS; ++s) {
+        if (s + 1 < KS) {
+          multiply_with(af[s & 1], bf[s & 1], integral_constant<int, FRAGS>{},
+                        [&](int k) __attribute__((always_inline)) { fetch_piece(slot, s + 1, k, af[(s + 1) & 1], bf[(s + 1) & 1]); });
+        } else {
+          const int behind = n_st - 2 - j;
+          arrive(behind < C::ST - 2 ? behind : C::ST - 2);
+          const bool more = j + C::ST < n_st;
+          multiply_with(af[s & 1], bf[s & 1], integral_constant<int, FRAGS + C::PPW>{}, [&](int k) __attribute__((always_inline)) {
+            if (k < FRAGS) fetch_piece(next, 0, k, af[0], bf[0]);
+            else if (more) load_piece(j + C::ST, slot, k - FRAGS);
+          });
+        }
+      }
+      slot = next;
+    }
+    if (C::KG == 1 || (n_st - 1) * C::KG + kg < chunks) {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        if (s + 1 < KS)
+          multiply_with(af[s & 1], bf[s & 1], integral_constant<int, FRAGS>{},
+                        [&](int k) __attribute__((always_inline)) { fetch_piece(slot, s + 1, k, af[(s + 1) & 1], bf[(s + 1) & 1]); });
+        else multiply_with(af[s & 1], bf[s & 1], integral_constant<int, 0>{}, [](int) {});
+      }
     }
   }
 
@@ -692,10 +735,13 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
   constexpr int PASSES = C::PASSES;
   std::conditional_t<F16, half8, f32x4> c_ahead[AHEAD ? PASSES : 1];
   if constexpr (AHEAD) {
-    constexpr int EPL = 16 / ES, LPR = C::BNT / EPL, RPP = C::THREADS / LPR;
+    constexpr int EPL = 16 / ES, LPR = C::BNT / EPL, RPP = C::RPP;
 #pragma unroll
-    for (int pass = 0; pass < PASSES; ++pass)
-      c_ahead[pass] = *(const decltype(&c_ahead[0]))(Cin + (int64_t)(m0 + pass * RPP + tid / LPR) * N + n0 + (tid % LPR) * EPL);
+    for (int pass = 0; pass < PASSES; ++pass) {
+      int row = pass * RPP + tid / LPR;
+      if (C::BMT % RPP && row >= C::BMT) row = C::BMT - 1;   // (not stored)
+      c_ahead[pass] = *(const decltype(&c_ahead[0]))(Cin + (int64_t)(m0 + row) * N + n0 + (tid % LPR) * EPL);
+    }
   }
   __syncthreads();
 #pragma unroll
@@ -711,15 +757,16 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
         *(f32x4 *)(smem + (kg * C::BMT + wm * C::TM + mb * FB + c) * C::E_PITCH + (wn * C::TN + nb * FB + 8 * i + 4 * g) * 4) = v4;
       }
   __syncthreads();
-  constexpr int EPL = 16 / ES, LPR = C::BNT / EPL, RPP = C::THREADS / LPR;
+  constexpr int EPL = 16 / ES, LPR = C::BNT / EPL, RPP = C::RPP;
   using OutV = std::conditional_t<F16, half8, f32x4>;
   const bool with_c = AHEAD || (PASSES == 1 && Cin != nullptr && beta != 0.f);   // (several passes meet a C in the AHEAD kernels only)
   const int e_row = tid / LPR, e_col = (tid % LPR) * EPL;
-  static_assert(C::BMT % RPP == 0 || RPP > C::BMT, "whole passes");
+  static_assert(C::BMT % RPP == 0 || RPP > C::BMT || C::EDGES, "whole passes");
 #pragma unroll
   for (int pass = 0; pass < PASSES; ++pass) {
     const int row = pass * RPP + e_row;
-    if (RPP > C::BMT && row >= C::BMT) break;
+    if (C::BMT % RPP && row >= C::BMT) break;
+    if (C::EDGES && (e_row >= RPP || m0 + row < m_own || n0 + e_col < n_own)) continue;
     const int64_t off = (int64_t)(m0 + row) * N + n0 + e_col;
     float v[EPL];
 #pragma unroll
@@ -751,10 +798,20 @@ __device__ __forceinline__ void gemm_tile(const typename C::T *__restrict__ A, c
 // the bytes in flight).
 template <bool NN, int ROWS, int COLS> struct HTile;
 template <bool NN> struct HTile<NN, 256, 128> : TileCfg<_Float16, NN, 4, 2, 64, 64, 1, 3> {};
+template <bool NN> struct HTile<NN, 192, 128> : TileCfg<_Float16, NN, 4, 2, 48, 64, 1, 3> {};
+template <bool NN> struct HTile<NN, 128, 192> : TileCfg<_Float16, NN, 2, 4, 64, 48, 1, 3> {};
+template <bool NN> struct HTile<NN, 96, 128> : TileCfg<_Float16, NN, 2, 2, 48, 64, 2, 2> {};
+template <bool NN> struct HTile<NN, 96, 96> : TileCfg<_Float16, NN, 2, 2, 48, 48, 2, 3> {};
+template <bool NN> struct HTile<NN, 96, 64> : TileCfg<_Float16, NN, 2, 2, 48, 32, 2, 4> {};
+template <bool NN> struct HTile<NN, 64, 32> : TileCfg<_Float16, NN, 2, 1, 32, 32, 4, 3> {};
 template <bool NN> struct HTile<NN, 128, 128> : TileCfg<_Float16, NN, 2, 2, 64, 64, 2, 2> {};
 template <bool NN> struct HTile<NN, 128, 64> : TileCfg<_Float16, NN, 2, 2, 64, 32, 2, 3> {};
 template <bool NN> struct HTile<NN, 64, 64> : TileCfg<_Float16, NN, 2, 2, 32, 32, 2, 4> {};
 template <bool NN> struct HTile<NN, 32, 32> : TileCfg<_Float16, NN, 1, 1, 32, 32, 4, 4> {};
+// ... and those whose two groups share K tiles
+template <bool NN, int ROWS> struct HShared;
+template <bool NN> struct HShared<NN, 128> : TileCfg<_Float16, NN, 2, 2, 64, 64, 2, 5, 16, 1, true> {};
+template <bool NN> struct HShared<NN, 96> : TileCfg<_Float16, NN, 2, 2, 48, 64, 2, 5, 16, 1, true> {};
 template <int EDGE> struct FTile;
 // ... and the two tiles of gemm_kernel_f32_mix, 32 KB of LDS each: 4 waves of 32 x 32 and of 16 x 16
 template <int SETS> struct FMix64 : TileCfg<float, false, 2, 2, 32, 32, 1, 2, 32, SETS> {};
@@ -775,6 +832,21 @@ __global__ void __launch_bounds__((HTile<NN, ROWS, COLS>::THREADS))
 gemm_kernel16_tile_c(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
                      _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta, int block0) {
   gemm_tile<HTile<NN, ROWS, COLS>, true>(A, B, Cin, D, M, N, K, alpha, beta, block0, blockIdx.x, gridDim.x);
+}
+
+// ROWS x 128
+template <bool NN, int ROWS>
+__global__ void __launch_bounds__((HShared<NN, ROWS>::THREADS))
+gemm_kernel16_shared(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
+                     _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta, int block0) {
+  gemm_tile<HShared<NN, ROWS>>(A, B, Cin, D, M, N, K, alpha, beta, block0, blockIdx.x, gridDim.x);
+}
+
+template <bool NN, int ROWS>
+__global__ void __launch_bounds__((HShared<NN, ROWS>::THREADS))
+gemm_kernel16_shared_c(const _Float16 *__restrict__ A, const _Float16 *__restrict__ B, const _Float16 *__restrict__ Cin,
+                       _Float16 *__restrict__ D, int M, int N, int K, float alpha, float beta, int block0) {
+  gemm_tile<HShared<NN, ROWS>, true>(A, B, Cin, D, M, N, K, alpha, beta, block0, blockIdx.x, gridDim.x);
 }
 
 template <int EDGE>
@@ -842,31 +914,41 @@ hipError_t launch_blocks(const GemmArgs &g, hipStream_t s, int tiles) {
   return hipGetLastError();
 }
 
-// `blocks` 256 x 256 blocks from block0 on, in tiles of configuration C by kernel Kern
+// tiles of configuration C by kernel Kern, of the 256 x 256 blocks from block0 on (EDGES: all that there are)
 template <class C, auto Kern>
-hipError_t launch_tiles(const GemmArgs &g, hipStream_t s, int block0, int blocks) {
+hipError_t launch_tiles(const GemmArgs &g, hipStream_t s, int block0, int tiles) {
   const hipError_t e = prepare_kernel<Kern, C::LDS_BYTES>();
   if (e != hipSuccess) return e;
   using T = typename C::T;
-  hipLaunchKernelGGL(Kern, dim3(blocks * C::SUB), dim3(C::THREADS), C::LDS_BYTES, s, (const T *)g.A, (const T *)g.B, (const T *)g.C,
+  hipLaunchKernelGGL(Kern, dim3(tiles), dim3(C::THREADS), C::LDS_BYTES, s, (const T *)g.A, (const T *)g.B, (const T *)g.C,
                      (T *)g.D, g.M, g.N, g.K, g.alpha, g.beta, block0);
   return hipGetLastError();
 }
 template <bool NN, int ROWS, int COLS>
-hipError_t launch_tiles16(const GemmArgs &g, hipStream_t s, int block0, int blocks) {
+hipError_t launch_edge16(const GemmArgs &g, hipStream_t s, int tiles, int block0 = 0) {
   using C = HTile<NN, ROWS, COLS>;
   if constexpr (C::PASSES > 1) {
-    if (g.C && g.beta != 0.f) return launch_tiles<C, gemm_kernel16_tile_c<NN, ROWS, COLS>>(g, s, block0, blocks);
+    if (g.C && g.beta != 0.f) return launch_tiles<C, gemm_kernel16_tile_c<NN, ROWS, COLS>>(g, s, block0, tiles);
   }
-  return launch_tiles<C, gemm_kernel16_tile<NN, ROWS, COLS>>(g, s, block0, blocks);
+  return launch_tiles<C, gemm_kernel16_tile<NN, ROWS, COLS>>(g, s, block0, tiles);
+}
+template <bool NN, int ROWS, int COLS>
+hipError_t launch_tiles16(const GemmArgs &g, hipStream_t s, int block0, int blocks) {
+  return launch_edge16<NN, ROWS, COLS>(g, s, blocks * HTile<NN, ROWS, COLS>::SUB, block0);
+}
+template <bool NN, int ROWS>
+hipError_t launch_shared(const GemmArgs &g, hipStream_t s, int tiles, int block0) {
+  using C = HShared<NN, ROWS>;
+  if (g.C && g.beta != 0.f) return launch_tiles<C, gemm_kernel16_shared_c<NN, ROWS>>(g, s, block0, tiles);
+  return launch_tiles<C, gemm_kernel16_shared<NN, ROWS>>(g, s, block0, tiles);
 }
 template <int EDGE>
 hipError_t launch_tiles32(const GemmArgs &g, hipStream_t s, int blocks) {
   using C = FTile<EDGE>;
   if constexpr (C::PASSES > 1) {
-    if (g.C && g.beta != 0.f) return launch_tiles<C, gemm_kernel_f32_c<EDGE>>(g, s, 0, blocks);
+    if (g.C && g.beta != 0.f) return launch_tiles<C, gemm_kernel_f32_c<EDGE>>(g, s, 0, blocks * C::SUB);
   }
-  return launch_tiles<C, gemm_kernel_f32<EDGE>>(g, s, 0, blocks);
+  return launch_tiles<C, gemm_kernel_f32<EDGE>>(g, s, 0, blocks * C::SUB);
 }
 
 // What the choice names (gemm_choice.h).
@@ -874,6 +956,9 @@ template <bool NN>
 hipError_t launch_f16(const GemmArgs &g, hipStream_t s) {
   const GemmChoice c = choose_gemm_f16(g.M, g.N, g.K, g.batch);
   hipError_t e = hipSuccess;
+  if (c.rows == 96) return c.cols == 64 ? launch_edge16<NN, 96, 64>(g, s, c.tiles) : c.cols == 96 ? launch_edge16<NN, 96, 96>(g, s, c.tiles) : g.K >= kSharedFrom ? launch_shared<NN, 96>(g, s, c.tiles, 0) : launch_edge16<NN, 96, 128>(g, s, c.tiles);
+  if (c.rows == 128) return launch_edge16<NN, 128, 192>(g, s, c.tiles);
+  if (c.rows == 192 && c.cols == 128) return launch_edge16<NN, 192, 128>(g, s, c.tiles);
   if (c.rows == 256 && c.cols == 256) e = launch_blocks<NN, 8, 4>(g, s, c.tiles);
   else if (c.rows == 256) e = launch_blocks<NN, 8, 3>(g, s, c.tiles);
   else if (c.rows == 320) e = launch_blocks<NN, 10, 4>(g, s, c.tiles);
@@ -882,9 +967,11 @@ hipError_t launch_f16(const GemmArgs &g, hipStream_t s) {
   if (e != hipSuccess || !c.tail_blocks) return e;
   const int from = c.tiles, left = c.tail_blocks;
   if (c.tail_rows == 32) return launch_tiles16<NN, 32, 32>(g, s, from, left);
+  if (c.tail_rows == 64 && c.tail_cols == 32) return launch_tiles16<NN, 64, 32>(g, s, from, left);
   if (c.tail_rows == 64) return launch_tiles16<NN, 64, 64>(g, s, from, left);
   if (c.tail_rows == 256) return launch_tiles16<NN, 256, 128>(g, s, from, left);
-  return c.tail_cols == 64 ? launch_tiles16<NN, 128, 64>(g, s, from, left) : launch_tiles16<NN, 128, 128>(g, s, from, left);
+  if (c.tail_cols == 64) return launch_tiles16<NN, 128, 64>(g, s, from, left);
+  return g.K >= kSharedFrom ? launch_shared<NN, 128>(g, s, left * HShared<NN, 128>::SUB, from) : launch_tiles16<NN, 128, 128>(g, s, from, left);
 }
 
 template <int SETS> constexpr int kMixLds = FMix64<SETS>::LDS_BYTES > FMix32<SETS>::LDS_BYTES ? FMix64<SETS>::LDS_BYTES : FMix32<SETS>::LDS_BYTES;
@@ -909,6 +996,12 @@ hipError_t launch_f32(const GemmArgs &g, hipStream_t s) {
   return edge == 64 ? launch_tiles32<64>(g, s, blocks) : launch_tiles32<32>(g, s, blocks);
 }
 
+template <bool NN, int ROWS, int COLS>
+hipError_t prepare_tile() {
+  constexpr int lds = HTile<NN, ROWS, COLS>::LDS_BYTES;
+  const hipError_t e = prepare_kernel<gemm_kernel16_tile<NN, ROWS, COLS>, lds>();
+  return e != hipSuccess ? e : prepare_kernel<gemm_kernel16_tile_c<NN, ROWS, COLS>, lds>();
+}
 template <bool NN>
 hipError_t prepare_f16() {
   const hipError_t e[] = {prepare_kernel<block_kernel<NN, 8, 4>(), BlockCfg<8, 4>::LDS_BYTES>(),
@@ -916,12 +1009,11 @@ hipError_t prepare_f16() {
                           prepare_kernel<block_kernel<NN, 6, 4>(), BlockCfg<6, 4>::LDS_BYTES>(),
                           prepare_kernel<block_kernel<NN, 6, 3>(), BlockCfg<6, 3>::LDS_BYTES>(),
                           prepare_kernel<block_kernel<NN, 10, 4>(), BlockCfg<10, 4>::LDS_BYTES>(),
-                          prepare_kernel<gemm_kernel16_tile<NN, 256, 128>, HTile<NN, 256, 128>::LDS_BYTES>(),
-                          prepare_kernel<gemm_kernel16_tile<NN, 128, 128>, HTile<NN, 128, 128>::LDS_BYTES>(),
-                          prepare_kernel<gemm_kernel16_tile<NN, 128, 64>, HTile<NN, 128, 64>::LDS_BYTES>(),
-                          prepare_kernel<gemm_kernel16_tile_c<NN, 256, 128>, HTile<NN, 256, 128>::LDS_BYTES>(),
-                          prepare_kernel<gemm_kernel16_tile_c<NN, 128, 128>, HTile<NN, 128, 128>::LDS_BYTES>(),
-                          prepare_kernel<gemm_kernel16_tile_c<NN, 128, 64>, HTile<NN, 128, 64>::LDS_BYTES>(),
+                          prepare_tile<NN, 256, 128>(), prepare_tile<NN, 128, 128>(), prepare_tile<NN, 128, 64>(),
+                          prepare_tile<NN, 192, 128>(), prepare_tile<NN, 128, 192>(), prepare_tile<NN, 96, 128>(), prepare_tile<NN, 96, 96>(), prepare_tile<NN, 96, 64>(),
+                          prepare_kernel<gemm_kernel16_shared<NN, 128>, HShared<NN, 128>::LDS_BYTES>(), prepare_kernel<gemm_kernel16_shared_c<NN, 128>, HShared<NN, 128>::LDS_BYTES>(),
+                          prepare_kernel<gemm_kernel16_shared<NN, 96>, HShared<NN, 96>::LDS_BYTES>(), prepare_kernel<gemm_kernel16_shared_c<NN, 96>, HShared<NN, 96>::LDS_BYTES>(),
+                          prepare_kernel<gemm_kernel16_tile<NN, 64, 32>, HTile<NN, 64, 32>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 64, 64>, HTile<NN, 64, 64>::LDS_BYTES>(),
                           prepare_kernel<gemm_kernel16_tile<NN, 32, 32>, HTile<NN, 32, 32>::LDS_BYTES>()};
   for (hipError_t x : e)

@@ -5,6 +5,7 @@
 namespace cfk {
 
 constexpr int kCus = 256;
+constexpr int kSharedFrom = 1088;   // K from which tiles of 96 x 128 and 128 x 128 run with groups that share K tiles (below)
 
 // A first launch of `tiles` macro tiles of rows x cols, and a second one of `tail_blocks` blocks of 256 x 256, the last ones of the batch, in
 // tiles of tail_rows x tail_cols; either may be missing (0).
@@ -35,6 +36,32 @@ inline GemmChoice gemm_blocks_and_tiles(int blocks) {
   return c;
 }
 
+// fp16, up to half a round of 256 x 256 blocks: one round of tiles, the smaller the better.  Between the sizes that divide a block lie others (the
+// last ones against the edges of M x N), taken from 512 of K on where the CUs hold them all at once.  Time relative to the next larger
+// size that divides a block, K=512 to 8192, TN and NN, with and without C, 500 drawn products: 64 x 32 0.89 to 0.93 (5 to 8 blocks), 96 x 64 0.90 to
+// 0.95 (17 to 24), 96 x 96 0.69 to 0.78, 96 x 128 0.92 to 0.94 (33 to 48), 128 x 192 and 192 x 128 0.89 to 0.95 (65 to 96).  us: 768 x 3072 x 4800 NN with C
+// 41.6 -> 29.7; M=N=1536 K=2048 TN 19.7 -> 13.6; 512 x 1024 x 2240 8.4 -> 6.8; 3840 x 1024 x 2048 21.3 -> 20.1.  (Measured and not built: 128 x 96 0.94 to 0.99, 64 x 96 0.95 to 0.99 of the larger size.)
+// What bounds the smaller ones is the bytes that a CU gets from the L2, 59 to 70 a nanosecond.  The two with 128 columns, of which two K
+// tiles a turn leave room for one turn ahead in the LDS, waited for them: with both groups at one K tile and four ahead 0.87 of the time
+// at 128 x 128 and 0.85 at 96 x 128 from 1536 of K on, 0.93 from 1088 (worst 1.10, operands of 10 us in the L2), 1.05 to 1.10 at 512 to 768.  The others have three
+// or four turns in the LDS and lose by it: 128 x 64 0.99 to 1.09, 96 x 96 1.01 to 1.03, 64 x 64 and 96 x 64 1.03 to 1.21.
+inline GemmChoice choose_gemm_f16_round(int M, int N, int K, int batch, int blocks) {
+  const auto tiles = [&](int r, int c) { return (int)((long long)((M + r - 1) / r) * ((N + c - 1) / c) * batch); };
+  const auto in = [&](int from, int to) { return blocks >= from && blocks <= to; };
+  if (K >= 512) {
+    if (in(5, 8)) return GemmChoice{0, 0, 0, 64, 32, blocks};
+    if (in(17, 24) && tiles(96, 64) <= kCus) return GemmChoice{96, 64, tiles(96, 64), 0, 0, 0};
+    if (in(33, 48) && tiles(96, 96) <= kCus) return GemmChoice{96, 96, tiles(96, 96), 0, 0, 0};
+    if (in(33, 48) && tiles(96, 128) <= kCus) return GemmChoice{96, 128, tiles(96, 128), 0, 0, 0};
+    if (in(65, 96)) {
+      const int wide = tiles(128, 192), high = tiles(192, 128);
+      if (wide <= high && wide <= kCus) return GemmChoice{128, 192, wide, 0, 0, 0};
+      if (high <= kCus) return GemmChoice{192, 128, high, 0, 0, 0};
+    }
+  }
+  return gemm_blocks_and_tiles(blocks);
+}
+
 // fp16.  From half a round of 256 x 256 blocks on: rounds of other macro tiles where these waste less of the chip.  Times in rounds of 256 x 256
 // tiles; one of which a share f is filled takes (1 + f)/2, because the idle CUs leave the others their power.
 // Measured, every tile for 842 drawn products of 129 to 1040 blocks, TN and NN, with and without C, D the same and three in turn; a full round,
@@ -48,8 +75,8 @@ inline GemmChoice gemm_blocks_and_tiles(int blocks) {
 // (64.3 against 61.8 for a round of 256 x 128).
 inline GemmChoice choose_gemm_f16(int M, int N, int K, int batch) {
   const int blocks = (M / 256) * (N / 256) * batch;
+  if (blocks <= kCus / 2) return choose_gemm_f16_round(M, N, K, batch, blocks);
   GemmChoice choice = gemm_blocks_and_tiles(blocks);
-  if (blocks <= kCus / 2) return choice;
   const auto rounds = [](long long tiles) {
     const int part = (int)(tiles % kCus);
     return (double)(tiles / kCus) + (part ? 0.5 + 0.5 * part / kCus : 0.0);
