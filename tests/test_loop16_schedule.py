@@ -357,7 +357,8 @@ class Checker:
 
 
 @pytest.mark.parametrize("shape,rowsum,fold", [("d128", "mfma", False), ("d128", "mfma", True), ("d128", "add", True), ("d128w4", "add", True), ("d128", "add", False), ("d128", "dot", False),
-                                               ("d256", "add", True), ("d256", "add", False), ("d64", "mfma", True), ("d64", "mfma", False), ("d64w4", "mfma", True)])
+                                               ("d256", "add", True), ("d256", "add", False), ("d64", "mfma", True), ("d64", "mfma", False), ("d64w4", "mfma", True),
+                                               ("d128w4", "add", False), ("d64w4", "mfma", False)])
 @pytest.mark.parametrize("n_tiles", [8, 12, 16, 32, 64])
 def test_loop_is_correct_symbolically(n_tiles, shape, rowsum, fold):
     g = _gen()
@@ -386,10 +387,12 @@ def _run_with_late_barrier(c, prog):
 
 @pytest.mark.parametrize("shape", ["d128", "d128w4", "d256", "d64", "d64w4"])
 @pytest.mark.parametrize("n_tiles", [7, 8, 9, 10, 11, 13, 14, 15, 16, 33, 34, 35])
-def test_any_number_of_tiles(n_tiles, shape):
+@pytest.mark.parametrize("fold", [True, False])   # (False: the loops with a multiply-add per score, which take most lengths with tiles left over)
+def test_any_number_of_tiles(n_tiles, shape, fold):
     g = _gen()
-    g.SHAPE, g.ROWSUM = shape, ("mfma" if shape.startswith("d64") else "add")
+    g.SHAPE, g.ROWSUM, g.FOLD = shape, ("mfma" if shape.startswith("d64") else "add"), fold
     g.configure()
+    assert g.FOLDED == fold
     prog = g.program(n_tiles)
     assert len(prog) == len(sum(g.schedule(n_tiles), []))   # (the turns of the loop add up to all tiles)
     _run_with_late_barrier(Checker(g, n_tiles), prog)
