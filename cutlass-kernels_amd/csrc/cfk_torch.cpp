@@ -171,4 +171,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "cfk_torch", nullptr, -1, methods};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_cfk_torch(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_cfk_torch(void) {
+  PyObject *m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", CFK_TORCH_VERSION) == 0) return m;   // (torch's C++ interface holds for one version)
+  Py_XDECREF(m);
+  return nullptr;
+}

@@ -13,13 +13,14 @@ import math
 import os
 import struct
 import subprocess
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_HERE, "libcfk_fmha.so")
 _lib = None
 _launch = None   # (fmha, fmha with workspace, gemm): the launching entry points taking their parameter block as bytes
 _BINDING_PATH = os.path.join(_HERE, "cfk_torch.so")
-_native = None   # csrc/cfk_torch.cpp: plain calls without the interpreter between their steps
+_native = None   # csrc/cfk_torch.cpp, where it can be loaded: plain calls without the interpreter between their steps
 _torch = None
 
 CFK_FP16 = 1
@@ -193,12 +194,18 @@ def fmha_forward_kernel(dtype, batch, heads, seqlen_q, seqlen_kv, head_dim, v_la
     return buf.value.decode()
 
 
-def _load_native(l):
-    if not os.path.exists(_BINDING_PATH):
-        raise RuntimeError(f"{_BINDING_PATH} is missing: build it first (make -C {os.path.join(_HERE, 'csrc')})")
-    loader = importlib.machinery.ExtensionFileLoader("cfk_torch", _BINDING_PATH)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("cfk_torch", loader))
-    loader.exec_module(module)
+def _load_native(l, torch_version):
+    """The extension, or None where it cannot serve -- not built, or built against another torch: every call then goes through ctypes."""
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("cfk_torch", _BINDING_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("cfk_torch", loader))
+        loader.exec_module(module)
+        if getattr(module, "torch_version", None) != torch_version:
+            raise ImportError("it was built against another torch")
+    except ImportError as e:
+        warnings.warn(f"{_BINDING_PATH} is not used with torch {torch_version}: {e} (make -C {os.path.join(_HERE, 'csrc')} builds it); small "
+                      "calls take up to 2 us longer on the host", RuntimeWarning, stacklevel=3)
+        return None
     module.setup(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (l.cfk_fmha_forward_or_workspace, l.cfk_fmha_forward_ws, l.cfk_gemm)))
     return module
 
@@ -210,7 +217,7 @@ def _launchers():
         import torch
         l = lib()
         _torch = torch
-        _native = _load_native(l)
+        _native = _load_native(l, str(torch.__version__))
         _launch = (ctypes.CFUNCTYPE(ctypes.c_int64, ctypes.c_char_p, ctypes.c_void_p)(("cfk_fmha_forward_or_workspace", l)),
                    ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_char_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p)(("cfk_fmha_forward_ws", l)),
                    ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_char_p, ctypes.c_void_p)(("cfk_gemm", l)))

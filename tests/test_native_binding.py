@@ -1,12 +1,14 @@
 """The launching calls as native code (csrc/cfk_torch.cpp) against the same calls in Python: the same results for plain calls, and the
 same errors for the others, which the native code leaves to Python."""
 import contextlib
+import os
+import subprocess
 import types
 
 import pytest
 import torch
 
-from _util import pkg
+from _util import ROOT, pkg
 
 f = pkg.fmha
 
@@ -25,6 +27,40 @@ def test_calls_that_are_not_plain_are_left_to_python():
         assert f._native.gemm(*args) is None
     for args in [(s, s, s, None, None, 1.0, 1.0, 1.0, 0, None), (s.to("meta"),) * 3 + (None, None, 1.0, 1.0, 1.0, 0, None), (None,) * 10, ()]:
         assert f._native.fmha(*args) is None
+
+
+@pytest.mark.parametrize("why", ["missing", "no library", "other torch", "older build"])
+def test_calls_go_through_ctypes_where_the_extension_cannot_serve(why, monkeypatch, tmp_path):
+    path, version = tmp_path / "cfk_torch.so", str(torch.__version__)
+    if why == "no library":
+        path.write_bytes(b"not an ELF file")
+    if why == "older build":     # (no version in it)
+        (tmp_path / "m.c").write_text("#include <Python.h>\nstatic struct PyModuleDef m = {PyModuleDef_HEAD_INIT, \"cfk_torch\", 0, -1, 0};\n"
+                                      "PyMODINIT_FUNC PyInit_cfk_torch(void) { return PyModule_Create(&m); }\n")
+        subprocess.run(["gcc", "-shared", "-fPIC", "-I", __import__("sysconfig").get_paths()["include"], "-o", str(path), str(tmp_path / "m.c")], check=True)
+    if why != "other torch":
+        monkeypatch.setattr(f, "_BINDING_PATH", str(path))
+    else:
+        version = "0.4.1"
+    with pytest.warns(RuntimeWarning, match="cfk_torch.so is not used"):
+        assert f._load_native(pkg.lib(), version) is None
+    monkeypatch.setattr(f, "_native", None)
+    h = torch.zeros((256, 64), dtype=torch.float16)
+    with pytest.raises(ValueError):    # (the call is made in Python, which refuses a CPU tensor)
+        pkg.gemm(h, h)
+
+
+def _plan(*args):
+    r = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "cutlass-kernels_amd", "csrc"), *args], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    assert "libcfk_fmha.so" in r.stdout
+    return "cfk_torch.so" in r.stdout
+
+
+def test_the_library_builds_without_torch_or_a_host_compiler():
+    assert _plan()
+    assert not _plan("PYTHON=false") and not _plan("PYTHON=no-such-python") and not _plan("CXX=no-such-compiler")
+    assert not _plan("TORCH=/nowhere") and not _plan("PYINC=/nowhere")
 
 
 def _gemm_calls():
