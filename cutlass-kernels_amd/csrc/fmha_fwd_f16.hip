@@ -83,10 +83,11 @@ float round_us(const HandTimes &h, int units, int tiles) {
   const float busy = 2.f * units / kCus - 1.f;
   return units ? h.round + tiles * (h.low + (h.full - h.low) * (busy > 0.f ? busy : 0.f)) : 0.f;
 }
-float fma_us(const Call &c, const HandTimes &h) {
+float fma_issue_us(const Call &c, const HandTimes &h) {
   const int items = c.items(h.bm);
-  return either(h.first + items / kCus * round_us(h, kCus, c.tiles()) + round_us(h, items % kCus, c.tiles()), c.mbytes() / 3.4f);
+  return h.first + items / kCus * round_us(h, kCus, c.tiles()) + round_us(h, items % kCus, c.tiles());
 }
+float fma_us(const Call &c, const HandTimes &h) { return either(fma_issue_us(c, h), c.mbytes() / 3.4f); }
 // the same with the items from `from` on cut into n units along the keys, and the merge of their results
 float fma_cut_us(const Call &c, const HandTimes &h, int n, int from) {
   const int units = n * (c.items(h.bm) - from);
@@ -102,17 +103,31 @@ float compiled_us(const Call &c, bool m16) {
   return c.head_dim == 64 ? 3.33f * ceilf(x / 3) - 0.2f + either(c.tiles() * per_tile, c.mbytes() / 3.42f)
                           : 6.57f * ceilf(x / 2) - 2.73f + either(c.tiles() * per_tile, c.mbytes() / 3.93f);
 }
-// rows of the FmaCfg build to take instead of a compiler-scheduled one, 0: none; *us: the time of the better one
-int fma_rows(const Call &c, bool m16, float *us) {
-  int bm = 0;
+// rows of the FmaCfg build to take instead of a compiler-scheduled one, 0: none; *us: the least of the sums, *rows_of_sum: whose it is
+int fma_rows(const Call &c, bool m16, float *us, int *rows_of_sum) {
+  int bm = *rows_of_sum = 0;
   *us = compiled_us(c, m16);
   float best = 0.97f * *us;
   for (int rows : {256, 128}) {
     if (rows == 128 && c.skv < 1024) continue;   // (0.98 to 1.06 of the time there)
     // (a last 256-row tile that is filled to half or less in every other tile -- 320, 352, 384 rows -- gained nothing: 0.99 to 1.08)
     if (rows == 256 && 2 * c.items(128) <= 3 * c.items(256)) continue;
-    const float t = fma_us(c, fma_times(c.head_dim, rows));
-    if (t < best) bm = rows, best = *us = t;
+    const HandTimes h = fma_times(c.head_dim, rows);
+    const float t = fma_us(c, h);
+    if (t >= best) continue;
+    best = *us = t, *rows_of_sum = rows;
+    // Where the sum says less and the calls took more (540 drawn calls, time relative to the compiler-scheduled build):
+    // 128 rows: more than a round of items 0.99 to 1.37 (300 heads of 128 rows, 1152 keys, head dim 64 24.0 -> 32.8 us; 96 heads of 608, 2048 keys, head dim 128
+    // 72.8 -> 75.3); a round or less: head dim 128 below 1216 keys 0.99 to 1.02; head dim 64 below 1600 keys and few rows a head, so that reading K and V
+    // takes as long as the multiplies, 0.98 to 1.16 (222 heads of 128 rows, 1216 keys 16.1 -> 18.6).  The others 0.92 to 1.00.
+    // 256 rows: head dim 128, up to half a round behind one whole round, below 896 keys 0.99 to 1.13 (336 heads of 224 rows, 768 keys 51.7 -> 57.1; 32 of 2912,
+    // 704 keys 39.8 -> 41.6), with more 0.93 to 1.01; head dim 64, a round or less below 768 keys, reading K and V, 0.96 to 1.05.  The others 0.73 to 1.02.
+    const int items = c.items(rows);
+    const bool reading = c.mbytes() / 3.4f > 0.8f * fma_issue_us(c, h);   // (or nearly as long)
+    const bool slower = rows == 128           ? items > kCus || (c.head_dim == 128 ? c.skv < 1216 : reading && c.skv < 1600)
+                        : c.head_dim == 128 ? items > kCus && 2 * items <= 3 * kCus && c.skv < 896
+                                            : items <= kCus && reading && c.skv < 768;
+    bm = slower ? 0 : rows;
   }
   return bm;
 }
@@ -126,7 +141,8 @@ void select_f16(int head_dim, int sq, int skv, int bh, F &&f) {
       // whose nine tiles are all in front of the loop and behind it)
       if (hand_loops_allowed() && fits<F256>(sq, skv) && !(head_dim == 128 && skv < 640) && !(problem_size(sq, bh) == 2 && skv < 1280)) {
         float us;
-        const int rows = fma_rows(Call{head_dim, sq, skv, bh}, C::M16, &us);
+        int sum;
+        const int rows = fma_rows(Call{head_dim, sq, skv, bh}, C::M16, &us, &sum);
         if (rows == 256) return f(F256{});
         if (rows == 128) return f(F128{});
       }
@@ -209,7 +225,9 @@ bool plan_fmha_f16_split(int head_dim, int sq, int skv, int bh, const FmhaPlan &
   if (head_dim != 256 && !(plan.hand && !plan.fma)) {
     const Call call{head_dim, sq, skv, bh};
     float us;
-    fma_rows(call, plan.mfma == 16, &us);
+    int rows;
+    fma_rows(call, plan.mfma == 16, &us, &rows);
+    if (rows) fma_rows(call, true, &us, &rows);   // (where a FmaCfg sum is the least, cuts were fitted beside the sum of fmha_fwd_kernel16)
     us *= 0.95f;
     KeySplit best{};
     for (int bm : {256, 128}) {

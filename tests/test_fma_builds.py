@@ -54,6 +54,20 @@ def test_which_calls_take_them_without_gpu():
         assert f.fmha_forward_kernel(f.CFK_FP16, *call).startswith("fmha_fwd_kernel16p<"), call
 
 
+# where the sums over rounds say less time for these builds and the calls took more: 1.02 to 1.37 of the compiler-scheduled builds' (fmha_fwd_f16.hip)
+SLOWER = [(5, 60, 128, 1152, 64), (8, 43, 128, 1472, 64), (6, 37, 128, 1216, 64), (7, 24, 96, 1088, 64), (8, 30, 160, 640, 64), (3, 54, 256, 576, 64),
+          (4, 24, 608, 1728, 128), (8, 18, 576, 1216, 128), (3, 48, 288, 3520, 128), (3, 20, 288, 1152, 128), (7, 48, 224, 768, 128), (8, 4, 2912, 704, 128)]
+FASTER = [(3, 27, 224, 1408, 64), (8, 10, 192, 1856, 64), (7, 29, 160, 1024, 64), (5, 27, 160, 832, 64), (6, 17, 160, 1728, 128), (3, 32, 192, 1856, 128),
+          (2, 22, 2208, 640, 128), (5, 38, 192, 2112, 128), (8, 20, 160, 2944, 128)]   # 0.82 to 0.96, on the other side of the lines
+
+
+def test_calls_that_these_builds_lose_stay_compiler_scheduled_without_gpu():
+    for call in SLOWER:
+        assert f.fmha_forward_kernel(f.CFK_FP16, *call).startswith(("fmha_fwd_kernel<", "fmha_fwd_kernel16<")), call
+    for call in FASTER:
+        assert f.fmha_forward_kernel(f.CFK_FP16, *call).startswith("fmha_fwd_kernel16f<"), call
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,Sq,Skv,D", [(2, 18, 2016, 3200, 128), (1, 50, 192, 1984, 128), (1, 18, 3840, 3264, 64), (1, 4, 1504, 4672, 256)])
 @pytest.mark.parametrize("keys", ["plain", "climbing", "masked"])
