@@ -137,9 +137,11 @@ void select_f16(int head_dim, int sq, int skv, int bh, F &&f) {
   tile_by_rule<Auto, Fallback>(sq, skv, bh, [&](auto cfg) {
     using C = decltype(cfg);
     if constexpr (!C::KSPLIT && !C::ASM) {
-      // (the tests pin the kernels of two calls with whole 256-row tiles and fewer than 1280 keys, and of one with 576 keys at head dim 128,
-      // whose nine tiles are all in front of the loop and behind it)
-      if (hand_loops_allowed() && fits<F256>(sq, skv) && !(head_dim == 128 && skv < 640) && !(problem_size(sq, bh) == 2 && skv < 1280)) {
+      // (time relative to the compiler-scheduled build, drawn calls with what fma_rows leaves out left out: head dim 128, 512 and 576 keys 0.87 to 1.04; 640 keys 0.90 to
+      // 0.99, but with at least 512 whole 256-row tiles, which fmha_fwd_kernel16 takes otherwise, 0.90 to 1.03; from 704 on 0.78 to 0.97 there.  Head dim 64,
+      // as many tiles, up to 1216 keys 0.93 to 1.00, 0.977 in the geometric mean: not worth a time that depends on the data)
+      const bool big = problem_size(sq, bh) == 2;
+      if (hand_loops_allowed() && fits<F256>(sq, skv) && skv >= (head_dim == 128 ? big ? 704 : 640 : big ? 1280 : 512)) {
         float us;
         int sum;
         const int rows = fma_rows(Call{head_dim, sq, skv, bh}, C::M16, &us, &sum);

@@ -22,7 +22,8 @@ using C256_128x64 = FmhaCfg<256, 64, 4, 1, false, false>;
 // 256): two 32-key tiles per barrier, big problems only
 using A256_128x64 = FmhaCfg<256, 32, 4, 1, false, false, false, false, 2, 0, true, true>;
 // ... with a multiply-add per score: every key length above 512 that the former does not take (145 drawn calls, time relative to the
-// compiler-scheduled build: 512 to 1023 keys 0.84 to 1.01, from 1024 on 0.79 to 0.94, with the keys of some items cut 0.34 to 0.94)
+// compiler-scheduled build: 512 to 1023 keys 0.84 to 1.01, from 1024 on 0.79 to 0.94, with the keys of some items cut 0.34 to 0.94; 64 with an odd number of
+// 32-key tiles 0.82 to 0.94, cut 0.18 to 0.80: 2 x 8 heads 8192 x 8160 1096 -> 901 us, 20 heads of 1536, 12000 keys 1132 -> 853)
 using F256_128x64 = FmaCfg<A256_128x64>;
 // few query rows: the waves of a workgroup split the keys (not by wish)
 using K256_32x32 = KsCfg<256, 4>;

@@ -992,8 +992,8 @@ constexpr bool fits(int sq, int skv) {
 template <class C>
 constexpr bool hand_loop_pays(long long items, int skv) {
   if (!C::QK8) {
-    // (the other head dims: fmha_fwd_f16.hip.  The tests pin the kernels of 512 keys, where this one is no faster, and of 8160)
-    if (C::FMA) return C::D == 256 && skv > 512 && skv % 64 == 0;
+    // (the other head dims: fmha_fwd_f16.hip.  Head dim 256, what the build with the scale in Q leaves: fmha_fwd_f16_d256.hip)
+    if (C::FMA) return C::D == 256 && skv > 512;
     if (C::D == 256) return skv >= 1024;
     // (which calls fold the scale into Q is a matter of exactness -- fmha_fwd_kernel16p.h: kFold -- and drawn where these loops took whole
     // groups of four tiles only: from 2048 keys on with few tiles behind the last one; what is left is for the FmaCfg builds)

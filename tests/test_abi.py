@@ -194,10 +194,18 @@ def test_predictable_latency_option_changes_the_choice_of_kernel_without_gpu():
     # and a leftover tile on top stay compiler-scheduled)
     assert "kernel16p<" not in f.fmha_forward_kernel(f.CFK_FP16, 1, 40, 2048, 2048 + 64, 128)
     assert "kernel16p<" not in f.fmha_forward_kernel(f.CFK_FP16, 8, 17, 896, 3520, 64)
-    # big problems with short keys: the compiler-scheduled 256-row builds need key length to pay (fp16 below 1152 keys and
-    # e4m3 below 2048 take 128-row tiles)
-    assert f.fmha_forward_kernel(f.CFK_FP16, 8, 27, 1536, 896, 128) == "fmha_fwd_kernel16<128,64,4,2,0,0,0,0,1,0,1,0>"
-    assert f.fmha_forward_kernel(f.CFK_FP16, 8, 32, 2048, 1216, 128) == "fmha_fwd_kernel16<128,64,8,2,0,0,0,0,1,0,1,0>"
+    # big problems with short keys: the loop with a multiply-add per score from 704 keys on at head dim 128; below, and at head dim 64 below
+    # 1280, the 16x16-MFMA builds.  The compiler-scheduled 256-row builds need key length to pay (e4m3 below 2048 takes 128-row tiles)
+    assert f.fmha_forward_kernel(f.CFK_FP16, 8, 27, 1536, 896, 128) == "fmha_fwd_kernel16f<128,64,8,2,0,0,0,0,2,0,1,1>"
+    assert f.fmha_forward_kernel(f.CFK_FP16, 8, 32, 2048, 1216, 128) == "fmha_fwd_kernel16f<128,64,8,2,0,0,0,0,2,0,1,1>"
+    assert f.fmha_forward_kernel(f.CFK_FP16, 8, 27, 1536, 640, 128) == "fmha_fwd_kernel16<128,64,4,2,0,0,0,0,1,0,1,0>"
+    assert f.fmha_forward_kernel(f.CFK_FP16, 8, 27, 1536, 896, 64) == "fmha_fwd_kernel16<64,64,4,3,0,0,0,0,1,0,1,0>"
+    f.set_option(f.CFK_OPT_PREDICTABLE_LATENCY, 1)   # (... whose compiler-scheduled builds take 128 rows below 1152 keys, and 256 from there on)
+    try:
+        assert f.fmha_forward_kernel(f.CFK_FP16, 8, 27, 1536, 896, 128) == "fmha_fwd_kernel16<128,64,4,2,0,0,0,0,1,0,1,0>"
+        assert f.fmha_forward_kernel(f.CFK_FP16, 8, 32, 2048, 1216, 128) == "fmha_fwd_kernel16<128,64,8,2,0,0,0,0,1,0,1,0>"
+    finally:
+        f.set_option(f.CFK_OPT_PREDICTABLE_LATENCY, 0)
     assert f.fmha_forward_kernel(f.CFK_FP8_E4M3, 8, 32, 2048, 1024, 128) == "fmha_fwd_kernel<128,64,4,2,1,1,0,0,1,0,0,0>"
     assert f.fmha_forward_kernel(f.CFK_FP8_E4M3, 8, 32, 2048, 2048, 128) == "fmha_fwd_kernel<128,64,8,2,1,1,0,0,2,0,0,0>"
     # the compiler-scheduled 256-row builds for e4m3 Q and K (one 8-wave workgroup per CU) while their rounds of 256 items fill

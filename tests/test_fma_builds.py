@@ -40,7 +40,7 @@ def test_forced_builds_match_the_oracle(wish):
 
 def test_which_calls_take_them_without_gpu():
     # where a sum over rounds says less time than for a compiler-scheduled build; not for callers that want a run time independent of the data
-    calls = [(7, 23, 192, 6400, 64), (6, 18, 2560, 1856, 128), (2, 8, 8192, 4160, 256)]
+    calls = [(7, 23, 192, 6400, 64), (6, 18, 2560, 1856, 128), (2, 8, 8192, 4160, 256), (2, 8, 8192, 8160, 256), (2, 5, 4224, 544, 256), (3, 26, 3328, 1088, 128)]
     for call in calls:
         assert f.fmha_forward_kernel(f.CFK_FP16, *call).startswith("fmha_fwd_kernel16f<"), call
     f.set_option(f.CFK_OPT_PREDICTABLE_LATENCY, 1)
@@ -69,7 +69,7 @@ def test_calls_that_these_builds_lose_stay_compiler_scheduled_without_gpu():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,H,Sq,Skv,D", [(2, 18, 2016, 3200, 128), (1, 50, 192, 1984, 128), (1, 18, 3840, 3264, 64), (1, 4, 1504, 4672, 256)])
+@pytest.mark.parametrize("B,H,Sq,Skv,D", [(2, 18, 2016, 3200, 128), (1, 50, 192, 1984, 128), (1, 18, 3840, 3264, 64), (1, 4, 1504, 4672, 256), (1, 4, 1216, 1696, 256)])
 @pytest.mark.parametrize("keys", ["plain", "climbing", "masked"])
 def test_cut_calls(B, H, Sq, Skv, D, keys):
     import torch

@@ -26,7 +26,7 @@ CASES = {
     "128x128": ["f16:2,224,2,64,256", "f8:2,160,2,64,2048", "hyb:2,160,2,64,512", "f16:1,512,2,64", "f16:1,512,2,128", "f16:1,384,2,128", "f8:1,2048,2,64", "f8:1,2048,2,128",
                 "f8:1,2048,1,256", "hyb:1,512,2,64", "f8climb:1,256,2,64,4096", "f8climb:1,256,2,128,4096", "f8climb:1,128,1,256,4096", "f8:1,4096,1,64", "f8:1,4096,1,128"],
     "256x128": ["f8:1,3072,1,128", "f8climb:1,256,2,128,3072", "f16:2,416,2,128,384", "f8:2,1184,2,128,2048", "f16:1,512,2,64", "f16:1,512,2,128", "f16:1,768,2,128,384", "f8:1,2048,2,128", "hyb:1,512,2,128", "f8climb:1,256,2,128,4096", "f8:1,4096,1,128"],
-    "128x32": ["f16:1,256,2,256", "hyb:1,256,2,256", "f16:2,96,2,256,256", "hyb:2,224,2,256,256"],
+    "128x32": ["f16:1,256,2,256", "hyb:1,256,2,256", "f16:2,96,2,256,256", "hyb:2,224,2,256,256", "f16:2,160,2,256,1056", "f16climb:1,256,2,256,992"],   # (33 and 31 key tiles)
     # the fp16 builds on 16x16x32 MFMAs
     "128x64/16": ["f16:1,512,2,64", "f16:1,512,2,128", "f16:2,384,3,128,192", "f16:1,256,2,64,64", "f16climb:1,256,2,64,512",
                   "f16climb:1,384,2,128", "f16climb:1,128,1,128,64"],
@@ -146,7 +146,7 @@ def test_tile_wish_is_honoured_by_the_plan_without_gpu():
     assert f.fmha_forward_plan(f.CFK_FP16, 1, 2, 96, 192, 64)[:2] == (32, 64)                       # query rows a multiple of 32
     assert f.fmha_forward_mfma(f.CFK_FP16, 2, 8, 8192, 8192, 256) == 16                             # hand-scheduled, 16x16x32
     assert f.fmha_forward_kernel(f.CFK_FP16, 2, 8, 8192, 8192, 256) == "fmha_fwd_kernel16p<256,32,4,1,0,0,0,0,2,0,1,1>"
-    assert f.fmha_forward_kernel(f.CFK_FP16, 2, 8, 8192, 8160, 256) == "fmha_fwd_kernel<256,32,4,1,0,0,0,0,1,0,0,0>"   # key length % 128 != 0
+    assert f.fmha_forward_kernel(f.CFK_FP16, 2, 8, 8192, 8160, 256) == "fmha_fwd_kernel16f<256,32,4,1,0,0,0,0,2,0,1,1>"   # key length % 128 != 0
     assert f.fmha_forward_mfma(f.CFK_FP16, 2, 4, 1536, 1024, 256) == 16                             # ... from 1024 keys on
     assert f.fmha_forward_mfma(f.CFK_FP16, 2, 4, 1536, 512, 256) == 32                              # below: 32x32
     assert f.fmha_forward_mfma(f.CFK_FP8_E4M3, 4, 16, 4096, 4096, 128) == 32
