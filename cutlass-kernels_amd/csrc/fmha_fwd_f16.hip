@@ -62,7 +62,7 @@ using All128 = CfgList<C128_128x64, N128_128x64, C128_256x64P, C128_256x64, N128
 // hand-scheduled one walks rounds of 256 items, in which a tile takes `low` us while at most half of the CUs work and more the more do,
 // up to `full`; either may instead be bound by reading K and V.  Fitted to 299 drawn calls of at least 512 keys, N(0,1) (rms of
 // the error: 3 to 4 % at head dim 64, 5 to 7 % at 128; where one sum is off, the other mostly is by as much).  The choice takes 0.947 of the
-// time of the compiler-scheduled builds (geometric mean; the best choice for each 0.940), worst 1.04.  us, compiler-scheduled -> chosen:
+// time of the compiler-scheduled builds (geometric mean; the best choice for each 0.940); kinds of call on which it was wrong: fma_rows.  us, compiler-scheduled -> chosen:
 // head dim 64, 80 heads of 1696 rows, 3520 keys 144.9 -> 135.1; 161 of 192, 6400 keys 113.4 -> 94.5; head dim 128, 108 of 2560, 1856 keys
 // 277.5 -> 243.3; 168 of 704, 1664 keys 125.2 -> 107.8; 36 of 2016, 3200 keys 146.4 -> 117.3 (last round cut along the keys).
 struct Call {

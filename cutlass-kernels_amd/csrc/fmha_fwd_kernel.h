@@ -1055,10 +1055,12 @@ bool first_fit(CfgList<Cs...>, int sq, int skv, long long bh, int size, TileWish
     // sixteenth for e4m3)
     const long long padded = (long long)((sq + C::BM - 1) / C::BM) * C::BM;
     const bool tight = C::BM <= 128 || (padded - sq) * (C::QK8 ? 16 : C::D == 64 ? 8 : 4) <= padded;
-    // (... and the fp16 256-row builds while what they lose -- to idle rows, to key tiles behind the last group of four
-    // (each about 2.5 tile times more) and to a last round of work items that leaves CUs idle (the 128-row builds
-    // lose about half as much to theirs) -- adds up to at most a quarter: over three draws of 100 problem sizes,
-    // automatic choice against CFK_FMHA_HANDLOOP=0, every choice that lost more than the noise summed to 0.29 or more)
+    // (... and the fp16 256-row builds with the scale folded into Q while idle rows, a last round of work items that leaves CUs idle (the 128-row
+    // builds lose about half as much to theirs) and 2.5 tile times for each key tile behind the last group of four add up to at most a quarter:
+    // over three draws of 100 problem sizes, automatic choice against CFK_FMHA_HANDLOOP=0, every choice that lost more than the noise
+    // summed to 0.29 or more.  The loops ran those last tiles outside, at that price, when the line was drawn; they no longer do, but a call that the line
+    // keeps off has its Q rounded once and is not to lose that: it is for the FmaCfg builds, fmha_fwd_f16.hip.  So the term says which calls
+    // fold the scale into Q, not what a tile costs)
     bool stacked_ok = true;
     if (C::ASM && !C::QK8 && C::BM > 128) {
       const long long items = bh * (padded / C::BM), rounds = (items + 255) / 256;

@@ -41,9 +41,14 @@ inline GemmChoice gemm_blocks_and_tiles(int blocks) {
 // size that divides a block, K=512 to 8192, TN and NN, with and without C, 500 drawn products: 64 x 32 0.89 to 0.93 (5 to 8 blocks), 96 x 64 0.90 to
 // 0.95 (17 to 24), 96 x 96 0.69 to 0.78, 96 x 128 0.92 to 0.94 (33 to 48), 128 x 192 and 192 x 128 0.89 to 0.95 (65 to 96).  us: 768 x 3072 x 4800 NN with C
 // 41.6 -> 29.7; M=N=1536 K=2048 TN 19.7 -> 13.6; 512 x 1024 x 2240 8.4 -> 6.8; 3840 x 1024 x 2048 21.3 -> 20.1.  (Measured and not built: 128 x 96 0.94 to 0.99, 64 x 96 0.95 to 0.99 of the larger size.)
-// What bounds the smaller ones is the bytes that a CU gets from the L2, 59 to 70 a nanosecond.  The two with 128 columns, of which two K
-// tiles a turn leave room for one turn ahead in the LDS, waited for them: with both groups at one K tile and four ahead 0.87 of the time
-// at 128 x 128 and 0.85 at 96 x 128 from 1536 of K on, 0.93 from 1088 (worst 1.10, operands of 10 us in the L2), 1.05 to 1.10 at 512 to 768.  The others have three
+// What bounds the smaller ones: 3.2 to 3.4 us of launch, first stage, sums and stores, and then the bytes that a CU gets from the L2, of 154 a nanosecond that the copies
+// could bring.  M=N=1024 NN in tiles of 64 x 64, us at K=512, 1024, 2048, 4096: 4.5, 5.9, 8.3, 15.7 on one set of operands, 4.6, 6.3, 9.4, 15.7 on three in turn:
+// 105 and 85 bytes a nanosecond between 1024 and 2048, where eight turns and more come out of the L2 or the memory behind it, 71 and 83 between 2048 and 4096.
+// The two with 128 columns, of which two K tiles a turn leave room for one turn ahead in the LDS, waited for them.  With both groups at one K tile and four ahead,
+// K=1088 to 2048, 185 products of 33 to 64 blocks, operands changing from call to call 0.85 to 0.96 of the time (0.918 in the geometric mean); the same operands
+// again and again 0.84 to 0.99, but 1.02 to 1.10 in 18 of 145 whose share of the operands lies in each XCD's L2 from the call before (up to about 3.9 of its 4 MB:
+// 1024 x 2304 x 1280 TN 9.8 -> 10.7 us), where there is no way to hide and the barrier every K-step is left.  A line drawn by that size gave
+// those back and cost the same products 0.06 to 0.12 on operands that change.  1.05 to 1.10 at K=512 to 768.  The other tiles have three
 // or four turns in the LDS and lose by it: 128 x 64 0.99 to 1.09, 96 x 96 1.01 to 1.03, 64 x 64 and 96 x 64 1.03 to 1.21.
 inline GemmChoice choose_gemm_f16_round(int M, int N, int K, int batch, int blocks) {
   const auto tiles = [&](int r, int c) { return (int)((long long)((M + r - 1) / r) * ((N + c - 1) / c) * batch); };

@@ -171,10 +171,11 @@ int cfk_gemm(const cfk_gemm_params *p, void *stream);
 /* Process-wide options (read by every later call; set them before launching from several threads).  No counterpart in the
  * reference, whose choices of this kind are compile-time macros (src/fmha-pipeline/README.md:11-28). */
 typedef enum cfk_option {
-  /* 1: no optimistic first pass.  Two kernels first walk the keys with a softmax reference point fixed by the first key
+  /* 1: no optimistic first pass.  Some kernels first walk the keys with a softmax reference point fixed by the first key
    * tile (no row max per tile) and, only if some weight left the range of P's type, walk them again tracking the running
-   * max as the reference does on every tile (online_softmax.h:123-165): e4m3 P from 3072 keys on, and fp16 problems
-   * with more work items than half the CUs.  On scores that climb along the key axis that costs up to twice the time.  With this option
+   * max as the reference does on every tile (online_softmax.h:123-165): e4m3 P from 3072 keys on, and fp16 from 512 keys on wherever
+   * cfk_fmha_forward_kernel names fmha_fwd_kernel16p or 16f or keys are split over workgroups of 128 rows and more.  On scores that climb along the key axis
+   * that costs up to twice the time of the kernels that run with this option, 2.7 times at head dim 256 in fp16.  With this option
    * no call takes such a pass: the same results to rounding (a few per cent slower on ordinary data).  The run time
    * then does not depend on the data, with one exception: fp16 at head dims 64 and 128, query lengths that are multiples of 256 and
    * at least 512 tiles of 256 rows, whose 16x16-MFMA build tests the row sum in place of a row max and repeats the scores of a tile

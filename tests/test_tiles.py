@@ -42,7 +42,7 @@ CASES = {
                     # ... its head-dim-64 shape (row sum on the matrix pipe)
                     "f16nt:1,512,2,64", "f16nt:1,256,3,64,768", "f16nt:3,2048,16,64", "f16ntclimb:1,512,2,64,768", "f16ntclimb:5,1024,16,64",
                     "f16:1,512,2,64", "f16climb:1,512,2,64,1024",
-                    # ... key lengths with one to three tiles behind the last group of four (taken outside the generated loop)
+                    # ... key lengths with one to three tiles behind the last group of four (which the loop's tails take)
                     "f16nt:1,512,2,128,576", "f16nt:2,2048,16,128,2240", "f16nt:1,256,3,128,640", "f16ntclimb:1,512,2,128,704",
                     "f16nt:1,512,2,64,640", "f16nt:3,2048,16,64,2112", "f16ntclimb:1,512,2,64,576", "f16ntclimb:1,512,2,64,640",
                     "f16ntclimb:1,512,2,128,576", "f16ntclimb:1,512,2,64,704",    # (the spike key inside the loop's tiles, and behind them)
